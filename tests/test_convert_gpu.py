@@ -557,6 +557,17 @@ def test_csr2csc_value_sizes_and_key_widths_over_whole_tiles(osa, gpu_ctx, m, n,
                     base)
 
 
+@pytest.mark.parametrize("tiles", [1, 2, 5, 7, 8, 9, 23])
+def test_csr2csc_fewer_tiles_than_dies_and_a_few_more(osa, gpu_ctx, tiles):
+    """A sort pass shares its tiles out to the eight dies (a range each): fewer tiles than dies, as many, one more,
+    ranges of unequal length; the entry count a whole number of tiles and one either side.  Exact."""
+    rng = np.random.default_rng(tiles)
+    for nnz in (3840 * tiles - 1, 3840 * tiles, 3840 * tiles + 1):
+        rowptr = np.array([0, nnz // 3, nnz], np.int32)
+        run_csr2csc(osa, gpu_ctx, 2, 300_000, rowptr, rng.integers(0, 300_000, nnz).astype(np.int32),
+                    rng.uniform(-1, 1, nnz).astype(np.float32), np.float32, True, 0)
+
+
 def test_csr2csc_twice_is_sorted_csr(osa, gpu_ctx):
     """Size-independent property at a large size: CSR -> CSC -> CSR equals the row-sorted matrix (checked against
     csrsort on the GPU and the oracle on the host)."""
