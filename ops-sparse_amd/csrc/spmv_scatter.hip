@@ -315,7 +315,7 @@ __device__ __forceinline__ float WidenOne(ValT v)
     return static_cast<float>(ToAcc<double, ValT>(v));
 }
 
-// Pass 1: the products of the pieces blockIdx.x, blockIdx.x + gridDim.x, ... written to `inter` in panel order.  One
+// Pass 1: the products of a workgroup's pieces (a step apart, below) written to `inter` in panel order.  One
 // workgroup a compute unit (the staging area is most of its LDS), so nothing else would cover the time a piece's
 // loads are on their way: the workgroup asks for the next piece's values and slots before it writes the current one
 // out (one piece after the other: 309 us on the 8 M x 8 M power-law matrix).
@@ -357,11 +357,18 @@ __global__ __launch_bounds__(kThreads) void ScatterProductsKernel(const ValT *__
             }
         }
     };
-    int32_t q = blockIdx.x;
-    if (q < Q) {
+    // The workgroups of an XCD take neighbouring pieces in the same turn: their chunks of a panel follow one another in
+    // memory, and the line between two chunks is completed in the L2 the workgroups share (5 M x 5 M power-law matrix,
+    // 39 M entries: 158 -> 147 us).
+    const uint32_t xcds = gridDim.x < kNumXcd ? gridDim.x : kNumXcd;
+    const uint32_t xcd = blockIdx.x % xcds;
+    const int32_t step = static_cast<int32_t>((gridDim.x - xcd + xcds - 1) / xcds);
+    const int32_t qEnd = static_cast<int32_t>(static_cast<int64_t>(Q) * (xcd + 1) / xcds);
+    int32_t q = static_cast<int32_t>(static_cast<int64_t>(Q) * xcd / xcds + blockIdx.x / xcds);
+    if (q < qEnd) {
         fetch(q);
     }
-    for (; q < Q; q += gridDim.x) {
+    for (; q < qEnd; q += step) {
         const int64_t first = static_cast<int64_t>(q) * kPiece;
         const int32_t count = nnz - first < kPiece ? static_cast<int32_t>(nnz - first) : kPiece;
         for (int32_t p = t; p <= P; p += kThreads) {
@@ -391,8 +398,8 @@ __global__ __launch_bounds__(kThreads) void ScatterProductsKernel(const ValT *__
             }
         }
         __syncthreads();
-        if (q + static_cast<int32_t>(gridDim.x) < Q) {
-            fetch(q + static_cast<int32_t>(gridDim.x));
+        if (q + step < qEnd) {
+            fetch(q + step);
         }
         // a wavefront a chunk: the piece's products of one panel, contiguous in the staging area and in memory
         // (four chunks at a time, their look-ups and LDS reads issued together, changed nothing: the kernel runs at
