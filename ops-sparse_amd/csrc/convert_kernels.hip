@@ -16,10 +16,13 @@
 // Building blocks:
 //   * a three-kernel inclusive scan of int32 (tile sums, one-workgroup scan of the
 //     sums, tile rescan), in place if wanted;
-//   * a least-significant-digit radix sort of (key, payload) pairs, four bits a
-//     pass.  A thread owns consecutive items of its tile, counts them per digit,
-//     the workgroup scans the 16 x 256 counters digit-major, and every item goes to
-//     digit base + number of earlier items with its digit: stable by construction;
+//   * least-significant-digit radix sorts of (key, payload) pairs: one of up to ten
+//     bits a pass, whose tiles are ordered in LDS and leave as runs of whole lines
+//     (csr2csc, coosort), and one of four bits a pass (the SpMV layouts, csrsort of
+//     very long rows).  In the latter a thread owns consecutive items of its tile,
+//     counts them per digit, the workgroup scans the 16 x 256 counters digit-major,
+//     and every item goes to digit base + number of earlier items with its digit:
+//     stable by construction;
 //   * bitonic sorts of 64-bit (column, position) keys in registers (a wavefront per
 //     row of up to 64 entries) and in LDS (a workgroup per row of up to 2048); the
 //     position in the low half makes every key distinct, so any correct sort is
@@ -141,6 +144,71 @@ __global__ __launch_bounds__(kBlockThreads) void ScanApplyKernel(const int32_t *
         if (first + i < n) {
             out[first + i] = before + v[i];
         }
+    }
+}
+
+// The same in one launch: one workgroup, a thread takes kScanOneItems consecutive elements of a chunk.  For arrays of up
+// to kScanOneMost elements, where the three launches above are three times the 4 us between two dependent kernels.
+constexpr int kScanOneThreads = 1024;
+constexpr int kScanOneItems = 16;
+constexpr int64_t kScanOneMost = int64_t{4} * kScanOneThreads * kScanOneItems;
+
+__global__ __launch_bounds__(kScanOneThreads) void ScanOneKernel(const int32_t *in, int32_t *out, int64_t n, int32_t add)
+{
+    // A chunk passes through LDS: memory is read and written a line a wavefront, the threads take consecutive elements.
+    // (one word of padding after every kScanOneItems: the threads' strides fall on all banks)
+    __shared__ int32_t chunk[kScanOneThreads * (kScanOneItems + 1)];
+    __shared__ int32_t waveSums[kScanOneThreads / kWave];
+    const int32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    int32_t carry = add;
+    for (int64_t c0 = 0; c0 < n; c0 += kScanOneThreads * kScanOneItems) {
+        int32_t v[kScanOneItems];
+#pragma unroll
+        for (int i = 0; i < kScanOneItems; ++i) {
+            const int64_t p = c0 + i * kScanOneThreads + tid;
+            v[i] = in[p < n ? p : n - 1];
+        }
+#pragma unroll
+        for (int i = 0; i < kScanOneItems; ++i) {
+            const int32_t p = i * kScanOneThreads + tid;
+            chunk[p + p / kScanOneItems] = c0 + p < n ? v[i] : 0;
+        }
+        __syncthreads();
+        int32_t sum = 0;
+#pragma unroll
+        for (int i = 0; i < kScanOneItems; ++i) {
+            sum += chunk[tid * (kScanOneItems + 1) + i];
+            v[i] = sum;
+        }
+        int32_t incl = sum;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int32_t up = __shfl_up(incl, off, kWave);
+            incl += lane >= off ? up : 0;
+        }
+        if (lane == kWave - 1) {
+            waveSums[wave] = incl;
+        }
+        __syncthreads();
+        int32_t base = carry + incl - sum;
+#pragma unroll
+        for (int w = 0; w < kScanOneThreads / kWave; ++w) {
+            base += w < wave ? waveSums[w] : 0;
+            carry += waveSums[w];
+        }
+#pragma unroll
+        for (int i = 0; i < kScanOneItems; ++i) {
+            chunk[tid * (kScanOneItems + 1) + i] = base + v[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kScanOneItems; ++i) {
+            const int32_t p = i * kScanOneThreads + tid;
+            if (c0 + p < n) {
+                out[c0 + p] = chunk[p + p / kScanOneItems];
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -445,23 +513,32 @@ __global__ __launch_bounds__(kBlockThreads) void RadixScatterKernel(
     }
 }
 
-// ----------------------------------------------- radix sort, 8 bits a pass
-// csr2csc's passes.  Sixteen times as many buckets as the 4-bit pass, so a tile's items for one bucket are few:
-// written straight from the lanes that hold them they would leave as scattered 12-byte pieces.  The tile is
-// therefore ordered by its 8-bit digit inside LDS first and written out in that order: neighbouring lanes then
-// write neighbouring addresses of one bucket's run.  What is ordered is one word an item, (digit, slot in the
-// tile), by two stable 4-bit splits; the items themselves stay where the loads put them and are fetched by slot at
-// the end.  A thread counts its items' digits in one 64-bit register, four bits a digit: the instruction count,
-// not the memory system, bounds this kernel, and a counter per digit selected by comparisons costs ten times more.
+// ----------------------------------------- radix sort, up to 10 bits a pass
+// The passes of csr2csc and coosort over (key, row, value) triples.  A pass reads 12 bytes an entry and writes 12, so
+// the number of passes is what counts, and with it the number of buckets a pass may have: with 1024 of them a tile's
+// run in a bucket is eight entries.  Such runs reach memory as whole lines all the same, because the workgroups of an
+// XCD work on neighbouring tiles at the same time: their runs of a bucket follow one another, and the lines between
+// them are completed in the L2 that the workgroups share.
+//
+// Inside a workgroup: a wavefront takes 512 consecutive entries of the tile, 64 at a time, and finds every lane's peers
+// (the lanes with its digit) from one ballot a digit bit; a counter a digit and wavefront in LDS carries the count from
+// one 64 to the next.  The running sums of those counters over (digit, wavefront) are where a wavefront's entries of a
+// digit start in the ordered tile; the entries are put there in LDS and leave in that order, neighbouring lanes writing
+// neighbouring addresses.
+//
+// Measured on 33.5 M entries: 190 us a pass over 128 buckets, 4.5 TB/s (448 MB written for 402 of entries), 275 us over
+// 1024; 285 us over 128 while tiles of 3840 were ordered by two 4-bit splits and every workgroup walked a range of its
+// own.  What is left is the length of a turn: one workgroup of 1024 a compute unit, six barriers a tile.
 
-constexpr int kWideBits = 8;
-constexpr int kWideDigits = 1 << kWideBits;
-constexpr int kWideItems = 15;                              // items a thread ranks: a 4-bit counter holds them,
-                                                            // and an odd stride over LDS has no bank conflicts
-constexpr int kWideTile = kBlockThreads * kWideItems;      // 3840
-constexpr int kWideSlotBits = 12;
-static_assert(kWideTile <= (1 << kWideSlotBits), "a slot number fits its field");
-static_assert(kWideDigits == kBlockThreads, "one thread per digit");
+constexpr int kWideItems = 8;      // entries of a thread
+constexpr int kWideMaxBits = 10;   // ... of a digit
+
+template <int T>
+struct WideShape {
+    static constexpr int kTile = T * kWideItems;
+    static constexpr int kWaves = T / kWave;
+    static constexpr int kPer = (1 << kWideMaxBits) > T ? (1 << kWideMaxBits) / T : 1;  // digits of a thread
+};
 
 // key - keyBase in wrap-around arithmetic (the keys of a COO sort may span the whole int32 range).
 __device__ __forceinline__ int32_t Rebased(int32_t key, int32_t keyBase)
@@ -469,40 +546,66 @@ __device__ __forceinline__ int32_t Rebased(int32_t key, int32_t keyBase)
     return static_cast<int32_t>(static_cast<uint32_t>(key) - static_cast<uint32_t>(keyBase));
 }
 
-// A pass's digit: `mask` = 2^bits - 1 with bits <= kWideBits (the passes of a sort share its key bits evenly).
-__device__ __forceinline__ int32_t WideDigit(int32_t key, int32_t shift, int32_t mask)
+// A pass's digit: `mask` = 2^bits - 1 with bits <= kWideMaxBits (the passes of a sort share its key bits evenly).
+__device__ __forceinline__ uint32_t WideDigit(int32_t key, int32_t shift, int32_t mask)
 {
-    return static_cast<int32_t>((static_cast<uint32_t>(key) >> shift) & static_cast<uint32_t>(mask));
+    return (static_cast<uint32_t>(key) >> shift) & static_cast<uint32_t>(mask);
 }
 
-// table[1 + digit * numTiles + tile] = items of that digit in the tile (see RadixCountKernel).  A workgroup counts
-// kWideCountTiles consecutive tiles and writes their counts of one digit side by side: a tile a workgroup leaves
-// the table written four bytes at a time, a cache line for each.
-constexpr int kWideCountTiles = 8;
-
-__global__ __launch_bounds__(kBlockThreads) void WideCountKernel(const int32_t *__restrict__ keys, int64_t n,
-                                                                int32_t keyBase, int32_t shift, int32_t mask,
-                                                                int32_t *__restrict__ table, int64_t numTiles)
+// Exclusive scan of one value a thread over a workgroup of T threads; its barriers order LDS only.
+template <int T>
+__device__ __forceinline__ int32_t WideBlockScan(int32_t v, int32_t *waveSums)
 {
-    __shared__ int32_t hist[kWideCountTiles][kWideDigits];
+    const int32_t lane = threadIdx.x % kWave;
+    const int32_t wave = threadIdx.x / kWave;
+    int32_t incl = v;
 #pragma unroll
-    for (int j = 0; j < kWideCountTiles; ++j) {
-        hist[j][threadIdx.x] = 0;
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int32_t up = __shfl_up(incl, off, kWave);
+        incl += lane >= off ? up : 0;
     }
-    __syncthreads();
-    const int64_t firstTile = static_cast<int64_t>(blockIdx.x) * kWideCountTiles;
+    if (lane == kWave - 1) {
+        waveSums[wave] = incl;
+    }
+    LdsBarrier();
+    int32_t base = 0;
+#pragma unroll
+    for (int w = 0; w < T / kWave; ++w) {
+        base += w < wave ? waveSums[w] : 0;
+    }
+    return base + incl - v;
+}
+
+// table[1 + digit * numTiles + tile] = entries of that digit in the tile (table[0] = 0: an inclusive scan of the table
+// then leaves, at the same place shifted down by one, the first output position of every (digit, tile)).  A workgroup
+// counts kWideCountTiles consecutive tiles and writes their counts of one digit side by side.
+constexpr int kWideCountTiles = 4;
+
+template <int T>
+__global__ __launch_bounds__(T) void WideCountKernel(const int32_t *__restrict__ keys, int64_t n, int32_t keyBase,
+                                                     int32_t shift, int32_t mask, int32_t *__restrict__ table,
+                                                     int64_t numTiles)
+{
+    constexpr int kTile = WideShape<T>::kTile;
+    __shared__ int32_t hist[kWideCountTiles << kWideMaxBits];
+    const int32_t digits = mask + 1;
+    for (int32_t i = threadIdx.x; i < kWideCountTiles * digits; i += T) {
+        hist[i] = 0;
+    }
+    const int64_t firstTile = static_cast<int64_t>(XcdContiguousTile(blockIdx.x, gridDim.x)) * kWideCountTiles;
     // The keys of a tile are loaded, all of them, a tile ahead of their counting: the compiler keeps a load and the
     // LDS atomic after it in program order, and an atomic straight behind its load is a round trip to memory for
-    // every item.  No branch around a load: an item past the end reads the last key and counts for nothing.
+    // every entry.  No branch around a load: an entry past the end reads the last key and counts for nothing.
     int32_t key[2][kWideItems];
     auto fetch = [&](int j) {
 #pragma unroll
         for (int i = 0; i < kWideItems; ++i) {
-            const int64_t at = (firstTile + j) * kWideTile + i * kBlockThreads + threadIdx.x;
+            const int64_t at = (firstTile + j) * kTile + i * T + threadIdx.x;
             key[j & 1][i] = keys[at < n ? at : n - 1];
         }
     };
     fetch(0);
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < kWideCountTiles; ++j) {
         if (j + 1 < kWideCountTiles) {
@@ -510,26 +613,26 @@ __global__ __launch_bounds__(kBlockThreads) void WideCountKernel(const int32_t *
         }
 #pragma unroll
         for (int i = 0; i < kWideItems; ++i) {
-            const int64_t at = (firstTile + j) * kWideTile + i * kBlockThreads + threadIdx.x;
-            atomicAdd(&hist[j][WideDigit(Rebased(key[j & 1][i], keyBase), shift, mask)], at < n ? 1 : 0);
+            const int64_t at = (firstTile + j) * kTile + i * T + threadIdx.x;
+            atomicAdd(&hist[j * digits + WideDigit(Rebased(key[j & 1][i], keyBase), shift, mask)], at < n ? 1 : 0);
         }
     }
     __syncthreads();
-    // lanes j = 0 .. kWideCountTiles - 1 of a group write neighbouring tiles of one digit
-    constexpr int kDigitsAtOnce = kBlockThreads / kWideCountTiles;
-    const int32_t j = threadIdx.x % kWideCountTiles;
-#pragma unroll
-    for (int d0 = 0; d0 < kWideDigits; d0 += kDigitsAtOnce) {
-        const int32_t d = d0 + threadIdx.x / kWideCountTiles;
-        if (firstTile + j < numTiles) {
-            table[1 + static_cast<int64_t>(d) * numTiles + firstTile + j] = hist[j][d];
+    // the lanes of a group of kWideCountTiles write neighbouring tiles of one digit
+    for (int32_t i = threadIdx.x; i < kWideCountTiles * digits; i += T) {
+        const int64_t tile = firstTile + i % kWideCountTiles;
+        if (tile < numTiles) {
+            const int32_t d = i / kWideCountTiles;
+            table[1 + static_cast<int64_t>(d) * numTiles + tile] = hist[i % kWideCountTiles * digits + d];
         }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        table[0] = 0;
     }
 }
 
 // Between two passes the n (row, value) pairs lie as n rows followed by n values in the 8 n bytes of their buffer:
-// 4-byte stores to a bucket's run, as for the keys (8-byte stores of whole pairs to such short runs took half as
-// long again).
+// 4-byte stores to a bucket's run, as for the keys.
 template <typename P>
 __device__ __forceinline__ auto WideRows(P *pairs)
 {
@@ -541,200 +644,248 @@ __device__ __forceinline__ auto WideVals(P *pairs, int64_t n)
     return reinterpret_cast<std::conditional_t<std::is_const<P>::value, const uint32_t, uint32_t> *>(pairs) + n;
 }
 
-// A tile's items as the loads deliver them, lane t holding slots t, t + 256, ...
+// A tile's entries as the loads deliver them: lane l of wavefront w holds entries 512 w + l, 512 w + 64 + l, ...
+template <int T>
 struct WideTileRegs {
     int32_t key[kWideItems];
     RadixPair pay[kWideItems];
-    int32_t first, next;  // prefix[digit tid][tile] and the entry after it
+    int32_t first[WideShape<T>::kPer];  // first output position of the thread's digits
 };
 
-template <int Mode, int VB, bool Full>
-__device__ __forceinline__ void WideFetch(WideTileRegs &r, int64_t tile, const int32_t *__restrict__ keysIn,
+template <int T, int Mode, int VB, bool Full>
+__device__ __forceinline__ void WideFetch(WideTileRegs<T> &r, int64_t tile, const int32_t *__restrict__ keysIn,
                                           const RadixPair *__restrict__ pairsIn, int64_t n, int32_t keyBase,
                                           int32_t shift, int32_t mask, const int32_t *__restrict__ prefix,
                                           int64_t numTiles, const RadixPairIo &io)
 {
+    constexpr int kPer = WideShape<T>::kPer;
     const int tid = threadIdx.x;
-    const int64_t tile0 = tile * kWideTile;
-    const int64_t flat = static_cast<int64_t>(tid) * numTiles + tile;
-    r.first = prefix[flat];
-    r.next = prefix[flat + 1];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int32_t d = tid * kPer + j;
+        r.first[j] = prefix[static_cast<int64_t>(d <= mask ? d : mask) * numTiles + tile];
+    }
+    const int64_t wave0 = tile * WideShape<T>::kTile + tid / kWave * (kWave * kWideItems) + tid % kWave;
 #pragma unroll
     for (int i = 0; i < kWideItems; ++i) {
-        const int64_t at = tile0 + i * kBlockThreads + tid;
-        // a slot past the end gets the largest digit, so that it sorts behind every real item
+        const int64_t at = wave0 + i * kWave;
+        // a slot past the end gets the largest digit, so that it sorts behind every real entry
         r.key[i] = static_cast<int32_t>(static_cast<uint32_t>(mask) << shift);
         r.pay[i] = RadixPair{0, 0u};
         if (Full || at < n) {
-            r.key[i] = Rebased(keysIn[at], keyBase);
+            r.key[i] = Rebased(LoadStream(keysIn + at), keyBase);
             if (Mode == kPayPairFirst) {
-                r.pay[i].row = io.rowSrc[at];
+                r.pay[i].row = LoadStream(io.rowSrc + at);
                 if (VB == 4) {
-                    r.pay[i].val = static_cast<const uint32_t *>(io.valSrc)[at];
+                    r.pay[i].val = LoadStream(static_cast<const uint32_t *>(io.valSrc) + at);
                 } else if (VB == 2) {
                     r.pay[i].val = static_cast<const uint16_t *>(io.valSrc)[at];
                 } else if (VB == 1) {
                     r.pay[i].val = static_cast<const uint8_t *>(io.valSrc)[at];
                 }
             } else {
-                r.pay[i] = RadixPair{WideRows(pairsIn)[at], WideVals(pairsIn, n)[at]};
+                r.pay[i] = RadixPair{LoadStream(WideRows(pairsIn) + at), LoadStream(WideVals(pairsIn, n) + at)};
             }
         }
     }
 }
 
+template <int T>
 struct WideLds {
-    int32_t key[kWideTile];
-    __align__(8) RadixPair pay[kWideTile];
-    uint32_t word[kWideTile];
-    int32_t counters[kCounterSlots];
-    int32_t waveSums[kBlockThreads / kWave];
-    int32_t outOf[kWideDigits];  // output position less slot in the ordered tile, for the items of a digit
+    union {
+        int32_t counters[WideShape<T>::kWaves << kWideMaxBits];  // [wavefront][digit]
+        struct {
+            int32_t key[WideShape<T>::kTile];
+            int32_t row[WideShape<T>::kTile];
+            uint32_t val[WideShape<T>::kTile];
+        };
+    };
+    int32_t outOf[1 << kWideMaxBits];  // output position less slot in the ordered tile, for the entries of a digit
+    int32_t waveSums[WideShape<T>::kWaves];
 };
 
-// Orders the tile held in LDS (key, pay filled, barrier not yet passed) and writes it out.  Ends with the stores
-// issued and no barrier behind them.
-template <int Mode, int VB, bool Full>
-__device__ __forceinline__ void WideOrderAndWrite(WideLds &lds, int32_t first, int32_t next, int64_t tile, int64_t n,
-                                                  int32_t shift, int32_t mask, int32_t *__restrict__ keysOut,
-                                                  RadixPair *__restrict__ pairsOut, const RadixPairIo &io)
+// Puts the tile held in registers into the LDS arrays in the order of its digits.  Ends with a barrier.
+template <int T>
+__device__ __forceinline__ void WideOrder(WideLds<T> &lds, const WideTileRegs<T> &r, int32_t shift, int32_t mask,
+                                          int32_t bits)
 {
-    const int tid = threadIdx.x;
+    constexpr int kPer = WideShape<T>::kPer, kWaves = WideShape<T>::kWaves;
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int32_t digits = mask + 1;
+    int32_t *mine = lds.counters + tid / kWave * digits;
+    for (int32_t d = lane; d < digits; d += kWave) {
+        mine[d] = 0;
+    }
+    uint32_t dig[kWideItems];
+    uint64_t peers[kWideItems];
+#pragma unroll
+    for (int i = 0; i < kWideItems; ++i) {
+        dig[i] = WideDigit(r.key[i], shift, mask);
+        peers[i] = ~uint64_t{0};
+    }
+    for (int32_t b = 0; b < bits; ++b) {
+#pragma unroll
+        for (int i = 0; i < kWideItems; ++i) {
+            const uint32_t ones = static_cast<uint32_t>(__builtin_amdgcn_sbfe(dig[i], b, 1));  // the bit in every place
+            const uint64_t m = __ballot(ones != 0);
+            // peers & ~(m ^ ones)
+            const uint32_t lo = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(peers[i]), static_cast<uint32_t>(m), ones, 0x90);
+            const uint32_t hi = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(peers[i] >> 32), static_cast<uint32_t>(m >> 32), ones, 0x90);
+            peers[i] = (static_cast<uint64_t>(hi) << 32) | lo;
+        }
+    }
+    // (a wavefront's own counters: LDS serves a wavefront's instructions in their order)
+    uint32_t rank[kWideItems];
+#pragma unroll
+    for (int i = 0; i < kWideItems; ++i) {
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(peers[i] >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(peers[i]), 0));
+        const uint32_t before = static_cast<uint32_t>(mine[dig[i]]);
+        rank[i] = before + below;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        if (below == 0) {
+            mine[dig[i]] = static_cast<int32_t>(before + __popcll(peers[i]));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+    }
+    LdsBarrier();
     {
-        // where the tile's run of digit `tid` starts in the ordered tile, from the lengths of the runs before it
-        int32_t total;
-        const int32_t start = BlockExclusiveScan(next - first, lds.waveSums, &total);  // has barriers
-        lds.outOf[tid] = first - start;
-    }
-    // a thread takes kWideItems consecutive slots of the current order
-    uint32_t word[kWideItems];
+        // digits of this thread: the counters become the start of every (digit, wavefront) in the ordered tile (read
+        // twice rather than kept: the registers hold two tiles)
+        int32_t sum = 0;
 #pragma unroll
-    for (int i = 0; i < kWideItems; ++i) {
-        const int32_t p = tid * kWideItems + i;
-        word[i] = (static_cast<uint32_t>(WideDigit(lds.key[p], shift, mask)) << kWideSlotBits) | static_cast<uint32_t>(p);
-    }
+        for (int j = 0; j < kPer; ++j) {
+            const int32_t d = tid * kPer + j;
+            if (d < digits) {
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const int32_t at = kWideSlotBits + half * kRadixBits;
-        uint64_t packed = 0;  // the thread's count of digit d in bits [4 d, 4 d + 4)
-        int32_t earlier[kWideItems];
-#pragma unroll
-        for (int i = 0; i < kWideItems; ++i) {
-            const uint32_t sh = ((word[i] >> at) & (kRadixDigits - 1)) * 4;
-            earlier[i] = static_cast<int32_t>((packed >> sh) & 15);
-            packed += uint64_t{1} << sh;
-        }
-#pragma unroll
-        for (int d = 0; d < kRadixDigits; ++d) {
-            lds.counters[Padded(d * kBlockThreads + tid)] = static_cast<int32_t>((packed >> (4 * d)) & 15);
-        }
-        LdsBarrier();
-        ScanDigitCounters(lds.counters, lds.waveSums);  // counters[d][t]: slots before thread t's first item of d
-#pragma unroll
-        for (int i = 0; i < kWideItems; ++i) {
-            const int32_t d = static_cast<int32_t>((word[i] >> at) & (kRadixDigits - 1));
-            lds.word[lds.counters[Padded(d * kBlockThreads + tid)] + earlier[i]] = word[i];
-        }
-        LdsBarrier();
-        if (half == 0) {
-#pragma unroll
-            for (int i = 0; i < kWideItems; ++i) {
-                word[i] = lds.word[tid * kWideItems + i];
-            }
-        }
-    }
-    const int64_t tile0 = tile * kWideTile;
-    const int32_t valid = Full ? kWideTile : static_cast<int32_t>(n - tile0);
-#pragma unroll
-    for (int i = 0; i < kWideItems; ++i) {
-        const int32_t p = i * kBlockThreads + tid;
-        if (Full || p < valid) {  // the real items are the first `valid` slots of the ordered tile
-            const uint32_t w = lds.word[p];
-            const int32_t slot = static_cast<int32_t>(w & ((1u << kWideSlotBits) - 1));
-            const int64_t dst = static_cast<int64_t>(lds.outOf[w >> kWideSlotBits] + p);
-            const RadixPair out = lds.pay[slot];
-            keysOut[dst] = lds.key[slot];
-            if (Mode == kPayPairLast) {
-                io.rowOut[dst] = out.row;
-                if (VB == 4) {
-                    static_cast<uint32_t *>(io.valOut)[dst] = out.val;
-                } else if (VB == 2) {
-                    static_cast<uint16_t *>(io.valOut)[dst] = static_cast<uint16_t>(out.val);
-                } else if (VB == 1) {
-                    static_cast<uint8_t *>(io.valOut)[dst] = static_cast<uint8_t>(out.val);
+                for (int w = 0; w < kWaves; ++w) {
+                    sum += lds.counters[w * digits + d];
                 }
-            } else {
-                WideRows(pairsOut)[dst] = out.row;
-                WideVals(pairsOut, n)[dst] = out.val;
+            }
+        }
+        int32_t run = WideBlockScan<T>(sum, lds.waveSums);
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const int32_t d = tid * kPer + j;
+            if (d < digits) {
+                lds.outOf[d] = r.first[j] - run;
+                constexpr int kAtOnce = 4;
+#pragma unroll
+                for (int w0 = 0; w0 < kWaves; w0 += kAtOnce) {
+                    int32_t count[kAtOnce];
+#pragma unroll
+                    for (int w = 0; w < kAtOnce; ++w) {
+                        count[w] = lds.counters[(w0 + w) * digits + d];
+                    }
+#pragma unroll
+                    for (int w = 0; w < kAtOnce; ++w) {
+                        lds.counters[(w0 + w) * digits + d] = run;
+                        run += count[w];
+                    }
+                }
             }
         }
     }
+    LdsBarrier();
+#pragma unroll
+    for (int i = 0; i < kWideItems; ++i) {
+        rank[i] += static_cast<uint32_t>(mine[dig[i]]);
+    }
+    LdsBarrier();  // the counters make room for the entries
+#pragma unroll
+    for (int i = 0; i < kWideItems; ++i) {
+        lds.key[rank[i]] = r.key[i];
+        lds.row[rank[i]] = r.pay[i].row;
+        lds.val[rank[i]] = r.pay[i].val;
+    }
+    LdsBarrier();
 }
 
-template <bool Full>
-__device__ __forceinline__ void WideStage(WideLds &lds, const WideTileRegs &r)
+// Writes the ordered tile out.  Ends with the stores issued and no barrier behind them.
+template <int T, int Mode, int VB, bool Full>
+__device__ __forceinline__ void WideWrite(const WideLds<T> &lds, int64_t tile, int64_t n, int32_t shift, int32_t mask,
+                                          int32_t *__restrict__ keysOut, RadixPair *__restrict__ pairsOut,
+                                          const RadixPairIo &io)
 {
+    const int tid = threadIdx.x;
+    const int32_t valid = Full ? WideShape<T>::kTile : static_cast<int32_t>(n - tile * WideShape<T>::kTile);
 #pragma unroll
     for (int i = 0; i < kWideItems; ++i) {
-        const int32_t p = i * kBlockThreads + threadIdx.x;
-        lds.key[p] = r.key[i];
-        lds.pay[p] = r.pay[i];
+        const int32_t p = i * T + tid;
+        if (Full || p < valid) {  // the real entries are the first `valid` slots of the ordered tile
+            const int32_t key = lds.key[p];
+            const int64_t dst = static_cast<int64_t>(lds.outOf[WideDigit(key, shift, mask)] + p);
+            keysOut[dst] = key;
+            if (Mode == kPayPairLast) {
+                io.rowOut[dst] = lds.row[p];
+                if (VB == 4) {
+                    static_cast<uint32_t *>(io.valOut)[dst] = lds.val[p];
+                } else if (VB == 2) {
+                    static_cast<uint16_t *>(io.valOut)[dst] = static_cast<uint16_t>(lds.val[p]);
+                } else if (VB == 1) {
+                    static_cast<uint8_t *>(io.valOut)[dst] = static_cast<uint8_t>(lds.val[p]);
+                }
+            } else {
+                WideRows(pairsOut)[dst] = lds.row[p];
+                WideVals(pairsOut, n)[dst] = lds.val[p];
+            }
+        }
     }
 }
 
 // One pass; the payload modes are those of RadixScatterKernel (pairs only), VB the bytes of a value in the arrays
 // that the first pass reads and the last one writes (a template parameter: a branch on it among the loads would
-// leave the compiler unable to count what is in flight).  prefix is the scanned table:
-// prefix[digit * numTiles + tile] is the first output position of the tile's items of that digit, and the entry
-// after it, in that same flat order, ends them.  A workgroup takes full tiles a step apart (below) and has the loads
-// of its next tile in flight while it orders and writes the current one (with two workgroups on a compute unit and a
-// tile's phases one after another, a tile fetched only when its turn comes leaves the memory system idle most of the
-// time: 3.2 TB/s for a pass that does nothing but copy).  The tile that the end of the array cuts short is done last,
+// leave the compiler unable to count what is in flight).  prefix is the scanned table of WideCountKernel:
+// prefix[digit * numTiles + tile] is the first output position of the tile's entries of that digit.  Every XCD has a
+// range of tiles, its workgroups take neighbouring tiles of it in the same turn, and a workgroup has the loads of its
+// next tile in flight while it writes the current one.  The tile that the end of the array cuts short is done last,
 // by workgroup 0, with bounds checks.
-template <int Mode, int VB>
-__global__ __launch_bounds__(kBlockThreads) void WideScatterKernel(
+template <int T, int Mode, int VB>
+__global__ __launch_bounds__(T) void WideScatterKernel(
     const int32_t *__restrict__ keysIn, const RadixPair *__restrict__ pairsIn, int32_t *__restrict__ keysOut,
-    RadixPair *__restrict__ pairsOut, int64_t n, int32_t keyBase, int32_t shift, int32_t mask,
+    RadixPair *__restrict__ pairsOut, int64_t n, int32_t keyBase, int32_t shift, int32_t mask, int32_t bits,
     const int32_t *__restrict__ prefix, int64_t numTiles, RadixPairIo io)
 {
-    __shared__ WideLds lds;
-    const int64_t fullTiles = n / kWideTile;
-    WideTileRegs r;
-    // Every XCD has a range of tiles and its workgroups take neighbouring tiles of it in the same turn: the runs that
-    // they write into a bucket follow one another, so the line that one run leaves half written is completed by the
-    // next while it is still in the L2 they share, and memory sees whole lines.  (A range of consecutive tiles to
-    // each workgroup keeps 64 x 128 x 3 half-written lines open in an L2, 3 MiB of its 4, and they are evicted as
-    // they are: a pass over 33.5 M entries 285 us against 200.)
+    __shared__ WideLds<T> lds;
+    const int64_t fullTiles = n / WideShape<T>::kTile;
+    WideTileRegs<T> r;
     const uint32_t xcds = gridDim.x < kNumXcd ? gridDim.x : kNumXcd;
     const uint32_t xcd = blockIdx.x % xcds;
     const int64_t step = (gridDim.x - xcd + xcds - 1) / xcds;
     const int64_t tileEnd = fullTiles * (xcd + 1) / xcds;
     int64_t tile = fullTiles * xcd / xcds + blockIdx.x / xcds;
-    auto turn = [&]() {
-        WideStage<true>(lds, r);
-        const int32_t first = r.first, next = r.next;
-        // the next tile's loads (the last turn fetches its own tile again rather than branch around the loads:
-        // a wait for "all but the stores issued since" needs one straight path)
+    // The loads of the next tile are on their way while the current one is ordered and written: two sets of registers
+    // used in turn.  (The last turn fetches its own tile again rather than branch around the loads: a wait for "all
+    // but what was issued since" needs one straight path.)
+    auto turn = [&](WideTileRegs<T> &now, WideTileRegs<T> &next) {
         const int64_t ahead = tile + step < tileEnd ? tile + step : tile;
-        WideFetch<Mode, VB, true>(r, ahead, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
+        WideFetch<T, Mode, VB, true>(next, ahead, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
         __builtin_amdgcn_sched_barrier(0);  // the loads are issued here, not where the scheduler finds room later
-        WideOrderAndWrite<Mode, VB, true>(lds, first, next, tile, n, shift, mask, keysOut, pairsOut, io);
+        WideOrder<T>(lds, now, shift, mask, bits);
+        WideWrite<T, Mode, VB, true>(lds, tile, n, shift, mask, keysOut, pairsOut, io);
         LdsBarrier();  // the tile's LDS is free again
         tile += step;
     };
     if (tile < tileEnd) {
-        WideFetch<Mode, VB, true>(r, tile, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
+        WideFetch<T, Mode, VB, true>(r, tile, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
+        WideTileRegs<T> other;
         // the first turn stands outside the loop: entered from here, with no stores behind the loads, the loop's
         // wait for the loads would be a wait for everything, the stores of the turn before included
-        turn();
+        turn(r, other);
         while (tile < tileEnd) {
-            turn();
+            turn(other, r);
+            if (tile >= tileEnd) {
+                break;
+            }
+            turn(r, other);
         }
     }
     if (blockIdx.x == 0 && fullTiles < numTiles) {
-        WideFetch<Mode, VB, false>(r, fullTiles, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
-        WideStage<false>(lds, r);
-        WideOrderAndWrite<Mode, VB, false>(lds, r.first, r.next, fullTiles, n, shift, mask, keysOut, pairsOut, io);
+        WideFetch<T, Mode, VB, false>(r, fullTiles, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
+        WideOrder<T>(lds, r, shift, mask, bits);
+        WideWrite<T, Mode, VB, false>(lds, fullTiles, n, shift, mask, keysOut, pairsOut, io);
     }
 }
 
@@ -1200,6 +1351,10 @@ void LaunchInclusiveScan(const int32_t *in, int32_t *out, int64_t count, int32_t
     if (count <= 0) {
         return;
     }
+    if (count <= kScanOneMost) {
+        hipLaunchKernelGGL(ScanOneKernel, dim3(1), dim3(kScanOneThreads), 0, s, in, out, count, add);
+        return;
+    }
     const int64_t numTiles = ScanTiles(count);
     hipLaunchKernelGGL(ScanTileSumsKernel, dim3(static_cast<uint32_t>(numTiles)), dim3(kBlockThreads), 0, s, in, count,
                        tiles);
@@ -1285,56 +1440,74 @@ void LaunchRadixPairPass(int mode, const int32_t *keysIn, const void *pairsIn, i
     }
 }
 
-int64_t WideTiles(int64_t n) { return (n + kWideTile - 1) / kWideTile; }
-int64_t WideTableInts(int64_t n) { return static_cast<int64_t>(kWideDigits) * WideTiles(n) + 1; }
-
-// Workgroups of the 8-bit scatter pass: two a compute unit, which is what their LDS allows to be resident.
-static uint32_t WideScatterBlocks(int64_t n)
+// Threads of the wide pass' workgroups.  Large ones write long runs, small ones occupy the chip with few entries (csr2csc
+// of 2.7 M entries: 171 us with 1024 threads, 125 with 512, 134 with 256; of 250 K: 99, 86 and 68; of 33.5 M: 790, 870
+// and 980).
+int WideThreads(int64_t n)
 {
-    static const int64_t resident = [] {
-        int dev = 0;
-        hipDeviceProp_t prop;
-        int64_t cus = 256;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
-            prop.multiProcessorCount > 0) {
-            cus = prop.multiProcessorCount;
-        } else {
+    return n >= (int64_t{1} << 23) ? 1024 : n >= (int64_t{1} << 20) ? 512 : 256;
+}
+int64_t WideTiles(int64_t n)
+{
+    const int64_t tile = static_cast<int64_t>(WideThreads(n)) * kWideItems;
+    return (n + tile - 1) / tile;
+}
+int64_t WideTableInts(int64_t n) { return (WideTiles(n) << kWideMaxBits) + 1; }
+
+// Passes of a sort of n entries over `keyBits` bits of key, and the bits each takes.  At least two: a first pass that
+// reads the sources and a last one that writes the outputs.  The passes share the key's bits evenly: the fewer buckets
+// a pass has, the longer the runs its tiles write.  (Nine bits at most where the workgroups are large: 20 bits of 33.5 M
+// keys in three passes of 7, 775 us, against two of 10, 784; in ten bits the counts and their table cost more, too.)
+struct WidePasses {
+    int32_t passes, bits;
+};
+WidePasses WidePassesOf(int32_t keyBits, int64_t n)
+{
+    const int32_t most = WideThreads(n) == 1024 ? 9 : kWideMaxBits;
+    const int32_t passes = keyBits <= 2 * most ? 2 : (keyBits + most - 1) / most;
+    return {passes, (keyBits + passes - 1) / passes};
+}
+
+// Workgroups of the scatter pass: as many as are resident (LDS and registers).
+uint32_t WideScatterBlocks(int64_t n, int threads)
+{
+    static const int64_t cus = [] {
+        int dev = 0, count = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || count <= 0) {
             (void)hipGetLastError();
+            return int64_t{256};
         }
-        const char *env = std::getenv("OPS_SPARSE_WIDE_BLOCKS_PER_CU");  // tuning override
-        const int64_t perCu = env != nullptr && std::atoi(env) > 0 ? std::atoi(env) : 2;
-        return cus * perCu;
+        return static_cast<int64_t>(count);
     }();
-    const int64_t fullTiles = n / kWideTile;
+    const int64_t resident = cus * (1024 / threads);
+    const int64_t fullTiles = n / (static_cast<int64_t>(threads) * kWideItems);
     return static_cast<uint32_t>(fullTiles < 1 ? 1 : (fullTiles < resident ? fullTiles : resident));
 }
 
-// One 8-bit pass carrying csr2csc's (row, value) pairs; table: WideTableInts(n) ints.
-void LaunchWidePairPass(int mode, const int32_t *keysIn, const void *pairsIn, int32_t *keysOut, void *pairsOut,
-                        int64_t n, int32_t keyBase, int32_t shift, int32_t bits, int32_t *table, int32_t *scratch,
-                        const RadixPairIo &io, hipStream_t s)
+// One pass carrying (row, value) pairs; table: WideTableInts(n) ints.
+template <int T>
+void LaunchWidePairPassOf(int mode, const int32_t *keysIn, const void *pairsIn, int32_t *keysOut, void *pairsOut,
+                          int64_t n, int32_t keyBase, int32_t shift, int32_t bits, int32_t *table, int32_t *scratch,
+                          const RadixPairIo &io, hipStream_t s)
 {
-    if (n <= 0) {
-        return;
-    }
     const int32_t mask = (1 << bits) - 1;
     const int64_t numTiles = WideTiles(n);
     const auto *pin = static_cast<const RadixPair *>(pairsIn);
     auto *pout = static_cast<RadixPair *>(pairsOut);
-    LaunchFill(table, 1, 0, s);
-    hipLaunchKernelGGL(WideCountKernel, dim3(static_cast<uint32_t>((numTiles + kWideCountTiles - 1) / kWideCountTiles)),
-                       dim3(kBlockThreads), 0, s, keysIn, n, keyBase, shift, mask, table, numTiles);
-    LaunchInclusiveScan(table, table, WideTableInts(n), 0, scratch, s);
-    const auto grid = dim3(WideScatterBlocks(n));
-#define OPSPARSE_WIDE_SCATTER(MODE, VB)                                                                              \
-    hipLaunchKernelGGL((WideScatterKernel<MODE, VB>), grid, dim3(kBlockThreads), 0, s, keysIn, pin, keysOut, pout, n, \
-                       keyBase, shift, mask, table, numTiles, io)
-#define OPSPARSE_WIDE_SCATTER_BY_VALUE(MODE)                                                                         \
-    switch (io.valueBytes) {                                                                                         \
-        case 4: OPSPARSE_WIDE_SCATTER(MODE, 4); break;                                                               \
-        case 2: OPSPARSE_WIDE_SCATTER(MODE, 2); break;                                                               \
-        case 1: OPSPARSE_WIDE_SCATTER(MODE, 1); break;                                                               \
-        default: OPSPARSE_WIDE_SCATTER(MODE, 0); break;                                                              \
+    hipLaunchKernelGGL(WideCountKernel<T>, dim3(static_cast<uint32_t>((numTiles + kWideCountTiles - 1) / kWideCountTiles)),
+                       dim3(T), 0, s, keysIn, n, keyBase, shift, mask, table, numTiles);
+    LaunchInclusiveScan(table, table, (numTiles << bits) + 1, 0, scratch, s);
+    const auto grid = dim3(WideScatterBlocks(n, T));
+#define OPSPARSE_WIDE_SCATTER(MODE, VB)                                                                               \
+    hipLaunchKernelGGL((WideScatterKernel<T, MODE, VB>), grid, dim3(T), 0, s, keysIn, pin, keysOut, pout, n, keyBase, \
+                       shift, mask, bits, table, numTiles, io)
+#define OPSPARSE_WIDE_SCATTER_BY_VALUE(MODE)                                                                          \
+    switch (io.valueBytes) {                                                                                          \
+        case 4: OPSPARSE_WIDE_SCATTER(MODE, 4); break;                                                                \
+        case 2: OPSPARSE_WIDE_SCATTER(MODE, 2); break;                                                                \
+        case 1: OPSPARSE_WIDE_SCATTER(MODE, 1); break;                                                                \
+        default: OPSPARSE_WIDE_SCATTER(MODE, 0); break;                                                               \
     }
     switch (mode) {
         case kPayPairFirst:
@@ -1349,6 +1522,20 @@ void LaunchWidePairPass(int mode, const int32_t *keysIn, const void *pairsIn, in
     }
 #undef OPSPARSE_WIDE_SCATTER_BY_VALUE
 #undef OPSPARSE_WIDE_SCATTER
+}
+
+void LaunchWidePairPass(int mode, const int32_t *keysIn, const void *pairsIn, int32_t *keysOut, void *pairsOut,
+                        int64_t n, int32_t keyBase, int32_t shift, int32_t bits, int32_t *table, int32_t *scratch,
+                        const RadixPairIo &io, hipStream_t s)
+{
+    if (n <= 0) {
+        return;
+    }
+    const int threads = WideThreads(n);
+    const auto launch = threads == 1024  ? LaunchWidePairPassOf<1024>
+                        : threads == 512 ? LaunchWidePairPassOf<512>
+                                         : LaunchWidePairPassOf<256>;
+    launch(mode, keysIn, pairsIn, keysOut, pairsOut, n, keyBase, shift, bits, table, scratch, io, s);
 }
 
 void LaunchGatherByPosition(const int32_t *pos, const int32_t *rowOfPos, const uint32_t *srcVal, int64_t nnz,
@@ -1385,14 +1572,13 @@ int32_t KeyBits(int64_t n)
 
 struct Csr2CscLayout {
     int64_t keysA, keysB, payA, payB, rowOfPos, table, tiles, bytes;
-    int64_t numTiles, tableCount;
+    int64_t tableCount;
 };
 
 Csr2CscLayout LayoutCsr2Csc(int64_t n, int64_t nnz)
 {
     Csr2CscLayout l{};
-    l.numTiles = (nnz + kWideTile - 1) / kWideTile;
-    l.tableCount = static_cast<int64_t>(kWideDigits) * l.numTiles + 1;
+    l.tableCount = WideTableInts(nnz);
     int64_t off = 0;
     const int64_t arr = Align256(4 * nnz);
     l.keysA = off; off += arr;
@@ -1647,12 +1833,7 @@ int opsparse_csr2csc_launch(int64_t m, int64_t n, int64_t nnz, const void *csrVa
     // position at the end, which cost two cache-line fills per entry (33.5 M entries: 2.9 -> 1.9 ms).
     // Up to eight bits a pass, the tile ordered through LDS before it leaves (33.5 M entries over 2^20 columns:
     // three passes instead of five, 1.2 ms).
-    const int32_t keyBits = KeyBits(n);
-    int32_t passes = (keyBits + kWideBits - 1) / kWideBits;
-    passes = passes < 2 ? 2 : passes;  // a first pass that reads the sources and a last one that writes the outputs
-    // the passes share the key's bits evenly (20 bits: 7, 7, 6 rather than 8, 8, 4): the fewer buckets a pass has,
-    // the longer the runs its tiles write, and short runs are what the memory side is slow at
-    const int32_t perPass = (keyBits + passes - 1) / passes;
+    const auto [passes, perPass] = WidePassesOf(KeyBits(n), nnz);
     const RadixPairIo io{rowOfPos, csrVal, cscRowInd, cscVal, valueBytes};
     const int32_t *keysIn = csrColInd;
     const void *pairsIn = nullptr;
@@ -1696,14 +1877,34 @@ __global__ __launch_bounds__(kBlockThreads) void CooRangeKernel(const int32_t *_
                                                                 int32_t *__restrict__ range)
 {
     int32_t lo[2] = {INT32_MAX, INT32_MAX}, hi[2] = {INT32_MIN, INT32_MIN};
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int32_t v[2] = {a[i], b[i]};
+    auto take = [&](int k, int32_t v) {
+        lo[k] = v < lo[k] ? v : lo[k];
+        hi[k] = v > hi[k] ? v : hi[k];
+    };
+    // four groups of four entries of each array asked for together; a group past the end re-reads the last whole one
+    constexpr int kAtOnce = 4;
+    const int64_t groups = n / 4, stride = static_cast<int64_t>(gridDim.x) * kBlockThreads;
+    const int64_t me = static_cast<int64_t>(blockIdx.x) * kBlockThreads + threadIdx.x;
+    for (int64_t i = me; i < groups; i += stride * kAtOnce) {
+        Int4U v[2][kAtOnce];
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            lo[k] = v[k] < lo[k] ? v[k] : lo[k];
-            hi[k] = v[k] > hi[k] ? v[k] : hi[k];
+        for (int j = 0; j < kAtOnce; ++j) {
+            const int64_t at = i + j * stride < groups ? i + j * stride : groups - 1;
+            v[0][j] = *reinterpret_cast<const Int4U *>(a + 4 * at);
+            v[1][j] = *reinterpret_cast<const Int4U *>(b + 4 * at);
         }
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                take(0, v[0][j][e]);
+                take(1, v[1][j][e]);
+            }
+        }
+    }
+    if (me < n - 4 * groups) {
+        take(0, a[4 * groups + me]);
+        take(1, b[4 * groups + me]);
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -1738,10 +1939,41 @@ __global__ __launch_bounds__(kBlockThreads) void CooRangeKernel(const int32_t *_
     }
 }
 
-__global__ __launch_bounds__(kBlockThreads) void CooRangeInitKernel(int32_t *range)
+// ... and range[4] = 0, counters[0 .. count) = 0 for the kernel below.
+__global__ __launch_bounds__(kBlockThreads) void CooRangeInitKernel(int32_t *range, int32_t *counters, int32_t count)
 {
-    if (threadIdx.x < 4) {
-        range[threadIdx.x] = (threadIdx.x & 1) ? INT32_MIN : INT32_MAX;
+    if (blockIdx.x == 0 && threadIdx.x < 5) {
+        range[threadIdx.x] = threadIdx.x == 4 ? 0 : (threadIdx.x & 1) ? INT32_MIN : INT32_MAX;
+    }
+    for (int32_t i = blockIdx.x * kBlockThreads + threadIdx.x; i < count; i += gridDim.x * kBlockThreads) {
+        counters[i] = 0;
+    }
+}
+
+// How long are the rows that the entries lie in?  Of `samples` evenly spaced entries, range[4] = the pairs that share a
+// row (a counter: the rows are hashed onto 2^bits of them): samples^2 / (2 n) x (mean row length over the entries).
+__global__ __launch_bounds__(kBlockThreads) void CooSampleKernel(const int32_t *__restrict__ primary, int64_t n,
+                                                                 int32_t samples, int32_t *__restrict__ counters,
+                                                                 int32_t bits, int32_t *__restrict__ range)
+{
+    const int32_t i = blockIdx.x * kBlockThreads + threadIdx.x;
+    int32_t pairs = 0;
+    if (i < samples) {
+        const uint32_t row = static_cast<uint32_t>(primary[static_cast<int64_t>(i) * n / samples]);
+        pairs = atomicAdd(counters + ((row * 0x9E3779B1u) >> (32 - bits)), 1);
+    }
+    __shared__ int32_t part[kBlockThreads / kWave];
+    pairs = GroupSum<kWave>(pairs);
+    if (threadIdx.x % kWave == 0) {
+        part[threadIdx.x / kWave] = pairs;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        pairs = 0;
+        for (int w = 0; w < kBlockThreads / kWave; ++w) {
+            pairs += part[w];
+        }
+        atomicAdd(range + 4, pairs);
     }
 }
 
@@ -1755,6 +1987,12 @@ __global__ __launch_bounds__(kBlockThreads) void CooRebaseKernel(int32_t *__rest
         b[i] = static_cast<int32_t>(static_cast<uint32_t>(b[i]) + static_cast<uint32_t>(addB));
     }
 }
+
+// From this many entries on a sample of the rows is taken, and rows of up to this mean length over the entries are
+// sorted by csrsort after one sort by row.
+constexpr int64_t kRowsFirstMin = int64_t{1} << 20;
+constexpr int32_t kRowSamples = 65536;
+constexpr double kRowsFirstLongest = 50.0;
 
 struct CoosortLayout {
     int64_t range, keysA, keysB, pairsA, pairsB, table, tiles, bytes;
@@ -1820,10 +2058,21 @@ int opsparse_coosort_launch(int64_t nnz, int32_t byRow, int32_t *cooRows, int32_
     int32_t *table = at(l.table), *tiles = at(l.tiles), *range = at(l.range);
     int32_t *primary = byRow != 0 ? cooRows : cooCols, *secondary = byRow != 0 ? cooCols : cooRows;
 
-    hipLaunchKernelGGL(CooRangeInitKernel, dim3(1), dim3(kBlockThreads), 0, s, range);
+    // (the counters of the sample: in the first key buffer, a power of two of them that fits)
+    int32_t sampleBits = 1;
+    while (sampleBits < 20 && (int64_t{2} << sampleBits) <= nnz) {
+        ++sampleBits;
+    }
+    const bool ask = nnz >= kRowsFirstMin;
+    hipLaunchKernelGGL(CooRangeInitKernel, dim3(ask ? 1024 : 1), dim3(kBlockThreads), 0, s, range, keys[0],
+                       ask ? 1 << sampleBits : 0);
     hipLaunchKernelGGL(CooRangeKernel, dim3(GridFor(nnz, kBlockThreads * 16, 2048)), dim3(kBlockThreads), 0, s, primary,
                        secondary, nnz, range);
-    int32_t r[4] = {0, 0, 0, 0};  // min / max of the primary key, of the secondary key
+    if (ask) {
+        hipLaunchKernelGGL(CooSampleKernel, dim3(kRowSamples / kBlockThreads), dim3(kBlockThreads), 0, s, primary, nnz,
+                           kRowSamples, keys[0], sampleBits, range);
+    }
+    int32_t r[5] = {0, 0, 0, 0, 0};  // min / max of the primary key, of the secondary key; pairs of the sample
     if (hipMemcpyAsync(r, range, sizeof(r), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         (void)hipGetLastError();
@@ -1834,9 +2083,7 @@ int opsparse_coosort_launch(int64_t nnz, int32_t byRow, int32_t *cooRows, int32_
     // One key's passes: the first reads (key, pair) from three arrays, the last writes three arrays.
     auto sortBy = [&](const int32_t *keySrc, int32_t keyBase, int32_t bits, const int32_t *pairRowSrc,
                       const void *pairValSrc, int32_t *keyDst, int32_t *pairRowDst, void *pairValDst) {
-        int32_t passes = (bits + kWideBits - 1) / kWideBits;
-        passes = passes < 2 ? 2 : passes;
-        const int32_t perPass = (bits + passes - 1) / passes;
+        const auto [passes, perPass] = WidePassesOf(bits, nnz);
         const RadixPairIo io{pairRowSrc, pairValSrc, pairRowDst, pairValDst, 4};
         const int32_t *keysIn = keySrc;
         const void *pairsIn = nullptr;
@@ -1851,12 +2098,32 @@ int opsparse_coosort_launch(int64_t nnz, int32_t byRow, int32_t *cooRows, int32_
             cur ^= 1;
         }
     };
+    const int32_t bitsS = RangeBits(r[2], r[3]), bitsP = RangeBits(r[0], r[1]);
+    const int64_t span = static_cast<int64_t>(r[1]) - r[0] + 1;
+    // (two rows that share a counter look like one: as many pairs of theirs as the counters would give anyway come off)
+    const double rowLength = (2.0 * r[4] / (static_cast<double>(kRowSamples) * kRowSamples) -
+                              1.0 / static_cast<double>(int64_t{1} << sampleBits)) * static_cast<double>(nnz);
+    if (ask && rowLength <= kRowsFirstLongest && span < nnz && r[2] >= 0 && r[3] < INT32_MAX) {
+        // Rows short enough for csrsort's registers: by row only, then every row by its secondary key in one pass over
+        // the entries instead of one a digit.
+        sortBy(primary, r[0], bitsP, secondary, perm, primary, secondary, perm);
+        int32_t *rowPtr = keys[0];  // the passes' buffers are free again
+        LaunchIndicesToOffsets(primary, nnz, span, 0, rowPtr, tiles, s);
+        const int rc = opsparse_csrsort_launch(span, static_cast<int64_t>(r[3]) + 1, nnz, 0, rowPtr, secondary, perm,
+                                               keys[1], static_cast<size_t>(l.table - l.keysB), stream);
+        if (rc != OPSPARSE_OK) {
+            return rc;
+        }
+        if (r[0] != 0) {
+            hipLaunchKernelGGL(CooRebaseKernel, dim3(GridFor(nnz, kBlockThreads * 8)), dim3(kBlockThreads), 0, s, primary,
+                               secondary, nnz, r[0], 0);
+        }
+        return CheckLaunch();
+    }
     // by the secondary key, (primary key, P) as the pair: the result stays in the workspace ...
     int32_t *midKeys = keys[1];                                   // (two or four passes: the last one writes buffer 1
     auto *midRows = static_cast<int32_t *>(pairs[1]);             //  only when their number is even)
-    const int32_t bitsS = RangeBits(r[2], r[3]), bitsP = RangeBits(r[0], r[1]);
-    const int32_t passesS = (bitsS + kWideBits - 1) / kWideBits < 2 ? 2 : (bitsS + kWideBits - 1) / kWideBits;
-    const int lastBuf = (passesS - 1) & 1;                        // buffer the last pass of that stage writes
+    const int lastBuf = (WidePassesOf(bitsS, nnz).passes - 1) & 1;                        // buffer the last pass of that stage writes
     midKeys = keys[lastBuf];
     midRows = static_cast<int32_t *>(pairs[lastBuf]);
     uint32_t *midVals = reinterpret_cast<uint32_t *>(pairs[lastBuf]) + nnz;

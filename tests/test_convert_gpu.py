@@ -450,6 +450,26 @@ def test_coosort_signed_indices_custom_perm_and_sorted_input(osa, gpu_ctx, by_ro
     run_coosort(osa, gpu_ctx, 200, 250, r[::-1], c[::-1], by_row)                              # reversed
 
 
+@pytest.mark.parametrize("nnz,m,n,least_row,what", [
+    ((1 << 20) - 1, 60_000, 1 << 20, 0, "too few entries to ask"), (1 << 20, 60_000, 1 << 20, 7, "short rows"),
+    ((1 << 20) + 5, 60_000, 3, 0, "short rows, repeated pairs"), (1_500_000, 60_000, 5000, -9, "short rows, base < 0"),
+    (1_500_000, 9_000, 5000, 0, "rows beyond the bound"), (1_500_000, 60_000, 5000, 0, "one long row among short ones"),
+    (1_100_000, 1_500_000, 5000, 0, "fewer entries than rows"), (1_500_000, 60_000, 5000, 0, "negative secondary keys")])
+@pytest.mark.parametrize("by_row", [True, False])
+def test_coosort_by_short_rows_and_where_they_are_not(osa, gpu_ctx, nnz, m, n, least_row, what, by_row):
+    """From 2^20 entries on a sample of the rows decides: one sort by row and csrsort inside the rows, or a pass for every
+    digit of both keys; both give the golden's order, row by row and column by column, P included."""
+    rng = np.random.default_rng(nnz + m)
+    primary, secondary = rng.integers(0, m, nnz) + least_row, rng.integers(0, n, nnz)
+    if what == "one long row among short ones":
+        primary[rng.integers(0, nnz, 100_000)] = 77
+    if what == "negative secondary keys":
+        secondary -= 100
+    rows, cols = (primary, secondary) if by_row else (secondary, primary)
+    run_coosort(osa, gpu_ctx, max(m, n), max(m, n), rows, cols, by_row,
+                perm=rng.permutation(nnz).astype(np.int32))
+
+
 def test_coosort_then_coo2csr_is_csr2csc(osa, gpu_ctx):
     """Sorting a matrix's COO triples by column and compressing the column indices gives its CSC form: the same
     row indices, values (through P) and column offsets as aclsparseCsr2cscEx2's oracle."""
@@ -559,13 +579,25 @@ def test_csr2csc_value_sizes_and_key_widths_over_whole_tiles(osa, gpu_ctx, m, n,
 
 @pytest.mark.parametrize("tiles", [1, 2, 5, 7, 8, 9, 23])
 def test_csr2csc_fewer_tiles_than_dies_and_a_few_more(osa, gpu_ctx, tiles):
-    """A sort pass shares its tiles out to the eight dies (a range each): fewer tiles than dies, as many, one more,
-    ranges of unequal length; the entry count a whole number of tiles and one either side.  Exact."""
+    """A sort pass shares its tiles (2 048 entries at these sizes) out to the eight dies, a range each: fewer tiles than
+    dies, as many, one more, ranges of unequal length; the entry count a whole number of tiles and one either side."""
     rng = np.random.default_rng(tiles)
-    for nnz in (3840 * tiles - 1, 3840 * tiles, 3840 * tiles + 1):
+    for nnz in (2048 * tiles - 1, 2048 * tiles, 2048 * tiles + 1):
         rowptr = np.array([0, nnz // 3, nnz], np.int32)
         run_csr2csc(osa, gpu_ctx, 2, 300_000, rowptr, rng.integers(0, 300_000, nnz).astype(np.int32),
                     rng.uniform(-1, 1, nnz).astype(np.float32), np.float32, True, 0)
+
+
+@pytest.mark.parametrize("val_type,numeric", [("FP32", True), ("FP16", True), ("INT8", True), ("FP32", False)])
+@pytest.mark.parametrize("n,nnz", [(1 << 20, (1 << 20) - 1), (1 << 20, 1 << 20), (5_000_000, (1 << 20) + 4097),
+                                   (1 << 18, (1 << 23) - 3), (1 << 20, 1 << 23), (5_000_000, (1 << 23) + 8193)])
+def test_csr2csc_either_side_of_the_workgroup_sizes(osa, gpu_ctx, n, nnz, val_type, numeric):
+    """The passes run in workgroups of 256, 512 and 1024 threads by entry count: either side of the two bounds, whole
+    tiles and a few entries more, 18 - 23 column bits (two and three passes), every value size."""
+    rng = np.random.default_rng(nnz + n)
+    rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, 999)), [nnz]]).astype(np.int32)
+    run_csr2csc(osa, gpu_ctx, 1000, n, rowptr, rng.integers(0, n, nnz).astype(np.int32),
+                _typed(rng.uniform(-1, 1, nnz).astype(np.float32), val_type), NP_TYPE[val_type], numeric, 0)
 
 
 def test_csr2csc_twice_is_sorted_csr(osa, gpu_ctx):
