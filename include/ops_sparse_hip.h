@@ -80,13 +80,14 @@ typedef OPSPARSE_ABI_ENUM(OpsparseSpmvKernel) {
                                       read in place, in an order that the layout fixes: the same bits at every
                                       call.  16 bytes of traffic per entry and no line-sized gathers; fp32 / fp16 /
                                       bf16 / int32, op(A) = A or (on a transposed copy) A^T */
-    OPSPARSE_SPMV_BLOCKED_LIVE = 7, /* the same two passes with the second one built for speed: it collects a row
-                                      block's values in LDS, streams the block's entries panel by panel against
-                                      them and adds into one fp64 accumulator a row with LDS atomics, in the order
-                                      the wavefronts get there: the last bit of a result may differ between two
-                                      calls.  The plan of aclsparseSpMVPreprocess under ACL_SPARSE_SPMV_ALG_DEFAULT,
-                                      whose results the reference lets vary; fp32 / fp16 / bf16, op(A) = A, values
-                                      read where the caller has them at every call */
+    OPSPARSE_SPMV_BLOCKED_LIVE = 7, /* the same two passes with a second one that collects a row block's values in LDS,
+                                      streams the block's entries panel by panel against them and adds into one fp64
+                                      accumulator a row with LDS atomics, in the order the wavefronts get there: the
+                                      last bit of a result may differ between two calls.  Takes rows of any length in
+                                      any order, where BLOCKED_GATHER refuses unsorted ones of more than 65 534
+                                      entries: what aclsparseSpMVPreprocess falls back to for those under
+                                      ACL_SPARSE_SPMV_ALG_DEFAULT; fp32 / fp16 / bf16, op(A) = A, values read where
+                                      the caller has them at every call */
     OPSPARSE_SPMV_SCATTER_LIVE = 8  /* op(A) = A^T with y larger than an L2, the mirror image: pieces of the caller's
                                       arrays multiplied by x[row] and written out sorted by output panel (2^14
                                       columns) through LDS, then a workgroup a panel adds the products, kept exactly,
@@ -129,7 +130,7 @@ typedef struct OpsparseSpmvPlan {
     int32_t numEmptyRows;  /* BLOCKED_GATHER: rows without entries; a small kernel of their own writes beta * y there */
     int32_t streamedBlocks;/* BLOCKED_GATHER: 1: the layout keeps the values, in (block, panel) order, and a wavefront
                               streams a run of row blocks; 0: values read in row order through a window in LDS */
-    int32_t reserved0;
+    int32_t usedRowBlocks; /* BLOCKED_GATHER: the row block numbers below this one hold all rows */
     int64_t rows;
     int64_t nnz;
     int64_t partOff;       /* byte offsets into the workspace */
@@ -244,8 +245,8 @@ int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int
 /*
  * BLOCKED_LIVE analysis (fp32, fp16 or bf16 values and x, op(A) = A, values read in place at every launch): the
  * layout of the plan kernel OPSPARSE_SPMV_BLOCKED_LIVE, whose second kernel adds into LDS with atomics in the order
- * the wavefronts get there — the fastest plan for a matrix with scattered columns whose values change between
- * calls, for callers who do not need the last bit of a result to repeat.  Same applicability bounds as BLOCKED_GATHER
+ * the wavefronts get there.  The two byte counts are room for it and, in its place, for the BLOCKED_GATHER layout with
+ * live values of the same matrix.  Same applicability bounds as BLOCKED_GATHER
  * except that a chunk needs 8 entries on average; `flags`: OPSPARSE_BLOCKED_VALUES_F16 / _BF16 only.  Synchronises
  * `stream` twice.  No counterpart in the reference.
  */

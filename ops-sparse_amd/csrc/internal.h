@@ -155,7 +155,9 @@ OpsparseScalar MakeScalar(const void *p, aclDataType computeType, aclsparsePoint
 // re-stored layout to pay: with the values frozen, and with live values.
 constexpr int32_t kScatteredForFrozenLayout = 190;
 constexpr int32_t kScatteredForLiveLayout = 310;
-// Columns from which the ordered layout with live values (repeatable sums) is taken for op(A) = A.
+// Entries from which the default algorithm re-stores a matrix with scattered gathers, and columns from which a matrix of
+// fewer entries would where the sums have to repeat.
+constexpr int64_t kMinDefaultNnz = 7000000;
 constexpr int64_t kMinColsOrderedLive = int64_t{5} << 19;  // 2.6 M
 
 struct RestoredChoice {
@@ -174,7 +176,7 @@ void TrimToWorkspace(aclsparseHandle_t handle, RestoredChoice *choice, int64_t r
 // entries or more, an x the layout applies to, and a sample of the columns that says the gathers are scattered:
 // one short kernel and a synchronisation of the handle's stream), else none.  `repeatable`: the caller promises
 // the same bits from every execution (aclsparseSpMVOp): BLOCKED_GATHER; else BLOCKED_LIVE where it exists
-// (op(A) = A, floating-point values).
+// (op(A) = A, floating-point values), which AnalyseRestored takes for what BLOCKED_GATHER refuses.
 RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffsets, const int32_t *colInd, int64_t rows,
                               int64_t cols, int64_t nnz, bool transpose, int32_t valueType, bool repeatable);
 // The size-query record of a matrix (OpsparseSpmvSized): written by the queries, asked by Preprocess / createDescr.

@@ -15,7 +15,7 @@
 //            its panel's slice of x into LDS and writes xg[i] = x[col[i]] for
 //            the panel's entries: 2 bytes read, 4 bytes written per entry, both
 //            as linear streams.
-//   phase 2  rows are grouped into row blocks (at most 2^12 rows, cut also
+//   phase 2  rows are grouped into row blocks (at most 2^10 - 2^12 rows, cut also
 //            wherever the entry count passes a multiple of the entry window).
 //            The entries of a block are one contiguous piece of the values in
 //            row order, and a workgroup owns one block: it streams the block's
@@ -91,9 +91,6 @@ constexpr uint32_t kStreamPadRow = 0x7ffu;        // row field of a padding posi
 constexpr int kStreamRoundShift = 11;             // above the row: the turn of the entry among those of its row that
 constexpr uint32_t kStreamMaxRound = 31;          // one LDS instruction would add together (31: "31st or later")
 constexpr int32_t kMaxBlockEntries = 65534;       // a block's slots are 16 bits
-// Phase 2 holds the gathered x of a row block in a window of LDS (kRowsWindow entries: two workgroups then share a
-// compute unit).  The blocks are cut at three quarters of that (plus the row in which the cut falls), so that
-// nearly all of them fit one window.
 constexpr int64_t kMinEntries = 2000000;          // below this the ordinary kernels are as fast or faster
 // x of more than 2^18 elements.  An x of 1 - 4 MB fits an L2, but gathers scattered over it still cost the row-wise
 // kernels 5.5 us per million (the rate at which an L2 answers them).  Whether the gathers are scattered is for the
@@ -399,7 +396,19 @@ __device__ __forceinline__ void SegJoinWave(const SegEnds &ends, int waves, int 
 
 // ---- row blocks ------------------------------------------------------------------------------------------------
 
-constexpr int kRowsWindow = 14336;  // entries of a row block whose gathered x a phase-2 workgroup holds in LDS at a time
+// Windowed row blocks come in three sizes: the entries of a block whose gathered x a phase-2 workgroup holds in LDS at a
+// time (the window), the rows of a block at most, and the workgroup's threads.  Small blocks: more workgroups a compute
+// unit, whose waits for memory and at barriers fall at different times.  Large ones: longer chunks (less padding, fewer
+// lines of gathered x shared between blocks).  The layout takes the smallest whose chunks are long enough.  A call with
+// live values, small / middle / large: 31 M entries over 123 panels (20 / 37 / 73 a chunk) 159 / 166 / 176 us; 24 M over
+// 46 panels (64 a chunk and more) 96 / 109 / 118; 65 M over 256 panels (9.7 / 18 / 35) 343 / 335 / 334; 34 M over 256
+// (7.5 / 14 / 28) does not fit the small size and takes 243 / 254.
+struct RowsSize {
+    int32_t window, rowLog, threads;
+    int64_t chunk;  // entries of a (panel, block) chunk, on average, from which the size is taken
+};
+constexpr RowsSize kRowsSizes[] = {{4096, 10, 256, 10}, {7168, 11, 256, 8}, {14336, 12, 512, 0}};
+constexpr int kNumRowsSizes = 3;
 
 // What the workgroup of a row block needs to know before anything else, in one piece.
 struct BlockMeta {
@@ -751,7 +760,8 @@ __global__ __launch_bounds__(kBlockThreads) void BlockedLongDeferKernel(const in
 // phase 2 reads them from: the caller's (valueOffsets = its row offsets; a block then holds no long row except as
 // its last row, so that its other entries are one piece) or the compact copy (valueOffsets = offsets).
 // blockShort[b] = the former, for the scatter kernel.  panelStart[p] = first entry of panel p in panel order
-// (p = P: the number of entries there).  header[3] (zero before) = entries of the largest block.
+// (p = P: the number of entries there).  header[3] (zero before) = entries of the largest block,
+// header[6] (zero before) = number of the last block with rows, plus one.
 __global__ __launch_bounds__(kBlockThreads) void BlockedBlockTablesKernel(
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ valueOffsets, const int32_t *__restrict__ blockRow,
     const int32_t *__restrict__ dstStart, const int32_t *__restrict__ srcStart, const int32_t *__restrict__ longFirst,
@@ -781,6 +791,9 @@ __global__ __launch_bounds__(kBlockThreads) void BlockedBlockTablesKernel(
         m.pad = 0;
         meta[b] = m;
         atomicMax(header + 3, offsets[blockRow[b + 1]] - offsets[blockRow[b]]);
+        if (m.nRows > 0) {
+            atomicMax(header + 6, b + 1);
+        }
     }
 }
 
@@ -1115,8 +1128,10 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
     const int tid = threadIdx.x;
     // Neighbouring panels on one XCD: the pieces of a long row in panels p and p + 1 are neighbours in memory, and
     // the cache line they share is then fetched once, by the L2 both workgroups sit behind.
-    const int64_t p = splits == 1 ? XcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x / splits;
-    const int64_t part = splits == 1 ? 0 : blockIdx.x % splits;
+    // (a panel's parts as well: they read the same slice of x.)
+    const uint32_t place = XcdContiguousTile(blockIdx.x, gridDim.x);
+    const int64_t p = place / splits;
+    const int64_t part = place % splits;
     const int64_t c0 = p << kPanelLog;
     const int64_t cn = cols - c0 < kPanelCols ? cols - c0 : kPanelCols;
     const int64_t a = panelStart[p], e = panelStart[p + 1];
@@ -1416,10 +1431,9 @@ __device__ __forceinline__ AccT LongRowTotal(const uint64_t *__restrict__ from, 
     return sum;
 }
 
-constexpr int kRowsThreads = 512;  // threads of a phase-2 workgroup; two workgroups share a compute unit
 constexpr int kLaneRun = 16;        // consecutive entries a lane sums in one round of phase 2
 constexpr int kBigRound = kWave * kLaneRun;
-constexpr int kStagePasses = 3;     // passes over a block's positions whose loads a wavefront has in flight at a time
+constexpr int kStagePasses = 2;     // passes over a block's positions whose loads a wavefront has in flight at a time
 constexpr uint64_t kJoinMark = 0x7ff8dead0000beefull;  // rowSum of a row that the joining thread writes
 
 template <typename ValT, typename OutT>
@@ -1447,8 +1461,8 @@ struct BlockRowsArgs {
 // In block order every (panel, block) chunk starts on a multiple of kLaneEntries and is padded to one (padding
 // carries the slot kPadSlot); src8[d / 8] is where the eight positions from d on sit in panel order, i.e. in xg.
 // The block's entries are entries meta.base .. of `vals` in row order.  The tables of BlockedRowTablesKernel tell
-// their rows apart: the key of an entry is two reads and a population count.  A block of more than kRowsWindow
-// entries is worked a window at a time: its positions are read once per window.
+// their rows apart: the key of an entry is two reads and a population count.  A block of more entries than
+// the window is worked a window at a time: its positions are read once per window.
 //
 // A window, step by step.  (1) The gathered x of the block's positions is dropped at its slot of xwin.  (2) Every
 // lane takes kLaneRun consecutive entries of the window into registers; behind a barrier the window's memory serves
@@ -1456,22 +1470,23 @@ struct BlockRowsArgs {
 // begins and ends inside the lane is a row's sum and goes to rowSum.  The runs at the lanes' edges are joined by a
 // segmented scan over the wavefront, the ones at the wavefronts' edges by one thread (SegJoin), which writes those
 // rows itself.  (4) rowSum goes out, a key a lane.
-template <int kThreads, typename ValT, typename OutT, typename AccT>
-__global__ __launch_bounds__(kThreads, 2 * kThreads / kWave / 4) void SpmvBlockRowsKernel(
+template <int kSize, typename ValT, typename OutT, typename AccT>
+__global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 5 : 4) void SpmvBlockRowsKernel(
     const BlockRowsArgs<ValT, OutT> a)
 {
     constexpr bool kIntData = std::is_same<ValT, int32_t>::value;
-    constexpr int kW = kRowsWindow;
+    constexpr int kW = kRowsSizes[kSize].window, kThreads = kRowsSizes[kSize].threads;
+    constexpr int kBlockRows = 1 << kRowsSizes[kSize].rowLog;
     constexpr int kWaves = kThreads / kWave;
     constexpr int kMaxRounds = (kW / kBigRound + kWaves - 1) / kWaves;
     constexpr int kWords = kW / 32 + 1;              // of a window's bits, the bit behind its last entry included
     constexpr int kPassSpan = kWave * kLaneEntries;  // positions a wavefront takes per pass: eight a lane
-    constexpr int kOrdPer = (kRowBlockRows + 8 + 8 * kThreads - 1) / (8 * kThreads);  // 16-byte pieces of ordRow a thread
+    constexpr int kOrdPer = (kBlockRows + 8 + 8 * kThreads - 1) / (8 * kThreads);  // 16-byte pieces of ordRow a thread
     static_assert(kW % kBigRound == 0 && kWords <= kThreads, "a window is whole rounds; a word of its bits a thread");
-    static_assert(kW / 2 >= kRowBlockRows + 2, "a sum for every row of a block, and two more keys");
+    static_assert(kW / 2 >= kBlockRows + 2, "a sum for every row of a block, and two more keys");
     static_assert(kLaneEntries == 8 && kLaneRun == 16, "the unpacking below");
     __shared__ __align__(16) uint32_t xwin[kW];
-    __shared__ __align__(16) uint16_t ordRow[kRowBlockRows + 16];
+    __shared__ __align__(16) uint16_t ordRow[kBlockRows + 16];
     __shared__ uint32_t rowBits[kWords];
     __shared__ uint16_t bitPrefix[kWords];
     __shared__ SegEnds ends;
@@ -1485,9 +1500,8 @@ __global__ __launch_bounds__(kThreads, 2 * kThreads / kWave / 4) void SpmvBlockR
         return;  // a block number no row maps to
     }
     const int32_t row0 = m.row0, dBeg = m.dBeg, dEnd = m.dEnd, P = a.P;
-    const int32_t nRows = m.nRows < kRowBlockRows ? m.nRows : kRowBlockRows;
-    // ---- asked for at once: the rows of the keys, and the number of the block's entries (the last prefix count
-    // belongs to the word of the bit behind the last entry; the words are found through it)
+    const int32_t nRows = m.nRows < kBlockRows ? m.nRows : kBlockRows;
+    // ---- asked for at once: the rows of the keys
     Uint4 ordPiece[kOrdPer];
 #pragma unroll
     for (int u = 0; u < kOrdPer; ++u) {
@@ -1513,7 +1527,7 @@ __global__ __launch_bounds__(kThreads, 2 * kThreads / kWave / 4) void SpmvBlockR
     AccT pendSum = AccT(0);
     // (whatever the tables hold, a row outside the block is never written)
     auto outKey = [&](int32_t key, AccT sum) {
-        const uint16_t row = ordRow[static_cast<uint32_t>(key) < static_cast<uint32_t>(kRowBlockRows + 8) ? key : 0];
+        const uint16_t row = ordRow[static_cast<uint32_t>(key) < static_cast<uint32_t>(kBlockRows + 8) ? key : 0];
         if (static_cast<int32_t>(row) < nRows) {
             out(row, sum);
         }
@@ -1976,6 +1990,7 @@ int32_t ValueBytes(int32_t valueType) { return valueType == OPSPARSE_F16 || valu
 
 struct BlockedLayout {
     int32_t P, B, window, passes;
+    int32_t size;    // windowed blocks: which of kRowsSizes
     bool streamed;      // row blocks of 2^10 rows that a wavefront streams (values kept in block order), not windowed
     int32_t rowLog;     // rows of a block at most: 2^rowLog
     int64_t valDOff;    // streamed: the values in block order
@@ -2019,7 +2034,16 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
         const char *env = std::getenv("OPS_SPARSE_BLOCKED_WINDOW");
         return env != nullptr ? std::atoll(env) : 0;
     }();
-    int64_t window = cutEnv > 0 ? cutEnv : kRowsWindow * 7 / 8;
+    // (the blocks are cut at seven eighths of the window, plus the row in which the cut falls: nearly all fit one)
+    l.size = kNumRowsSizes - 1;
+    for (int i = 0; i < kNumRowsSizes - 1; ++i) {
+        const int64_t blocks = (rows >> kRowsSizes[i].rowLog) + nnz / (kRowsSizes[i].window * 7 / 8) + 1;
+        if (nnz / (P * blocks) >= kRowsSizes[i].chunk) {
+            l.size = i;
+            break;
+        }
+    }
+    int64_t window = cutEnv > 0 ? cutEnv : kRowsSizes[l.size].window * 7 / 8;
     window = window > kMaxBlockEntries / 2 ? kMaxBlockEntries / 2 : window;
     // Values that the layout keeps (frozen values, either op(A)) are kept in block order and streamed by a wavefront
     // a block; values read where the caller has them need the windowed blocks, which read them in row order.
@@ -2044,7 +2068,7 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
             window = cut;
         }
     }
-    l.rowLog = l.streamed ? kStreamRowLog : kRowBlockLog;
+    l.rowLog = l.streamed ? kStreamRowLog : kRowsSizes[l.size].rowLog;
     // The values a launch reads: the caller's own (live values, op(A) = A), the transposed copy (op(A) = A^T), or,
     // for op(A) = A with frozen values, a compact copy without the long rows' values, whose entries are stored a
     // second time with their values.
@@ -2189,6 +2213,26 @@ int WithValueType(int32_t valueType, Fn &&fn)
 
 }  // namespace
 
+// Workgroups a panel in phase 1.  One workgroup is resident a compute unit, so P x splits of them run in whole rounds:
+// the number of parts that makes rounds x (what a workgroup takes for its slice of x + its part of the entries)
+// smallest.  (4 M columns are 123 panels: 80 us in 369 thirds, two rounds, 53 us in 246 halves; 6 M columns, 184
+// panels, 72 % of the chip with one workgroup each.)
+int32_t GatherSplits(int64_t P, int64_t nnz)
+{
+    const double slice = 5.0, panel = 0.00036 * static_cast<double>(nnz) / static_cast<double>(P);  // us
+    int32_t best = 1;
+    double least = 0.0;
+    for (int32_t s = 1; s <= 64; ++s) {  // (2^18 columns, the fewest, are eight panels)
+        const double rounds = static_cast<double>((P * s + 255) / 256);
+        const double t = rounds * (slice + panel / s);
+        if (s == 1 || t < 0.98 * least) {
+            best = s;
+            least = t;
+        }
+    }
+    return best;
+}
+
 // valType: the type of the caller's values and of x (OPSPARSE_F32 / F16 / BF16 / I32); outType that of y: fp32, or
 // the values' own type.  a.rows outputs, a.cols inputs: the caller has exchanged them for op(A) = A^T.
 int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valType, int32_t outType, int32_t computeIsInt)
@@ -2211,7 +2255,7 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
     if (plan.numEmptyRows < 0 || plan.numEmptyRows > a.rows || plan.numLongRows < 0 || plan.numLongRows > l.maxLong) {
         return OPSPARSE_E_INVALID;
     }
-    if ((plan.streamedBlocks != 0) != l.streamed) {
+    if ((plan.streamedBlocks != 0) != l.streamed || plan.usedRowBlocks < 1 || plan.usedRowBlocks > l.B) {
         return OPSPARSE_E_INVALID;
     }
     auto *base = static_cast<unsigned char *>(a.ws);
@@ -2236,8 +2280,7 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
     }
     const int32_t *header = longRows ? ints(0) : nullptr;
     auto *longPartial = reinterpret_cast<uint64_t *>(base + l.longPartialOff);
-    // Few panels: several workgroups per panel, so that every CU has one.
-    const int32_t splits = l.P >= 192 ? 1 : (256 + l.P - 1) / l.P;
+    const int32_t splits = GatherSplits(l.P, a.nnz);
     return WithValueType(valType, [&](auto tag) {
         using ValT = decltype(tag);
         auto run = [&](auto accTag, auto outTag) {
@@ -2275,7 +2318,7 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
                 args.longRows = ints(l.longRowsOff);
                 args.B = l.B;
                 args.xgEntries = static_cast<int32_t>(a.nnz);
-                hipLaunchKernelGGL((SpmvBlockStreamKernel<ValT, OutT, AccT>), dim3(static_cast<uint32_t>(l.B)),
+                hipLaunchKernelGGL((SpmvBlockStreamKernel<ValT, OutT, AccT>), dim3(static_cast<uint32_t>(plan.usedRowBlocks)),
                                    dim3(kStreamThreads), 0, a.stream, args);
                 if (longRows) {  // (every long row is left to this kernel)
                     constexpr int kRowsPerBlock = kBlockThreads / kWave;
@@ -2304,8 +2347,17 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
             args.P = l.P;
             args.xgEntries = static_cast<int32_t>(a.nnz);
             args.valEntries = a.nnz;  // (the compact copy of a frozen plan has room for as many, and 16 bytes more)
-            hipLaunchKernelGGL((SpmvBlockRowsKernel<kRowsThreads, ValT, OutT, AccT>), dim3(static_cast<uint32_t>(l.B)),
-                               dim3(kRowsThreads), 0, a.stream, args);
+            // (the block numbers in use: they come first, and a die is given a range of them; with the numbers that no
+            // row maps to counted in, three of the eight dies had nothing to do: 258 us against 146)
+            const auto grid = dim3(static_cast<uint32_t>(plan.usedRowBlocks));
+            const auto threads = dim3(kRowsSizes[l.size].threads);
+            if (l.size == 0) {
+                hipLaunchKernelGGL((SpmvBlockRowsKernel<0, ValT, OutT, AccT>), grid, threads, 0, a.stream, args);
+            } else if (l.size == 1) {
+                hipLaunchKernelGGL((SpmvBlockRowsKernel<1, ValT, OutT, AccT>), grid, threads, 0, a.stream, args);
+            } else {
+                hipLaunchKernelGGL((SpmvBlockRowsKernel<2, ValT, OutT, AccT>), grid, threads, 0, a.stream, args);
+            }
             if (plan.numEmptyRows > 0) {
                 hipLaunchKernelGGL((SpmvEmptyRowsKernel<OutT, AccT>),
                                    dim3((plan.numEmptyRows + kBlockThreads - 1) / kBlockThreads), dim3(kBlockThreads), 0,
@@ -2559,7 +2611,8 @@ int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int
     if (rcScatter != OPSPARSE_OK) {
         return rcScatter;
     }
-    int32_t tail[3] = {0, 0, 0};  // entries of the largest row block, long rows summed on their own, rows without entries
+    // entries of the largest row block, long rows summed on their own, rows without entries, block numbers in use
+    int32_t tail[4] = {0, 0, 0, 0};
     if (hipMemcpyAsync(tail, status + 3, sizeof(tail), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         (void)hipGetLastError();
@@ -2583,6 +2636,7 @@ int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int
     p.numDeferredLongRows = tail[1];
     p.numEmptyRows = tail[2];
     p.streamedBlocks = l.streamed ? 1 : 0;
+    p.usedRowBlocks = tail[3];
     p.numLongRows = head[1];
     p.rows = rows;
     p.nnz = nnz;

@@ -579,8 +579,10 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
     const int tid = threadIdx.x;
     // Neighbouring panels on one XCD: the pieces of a long row in panels p and p + 1 are neighbours in memory, and
     // the cache line they share is then fetched once, by the L2 both workgroups sit behind.
-    const int64_t p = splits == 1 ? XcdContiguousTile(blockIdx.x, gridDim.x) : blockIdx.x / splits;
-    const int64_t part = splits == 1 ? 0 : blockIdx.x % splits;
+    // (a panel's parts as well: they read the same slice of x.)
+    const uint32_t place = XcdContiguousTile(blockIdx.x, gridDim.x);
+    const int64_t p = place / splits;
+    const int64_t part = place % splits;
     const int64_t c0 = p << kPanelLog;
     const int64_t cn = cols - c0 < kPanelCols ? cols - c0 : kPanelCols;
     const int64_t a = srcStart[p * B], e = srcStart[(p + 1) * B];
@@ -1269,8 +1271,7 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
     if (plan.liveValues == 0 || plan.transposed != 0 || a.vals == nullptr) {
         return OPSPARSE_E_INVALID;  // (this layout is the one with live values, for op(A) = A)
     }
-    // Few panels: several workgroups per panel, so that every CU has one.
-    const int32_t splits = l.P >= 192 ? 1 : (256 + l.P - 1) / l.P;
+    const int32_t splits = GatherSplits(l.P, a.nnz);
     // long rows: summed from the caller's own arrays (header[1] of them, counted by the analysis)
     const bool longRows = plan.numLongRows > 0;
     if (longRows && plan.liveValues != 0 && (a.vals == nullptr || a.colInd == nullptr)) {
@@ -1345,14 +1346,23 @@ using namespace opsparse::live_layout;
 
 extern "C" {
 
-size_t opsparse_spmv_csr_live_workspace_bytes(int64_t rows, int64_t cols, int64_t nnz)
-{
-    return static_cast<size_t>(MakeBlockedLayout(rows, cols, nnz).bytes);
-}
-
+// Room for this layout and, in the same buffer, for the ordered one with live values (spmv_blocked.hip), which
+// aclsparseSpMVPreprocess builds there where it applies.
 size_t opsparse_spmv_csr_live_resident_bytes(int64_t rows, int64_t cols, int64_t nnz)
 {
-    return static_cast<size_t>(MakeBlockedLayout(rows, cols, nnz).resident);
+    const BlockedLayout l = MakeBlockedLayout(rows, cols, nnz);
+    const size_t ordered = opsparse_spmv_csr_blocked_resident_bytes(rows, cols, nnz, OPSPARSE_BLOCKED_LIVE_VALUES);
+    const auto own = static_cast<size_t>(l.resident);
+    return l.P == 0 ? 0 : (own > ordered ? own : ordered);
+}
+
+size_t opsparse_spmv_csr_live_workspace_bytes(int64_t rows, int64_t cols, int64_t nnz)
+{
+    const BlockedLayout l = MakeBlockedLayout(rows, cols, nnz);
+    const size_t ordered = opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, OPSPARSE_BLOCKED_LIVE_VALUES) -
+                           opsparse_spmv_csr_blocked_resident_bytes(rows, cols, nnz, OPSPARSE_BLOCKED_LIVE_VALUES);
+    const auto own = static_cast<size_t>(l.bytes - l.resident);
+    return l.P == 0 ? 0 : opsparse_spmv_csr_live_resident_bytes(rows, cols, nnz) + (own > ordered ? own : ordered);
 }
 
 int opsparse_spmv_csr_live_analyse_split(const int32_t *rowOffsets, const int32_t *colInd, const void *csrValues,

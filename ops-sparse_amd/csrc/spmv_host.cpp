@@ -103,12 +103,12 @@ aclsparseStatus_t ValidateData(SpmvCall *c, aclDataType computeType)
 // CSR_ALG2 asks for one: the blocked-gather layout first, the column panels where that one does not fit the
 // matrix; both hold a copy of the values as they were at Preprocess.
 // ALG_DEFAULT / CSR_ALG1 get a layout with LIVE values (every call re-reads the caller's values, so nothing can go
-// stale) when the gathers of x are scattered: 0.35 ms against 1.1 ms for the merge path on an 8 M x 8 M power-law
-// matrix.  For op(A) = A and floating-point values that is the layout whose row blocks add with LDS atomics: these
-// algorithm values promise no bit-wise repeatable result (reference include/cann_ops_sparse.h:57-60, only CSR_ALG2
-// is "deterministic").  OPS_SPARSE_SPMV_REPEATABLE in the environment (read at every size query / Preprocess) asks
-// for the ordered layout there too: same bits from every call, about 0.5 ms on that matrix.  op(A) = A^T and
-// int32 values always get the ordered one.  GetBufferSize and Preprocess ask the same question of the same arrays
+// stale) when the gathers of x are scattered: 0.33 ms against 1.1 ms for the merge path on an 8 M x 8 M power-law
+// matrix.  Its rows are summed in an order that the layout fixes.  A matrix with a row that this layout refuses gets, for
+// op(A) = A and floating-point values, the one whose row blocks add with LDS atomics: these algorithm values promise no
+// bit-wise repeatable result (reference include/cann_ops_sparse.h:57-60, only CSR_ALG2 is "deterministic").
+// OPS_SPARSE_SPMV_REPEATABLE in the environment (read at every size query / Preprocess) rules that one out, and the
+// scatter layout of op(A) = A^T with it.  GetBufferSize and Preprocess ask the same question of the same arrays
 // (a sample of the column indices, one short kernel and a synchronisation), so they agree on the size.
 using Restored = opsparse::RestoredChoice;
 
@@ -277,11 +277,12 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
     // against 44 with the layout; 1.5 M x 4: 51 against 57; 2 M x 4: 87 against 71).  Tuning override, read at
     // every call: OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ.
     const char *minEnv = std::getenv("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ");
-    if (nnz < (minEnv != nullptr ? std::atoll(minEnv) : 7000000LL)) {
+    if (nnz < (minEnv != nullptr ? std::atoll(minEnv) : kMinDefaultNnz)) {
         return {0, 0, false};
     }
     // Results that may differ in the last bit between calls (the reference's ALG_DEFAULT / CSR_ALG1 of aclsparseSpMV)
-    // get the layout whose row blocks add with atomics, where there is one: op(A) = A, floating-point data.
+    // may fall back to the layout whose row blocks add with atomics, where there is one: op(A) = A, floating-point data.
+    // Its bytes are room for the ordered one, too.
     const bool atomics = !repeatable && !transpose && valueType != OPSPARSE_I32;
     const size_t bytes =
         atomics ? opsparse_spmv_csr_live_workspace_bytes(rows, cols, nnz)
@@ -289,13 +290,12 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
     if (bytes == 0) {
         return {0, 0, false};
     }
-    // The ordered layout reads the values through a window in LDS and is about half again as slow as the one with
-    // atomics: against the row-wise kernels on the caller's arrays it only wins where x is out of reach of the
-    // caches (x of 3 M elements: 363 us against 447 for 3 M rows of 12, 177 against 392 for 4000 rows of 8000; x of
-    // 2.2 M: 112 against 87 for 2 M rows of 4; x of 1 M and less: slower throughout).  (op(A) = A^T replaces atomics
-    // on y and keeps the bounds of AnalyseRestored.)
+    // Repeatable sums of fewer than 7 M entries (the bound above, whatever it was overridden with): the row-wise kernels'
+    // sums repeat as they are, and only an x out of reach of the caches makes them slower than the layout.  (op(A) = A^T
+    // replaces atomics on y and keeps the bounds of AnalyseRestored.)
     const char *minColsEnv = std::getenv("OPS_SPARSE_ORDERED_LIVE_MIN_COLS");  // tuning override, read at every call
-    if (!atomics && !transpose && cols < (minColsEnv != nullptr ? std::atoll(minColsEnv) : kMinColsOrderedLive)) {
+    const int64_t minCols = minColsEnv != nullptr ? std::atoll(minColsEnv) : nnz < kMinDefaultNnz ? kMinColsOrderedLive : 0;
+    if (!atomics && !transpose && cols < minCols) {
         return {0, 0, false};
     }
     // scattered gathers (op(A) = A^T: scattered updates of y)?  Not under stream capture (nothing may synchronise there) and not without a workspace.
@@ -364,7 +364,24 @@ int AnalyseRestored(int32_t kernel, const int32_t *rowOffsets, const int32_t *co
         return opsparse_spmv_csr_analyse(rowOffsets, rows, cols, nnz, buffer, bytes, OPSPARSE_SPMV_AUTO, plan, stream);
     }
     if (kernel == OPSPARSE_SPMV_BLOCKED_LIVE) {
+        // The layout whose rows are summed in order, in the same buffer: it has become the faster one (31 M entries
+        // over 4 M columns 159 us against 182 with atomics, 32 M over 1 M 113 against 132, 65 M over 8 M 335 against
+        // 339) and its results repeat.  The atomics one takes the matrices that it refuses: a row of more than 65 534
+        // entries that cannot go the long rows' way.
         const int32_t flags = BlockedFlags(false, true, valueType);
+        const size_t need = opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, flags);
+        const size_t keep = opsparse_spmv_csr_blocked_resident_bytes(rows, cols, nnz, flags);
+        int rc = OPSPARSE_E_UNSUPPORTED;
+        if (need > 0 && scratchBytes > 0 && keep <= bytes && need - keep <= scratchBytes) {
+            rc = opsparse_spmv_csr_blocked_analyse_split(rowOffsets, colInd, values, rows, cols, nnz, flags, buffer, bytes,
+                                                         scratch, scratchBytes, plan, stream);
+        } else if (need > 0 && scratchBytes == 0 && need <= bytes) {
+            rc = opsparse_spmv_csr_blocked_analyse(rowOffsets, colInd, values, rows, cols, nnz, flags, buffer, bytes, plan,
+                                                   stream);
+        }
+        if (rc != OPSPARSE_E_UNSUPPORTED) {
+            return rc;
+        }
         return scratchBytes > 0 ? opsparse_spmv_csr_live_analyse_split(rowOffsets, colInd, values, rows, cols, nnz, flags,
                                                                        buffer, bytes, scratch, scratchBytes, plan, stream)
                                 : opsparse_spmv_csr_live_analyse(rowOffsets, colInd, values, rows, cols, nnz, flags, buffer,

@@ -829,3 +829,86 @@ def test_buffer_holds_only_what_the_calls_keep_when_the_handle_lends_the_scratch
         run(state)                                             # the ordinary plan, inside the smaller buffer
     finally:
         L.aclsparseSetWorkspace(handle.h, None, 0)
+
+
+SIZES = {"small": (260_000, 300_000), "middle": (200_000, 9_830_400), "large": (200_000, 22_900_000)}
+
+
+@pytest.mark.parametrize("size", list(SIZES))
+@pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.float16, torch.float32),
+                                       (torch.float16, torch.float16), (torch.bfloat16, torch.float32),
+                                       (torch.bfloat16, torch.bfloat16), (torch.int32, torch.int32),
+                                       (torch.int32, torch.float32)])
+def test_every_size_of_the_windowed_row_blocks(osa, gpu_ctx, size, dtype, out):
+    """The windowed blocks come in three sizes by how many entries a (panel, block) chunk gets (10, 300 and 699 panels
+    here): blocks of up to 1024, 2048 and 4096 rows and 4096, 7168 and 14 336 entries a window.  Rows of 0 - 22 entries;
+    a run of empty rows longer than a block; rows of 5000 and 20 000 unsorted entries, which fill several windows; a row of
+    20 000 ascending ones (a long row).  Every type of values and of y."""
+    dev, stream, handle = gpu_ctx
+    rows, cols = SIZES[size]
+    rng = np.random.default_rng(len(size) + 3 * (dtype == torch.float16))
+    lengths = rng.integers(0, 23, rows)
+    lengths[5000:9500] = 0
+    lengths[[7, 1023, 1024, rows - 1]] = [5000, 20_000, 20_000, 5000]
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(0, cols, nnz).astype(np.int32)
+    colind[rowptr[1024]:rowptr[1025]].sort()
+    integer, int_sums = dtype == torch.int32, out == torch.int32
+    if integer:
+        big = 50_000 if int_sums else 2_000
+        val, x = rng.integers(-big, big, nnz).astype(np.int32), rng.integers(-big, big, cols).astype(np.int32)
+        y0 = rng.integers(-9, 9, rows).astype(np.int32) if int_sums else rng.uniform(-1, 1, rows).astype(np.float32)
+    else:
+        rnd = lambda a, t: torch.from_numpy(a.astype(np.float32)).to(t).float().numpy()
+        val, x = rnd(rng.uniform(-1, 1, nnz), dtype), rnd(rng.uniform(-1, 1, cols), dtype)
+        y0 = rnd(rng.uniform(-1, 1, rows), out)
+    dev_as = lambda a, t: to_dev(a, dev) if t == torch.int32 else to_dev(a, dev).to(t)
+    d_val, d_y = dev_as(val, dtype), dev_as(y0, out)
+    A = osa.Csr(rows, cols, to_dev(rowptr, dev), to_dev(colind, dev), d_val)
+    op = osa.SpmvOp(handle, A, osa.DnVec(dev_as(x, dtype)), osa.DnVec(d_y),
+                    compute_type=osa.ACL_INT32 if int_sums else osa.ACL_FLOAT)
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, nnz)
+    alpha, beta = (3, -2) if int_sums else (1.5, -0.5)
+    op(alpha, beta)
+    stream.synchronize()
+    if int_sums:
+        assert np.array_equal(d_y.cpu().numpy(), oracle.spmv_i32(rows, rowptr, colind, val, x, y0, alpha, beta))
+        return
+    gold = oracle.spmv_f64(rows, cols, rowptr, colind, val.astype(np.float32), x.astype(np.float32), y0, alpha, beta)
+    got = d_y.float().cpu().numpy()
+    if out == torch.float32:
+        assert oracle.max_rel_err(got, gold) <= 1e-5
+    else:  # the fp64 sum rounded once: half a unit in the last place
+        half_ulp = 2.0 ** -11 if out == torch.float16 else 2.0 ** -8
+        assert np.all(np.abs(got - gold) <= 1.001 * half_ulp * np.maximum(np.abs(gold), 2.0 ** -14))
+
+
+@pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.float16, torch.float32),
+                                       (torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16)])
+def test_default_plan_of_a_row_too_long_for_the_ordered_blocks(osa, gpu_ctx, dtype, out):
+    """A row of 70 000 entries whose columns do not ascend fits no ordered row block: the default plan then takes the
+    layout whose blocks are summed with atomics, in the same buffer."""
+    dev, stream, handle = gpu_ctx
+    rows, cols = 300_000, 1_400_000
+    rng = np.random.default_rng(51)
+    lengths = rng.integers(0, 20, rows)
+    lengths[123_456] = 70_000
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(0, cols, nnz).astype(np.int32)
+    rnd = lambda a, t: torch.from_numpy(a.astype(np.float32)).to(t).float().numpy()
+    val, x, y0 = rnd(rng.uniform(-1, 1, nnz), dtype), rnd(rng.uniform(-1, 1, cols), dtype), rnd(rng.uniform(-1, 1, rows), out)
+    d_y = to_dev(y0, dev).to(out)
+    A = osa.Csr(rows, cols, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev).to(dtype))
+    op = osa.SpmvOp(handle, A, osa.DnVec(to_dev(x, dev).to(dtype)), osa.DnVec(d_y))
+    assert op.buffer.numel() == osa.lib().opsparse_spmv_csr_live_workspace_bytes(rows, cols, nnz)
+    op(1.5, -0.5)
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, cols, rowptr, colind, val, x, y0, 1.5, -0.5)
+    got = d_y.float().cpu().numpy()
+    half_ulp = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[out]
+    if out == torch.float32:
+        assert oracle.max_rel_err(got, gold) <= 1e-5
+    else:
+        assert np.all(np.abs(got - gold) <= 1.001 * half_ulp * np.maximum(np.abs(gold), 2.0 ** -14))
