@@ -84,7 +84,13 @@ constexpr int32_t kStreamWindow = 65536;          // a block is also cut whereve
 constexpr int32_t kStreamMinWindow = 4096;        // (of this, where the matrix has few rows: MakeBlockedLayout)
 constexpr int64_t kStreamBlocksWanted = 8192;
 constexpr int64_t kStreamMinChunkEntries = 16;
-constexpr int64_t kStreamMaxRowPanelEntries = 16;
+constexpr int64_t kStreamMaxRowPanelEntries = 12;
+// Uneven rows: the mean length of an entry's row is this many times the mean row's, and such a row has half an entry or
+// more in a panel.  They meet themselves in the instructions of the stream: 4 M x 4 M power-law rows 155 us streamed,
+// 120 in windowed blocks, 300 K x 300 K ones 73 and 38; rows of 8 or 32 entries each 122 and 130, 106 and 113; 8 M
+// power-law rows with few long ones among them (a quarter of an entry in a panel) 251 and 302.
+constexpr double kStreamMaxUnevenness = 4.0;
+constexpr double kStreamUnevenRowPanelEntries = 0.5;
 constexpr int kStreamThreads = 64;                // a wavefront a workgroup: nothing is shared, nothing waits
 constexpr int kTurnThreads = 256;
 constexpr uint32_t kStreamPadRow = 0x7ffu;        // row field of a padding position (rows take 10 of its 11 bits)
@@ -897,6 +903,34 @@ __global__ __launch_bounds__(kTableThreads) void BlockedRowTablesKernel(const Bl
         if (last <= static_cast<uint32_t>(nRows) + 1) {
             ord[last] = kNoRow;  // the key of bit nB
         }
+    }
+}
+
+// sums[0] += the squared lengths, sums[1] += the lengths of the rows of fewer than `below` entries (zero before).
+__global__ __launch_bounds__(kBlockThreads) void RowSquaresKernel(const int32_t *__restrict__ rowOffsets, int64_t rows,
+                                                                  int32_t below, unsigned long long *__restrict__ sums)
+{
+    __shared__ unsigned long long part[2][kBlockThreads / kWave];
+    unsigned long long squares = 0, entries = 0;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+    for (int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; r < rows; r += stride) {
+        const int64_t n = rowOffsets[r + 1] - rowOffsets[r];
+        squares += n > 0 && n < below ? n * n : 0;
+        entries += n > 0 && n < below ? n : 0;
+    }
+    squares = GroupSum<kWave>(squares);
+    entries = GroupSum<kWave>(entries);
+    if (threadIdx.x % kWave == 0) {
+        part[0][threadIdx.x / kWave] = squares;
+        part[1][threadIdx.x / kWave] = entries;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned long long all = 0;
+        for (int w = 0; w < kBlockThreads / kWave; ++w) {
+            all += part[threadIdx.x][w];
+        }
+        atomicAdd(sums + threadIdx.x, all);
     }
 }
 
@@ -2016,7 +2050,10 @@ struct BlockedLayout {
 
 // Layout for a product with `rows` outputs and `cols` inputs (op(A) = A^T: the columns of A are the outputs).
 // 0 panels: the layout does not apply.
-BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool transposed, bool live, int32_t valueType)
+// `stream`: frozen values streamed, where their chunks are long enough for that (the analysis asks for one or the other
+// by how uneven the rows are).
+BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool transposed, bool live, int32_t valueType,
+                                bool stream)
 {
     BlockedLayout l{};
     if (rows <= 0 || cols <= 0 || nnz <= 0 || nnz > INT32_MAX || rows >= INT32_MAX || cols > INT32_MAX) {
@@ -2048,7 +2085,7 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
     // Values that the layout keeps (frozen values, either op(A)) are kept in block order and streamed by a wavefront
     // a block; values read where the caller has them need the windowed blocks, which read them in row order.
     const bool noStream = std::getenv("OPS_SPARSE_BLOCKED_NO_STREAM") != nullptr;  // tuning switch
-    l.streamed = !live && !noStream;
+    l.streamed = stream && !live && !noStream;
     if (l.streamed) {
         // Streamed blocks are cut by their rows; the entry cut is there for matrices of few, long rows, which would
         // otherwise make fewer blocks than the chip has wavefronts: about 8192 blocks of 4096 entries at least.
@@ -2060,7 +2097,7 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
         // block of 2^10 rows has a quarter of the entries of a windowed one: many panels and few entries a row
         // are the windowed blocks' case) and where a row does not put more than 16 entries into a panel on
         // average (such rows meet themselves in every instruction of the stream: 200 000 rows of 300 entries over
-        // 10 panels 326 us streamed, 247 us windowed; over 19 panels 234 against 254).
+        // 19 panels 228 us streamed, 202 us windowed; over 31 panels 200 either way).
         const int64_t blocks = ((rows + kStreamRows - 1) >> kStreamRowLog) + nnz / cut + 1;
         if (nnz / (P * blocks) < kStreamMinChunkEntries || nnz / rows / P > kStreamMaxRowPanelEntries) {
             l.streamed = false;
@@ -2244,7 +2281,7 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
         return OPSPARSE_E_UNSUPPORTED;
     }
     const bool transposed = plan.transposed != 0, live = plan.liveValues != 0;
-    const BlockedLayout l = MakeBlockedLayout(a.rows, a.cols, a.nnz, transposed, live, valType);
+    const BlockedLayout l = MakeBlockedLayout(a.rows, a.cols, a.nnz, transposed, live, valType, plan.streamedBlocks != 0);
     if (l.P == 0 || plan.numPanels != l.P || plan.numRowBlocks != l.B || plan.entryWindow != l.window) {
         return OPSPARSE_E_INVALID;
     }
@@ -2389,51 +2426,69 @@ using namespace opsparse;
 
 extern "C" {
 
-size_t opsparse_spmv_csr_blocked_workspace_bytes(int64_t rows, int64_t cols, int64_t nnz, int32_t flags)
+// Room for either form of the row blocks: which one frozen values get is for the analysis to say.
+static void BlockedBytes(int64_t rows, int64_t cols, int64_t nnz, int32_t flags, int64_t *resident, int64_t *scratch)
 {
     const bool t = (flags & OPSPARSE_BLOCKED_TRANSPOSE) != 0, live = (flags & OPSPARSE_BLOCKED_LIVE_VALUES) != 0;
     const int32_t vt = ValueTypeOfFlags(flags);
-    return static_cast<size_t>((t ? MakeBlockedLayout(cols, rows, nnz, true, live, vt)
-                                  : MakeBlockedLayout(rows, cols, nnz, false, live, vt)).bytes);
+    *resident = *scratch = 0;
+    for (const bool stream : {false, true}) {
+        const BlockedLayout l = MakeBlockedLayout(t ? cols : rows, t ? rows : cols, nnz, t, live, vt, stream);
+        *resident = l.resident > *resident ? l.resident : *resident;
+        *scratch = l.bytes - l.resident > *scratch ? l.bytes - l.resident : *scratch;
+    }
+}
+
+size_t opsparse_spmv_csr_blocked_workspace_bytes(int64_t rows, int64_t cols, int64_t nnz, int32_t flags)
+{
+    int64_t resident, scratch;
+    BlockedBytes(rows, cols, nnz, flags, &resident, &scratch);
+    return static_cast<size_t>(resident + scratch);
 }
 
 size_t opsparse_spmv_csr_blocked_resident_bytes(int64_t rows, int64_t cols, int64_t nnz, int32_t flags)
 {
-    const bool t = (flags & OPSPARSE_BLOCKED_TRANSPOSE) != 0, live = (flags & OPSPARSE_BLOCKED_LIVE_VALUES) != 0;
-    const int32_t vt = ValueTypeOfFlags(flags);
-    return static_cast<size_t>((t ? MakeBlockedLayout(cols, rows, nnz, true, live, vt)
-                                  : MakeBlockedLayout(rows, cols, nnz, false, live, vt)).resident);
+    int64_t resident, scratch;
+    BlockedBytes(rows, cols, nnz, flags, &resident, &scratch);
+    return static_cast<size_t>(resident);
 }
 
-int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int32_t *colInd, const void *csrValues,
-                                      int64_t rows, int64_t cols, int64_t nnz, int32_t flags, void *workspace,
-                                      size_t workspaceBytes, void *scratchSpace, size_t scratchBytes,
-                                      OpsparseSpmvPlan *plan, void *stream)
+// `unevenToWindows`: frozen values of uneven rows go into windowed blocks where both forms apply.
+static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, const void *csrValues, int64_t rows,
+                          int64_t cols, int64_t nnz, int32_t flags, void *workspace, size_t workspaceBytes,
+                          void *scratchSpace, size_t scratchBytes, bool unevenToWindows, OpsparseSpmvPlan *plan, void *stream)
 {
     if (plan == nullptr || rowOffsets == nullptr || colInd == nullptr || csrValues == nullptr) {
         return OPSPARSE_E_INVALID;
     }
+    const int32_t *callersOffsets = rowOffsets, *callersColumns = colInd;
+    const void *callersValues = csrValues;
     const bool transposed = (flags & OPSPARSE_BLOCKED_TRANSPOSE) != 0, live = (flags & OPSPARSE_BLOCKED_LIVE_VALUES) != 0;
     const int32_t valueType = ValueTypeOfFlags(flags);
     const int64_t outputs = transposed ? cols : rows, inputs = transposed ? rows : cols;
-    const BlockedLayout l = MakeBlockedLayout(outputs, inputs, nnz, transposed, live, valueType);
-    if (l.P == 0) {
+    // (where both forms apply they differ in what follows the transposed copy, which comes first in either)
+    const BlockedLayout windowed = MakeBlockedLayout(outputs, inputs, nnz, transposed, live, valueType, false);
+    const BlockedLayout streamed = MakeBlockedLayout(outputs, inputs, nnz, transposed, live, valueType, true);
+    if (streamed.P == 0 && windowed.P == 0) {
         return OPSPARSE_E_UNSUPPORTED;
     }
+    BlockedLayout l = streamed.P != 0 ? streamed : windowed;
+    int64_t resident, scratchNeed;
+    BlockedBytes(rows, cols, nnz, flags, &resident, &scratchNeed);
     // what the launches keep goes into `workspace`, what only the analysis needs into `scratchSpace`
-    if (workspace == nullptr || static_cast<int64_t>(workspaceBytes) < l.resident || scratchSpace == nullptr ||
-        static_cast<int64_t>(scratchBytes) < l.bytes - l.resident) {
+    if (workspace == nullptr || static_cast<int64_t>(workspaceBytes) < resident || scratchSpace == nullptr ||
+        static_cast<int64_t>(scratchBytes) < scratchNeed) {
         return OPSPARSE_E_WORKSPACE;
     }
     auto s = static_cast<hipStream_t>(stream);
     auto *residentBase = static_cast<unsigned char *>(workspace);
     auto *scratchBase = static_cast<unsigned char *>(scratchSpace);
-    const int64_t residentEnd = l.resident;
-    auto at = [&](int64_t off) { return off < residentEnd ? residentBase + off : scratchBase + (off - residentEnd); };
+    auto at = [&](int64_t off) { return off < l.resident ? residentBase + off : scratchBase + (off - l.resident); };
     auto ints = [&](int64_t off) { return reinterpret_cast<int32_t *>(at(off)); };
     int32_t *status = ints(0);
-    // status, number of long rows, their entries, entries of the largest block, long rows summed on their own
-    LaunchFillI32(status, 8, 0, s);
+    // status, number of long rows, their entries, entries of the largest block, long rows summed on their own, rows
+    // without entries, block numbers in use; [8]: the rows' lengths squared and summed, 64 bits
+    LaunchFillI32(status, 16, 0, s);
     if (transposed) {
         // The CSC arrays of A are the CSR arrays of A^T: from here on the matrix is that copy.
         hipLaunchKernelGGL(CheckColumnsKernel, dim3(GridOf(nnz, kBlockThreads, 16384)), dim3(kBlockThreads), 0, s, colInd,
@@ -2469,6 +2524,25 @@ int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int
         csrValues = at(l.cscValOff);  // (live values: filled at every call; the analysis reads no value then)
     }
     // From here on: `outputs` rows, `inputs` columns, the arrays rowOffsets / colInd / csrValues.
+    bool fallsBack = false;
+    if (l.streamed && windowed.P != 0 && unevenToWindows) {
+        hipLaunchKernelGGL(RowSquaresKernel, dim3(GridOf(outputs, kBlockThreads * 16, 2048)), dim3(kBlockThreads), 0, s,
+                           rowOffsets, outputs, l.longMinRow > 0 ? l.longMinRow : INT32_MAX,
+                           reinterpret_cast<unsigned long long *>(status + 8));
+        unsigned long long sums[2] = {0, 0};
+        if (hipMemcpyAsync(sums, status + 8, sizeof(sums), hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess) {
+            (void)hipGetLastError();
+            return OPSPARSE_E_LAUNCH;
+        }
+        const double entries = sums[1] > 0 ? static_cast<double>(sums[1]) : 1.0;
+        const double weighted = static_cast<double>(sums[0]) / entries;  // mean length of an entry's row
+        if (weighted > kStreamMaxUnevenness * entries / static_cast<double>(outputs) &&
+            weighted > kStreamUnevenRowPanelEntries * static_cast<double>(l.P)) {
+            l = windowed;
+            fallsBack = true;
+        }
+    }
     const bool frozenCopy = !live && !transposed;
     int32_t *keys[2] = {ints(l.keys0Off), ints(l.keys1Off)};
     int32_t *poss[2] = {ints(l.pos0Off), ints(l.pos1Off)};
@@ -2622,7 +2696,10 @@ int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int
         return OPSPARSE_E_LAUNCH;
     }
     if (!l.streamed && tail[0] > kMaxBlockEntries) {
-        return OPSPARSE_E_UNSUPPORTED;  // a row too long for a block's 16-bit slots that cannot go the long rows' way
+        // a row too long for a block's 16-bit slots that cannot go the long rows' way (the streamed blocks take it)
+        return fallsBack ? AnalyseBlocked(callersOffsets, callersColumns, callersValues, rows, cols, nnz, flags, workspace,
+                                          workspaceBytes, scratchSpace, scratchBytes, false, plan, stream)
+                         : OPSPARSE_E_UNSUPPORTED;
     }
     OpsparseSpmvPlan p{};
     p.kernel = OPSPARSE_SPMV_BLOCKED_GATHER;
@@ -2643,6 +2720,15 @@ int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int
     p.bytes = l.bytes;
     *plan = p;
     return OPSPARSE_OK;
+}
+
+int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int32_t *colInd, const void *csrValues,
+                                            int64_t rows, int64_t cols, int64_t nnz, int32_t flags, void *workspace,
+                                            size_t workspaceBytes, void *scratchSpace, size_t scratchBytes,
+                                            OpsparseSpmvPlan *plan, void *stream)
+{
+    return AnalyseBlocked(rowOffsets, colInd, csrValues, rows, cols, nnz, flags, workspace, workspaceBytes, scratchSpace,
+                          scratchBytes, true, plan, stream);
 }
 
 int opsparse_spmv_csr_blocked_analyse(const int32_t *rowOffsets, const int32_t *colInd, const void *csrValues,

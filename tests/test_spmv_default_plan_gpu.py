@@ -912,3 +912,51 @@ def test_default_plan_of_a_row_too_long_for_the_ordered_blocks(osa, gpu_ctx, dty
         assert oracle.max_rel_err(got, gold) <= 1e-5
     else:
         assert np.all(np.abs(got - gold) <= 1.001 * half_ulp * np.maximum(np.abs(gold), 2.0 ** -14))
+
+
+@pytest.mark.parametrize("rows_are,streamed", [("even", 1), ("uneven", 0), ("uneven with one too long for a window", 1)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_frozen_values_are_streamed_unless_the_rows_are_uneven(osa, gpu_ctx, rows_are, streamed, transposed):
+    """Frozen values, chunks long enough for either form of the row blocks: even rows are streamed by a wavefront a block,
+    uneven ones take the windowed blocks, and a row of 70 000 entries whose columns do not ascend, which fits no
+    window, the streamed ones after all.  (op(A) = A^T: the rows are those of the transpose.)"""
+    dev, stream, handle = gpu_ctx
+    L = osa.lib()
+    rows, cols = 300_000, 320_000
+    rng = np.random.default_rng(61)
+    lengths = np.full(rows, 9) if rows_are == "even" else rng.choice([1, 2, 3, 400], rows, p=[0.4, 0.3, 0.28, 0.02])
+    if rows_are.startswith("uneven with"):
+        lengths[77] = 70_000
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(0, cols, nnz).astype(np.int32)
+    val = rng.uniform(-1, 1, nnz).astype(np.float32)
+    if transposed:
+        # the matrix handed over is the transpose; its entries of a column ascend by row, so that the long row of the
+        # product has ascending columns and goes the long rows' way in either form
+        import scipy.sparse as sp
+        t = sp.csr_matrix((val, colind, rowptr), shape=(rows, cols)).tocsc()
+        d_arrays, shape = (t.indptr.astype(np.int32), t.indices.astype(np.int32), t.data), (cols, rows)
+        streamed = 0 if rows_are.startswith("uneven") else streamed
+    else:
+        d_arrays, shape = (rowptr, colind, val), (rows, cols)
+    d = [to_dev(np.ascontiguousarray(a), dev) for a in d_arrays]
+    x, y0 = rng.uniform(-1, 1, cols).astype(np.float32), rng.uniform(-1, 1, rows).astype(np.float32)
+    flags = osa.OPSPARSE_BLOCKED_TRANSPOSE if transposed else 0
+    need = L.opsparse_spmv_csr_blocked_workspace_bytes(*shape, nnz, flags)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    plan = osa.OpsparseSpmvPlan()
+    pv = lambda t: ctypes.c_void_p(t.data_ptr())
+    sp_ = ctypes.c_void_p(stream.cuda_stream)
+    assert L.opsparse_spmv_csr_blocked_analyse(pv(d[0]), pv(d[1]), pv(d[2]), *shape, nnz, flags, pv(ws), need,
+                                               ctypes.byref(plan), sp_) == 0
+    assert plan.streamedBlocks == streamed
+    d_x, d_y = to_dev(x, dev), to_dev(y0, dev)
+    scalar = lambda v: osa.OpsparseScalar(v, None, 0, 0)
+    assert L.opsparse_spmv_csr_launch(ctypes.byref(plan), int(transposed), pv(d[0]), pv(d[1]), pv(d[2]), pv(d_x), pv(d_y),
+                                      *shape, nnz, scalar(1.5), scalar(-0.5), osa.OPSPARSE_F32, osa.OPSPARSE_F32, 0, pv(ws),
+                                      need, sp_) == 0
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, cols, rowptr, colind, val, x, y0, 1.5, -0.5)
+    assert oracle.max_rel_err(d_y.cpu().numpy(), gold) <= 1e-5
