@@ -89,8 +89,8 @@ typedef OPSPARSE_ABI_ENUM(OpsparseSpmvKernel) {
                                       ACL_SPARSE_SPMV_ALG_DEFAULT; fp32 / fp16 / bf16, op(A) = A, values read where
                                       the caller has them at every call */
     OPSPARSE_SPMV_SCATTER_LIVE = 8  /* op(A) = A^T with y larger than an L2, the mirror image: pieces of the caller's
-                                      arrays multiplied by x[row] and written out sorted by output panel (2^14
-                                      columns) through LDS, then a workgroup a panel adds the products, kept exactly,
+                                      arrays multiplied by x[row] and written out sorted by output panel (256 of
+                                      them, or a multiple) through LDS, then a workgroup a panel adds the products, kept exactly,
                                       into fp64 sums in LDS with atomics.  26 bytes of traffic per entry, none on y;
                                       fp32 / fp16 / bf16, values read where the caller has them; like the reference's
                                       transposed kernel the last bit of a result may differ between two calls */
@@ -265,7 +265,8 @@ int opsparse_spmv_csr_live_analyse_split(const int32_t *rowOffsets, const int32_
  * SCATTER_LIVE analysis (op(A) = A^T; fp32, fp16 or bf16 values and x, values read in place at every launch): the
  * layout of the plan kernel OPSPARSE_SPMV_SCATTER_LIVE.  Takes the place of the atomics on y of the reference's
  * transposed kernel (sparse/spmv/arch22/kernels/spmv_kernel.cpp:21-55).  It looks at the structure only: no value is
- * read or kept.  Applies from 128 output panels of 2^14 columns on (more than 2 M columns) up to 2^25 columns;
+ * read or kept.  Applies from 2^18 columns on up to 2^25 columns (plan->numPanels counts them in
+ * units of 2^14);
  * OPSPARSE_E_UNSUPPORTED also for a column with more than 8192 entries (all its products would queue for one
  * address of LDS) and for a piece (16 384 consecutive entries of fp32 values, 32 768 of 16-bit ones) that spans more
  * than 65 535 rows: the ordered layout

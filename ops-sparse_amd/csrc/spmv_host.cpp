@@ -310,7 +310,9 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
     int32_t scattered = 0;
     if (opsparse_spmv_csr_gathers_scattered(rowOffsets, colInd, rows, cols, nnz, handle->workspace(),
                                             handle->workspaceBytes(), &scattered, handle->stream) != OPSPARSE_OK ||
-        scattered < kScatteredForLiveLayout) {
+        scattered < (transpose ? kScatteredForFrozenLayout : kScatteredForLiveLayout)) {
+        // (op(A) = A^T would send every far entry to y as an atomic, 20 G/s: 300 K x 300 K with 24 random columns a row,
+        // of which no more than 31 % can be far, 361 us that way)
         return {0, 0, false};
     }
     return {atomics ? OPSPARSE_SPMV_BLOCKED_LIVE : OPSPARSE_SPMV_BLOCKED_GATHER, bytes, true};
@@ -393,7 +395,7 @@ int AnalyseRestored(int32_t kernel, const int32_t *rowOffsets, const int32_t *co
         // the layout that sorts the products by output panel through LDS and needs no transposed copy (the 8 M x 8 M
         // power-law matrix: 0.3 ms a call against 1.4 ms), where the matrix is one for it.  Its buffer is smaller
         // than the ordered layout's, which the size query answered with; where it does not apply (a column with
-        // thousands of entries, fewer than 2 M columns) the ordered layout over the transposed copy follows.
+        // thousands of entries) the ordered layout over the transposed copy follows.
         const int32_t flags = BlockedFlags(false, true, valueType);
         const size_t need = opsparse_spmv_csr_scatter_workspace_bytes(rows, cols, nnz, flags);
         const size_t keep = opsparse_spmv_csr_scatter_resident_bytes(rows, cols, nnz, flags);

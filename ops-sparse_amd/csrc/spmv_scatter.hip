@@ -8,8 +8,8 @@
 //
 //   pass 1   a workgroup takes a PIECE of consecutive entries of the caller's arrays (128 KiB of products: 16 384
 //            entries of fp32 values, 32 768 of fp16 / bf16): values (as they are at this call) and, from the layout,
-//            each entry's row and its slot in the piece sorted by output panel (2^14 columns of A = 128 KiB of fp64
-//            sums).  It multiplies by x[row] - consecutive entries share rows, so these loads are as good as linear
+//            each entry's row and its slot in the piece sorted by output panel (at most 20 000 columns of A,
+//            156 KiB of fp64 sums; 256 panels, or a multiple, of equal width).  It multiplies by x[row] - consecutive entries share rows, so these loads are as good as linear
 //            - drops the product at its slot of a staging area in LDS, and writes the staging area out one (panel,
 //            piece) chunk at a time: the products arrive in memory sorted by panel, a panel's in the order of the
 //            caller's arrays.  A product is kept exactly: fp64 for fp32 operands, fp32 for 16-bit ones.
@@ -38,11 +38,13 @@ namespace opsparse {
 namespace scatter_layout {
 
 constexpr int kThreads = 1024;                  // one workgroup a compute unit: it owns 128 KiB of LDS and more
-constexpr int kOutLog = 14;                     // columns of A per output panel: 128 KiB of fp64 sums
-constexpr int kOutCols = 1 << kOutLog;
+constexpr int kPanelSlots = 256;                // pass 2 runs a workgroup a compute unit: the output panels are made a
+                                                // whole number of rounds of them
+constexpr int kMaxOutCols = 20000;              // columns of A per output panel at most: 156 KiB of fp64 sums
+constexpr int kKeyLog = 15;                     // bits of a local column in the sort keys
 constexpr int kStageBytes = 128 << 10;          // the products of a piece staged in LDS
-constexpr int kMaxPanels = 2048;                // the chunk tables of a piece in LDS: 16 KiB
-constexpr int64_t kMinPanels = 128;             // fewer output panels would leave compute units idle in pass 2
+constexpr int kMaxPanels = 3800;                // the chunk tables of a piece in LDS
+constexpr int64_t kMinPanels = 16;              // of 2^14 columns: below 2^18 columns the products go to y as atomics
 constexpr int64_t kMaxChunks = int64_t{1} << 26;  // panels x pieces: the chunk tables
 // A column with more entries than this is left to the ordered layout over the transposed copy, which sums such a
 // column as a long row: here all its products would queue for one address of LDS.
@@ -54,6 +56,8 @@ typedef unsigned short Ushort4 __attribute__((ext_vector_type(4)));
 
 struct ScatterLayout {
     int32_t P, Q;  // output panels, pieces (0 panels: the layout does not apply)
+    int32_t W;     // columns of an output panel
+    int32_t units; // 2^14-column units of y, in which the bounds are stated (plan.numPanels)
     int32_t piece;  // entries of a piece
     // what the launches use (the first `resident` bytes)
     int64_t metaOff;       // uint32 per entry: slot in the piece's panel order | (row - first row of the piece) << 16
@@ -95,14 +99,21 @@ ScatterLayout MakeLayout(int64_t rows, int64_t cols, int64_t nnz, int32_t valueT
     if (rows <= 0 || cols <= 0 || nnz <= 0 || nnz > INT32_MAX - 65536 || rows >= INT32_MAX || cols > (int64_t{1} << 25)) {
         return l;
     }
-    const int64_t P = (cols + kOutCols - 1) >> kOutLog;
+    // Panels of 2^14 columns made 306 workgroups of 5 M columns, two rounds of the chip for 1.2 rounds of work (pass 2
+    // 119 us, 83 with 256 panels), and left half of it idle below 2 M columns.
+    const int64_t rounds = (cols + kPanelSlots * kMaxOutCols - 1) / (kPanelSlots * kMaxOutCols);
+    const int64_t W = (cols + rounds * kPanelSlots - 1) / (rounds * kPanelSlots);
+    const int64_t P = (cols + W - 1) / W;
     const int pb = ProductBytes(valueType);
     const int64_t piece = kStageBytes / pb;
     const int64_t Q = (nnz + piece - 1) / piece;
-    if (P < MinPanels() || P > kMaxPanels || P * Q > kMaxChunks) {
+    const int64_t units = (cols + 16383) >> 14;
+    if (units < MinPanels() || P > kMaxPanels || P * Q > kMaxChunks) {
         return l;
     }
+    l.units = static_cast<int32_t>(units);
     l.P = static_cast<int32_t>(P);
+    l.W = static_cast<int32_t>(W);
     l.Q = static_cast<int32_t>(Q);
     l.piece = static_cast<int32_t>(piece);
     auto align = [](int64_t v) { return (v + 255) / 256 * 256; };
@@ -139,15 +150,19 @@ inline uint32_t GridOf(int64_t items, int64_t perBlock, int64_t cap)
 
 // ---------------------------------------------------------------------------------------------- analysis kernels
 
-// status[0] |= 1 for a column index outside [0, cols).
-__global__ __launch_bounds__(kBlockThreads) void ColumnRangeKernel(const int32_t *__restrict__ colInd, int64_t nnz, int64_t cols,
-                                                                   int32_t *__restrict__ status)
+// keys[i] = (output panel, column inside it) of entry i; status[0] |= 1 for a column index outside [0, cols).
+__global__ __launch_bounds__(kBlockThreads) void PanelKeysKernel(const int32_t *__restrict__ colInd, int64_t nnz, int64_t cols,
+                                                                 int32_t W, int32_t *__restrict__ keys,
+                                                                 int32_t *__restrict__ status)
 {
     const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
     bool bad = false;
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < nnz; i += stride) {
         const int32_t c = colInd[i];
-        bad = bad || c < 0 || c >= cols;
+        const bool out = c < 0 || c >= cols;
+        const int32_t p = out ? 0 : c / W;
+        keys[i] = out ? 0 : (p << kKeyLog) | (c - p * W);
+        bad = bad || out;
     }
     if (bad) {
         atomicOr(status, 1);
@@ -159,9 +174,9 @@ __global__ __launch_bounds__(kThreads) void ColumnMaxKernel(const uint16_t *__re
                                                             const int32_t *__restrict__ panelStart,
                                                             int32_t *__restrict__ status)
 {
-    __shared__ int32_t count[kOutCols];
+    __shared__ int32_t count[kMaxOutCols];
     const int t = threadIdx.x;
-    for (int32_t c = t; c < kOutCols; c += kThreads) {
+    for (int32_t c = t; c < kMaxOutCols; c += kThreads) {
         count[c] = 0;
     }
     __syncthreads();
@@ -171,7 +186,7 @@ __global__ __launch_bounds__(kThreads) void ColumnMaxKernel(const uint16_t *__re
     }
     __syncthreads();
     int32_t most = 0;
-    for (int32_t c = t; c < kOutCols; c += kThreads) {
+    for (int32_t c = t; c < kMaxOutCols; c += kThreads) {
         most = count[c] > most ? count[c] : most;
     }
     for (int off = kWave / 2; off > 0; off >>= 1) {
@@ -183,10 +198,10 @@ __global__ __launch_bounds__(kThreads) void ColumnMaxKernel(const uint16_t *__re
     }
 }
 
-// From the entries sorted by panel (key = column, payload = entry of the caller's arrays): the local column of every
+// From the entries sorted by panel (key = panel and local column, payload = entry of the caller's arrays): the local column of every
 // product, where every entry's product goes, and the number of entries of every (panel, piece) chunk.  A thread
 // takes eight consecutive sorted entries, which mostly share a chunk, and counts a run of them with one atomic.
-__global__ __launch_bounds__(kBlockThreads) void ChunkCountKernel(const int32_t *__restrict__ sortedCol,
+__global__ __launch_bounds__(kBlockThreads) void ChunkCountKernel(const int32_t *__restrict__ sortedKey,
                                                                   const int32_t *__restrict__ sortedEntry, int64_t nnz, int32_t Q,
                                                                   int32_t piece, uint16_t *__restrict__ colLocal,
                                                                   int32_t *__restrict__ dstOf, int32_t *__restrict__ count)
@@ -198,10 +213,10 @@ __global__ __launch_bounds__(kBlockThreads) void ChunkCountKernel(const int32_t 
         int32_t run = 0;
         for (int j = 0; j < kRun && s0 + j < nnz; ++j) {
             const int64_t s = s0 + j;
-            const int32_t c = sortedCol[s], i = sortedEntry[s];
-            colLocal[s] = static_cast<uint16_t>(c & (kOutCols - 1));
+            const int32_t c = sortedKey[s], i = sortedEntry[s];
+            colLocal[s] = static_cast<uint16_t>(c & ((1 << kKeyLog) - 1));
             dstOf[i] = static_cast<int32_t>(s);
-            const int64_t at = static_cast<int64_t>(c >> kOutLog) * Q + i / piece;
+            const int64_t at = static_cast<int64_t>(c >> kKeyLog) * Q + i / piece;
             if (at != chunk) {
                 if (run > 0) {
                     atomicAdd(count + chunk, run);
@@ -261,14 +276,14 @@ __global__ __launch_bounds__(kBlockThreads) void EntryMetaKernel(const int32_t *
                                                                  const int32_t *__restrict__ dstOf, const int32_t *__restrict__ chunkDst,
                                                                  const int32_t *__restrict__ pieceBase,
                                                                  const int32_t *__restrict__ pieceRow, int64_t nnz, int32_t P,
-                                                                 int32_t piece, uint32_t *__restrict__ meta,
+                                                                 int32_t W, int32_t piece, uint32_t *__restrict__ meta,
                                                                  int32_t *__restrict__ status)
 {
     const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
     bool wide = false;
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < nnz; i += stride) {
         const int64_t q = i / piece;
-        const int32_t p = colInd[i] >> kOutLog;
+        const int32_t p = colInd[i] / W;
         const int32_t slot = pieceBase[q * (P + 1) + p] + dstOf[i] - chunkDst[q * P + p];
         const int32_t rel = rowInd[i] - pieceRow[q];
         wide = wide || rel > 65535;
@@ -333,7 +348,7 @@ __global__ __launch_bounds__(kThreads) void ScatterProductsKernel(const ValT *__
     __shared__ int32_t base[kMaxPanels + 1];
     __shared__ int32_t dst[kMaxPanels];
     const int t = threadIdx.x;
-    const int wave = t / kWave, lane = t % kWave;
+    constexpr int kChunkLanes = 16;
     Uint4 m[kRounds];
     float v[kRounds][4];
     // values and slots of piece q into registers: every load is issued whatever the piece's length (those past its end
@@ -401,14 +416,12 @@ __global__ __launch_bounds__(kThreads) void ScatterProductsKernel(const ValT *__
         if (q + step < qEnd) {
             fetch(q + step);
         }
-        // a wavefront a chunk: the piece's products of one panel, contiguous in the staging area and in memory
-        // (four chunks at a time, their look-ups and LDS reads issued together, changed nothing: the kernel runs at
-        // the rate at which memory takes 256-byte pieces written to 512 places at once, 3.9 TB/s for reads and writes
-        // together, where the radix passes of the analysis, with 16 places, reach 2.6)
-        for (int32_t p = wave; p < P; p += kThreads / kWave) {
+        // kChunkLanes lanes a chunk: the piece's products of one panel, 32 or 64 on average, contiguous in the staging
+        // area and in memory (64 lanes a chunk: 166 us, 32 and 16: 155, on 39 M entries)
+        for (int32_t p = t / kChunkLanes; p < P; p += kThreads / kChunkLanes) {
             const int32_t s0 = base[p], s1 = base[p + 1];
             ProdT *out = inter + dst[p];
-            for (int32_t k = s0 + lane; k < s1; k += kWave) {
+            for (int32_t k = s0 + t % kChunkLanes; k < s1; k += kChunkLanes) {
                 out[k - s0] = stage[k];
             }
         }
@@ -420,13 +433,13 @@ __global__ __launch_bounds__(kThreads) void ScatterProductsKernel(const ValT *__
 template <typename OutT, typename ProdT>
 __global__ __launch_bounds__(kThreads) void ScatterSumKernel(const ProdT *__restrict__ inter, const uint16_t *__restrict__ colLocal,
                                                              const int32_t *__restrict__ panelStart, OutT *__restrict__ y,
-                                                             const OutT *__restrict__ yIn, int64_t cols, OpsparseScalar alphaS,
+                                                             const OutT *__restrict__ yIn, int64_t cols, int32_t W, OpsparseScalar alphaS,
                                                              OpsparseScalar betaS)
 {
-    __shared__ __align__(16) double acc[kOutCols];
+    extern __shared__ __align__(16) double acc[];  // W
     const int32_t p = blockIdx.x;
     const int t = threadIdx.x;
-    for (int32_t c = t; c < kOutCols; c += kThreads) {
+    for (int32_t c = t; c < W; c += kThreads) {
         acc[c] = 0.0;
     }
     __syncthreads();
@@ -461,8 +474,8 @@ __global__ __launch_bounds__(kThreads) void ScatterSumKernel(const ProdT *__rest
     }
     __syncthreads();
     const double alpha = ReadScalar<double>(alphaS), beta = ReadScalar<double>(betaS);
-    const int64_t c0 = static_cast<int64_t>(p) << kOutLog;
-    for (int32_t c = t; c < kOutCols && c0 + c < cols; c += kThreads) {
+    const int64_t c0 = static_cast<int64_t>(p) * W;
+    for (int32_t c = t; c < W && c0 + c < cols; c += kThreads) {
         double r = alpha * acc[c];
         if (beta != 0.0) {
             r += beta * ToAcc<double, OutT>(yIn[c0 + c]);
@@ -496,7 +509,7 @@ int Launch(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valType, int
         return OPSPARSE_E_UNSUPPORTED;  // y is fp32, or of the 16-bit type of the values
     }
     const ScatterLayout l = MakeLayout(a.rows, a.cols, a.nnz, valType);
-    if (l.P == 0 || plan.numPanels != l.P || plan.numRowBlocks != l.Q || plan.entryWindow != l.piece) {
+    if (l.P == 0 || plan.numPanels != l.units || plan.numRowBlocks != l.Q || plan.entryWindow != l.piece) {
         return OPSPARSE_E_INVALID;
     }
     if (a.ws == nullptr || static_cast<int64_t>(a.wsBytes) < l.resident || plan.bytes != l.bytes) {
@@ -521,9 +534,10 @@ int Launch(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valType, int
     auto sums = [&](auto outTag, auto prodTag) {
         using OutT = decltype(outTag);
         using ProdT = decltype(prodTag);
-        hipLaunchKernelGGL((ScatterSumKernel<OutT, ProdT>), dim3(static_cast<uint32_t>(l.P)), dim3(kThreads), 0, a.stream,
+        hipLaunchKernelGGL((ScatterSumKernel<OutT, ProdT>), dim3(static_cast<uint32_t>(l.P)), dim3(kThreads),
+                           static_cast<size_t>(l.W) * sizeof(double), a.stream,
                            static_cast<const ProdT *>(inter), colLocal, ints(l.panelStartOff), static_cast<OutT *>(a.y),
-                           static_cast<const OutT *>(a.yIn), a.cols, a.alpha, a.beta);
+                           static_cast<const OutT *>(a.yIn), a.cols, l.W, a.alpha, a.beta);
     };
     if (valType == OPSPARSE_F16) {
         products(Half{}, float{});
@@ -596,8 +610,8 @@ int opsparse_spmv_csr_scatter_analyse_split(const int32_t *rowOffsets, const int
 
     LaunchFillI32(status, 4, 0, s);
     LaunchFillI32(count, chunks + 1, 0, s);
-    hipLaunchKernelGGL(ColumnRangeKernel, dim3(GridOf(nnz, kBlockThreads, 16384)), dim3(kBlockThreads), 0, s, colInd, nnz, cols,
-                       status);
+    hipLaunchKernelGGL(PanelKeysKernel, dim3(GridOf(nnz, kBlockThreads, 16384)), dim3(kBlockThreads), 0, s, colInd, nnz, cols,
+                       l.W, keys[1], status);
     int32_t seen[2] = {0, 0};
     if (hipMemcpyAsync(seen, status, sizeof(seen), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
@@ -613,9 +627,9 @@ int opsparse_spmv_csr_scatter_analyse_split(const int32_t *rowOffsets, const int
         ++bits;
     }
     const int passes = bits == 0 ? 1 : (bits + 3) / 4;
-    const int32_t *keysIn = colInd, *payIn = nullptr;
+    const int32_t *keysIn = keys[1], *payIn = nullptr;
     for (int k = 0; k < passes; ++k) {
-        LaunchRadixPass(keysIn, payIn, keys[k & 1], pays[k & 1], nnz, 0, kOutLog + 4 * k, table, scan, s);
+        LaunchRadixPass(keysIn, payIn, keys[k & 1], pays[k & 1], nnz, 0, kKeyLog + 4 * k, table, scan, s);
         keysIn = keys[k & 1];
         payIn = pays[k & 1];
     }
@@ -630,7 +644,7 @@ int opsparse_spmv_csr_scatter_analyse_split(const int32_t *rowOffsets, const int
     hipLaunchKernelGGL(ColumnMaxKernel, dim3(static_cast<uint32_t>(l.P)), dim3(kThreads), 0, s, colLocal,
                        ints(l.panelStartOff), status);
     hipLaunchKernelGGL(EntryMetaKernel, dim3(GridOf(nnz, kBlockThreads, 16384)), dim3(kBlockThreads), 0, s, colInd, rowInd, dstOf,
-                       ints(l.chunkDstOff), ints(l.pieceBaseOff), ints(l.pieceRowOff), nnz, l.P, l.piece,
+                       ints(l.chunkDstOff), ints(l.pieceBaseOff), ints(l.pieceRowOff), nnz, l.P, l.W, l.piece,
                        reinterpret_cast<uint32_t *>(at(l.metaOff)), status);
     if (hipMemcpyAsync(seen, status, sizeof(seen), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess || CheckLaunch() != OPSPARSE_OK) {
@@ -647,7 +661,7 @@ int opsparse_spmv_csr_scatter_analyse_split(const int32_t *rowOffsets, const int
     p.kernel = OPSPARSE_SPMV_SCATTER_LIVE;
     p.rows = rows;
     p.nnz = nnz;
-    p.numPanels = l.P;
+    p.numPanels = l.units;
     p.numRowBlocks = l.Q;
     p.entryWindow = l.piece;
     p.transposed = 1;

@@ -231,3 +231,18 @@ def test_scatter_analysis_refusals(osa, gpu_ctx):
     assert analyse(rowptr, bad) == osa.OPSPARSE_E_INVALID
     assert analyse(*_matrix(rows, cols, 32, hot_column=9000)) == osa.OPSPARSE_E_UNSUPPORTED
     assert analyse(*_matrix(rows, cols, 33, empty_run=80_000)) == osa.OPSPARSE_E_UNSUPPORTED
+
+
+@pytest.mark.parametrize("cols", [300_000, 5_120_000, 5_120_001, 10_240_001])
+def test_output_panels_of_every_round_count(osa, gpu_ctx, cols):
+    """The output panels are 256, 512 or 768 of equal width, at most 20 000 columns: a few wide ones, the widest there are,
+    one column more (twice as many half as wide), three rounds; the last panel short."""
+    L = osa.lib()
+    rows = 1_400_000
+    rowptr, colind = _matrix(rows, cols, cols % 1000)
+    colind[-4:] = [cols - 1, 0, cols - 1, cols // 256]
+    st, buf, d, val, call, _ = _preprocess(osa, gpu_ctx, rowptr, colind, cols)
+    assert st == 0
+    scatter = L.opsparse_spmv_csr_scatter_workspace_bytes(rows, cols, colind.size, 0)
+    assert 0 < scatter < buf.numel() and _untouched_from(buf, scatter)
+    call(val, 1.5, -0.5)
