@@ -195,14 +195,18 @@ bool PrefersWholeRows(const aclsparseSpMatDescr *A, const OpsparseSpmmPlan &plan
     if ((rowBytes == 16 || rowBytes == 32) && plan.maxRowNnz <= 200) {
         return false;  // the kernel for a B of one or two 16-byte pieces a row takes these
     }
-    if (rowBytes > 512 || static_cast<double>(plan.maxRowNnz) > 4.0 * mean + 8.0) {
+    // (fp32, n = 256, local columns: 27-point mesh of 614 K rows 2142 / 936, band of 12 675 / 492, of 20 485 / 388; but
+    // 9-point 1229 / 1329)
+    const int64_t widest = elemBytes == 4 && mean >= 12.0 ? 1024 : 512;
+    if (rowBytes > widest || static_cast<double>(plan.maxRowNnz) > 4.0 * mean + 8.0) {
         return false;
     }
     if (elemBytes == 2) {
-        // fp16, whose slab kernel is the one tuned on c5, keeps the slabs except under local rows of 16 entries or
-        // more (us, slabs / rows: 27-point mesh n = 32 361 / 245, n = 64 459 / 399, n = 256 1401 / 1207; but 5-point
-        // n = 64 267 / 305, n = 128 508 / 614, 32 random columns a row n = 32 292 / 412)
-        if (mean < 16.0) {
+        // fp16 keeps the slabs, tuned on c5, except under local rows of 6 entries or more (us, slabs / rows, pipelined:
+        // 7-point mesh of 1.1 M rows n = 24 106 / 74, n = 32 110 / 84, n = 64 174 / 154, n = 256 641 / 597; 9-point
+        // n = 64 252 / 228; band of 12 n = 32 75 / 50, n = 128 176 / 184, n = 256 363 / 325; 32 random columns a row
+        // n = 32 292 / 412)
+        if (mean < 6.0) {
             return false;
         }
     } else {

@@ -46,6 +46,9 @@ constexpr int32_t kSegmentNnz = 256;  // entries per segment (128: c5 1.394 ms, 
 // under n = 16 / 32 / 64 instead of 107 / 181 / 431, a 27-point one 313 / 581 us under n = 32 / 64 instead of
 // 270 / 459; with one 107 / 212 / 508 and 274 / 492; random columns do not care.)
 constexpr int kSpmmRowsPerGroup = 2;
+// The same for the pipelined row kernel, at most (eight or 24: the same times within 3 %, but a 27-point mesh under
+// n = 128 804 us instead of 700).
+constexpr int32_t kPipelineTurns = 4;
 
 // Index of element (r, c) of a dense matrix with leading dimension ld.
 __device__ __forceinline__ int64_t DenseIndex(int64_t r, int64_t c, int64_t ld, bool colMajor)
@@ -268,6 +271,164 @@ __global__ __launch_bounds__(kBlockThreads) void SpmmRowSplitKernel(
                 *reinterpret_cast<CVec *>(out) = res;
             }
         }
+    }
+}
+
+// Rows of at most longRowNnz entries, one lane group per row, `turns` rows a group one after the other.
+// On a mesh or a band the rows of B come from the caches and what bounds the row kernel is the chain in front of a row's
+// sum - its bounds, its entries, its rows of B: on a 7-point mesh of 2 M rows under n = 32 a wavefront waited 70 % of its
+// time and the vector ALUs were busy 46 %.  So the chain is cut into three stages of
+// neighbouring turns: while the rows of B of turn i are on their way, the entries of turn i + 1 and the bounds of turn
+// i + 2 are asked for.  Their loads are unconditional (a position past the end re-reads an entry of the row, or of the
+// one in front of an empty row) and come after the gathers, so the wait for the gathers leaves them in flight.  The
+// offsets of the rows of B are worked out once an entry and travel through the lanes; all of a batch's shuffles stand
+// in front of its first load.
+template <typename ValT, typename CT, typename AccT, int V, int L, bool Small32>
+__global__ __launch_bounds__(kBlockThreads) void SpmmRowPipelineKernel(
+    const int32_t *__restrict__ rowOffsets, const int32_t *__restrict__ colInd, const ValT *__restrict__ vals,
+    const ValT *__restrict__ B, CT *__restrict__ C, int64_t rows, int32_t n, int64_t ldb, int64_t ldc,
+    int32_t longRowNnz, int32_t turns, OpsparseScalar alphaS, OpsparseScalar betaS, int32_t clampF16)
+{
+    typedef ValT BVec __attribute__((ext_vector_type(V)));
+    typedef CT CVec __attribute__((ext_vector_type(V), aligned(16)));
+    constexpr int kGroups = kBlockThreads / L;
+    constexpr int U = 8;                            // gathers of a lane in flight
+    constexpr int kPlaces = L < U ? U / L : 1;      // entries a lane holds of a chunk
+    constexpr int kEntries = kPlaces * L;           // entry j * L + lane of the chunk in place j
+
+    const AccT alpha = ReadScalar<AccT>(alphaS);
+    const AccT beta = ReadScalar<AccT>(betaS);
+    const bool betaZero = (beta == AccT(0));
+    const int32_t lane = threadIdx.x % L;
+    const int32_t group = threadIdx.x / L;
+    const uint32_t ldbBytes = static_cast<uint32_t>(ldb) * static_cast<uint32_t>(sizeof(ValT));
+    const int64_t first = static_cast<int64_t>(XcdContiguousTile(blockIdx.x, gridDim.x)) * turns * kGroups + group;
+
+    struct Bounds {
+        int32_t s, e;
+    };
+    struct Chunk {
+        uint32_t at[kPlaces];
+        ValT val[kPlaces];
+    };
+    // (a row past the end reads the last one's bounds; it is never summed or written)
+    auto loadBounds = [&](int64_t r) {
+        r = r < rows ? r : rows - 1;
+        return Bounds{rowOffsets[r], rowOffsets[r + 1]};
+    };
+    auto loadChunk = [&](int32_t p, int32_t e, Chunk &c) {
+        const int32_t lastAt = e > 0 ? e - 1 : 0;
+#pragma unroll
+        for (int j = 0; j < kPlaces; ++j) {
+            const int32_t mine = j * L + lane < e - p ? p + j * L + lane : lastAt;
+            c.at[j] = static_cast<uint32_t>(LoadStream(colInd + mine));
+            c.val[j] = LoadStream(vals + mine);
+        }
+    };
+
+    Bounds cur = loadBounds(first);
+    Chunk chunk;
+    loadChunk(cur.s, cur.e, chunk);
+    Bounds next = loadBounds(first + kGroups);
+    for (int32_t turn = 0; turn < turns; ++turn) {
+        const int64_t r = first + static_cast<int64_t>(turn) * kGroups;
+        const bool mine = r < rows && cur.e - cur.s <= longRowNnz;  // else past the end, or written by the segment kernels
+        const int32_t len = mine ? cur.e - cur.s : 0;
+        Chunk nextChunk;
+        Bounds nextButOne;
+        for (int32_t c0 = 0; c0 < n; c0 += L * V) {
+            const int32_t col = c0 + lane * V;
+            const bool active = col < n;
+            const int32_t colSafe = active ? col : 0;
+            const uint32_t colBytes = static_cast<uint32_t>(colSafe) * static_cast<uint32_t>(sizeof(ValT));
+            AccT acc[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                acc[i] = AccT(0);
+            }
+            // Adds entries [q0, q0 + U) of a chunk that holds cnt; `between` runs when their gathers have been issued.
+            auto addBatch = [&](const uint32_t (&at)[kPlaces], const float (&val)[kPlaces], int32_t q0, int32_t cnt,
+                                auto between) {
+                uint32_t to[U];
+                float v[U];
+                BVec b[U];
+#pragma unroll
+                for (int q = 0; q < U; ++q) {
+                    to[q] = __shfl(at[q / L], q0 + q % L, L);
+                    v[q] = __shfl(val[q / L], q0 + q % L, L);
+                }
+#pragma unroll
+                for (int q = 0; q < U; ++q) {
+                    if (q0 + q < cnt) {
+                        if constexpr (Small32) {
+                            b[q] = *reinterpret_cast<const BVec *>(reinterpret_cast<const char *>(B) + (to[q] + colBytes));
+                        } else {
+                            b[q] = *reinterpret_cast<const BVec *>(B + static_cast<int64_t>(to[q]) * ldb + colSafe);
+                        }
+                    }
+                }
+                between();
+#pragma unroll
+                for (int q = 0; q < U; ++q) {
+                    if (q0 + q < cnt) {
+                        const AccT vq = static_cast<AccT>(v[q]);
+#pragma unroll
+                        for (int i = 0; i < V; ++i) {
+                            acc[i] += vq * ToAcc<AccT>(b[q][i]);
+                        }
+                    }
+                }
+            };
+            uint32_t at[kPlaces];
+            float val[kPlaces];
+            auto unpack = [&](const Chunk &c) {
+#pragma unroll
+                for (int j = 0; j < kPlaces; ++j) {
+                    at[j] = Small32 ? c.at[j] * ldbBytes : c.at[j];
+                    val[j] = static_cast<float>(ToAcc<AccT>(c.val[j]));
+                }
+            };
+            unpack(chunk);
+            addBatch(at, val, 0, len, [&]() {
+                if (L < kWave || c0 == 0) {  // (below 64 lanes there is one tile of columns)
+                    loadChunk(next.s, next.e, nextChunk);
+                    nextButOne = loadBounds(r + 2 * kGroups);
+                }
+            });
+            for (int32_t q0 = U; q0 < (len < kEntries ? len : kEntries); q0 += U) {
+                addBatch(at, val, q0, len, []() {});
+            }
+            for (int32_t done = kEntries; done < len; done += kEntries) {
+                Chunk more;
+                loadChunk(cur.s + done, cur.e, more);
+                unpack(more);
+                const int32_t cnt = len - done < kEntries ? len - done : kEntries;
+                for (int32_t q0 = 0; q0 < cnt; q0 += U) {
+                    addBatch(at, val, q0, cnt, []() {});
+                }
+            }
+            if (active && mine) {
+                CT *out = C + r * ldc + col;
+                CVec res;
+                if (betaZero) {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) {
+                        res[i] = Epilogue<CT, AccT>::Apply(acc[i], alpha, beta, true, nullptr, clampF16 != 0);
+                    }
+                } else {
+                    const CVec old = *reinterpret_cast<const CVec *>(out);
+#pragma unroll
+                    for (int i = 0; i < V; ++i) {
+                        const CT o = old[i];
+                        res[i] = Epilogue<CT, AccT>::Apply(acc[i], alpha, beta, false, &o, clampF16 != 0);
+                    }
+                }
+                *reinterpret_cast<CVec *>(out) = res;
+            }
+        }
+        cur = next;
+        chunk = nextChunk;
+        next = nextButOne;
     }
 }
 
@@ -1437,6 +1598,52 @@ bool NoBinning()
 template <typename ValT, typename CT, typename AccT, int V, int L>
 void LaunchLongRows(const SpmmArgs &a);
 
+// B spans less than 4 GiB: the kernels address its rows by 32-bit byte offsets.
+bool Small32(const SpmmArgs &a, size_t elementBytes)
+{
+    return static_cast<uint64_t>(a.k) * static_cast<uint64_t>(a.ldb) * elementBytes < (1ull << 32);
+}
+
+// Whether the rows of an analysed matrix are worked by the pipelined kernel.  Two-byte elements: always, up to 32 lanes a
+// group (us, one row after the other / pipelined: 27-point mesh of 614 K rows, n = 32 155 / 132, n = 64 247 / 178, n = 256
+// 736 / 605; 7-point of 1.1 M rows 96 / 84, 174 / 154, 696 / 597; band of 20 57 / 46, 97 / 71, 307 / 255).  fp32, whose
+// other kernel keeps eight wavefronts on a SIMD where this one keeps five: rows of 16 entries on up to 8 lanes (27-point
+// n = 16 176 / 151, n = 32 165 / 153; 12 entries 66.4 / 66.7, 8 random ones 181 / 186), of 24 on 16 lanes (27-point
+// n = 64 263 / 249, 20 entries 105 / 111), and any on 32 (n = 128: 7-point 436 / 405, 9-point 659 / 580).
+template <typename ValT, int L>
+bool RowsArePipelined(const SpmmArgs &a)
+{
+    if (a.plan == nullptr || a.nnz <= 0 || a.rows <= 0 || L > 32) {
+        return false;
+    }
+    const int64_t shortest = sizeof(ValT) == 2 || L == 32 ? 0 : (L == 16 ? 24 : 16);
+    return a.nnz >= shortest * a.rows;
+}
+
+template <typename ValT, typename CT, typename AccT, int V, int L>
+int LaunchRowPipeline(const SpmmArgs &a, bool binned)
+{
+    constexpr int kGroups = kBlockThreads / L;
+    // Turns a workgroup: as many as leave the chip eight rounds of workgroups, up to kPipelineTurns.
+    const int64_t tiles = (a.rows + kGroups - 1) / kGroups;
+    const int64_t fill = tiles / (8 * 2048);
+    const int32_t turns = static_cast<int32_t>(fill < 1 ? 1 : (fill > kPipelineTurns ? kPipelineTurns : fill));
+    const uint32_t grid = static_cast<uint32_t>((tiles + turns - 1) / turns);
+    auto launch = [&](auto tag) {
+        constexpr bool kSmall = decltype(tag)::value;
+        hipLaunchKernelGGL((SpmmRowPipelineKernel<ValT, CT, AccT, V, L, kSmall>), dim3(grid), dim3(kBlockThreads), 0,
+                           a.stream, a.rowOffsets, a.colInd, static_cast<const ValT *>(a.vals),
+                           static_cast<const ValT *>(a.B), static_cast<CT *>(a.C), a.rows,
+                           static_cast<int32_t>(a.n), a.ldb, a.ldc, binned ? a.plan->longRowNnz : INT32_MAX, turns, a.alpha, a.beta, a.clampF16);
+    };
+    if (tiles > 0 && Small32(a, sizeof(ValT))) {
+        launch(std::true_type{});
+    } else if (tiles > 0) {
+        launch(std::false_type{});
+    }
+    return CheckLaunch();
+}
+
 template <typename ValT, typename CT, typename AccT, int V, int L>
 int LaunchRowSplit(const SpmmArgs &a)
 {
@@ -1445,7 +1652,17 @@ int LaunchRowSplit(const SpmmArgs &a)
     const int64_t rowsPerBlock = static_cast<int64_t>(kGroups) * kSpmmRowsPerGroup;
     const int64_t slots = a.rows;
     const uint32_t grid = static_cast<uint32_t>((slots + rowsPerBlock - 1) / rowsPerBlock);
-    if (slots > 0) {
+    bool pipelined = false;
+    if constexpr (std::is_same_v<AccT, double>) {
+        pipelined = RowsArePipelined<ValT, L>(a);
+        if (pipelined) {
+            const int rc = LaunchRowPipeline<ValT, CT, AccT, V, L>(a, binned);
+            if (rc != OPSPARSE_OK) {
+                return rc;
+            }
+        }
+    }
+    if (slots > 0 && !pipelined) {
         hipLaunchKernelGGL((SpmmRowSplitKernel<ValT, CT, AccT, V, L>), dim3(grid), dim3(kBlockThreads), 0, a.stream,
                            a.rowOffsets, a.colInd, static_cast<const ValT *>(a.vals),
                            static_cast<const ValT *>(a.B), static_cast<CT *>(a.C), slots, static_cast<int32_t>(a.n),
@@ -1510,7 +1727,7 @@ int LaunchSlab(const SpmmArgs &a)
         table ? reinterpret_cast<const int32_t *>(static_cast<unsigned char *>(a.ws) + a.plan->slabStartOff) : nullptr;
     const uint32_t grid = table ? static_cast<uint32_t>(a.plan->numSlabs) : static_cast<uint32_t>((a.rows + rps - 1) / rps);
     const int32_t longRowNnz = binned ? a.plan->longRowNnz : kSlabCap;
-    const bool small32 = static_cast<uint64_t>(a.k) * static_cast<uint64_t>(a.ldb) * sizeof(ValT) < (1ull << 32);
+    const bool small32 = Small32(a, sizeof(ValT));
     // Long rows: their segment workgroups ride in the same launch, the fix-up follows.
     constexpr int kGroups = kBlockThreads / L;
     // More columns than a lane group spans: one workgroup a (slab, tile of columns), the tiles of equal width (a

@@ -528,6 +528,61 @@ def test_kernel_choice_by_shape_and_width(osa, gpu_ctx, shape, n, monkeypatch):
     assert oracle.max_rel_err(got, gold) <= 1e-5
 
 
+def _banded(m, lengths, rng):
+    """Rows of the given lengths, their columns distinct and near the diagonal."""
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    row = np.repeat(np.arange(m), lengths)
+    place = np.arange(rowptr[-1]) - rowptr[row]
+    start = np.clip(np.arange(m) - 2 * lengths, 0, m - 4 * int(lengths.max()) - 4)
+    colind = start[row] + 4 * place + rng.integers(0, 4, rowptr[-1])
+    return rowptr, colind.astype(np.int32)
+
+
+@pytest.mark.parametrize("n,half", [(12, False), (16, False), (20, False), (32, False), (52, False), (64, False),
+                                    (100, False), (128, False), (256, False), (24, True), (40, True), (64, True),
+                                    (200, True), (256, True)])
+def test_pipelined_rows_of_every_length(osa, gpu_ctx, n, half):
+    """Local rows of 0 to 70 entries (first, last and a run of them empty; whole chunks, one entry more, one less; a
+    row count that leaves a tile unfinished) under every lane-group width, idle lanes among them.  The last entry of
+    some rows meets an infinite row of B, which their sums must show as an infinity: nothing past a row's end may be
+    added, not even multiplied by zero."""
+    rng = np.random.default_rng(n)
+    m = 5003
+    lengths = rng.integers(0, 71, m)
+    lengths[:3] = lengths[-2:] = lengths[700:790] = 0
+    lengths[10:16] = (8, 7, 9, 16, 32, 64)
+    rowptr, colind = _banded(m, lengths, rng)
+    val = rng.uniform(0.25, 1, colind.size).astype(np.float32)
+    B = rng.uniform(-1, 1, m * n).astype(np.float32)
+    if half:
+        val, B = (torch.from_numpy(a).to(torch.float16).float().numpy() for a in (val, B))
+    C0 = rng.uniform(-1, 1, m * n).astype(np.float32)
+    vd, cd = (torch.float16, torch.float32) if half else (None, None)
+    gold = oracle.spmm_f64(m, n, rowptr, colind, val, B, n, C0, n, 1.5, -0.5)
+    got = run_spmm(osa, gpu_ctx, m, m, n, rowptr, colind, val, B, n, C0, n, 1.5, -0.5, val_dtype=vd, c_dtype=cd)
+    assert oracle.max_rel_err(got, gold) <= 1e-5
+    target = colind[rowptr[14 + 1] - 1]
+    B.reshape(m, n)[target] = np.inf
+    meets = np.zeros(m, dtype=bool)
+    meets[np.repeat(np.arange(m), lengths)[colind == target]] = True
+    got = run_spmm(osa, gpu_ctx, m, m, n, rowptr, colind, val, B, n, C0, n, 1.5, 0.0, val_dtype=vd, c_dtype=cd)
+    assert meets[14] and np.all(np.isposinf(np.asarray(got, dtype=np.float64).reshape(m, n)[meets]))
+    assert np.all(np.isfinite(np.asarray(got, dtype=np.float64).reshape(m, n)[~meets]))
+
+
+def test_pipelined_rows_with_several_turns(osa, gpu_ctx):
+    """Enough rows of 128 columns that a lane group takes several, the last workgroup's last turns past the end."""
+    rng = np.random.default_rng(8)
+    m, n = 2 * 16384 * 8 + 13, 128
+    rowptr, colind = _banded(m, rng.integers(4, 10, m), rng)
+    val = rng.uniform(-1, 1, colind.size).astype(np.float32)
+    B = rng.uniform(-1, 1, m * n).astype(np.float32)
+    C0 = np.zeros(m * n, dtype=np.float32)
+    gold = oracle.spmm_f64(m, n, rowptr, colind, val, B, n, C0, n, 1.0, 0.0)
+    got = run_spmm(osa, gpu_ctx, m, m, n, rowptr, colind, val, B, n, C0, n, 1.0, 0.0)
+    assert oracle.max_rel_err(got, gold) <= 1e-5
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8])
 @pytest.mark.parametrize("b_rm,c_rm", [(True, True), (False, False), (True, False)])
 @pytest.mark.parametrize("half", [False, True])
