@@ -1959,7 +1959,13 @@ __global__ __launch_bounds__(kBlockThreads) void CooSampleKernel(const int32_t *
     const int32_t i = blockIdx.x * kBlockThreads + threadIdx.x;
     int32_t pairs = 0;
     if (i < samples) {
-        const uint32_t row = static_cast<uint32_t>(primary[static_cast<int64_t>(i) * n / samples]);
+        // one entry of every stretch, from a place of its own in each: entries in a periodic order (a long row at every
+        // other position, triples column by column) are seen as often as they are there
+        const int64_t first = static_cast<int64_t>(i) * n / samples, next = static_cast<int64_t>(i + 1) * n / samples;
+        uint32_t mix = static_cast<uint32_t>(i) * 0x85EBCA6Bu;
+        mix = (mix ^ (mix >> 15)) * 0xC2B2AE35u;
+        const int64_t place = static_cast<int64_t>(static_cast<uint64_t>(mix) * static_cast<uint64_t>(next - first) >> 32);
+        const uint32_t row = static_cast<uint32_t>(primary[first + place]);
         pairs = atomicAdd(counters + ((row * 0x9E3779B1u) >> (32 - bits)), 1);
     }
     __shared__ int32_t part[kBlockThreads / kWave];
@@ -2103,7 +2109,10 @@ int opsparse_coosort_launch(int64_t nnz, int32_t byRow, int32_t *cooRows, int32_
     // (two rows that share a counter look like one: as many pairs of theirs as the counters would give anyway come off)
     const double rowLength = (2.0 * r[4] / (static_cast<double>(kRowSamples) * kRowSamples) -
                               1.0 / static_cast<double>(int64_t{1} << sampleBits)) * static_cast<double>(nnz);
-    if (ask && rowLength <= kRowsFirstLongest && span < nnz && r[2] >= 0 && r[3] < INT32_MAX) {
+    // (nor can the rows be shorter than the entries over the rows' range, whatever the sample says: csrsort's scratch for
+    // short rows fits the passes' buffers, the one for a matrix of rows of thousands of entries would not)
+    const bool mayBeShort = static_cast<double>(nnz) <= kRowsFirstLongest * static_cast<double>(span);
+    if (ask && mayBeShort && rowLength <= kRowsFirstLongest && span < nnz && r[2] >= 0 && r[3] < INT32_MAX) {
         // Rows short enough for csrsort's registers: by row only, then every row by its secondary key in one pass over
         // the entries instead of one a digit.
         sortBy(primary, r[0], bitsP, secondary, perm, primary, secondary, perm);

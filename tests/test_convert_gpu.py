@@ -454,7 +454,8 @@ def test_coosort_signed_indices_custom_perm_and_sorted_input(osa, gpu_ctx, by_ro
     ((1 << 20) - 1, 60_000, 1 << 20, 0, "too few entries to ask"), (1 << 20, 60_000, 1 << 20, 7, "short rows"),
     ((1 << 20) + 5, 60_000, 3, 0, "short rows, repeated pairs"), (1_500_000, 60_000, 5000, -9, "short rows, base < 0"),
     (1_500_000, 9_000, 5000, 0, "rows beyond the bound"), (1_500_000, 60_000, 5000, 0, "one long row among short ones"),
-    (1_100_000, 1_500_000, 5000, 0, "fewer entries than rows"), (1_500_000, 60_000, 5000, 0, "negative secondary keys")])
+    (1_100_000, 1_500_000, 5000, 0, "fewer entries than rows"), (1_500_000, 60_000, 5000, 0, "negative secondary keys"),
+    (1 << 20, 60_000, 1 << 20, 0, "one row at every other place"), (1_200_000, 20_000, 60, 0, "column by column")])
 @pytest.mark.parametrize("by_row", [True, False])
 def test_coosort_by_short_rows_and_where_they_are_not(osa, gpu_ctx, nnz, m, n, least_row, what, by_row):
     """From 2^20 entries on a sample of the rows decides: one sort by row and csrsort inside the rows, or a pass for every
@@ -465,6 +466,10 @@ def test_coosort_by_short_rows_and_where_they_are_not(osa, gpu_ctx, nnz, m, n, l
         primary[rng.integers(0, nnz, 100_000)] = 77
     if what == "negative secondary keys":
         secondary -= 100
+    if what == "one row at every other place":
+        primary[1::2] = 77
+    if what == "column by column":
+        primary, secondary = np.arange(nnz) % m, np.arange(nnz) // m
     rows, cols = (primary, secondary) if by_row else (secondary, primary)
     run_coosort(osa, gpu_ctx, max(m, n), max(m, n), rows, cols, by_row,
                 perm=rng.permutation(nnz).astype(np.int32))
