@@ -2072,7 +2072,9 @@ int opsparse_coosort_launch(int64_t nnz, int32_t byRow, int32_t *cooRows, int32_
     const bool ask = nnz >= kRowsFirstMin;
     hipLaunchKernelGGL(CooRangeInitKernel, dim3(ask ? 1024 : 1), dim3(kBlockThreads), 0, s, range, keys[0],
                        ask ? 1 << sampleBits : 0);
-    hipLaunchKernelGGL(CooRangeKernel, dim3(GridFor(nnz, kBlockThreads * 16, 2048)), dim3(kBlockThreads), 0, s, primary,
+    // (two workgroups a compute unit keep memory busy, 5.8 TB/s; more of them cost their ends: 33.5 M entries 46 us with
+    // 512, 65 with 2048)
+    hipLaunchKernelGGL(CooRangeKernel, dim3(GridFor(nnz, kBlockThreads * 16, 512)), dim3(kBlockThreads), 0, s, primary,
                        secondary, nnz, range);
     if (ask) {
         hipLaunchKernelGGL(CooSampleKernel, dim3(kRowSamples / kBlockThreads), dim3(kBlockThreads), 0, s, primary, nnz,
