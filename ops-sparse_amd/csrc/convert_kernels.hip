@@ -2013,8 +2013,10 @@ CoosortLayout LayoutCoosort(int64_t nnz)
     l.keysB = off; off += Align256(4 * nnz);
     l.pairsA = off; off += Align256(8 * nnz);
     l.pairsB = off; off += Align256(8 * nnz);
-    l.table = off; off += Align256(4 * WideTableInts(nnz));
-    l.tiles = off; off += Align256(4 * ScanTiles(WideTableInts(nnz)));
+    const int64_t tableCount = WideTableInts(nnz);
+    l.table = off; off += Align256(4 * tableCount);
+    // (scanned are the table and, where the rows come first, the offsets of fewer than nnz rows: span + 1 <= nnz)
+    l.tiles = off; off += Align256(4 * ScanTiles(tableCount > nnz ? tableCount : nnz));
     l.bytes = off;
     return l;
 }

@@ -475,6 +475,35 @@ def test_coosort_by_short_rows_and_where_they_are_not(osa, gpu_ctx, nnz, m, n, l
                 perm=rng.permutation(nnz).astype(np.int32))
 
 
+@pytest.mark.parametrize("nnz,m", [(1 << 20, (1 << 20) - 1), ((1 << 20) + 3, 300_000), ((1 << 23) - 1, 7_000_000),
+                                   ((1 << 23) - 1, 2_700_000), (1 << 23, (1 << 23) - 1), ((1 << 23) + 5, 2_700_000),
+                                   ((1 << 23) + 5, 1_600_000), ((1 << 23) + 5, 1_150_000)])
+@pytest.mark.parametrize("by_row", [True, False])
+def test_coosort_of_short_rows_stays_inside_its_buffer(osa, gpu_ctx, nnz, m, by_row):
+    """One, three, five and seven entries a row, as many rows as there may be among them, either side of the entry counts
+    at which the sort's tables change their size: nothing behind the bytes that the size query asked for is written."""
+    dev, stream, handle = gpu_ctx
+    L = osa.lib()
+    rng = np.random.default_rng(nnz + m)
+    primary, secondary = rng.integers(0, m, nnz).astype(np.int32), rng.integers(0, 1 << 20, nnz).astype(np.int32)
+    primary[0], primary[-1] = m - 1, 0
+    rows, cols = (primary, secondary) if by_row else (secondary, primary)
+    perm = np.arange(nnz, dtype=np.int32)
+    d_r, d_c, d_p = dev_i32(rows, dev), dev_i32(cols, dev), dev_i32(perm, dev)
+    size = ctypes.c_size_t(0)
+    extent = max(m, 1 << 20)
+    assert L.aclsparseXcoosort_bufferSizeExt(handle.h, extent, extent, nnz, ptr(d_r), ptr(d_c), ctypes.byref(size)) == 0
+    guard = 1 << 16
+    buf = torch.full((size.value + guard,), 0x5A, dtype=torch.uint8, device=dev)
+    torch.cuda.synchronize()
+    fn = L.aclsparseXcoosortByRow if by_row else L.aclsparseXcoosortByColumn
+    assert fn(handle.h, extent, extent, nnz, ptr(d_r), ptr(d_c), ptr(d_p), ptr(buf)) == 0
+    stream.synchronize()
+    assert bool((buf[size.value:] == 0x5A).all())
+    for got, exp in zip((d_r, d_c, d_p), oracle.coosort(rows, cols, perm, by_row)):
+        assert np.array_equal(got.cpu().numpy(), exp)
+
+
 def test_coosort_then_coo2csr_is_csr2csc(osa, gpu_ctx):
     """Sorting a matrix's COO triples by column and compressing the column indices gives its CSC form: the same
     row indices, values (through P) and column offsets as aclsparseCsr2cscEx2's oracle."""

@@ -251,3 +251,13 @@ def test_measurement_launchers_refuse_bad_arguments(osa, L, ptr):
     assert L.opsparse_gather_launch(None, ptr, 4, None, None) == E_INVALID
     assert L.opsparse_gather_launch(ptr, None, 4, None, None) == E_INVALID
     assert L.opsparse_gather_launch(ptr, ptr, 0, None, None) == OK
+
+
+def test_coosort_buffer_has_room_for_the_offsets_scan_of_short_rows(L):
+    """coosort scans, besides its sort's table, the offsets of up to nnz - 1 rows; csr2csc's buffer for a matrix of nnz - 1
+    columns has room for the same scan, for a table of the same sort, and otherwise one array of nnz integers more and
+    256 bytes less."""
+    for nnz in (2, 100, 4095, (1 << 20) - 1, 1 << 20, 1_100_000, 4_194_304, (1 << 23) - 1, 1 << 23, 16_000_000,
+                20_963_328, 33_000_000, 400_000_000, (1 << 31) - 1):
+        array = (4 * nnz + 255) // 256 * 256
+        assert L.opsparse_coosort_workspace_bytes(nnz) - 256 + array >= L.opsparse_csr2csc_workspace_bytes(1, nnz - 1, nnz)
