@@ -1091,6 +1091,7 @@ __global__ __launch_bounds__(kBlockThreads) void SortShortRowsKernel(const int32
     }
     int64_t begin[R], len[R];
     int32_t col[R], pay[R];
+    uint32_t mids = 0, longs = 0;  // the group's rows for the lists
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int64_t row = row0 + r;
@@ -1104,13 +1105,8 @@ __global__ __launch_bounds__(kBlockThreads) void SortShortRowsKernel(const int32
             }
         }
         if (len[r] > G) {
-            if (g == 0) {
-                if (len[r] <= kSortWaveRow) {
-                    midList[atomicAdd(counters, 1)] = static_cast<int32_t>(row);
-                } else {
-                    longList[atomicAdd(counters + 1, 1)] = static_cast<int32_t>(row);
-                }
-            }
+            mids |= len[r] <= kSortWaveRow && g == 0 ? 1u << r : 0u;
+            longs |= len[r] > kSortWaveRow && g == 0 ? 1u << r : 0u;
             len[r] = 0;
         }
         col[r] = 0;
@@ -1127,6 +1123,35 @@ __global__ __launch_bounds__(kBlockThreads) void SortShortRowsKernel(const int32
         if (g < len[r]) {
             colInd[begin[r] + g] = col[r];
             perm[begin[r] + g] = pay[r];
+        }
+    }
+    // The listed rows of a workgroup take their places with one addition a list.  An addition a row, to the same two words,
+    // was served one after the other, 10 ns each: with 4.4 random entries a row, of which 4 % of the rows do not fit eight
+    // lanes, coosort of 33 M entries took 4257 us, 1552 now (2780 by the passes over both keys); equal rows as before.
+    __shared__ int32_t count[2], first[2];
+    if (threadIdx.x < 2) {
+        count[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    int32_t at[2] = {0, 0};
+    if (mids != 0) {
+        at[0] = atomicAdd(&count[0], __popc(mids));
+    }
+    if (longs != 0) {
+        at[1] = atomicAdd(&count[1], __popc(longs));
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 && count[threadIdx.x] > 0) {
+        first[threadIdx.x] = atomicAdd(counters + threadIdx.x, count[threadIdx.x]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if ((mids >> r & 1u) != 0) {
+            midList[first[0] + at[0]++] = static_cast<int32_t>(row0 + r);
+        }
+        if ((longs >> r & 1u) != 0) {
+            longList[first[1] + at[1]++] = static_cast<int32_t>(row0 + r);
         }
     }
 }

@@ -295,6 +295,23 @@ def test_csrsort_short_rows_every_group_size_and_key_width(osa, gpu_ctx, mean, n
     run_csrsort(osa, gpu_ctx, m, n, rowptr + base, colind + base, base=base)
 
 
+@pytest.mark.parametrize("base", [0, 1])
+def test_csrsort_lists_filled_by_whole_workgroups(osa, gpu_ctx, base):
+    """Rows of a few entries on average, so that a row gets eight lanes, with runs of rows too long for them: every row of
+    several workgroups on one list, on the other, on either in turn, one row of a workgroup, its first and its last."""
+    rng = np.random.default_rng(17)
+    m, n = 300_000, 50_000
+    lengths = rng.integers(0, 5, m)
+    lengths[256:1024] = 20                                   # (a workgroup takes 256 rows)
+    lengths[2048:2304] = 70
+    lengths[4096:4608:2], lengths[4097:4608:2] = 9, 65
+    lengths[[8192, 8703, 9000, m - 1]] = [9, 64, 65, 3000]
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    assert 2 * int(rowptr[-1]) // m <= 8
+    colind = rng.integers(0, n, int(rowptr[-1])).astype(np.int32)
+    run_csrsort(osa, gpu_ctx, m, n, rowptr + base, colind + base, base=base)
+
+
 def test_csrsort_many_rows(osa, gpu_ctx):
     """A million short rows (one wavefront each) with a power-law tail."""
     rng = np.random.default_rng(9)
