@@ -111,6 +111,14 @@ constexpr int64_t kLongChunkMeanFrozen = 4;
 constexpr int64_t kLongMinRowFrozen = 1024;
 constexpr int kLongLanes = 16;        // lanes that sum one (long row, panel) piece in phase 1
 constexpr int32_t kInBlockLongRows = 64;          // long rows a row block's own workgroup adds up at most
+// Live values: pieces of at least this many entries that are also longer than this many lane groups' shares of the
+// workgroup's long entries are added up by the whole workgroup.  A group takes 64 entries a round trip to memory, and the
+// hub of a graph has thousands in a panel where there are few panels: 400 K x 400 K power-law rows, 24 entries a row, the
+// longest 100 000, 105 us a call, 64 with it (77 by the merge path); 1 M x 1 M, 8.6 M entries, 96 and 63.  With four
+// shares instead of six, 1.3 M x 1.3 M and 24 entries a row 159 us, 155 by groups alone.
+constexpr int32_t kBigPiece = 2048;
+constexpr int32_t kBigPieceShares = 6;
+constexpr int32_t kMaxBigPieces = kBlkThreads / kLongLanes / kBigPieceShares + 1;
 constexpr int kLongTile = 3072;                   // long rows a phase-1 workgroup has in LDS at a time
 
 typedef float Float4 __attribute__((ext_vector_type(4)));
@@ -1340,14 +1348,74 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
     const int32_t gl = tid / kLongLanes, gt = tid % kLongLanes;
     const int32_t base = static_cast<int32_t>(c0);
     const int32_t *loTab = longChunk + p * maxLong, *hiTab = longChunk + (p + 1) * maxLong;
+    __shared__ int32_t waveEntries[kBlkThreads / kWave], bigPiece[kMaxBigPieces], numBigSeen;
+    __shared__ uint64_t waveSum[2][kBlkThreads / kWave];
     for (int32_t t0 = 0; t0 < numLong; t0 += kLongTile) {
         const int32_t tn = numLong - t0 < kLongTile ? numLong - t0 : kLongTile;
         __syncthreads();  // (the tile before is done with)
+        int32_t entries = 0;  // of the pieces of this thread that are the workgroup's
+        bool long1 = false;
         for (int32_t i = tid; i < tn; i += kBlkThreads) {
-            pieceLo[i] = loTab[t0 + i];
-            pieceHi[i] = hiTab[t0 + i];
+            const int32_t lo1 = loTab[t0 + i], hi1 = hiTab[t0 + i];
+            pieceLo[i] = lo1;
+            pieceHi[i] = hi1;
+            if (i % static_cast<int32_t>(splits) == static_cast<int32_t>(part)) {
+                entries += hi1 - lo1;
+                long1 = long1 || hi1 - lo1 >= kBigPiece;
+            }
         }
-        __syncthreads();
+        if (tid == 0) {
+            numBigSeen = 0;
+        }
+        int32_t numBig = 0;
+        if (__syncthreads_or(long1 ? 1 : 0) != 0) {
+            // Pieces that would keep their group busy long after the others are done (a hub of a graph over few panels)
+            // are taken out of the groups' turns: the whole workgroup adds them up, one after the other.
+            entries = GroupSum<kWave>(entries);
+            if (lane == 0) {
+                waveEntries[wave] = entries;
+            }
+            __syncthreads();
+            int64_t all = 0;
+            for (int w = 0; w < kBlkThreads / kWave; ++w) {
+                all += waveEntries[w];
+            }
+            const int64_t share = kBigPieceShares * all / kGroups;  // (so at most kMaxBigPieces are longer)
+            for (int32_t i = tid; i < tn; i += kBlkThreads) {
+                const int32_t len = pieceHi[i] - pieceLo[i];
+                if (i % static_cast<int32_t>(splits) == static_cast<int32_t>(part) && len >= kBigPiece && len > share) {
+                    bigPiece[atomicAdd(&numBigSeen, 1)] = i;
+                    pieceLo[i] = pieceHi[i] = -1;
+                }
+            }
+            __syncthreads();
+            numBig = numBigSeen;
+        }
+        // Group q of a piece [i0, i1) holds its entries 4 q .. 4 q + 3; the last group may be short.  A request
+        // is always four whole entries: it starts at most at i1 - 4 (never below 0), so the last group reads a
+        // few entries in front of its own, and a group past the end re-reads the last one; `add` takes only the
+        // entries that are the group's own.  No entry is ever fetched one by one.
+        auto request = [&](int32_t i0, int32_t i1, int32_t q, Int4U *c, Uint4 *v) {
+            int64_t at = i0 + 4 * static_cast<int64_t>(q);
+            at = at + 4 <= i1 ? at : static_cast<int64_t>(i1) - 4;
+            at = at < 0 ? 0 : at;
+            *c = __builtin_nontemporal_load(reinterpret_cast<const Int4U *>(colInd + at));
+            *v = LoadFourRaw(vals + at);
+        };
+        auto add = [&](int32_t i0, int32_t i1, int32_t q, const Int4U &c, const Uint4 &v, AccT *sum) {
+            const int64_t own = i0 + 4 * static_cast<int64_t>(q);  // first entry of the group
+            int64_t at = own + 4 <= i1 ? own : static_cast<int64_t>(i1) - 4;
+            at = at < 0 ? 0 : at;
+            const uint32_t mask = kPanelCols - 1;  // an entry of the group is in the panel by construction
+            const int32_t cs[4] = {c.x, c.y, c.z, c.w};
+            const uint32_t vs[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const AccT t = RawToAcc<AccT, kIntData>(vs[j]) *
+                               RawToAcc<AccT, kIntData>(xs[static_cast<uint32_t>(cs[j] - base) & mask]);
+                *sum += (at + j >= own && at + j < i1) ? t : AccT(0);
+            }
+        };
         // Groups of kLongLanes lanes take the rows of the tile in turn (a part of them when a panel has several
         // workgroups), each lane 16 bytes of either array per request.  Most pieces are a request or two long, so
         // what a group waits for is the round trip of each piece: the first request of the group's next piece is
@@ -1355,31 +1423,6 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
         const int32_t stride = static_cast<int32_t>(splits) * kGroups;
         int32_t k = static_cast<int32_t>(part) + static_cast<int32_t>(splits) * gl;
         if (k < tn) {
-            // Group q of a piece [i0, i1) holds its entries 4 q .. 4 q + 3; the last group may be short.  A request
-            // is always four whole entries: it starts at most at i1 - 4 (never below 0), so the last group reads a
-            // few entries in front of its own, and a group past the end re-reads the last one; `add` takes only the
-            // entries that are the group's own.  No entry is ever fetched one by one.
-            auto request = [&](int32_t i0, int32_t i1, int32_t q, Int4U *c, Uint4 *v) {
-                int64_t at = i0 + 4 * static_cast<int64_t>(q);
-                at = at + 4 <= i1 ? at : static_cast<int64_t>(i1) - 4;
-                at = at < 0 ? 0 : at;
-                *c = __builtin_nontemporal_load(reinterpret_cast<const Int4U *>(colInd + at));
-                *v = LoadFourRaw(vals + at);
-            };
-            auto add = [&](int32_t i0, int32_t i1, int32_t q, const Int4U &c, const Uint4 &v, AccT *sum) {
-                const int64_t own = i0 + 4 * static_cast<int64_t>(q);  // first entry of the group
-                int64_t at = own + 4 <= i1 ? own : static_cast<int64_t>(i1) - 4;
-                at = at < 0 ? 0 : at;
-                const uint32_t mask = kPanelCols - 1;  // an entry of the group is in the panel by construction
-                const int32_t cs[4] = {c.x, c.y, c.z, c.w};
-                const uint32_t vs[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const AccT t = RawToAcc<AccT, kIntData>(vs[j]) *
-                                   RawToAcc<AccT, kIntData>(xs[static_cast<uint32_t>(cs[j] - base) & mask]);
-                    *sum += (at + j >= own && at + j < i1) ? t : AccT(0);
-                }
-            };
             int32_t i0 = pieceLo[k], i1 = pieceHi[k];
             Int4U cFirst;
             Uint4 vFirst;
@@ -1407,7 +1450,7 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
                 for (int off = kLongLanes / 2; off > 0; off >>= 1) {
                     sum += __shfl_xor(sum, off, kLongLanes);
                 }
-                if (gt == 0) {
+                if (gt == 0 && i0 >= 0) {  // (i0 < 0: a piece for the whole workgroup)
                     longPartial[static_cast<int64_t>(t0 + k) * P + p] = AccToSlot(sum);
                 }
                 if (kn >= tn) {
@@ -1418,6 +1461,32 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
                 i1 = j1;
                 cFirst = cAhead;
                 vFirst = vAhead;
+            }
+        }
+        for (int32_t b = 0; b < numBig; ++b) {
+            const int32_t k1 = bigPiece[b];
+            const int32_t i0 = loTab[t0 + k1], i1 = hiTab[t0 + k1];
+            const int32_t n4 = (i1 - i0 + 3) >> 2;
+            AccT sum = AccT(0);
+            for (int32_t q = tid; q < n4; q += 2 * kBlkThreads) {
+                Int4U c[2];
+                Uint4 v[2];
+                request(i0, i1, q, &c[0], &v[0]);
+                request(i0, i1, q + kBlkThreads, &c[1], &v[1]);
+                add(i0, i1, q, c[0], v[0], &sum);
+                add(i0, i1, q + kBlkThreads, c[1], v[1], &sum);
+            }
+            sum = GroupSum<kWave>(sum);
+            if (lane == 0) {
+                waveSum[b & 1][wave] = AccToSlot(sum);
+            }
+            __syncthreads();  // (the other half of waveSum is written next: read before this barrier)
+            if (tid == 0) {
+                AccT all = AccT(0);
+                for (int w = 0; w < kBlkThreads / kWave; ++w) {
+                    all += SlotToAcc<AccT>(waveSum[b & 1][w]);
+                }
+                longPartial[static_cast<int64_t>(t0 + k1) * P + p] = AccToSlot(all);
             }
         }
     }

@@ -960,3 +960,53 @@ def test_frozen_values_are_streamed_unless_the_rows_are_uneven(osa, gpu_ctx, row
     stream.synchronize()
     gold = oracle.spmv_f64(rows, cols, rowptr, colind, val, x, y0, 1.5, -0.5)
     assert oracle.max_rel_err(d_y.cpu().numpy(), gold) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype,out", [(torch.float32, torch.float32), (torch.float16, torch.float32),
+                                       (torch.bfloat16, torch.bfloat16), (torch.int32, torch.int32)])
+def test_hubs_over_few_panels_are_summed_by_whole_workgroups(osa, gpu_ctx, dtype, out):
+    """Rows whose part of a panel is much longer than the other long rows': over all ten panels, inside one panel, the rest
+    of a division by four at every end; forty of them, more than one workgroup's share, beside 300 ordinary long rows.
+    The same bits at every call."""
+    dev, stream, handle = gpu_ctx
+    rows, cols = 200_000, 300_000
+    rng = np.random.default_rng(71)
+    lengths = rng.integers(0, 12, rows)
+    ordinary = rng.choice(np.arange(1000, rows), 300, replace=False)
+    lengths[ordinary] = rng.integers(2000, 4000, 300)
+    hubs = np.array([0, 1, 500, 501, 502, 503] + list(range(600, 634)) + [rows - 1])
+    lengths[hubs] = 30_000 + np.arange(hubs.size)
+    lengths[[0, 1, rows - 1]] = [100_001, 60_002, 50_003]
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(0, cols, nnz).astype(np.int32)
+    colind[rowptr[rows - 1]:] = rng.integers(40_000, 65_000, 50_003)
+    for r in np.concatenate([hubs, ordinary]):
+        colind[rowptr[r]:rowptr[r + 1]].sort()
+    if dtype == torch.int32:
+        val, x, y0 = (rng.integers(-50_000, 50_000, n).astype(np.int32) for n in (nnz, cols, rows))
+        dev_as, alpha, beta = lambda a, t: to_dev(a, dev), 3, -2
+    else:
+        rnd = lambda n, t: torch.from_numpy(rng.uniform(-1, 1, n).astype(np.float32)).to(t).float().numpy()
+        val, x, y0 = rnd(nnz, dtype), rnd(cols, dtype), rnd(rows, out)
+        dev_as, alpha, beta = lambda a, t: to_dev(a, dev).to(t), 1.5, -0.5
+    d_y = dev_as(y0, out)
+    A = osa.Csr(rows, cols, to_dev(rowptr, dev), to_dev(colind, dev), dev_as(val, dtype))
+    op = osa.SpmvOp(handle, A, osa.DnVec(dev_as(x, dtype)), osa.DnVec(d_y),
+                    compute_type=osa.ACL_INT32 if dtype == torch.int32 else osa.ACL_FLOAT)
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, nnz)
+    got = []
+    for _ in range(3):
+        d_y.copy_(dev_as(y0, out))
+        op(alpha, beta)
+        stream.synchronize()
+        got.append(d_y.cpu())
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    if dtype == torch.int32:
+        assert np.array_equal(got[0].numpy(), oracle.spmv_i32(rows, rowptr, colind, val, x, y0, alpha, beta))
+        return
+    gold = oracle.spmv_f64(rows, cols, rowptr, colind, val, x, y0, alpha, beta)
+    if out == torch.float32:
+        assert oracle.max_rel_err(got[0].numpy(), gold) <= 1e-5
+    else:  # the fp64 sum rounded once: half a unit in the last place
+        assert np.all(np.abs(got[0].float().numpy() - gold) <= 1.001 * 2.0 ** -8 * np.maximum(np.abs(gold), 2.0 ** -14))
