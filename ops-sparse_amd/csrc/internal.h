@@ -159,6 +159,8 @@ constexpr int32_t kScatteredForLiveLayout = 310;
 // fewer entries would where the sums have to repeat.
 constexpr int64_t kMinDefaultNnz = 7000000;
 constexpr int64_t kMinColsOrderedLive = int64_t{5} << 19;  // 2.6 M
+// The same for rows of fewer than six entries, whatever their number.
+constexpr int64_t kMinColsOrderedShortRows = int64_t{7} << 17;  // 0.9 M
 
 struct RestoredChoice {
     int32_t kernel;

@@ -291,10 +291,16 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
         return {0, 0, false};
     }
     // Repeatable sums of fewer than 7 M entries (the bound above, whatever it was overridden with): the row-wise kernels'
-    // sums repeat as they are, and only an x out of reach of the caches makes them slower than the layout.  (op(A) = A^T
-    // replaces atomics on y and keeps the bounds of AnalyseRestored.)
+    // sums repeat as they are, and only an x out of reach of the caches makes them slower than the layout.  Of more
+    // entries: only the shortest rows over the smallest x are faster row by row (us a call, row by row / layout, 8 M
+    // entries, 400 K, 600 K and 800 K columns: 2 a row 47 / 57, 47 / 57, 50 / 57; 4 a row 45 / 49, 46 / 49, 47 / 49; 6 a
+    // row 44 / 46, 45 / 45, 45 / 44; 1 M columns, 4 a row: 53 / 49).  (op(A) = A^T replaces atomics on y and keeps the
+    // bounds of AnalyseRestored.)
     const char *minColsEnv = std::getenv("OPS_SPARSE_ORDERED_LIVE_MIN_COLS");  // tuning override, read at every call
-    const int64_t minCols = minColsEnv != nullptr ? std::atoll(minColsEnv) : nnz < kMinDefaultNnz ? kMinColsOrderedLive : 0;
+    const int64_t minCols = minColsEnv != nullptr ? std::atoll(minColsEnv)
+                            : nnz < kMinDefaultNnz ? kMinColsOrderedLive
+                            : nnz < 6 * rows       ? kMinColsOrderedShortRows
+                                                   : 0;
     if (!atomics && !transpose && cols < minCols) {
         return {0, 0, false};
     }

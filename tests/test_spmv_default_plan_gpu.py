@@ -757,6 +757,29 @@ def test_ordered_live_layout_only_where_x_is_out_of_reach_of_the_caches(osa, gpu
     assert osa.SpmvOp(handle, A, osa.DnVec(d[3]), Y).buffer.numel() > plain
 
 
+@pytest.mark.parametrize("rows,per_row,cols,layout", [(1_450_000, 5, 910_000, False), (1_450_000, 5, 925_000, True),
+                                                      (1_200_000, 6, 600_000, True), (1_190_000, 6, 600_000, True),
+                                                      (1_160_000, 6, 600_000, False)])
+def test_spmvop_keeps_the_shortest_rows_over_a_small_x_row_by_row(osa, gpu_ctx, monkeypatch, rows, per_row, cols, layout):
+    """aclsparseSpMVOp's default from 7 M entries on: the ordered layout, but not for rows of fewer than six entries below
+    0.9 M columns.  (The last matrix has fewer than 7 M entries.)"""
+    dev, stream, handle = gpu_ctx
+    for name in ("OPS_SPARSE_ORDERED_LIVE_MIN_COLS", "OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ"):
+        monkeypatch.delenv(name)
+    rng = np.random.default_rng(rows + cols)
+    rowptr = (np.arange(rows + 1) * per_row).astype(np.int32)
+    colind = rng.integers(0, cols, rows * per_row).astype(np.int32)
+    val, x, y0 = (rng.uniform(-1, 1, n).astype(np.float32) for n in (colind.size, cols, rows))
+    A = osa.Csr(rows, cols, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev))
+    d_z = torch.zeros(rows, dtype=torch.float32, device=dev)
+    op = osa.SpmvOpPlan(handle, A, osa.DnVec(to_dev(x, dev)), osa.DnVec(to_dev(y0, dev)), osa.DnVec(d_z))
+    assert (op.buffer_bytes > 0) == layout
+    op(1.5, -0.5)
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, cols, rowptr, colind, val, x, y0, 1.5, -0.5)
+    assert oracle.max_rel_err(d_z.cpu().numpy(), gold) <= 1e-5
+
+
 @pytest.mark.parametrize("alg_name", ["default", "alg2", "spmvop_default"])
 def test_buffer_holds_only_what_the_calls_keep_when_the_handle_lends_the_scratch(osa, gpu_ctx, alg_name):
     """Two thirds of what a layout's analysis needs is scratch.  A handle that was given a workspace with room for it
