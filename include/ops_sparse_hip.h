@@ -137,7 +137,8 @@ typedef struct OpsparseSpmvPlan {
     int64_t carryOff;
     int64_t headOff;
     int64_t bytes;         /* workspace bytes this plan uses */
-    int64_t panelStart[OPSPARSE_SPMV_MAX_PANELS + 1]; /* COLUMN_PANELS: first entry of every panel */
+    int64_t panelStart[OPSPARSE_SPMV_MAX_PANELS + 1]; /* COLUMN_PANELS: first entry of every panel; BLOCKED_GATHER: [0] =
+                              entries of the fullest panel above the mean one */
 } OpsparseSpmvPlan;
 
 /* Bytes opsparse_spmv_csr_analyse / _launch may touch in `workspace`. */

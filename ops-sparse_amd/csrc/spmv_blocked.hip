@@ -775,7 +775,8 @@ __global__ __launch_bounds__(kBlockThreads) void BlockedLongDeferKernel(const in
 // its last row, so that its other entries are one piece) or the compact copy (valueOffsets = offsets).
 // blockShort[b] = the former, for the scatter kernel.  panelStart[p] = first entry of panel p in panel order
 // (p = P: the number of entries there).  header[3] (zero before) = entries of the largest block,
-// header[6] (zero before) = number of the last block with rows, plus one.
+// header[6] (zero before) = number of the last block with rows, plus one, header[7] (zero before) = entries of the
+// fullest panel.
 __global__ __launch_bounds__(kBlockThreads) void BlockedBlockTablesKernel(
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ valueOffsets, const int32_t *__restrict__ blockRow,
     const int32_t *__restrict__ dstStart, const int32_t *__restrict__ srcStart, const int32_t *__restrict__ longFirst,
@@ -788,6 +789,9 @@ __global__ __launch_bounds__(kBlockThreads) void BlockedBlockTablesKernel(
     }
     if (b <= P) {
         panelStart[b] = srcStart[static_cast<int64_t>(b) * B];
+    }
+    if (b < P) {
+        atomicMax(header + 7, srcStart[static_cast<int64_t>(b + 1) * B] - srcStart[static_cast<int64_t>(b) * B]);
     }
     if (b < B) {
         BlockMeta m;
@@ -2319,18 +2323,26 @@ int WithValueType(int32_t valueType, Fn &&fn)
 
 }  // namespace
 
-// Workgroups a panel in phase 1.  One workgroup is resident a compute unit, so P x splits of them run in whole rounds:
-// the number of parts that makes rounds x (what a workgroup takes for its slice of x + its part of the entries)
-// smallest.  (4 M columns are 123 panels: 80 us in 369 thirds, two rounds, 53 us in 246 halves; 6 M columns, 184
-// panels, 72 % of the chip with one workgroup each.)
-int32_t GatherSplits(int64_t P, int64_t nnz)
+// Workgroups a panel in phase 1.  One workgroup is resident a compute unit, so P x splits of them run in rounds of 256.  A
+// round of k workgroups with n entries each takes slice + n (a k + b): its slice of x, then what the memory takes for all
+// of its entries and a compute unit for its own (32 M entries: 10 workgroups 0.07 entries a ns, 46: 0.25, 123: 0.49, 230:
+// 0.64).  Taken is the number of parts for which the rounds add up to least.  (Charged as whole ones, the last rounds
+// came out too dear: 6 M columns, 184 panels, were cut in four, power-law rows 271 us a call, 246 uncut; 9.5 M columns
+// 151, 144 uncut.  4 M columns, 123 panels: 155 us in halves, 179 in thirds.)
+// `excess`: by how many entries the fullest panel exceeds the mean one, which the compute unit that has a part of it works
+// through alone.  Smaller parts soften that: the panels of op(A) = A^T differ as the rows of A do (4 M power-law rows of
+// 12 on average, transposed, values frozen: 188 us in halves, 173 in quarters; rows of even length 167 and 170).
+int32_t GatherSplits(int64_t P, int64_t nnz, int64_t excess)
 {
-    const double slice = 5.0, panel = 0.00036 * static_cast<double>(nnz) / static_cast<double>(P);  // us
+    const double slice = 5.0, a = 1.0e-6, b = 1.25e-4;  // us
     int32_t best = 1;
     double least = 0.0;
     for (int32_t s = 1; s <= 64; ++s) {  // (2^18 columns, the fewest, are eight panels)
-        const double rounds = static_cast<double>((P * s + 255) / 256);
-        const double t = rounds * (slice + panel / s);
+        const int64_t full = P * s / 256, rest = P * s % 256;
+        const double n = static_cast<double>(nnz) / static_cast<double>(P * s);
+        const double t = static_cast<double>(full) * (slice + n * (256 * a + b)) +
+                         (rest > 0 ? slice + n * (static_cast<double>(rest) * a + b) : 0.0) +
+                         static_cast<double>(excess) / s * b;
         if (s == 1 || t < 0.98 * least) {
             best = s;
             least = t;
@@ -2386,7 +2398,7 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
     }
     const int32_t *header = longRows ? ints(0) : nullptr;
     auto *longPartial = reinterpret_cast<uint64_t *>(base + l.longPartialOff);
-    const int32_t splits = GatherSplits(l.P, a.nnz);
+    const int32_t splits = GatherSplits(l.P, a.nnz, plan.panelStart[0]);
     return WithValueType(valType, [&](auto tag) {
         using ValT = decltype(tag);
         auto run = [&](auto accTag, auto outTag) {
@@ -2556,7 +2568,7 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
     auto ints = [&](int64_t off) { return reinterpret_cast<int32_t *>(at(off)); };
     int32_t *status = ints(0);
     // status, number of long rows, their entries, entries of the largest block, long rows summed on their own, rows
-    // without entries, block numbers in use; [8]: the rows' lengths squared and summed, 64 bits
+    // without entries, block numbers in use, entries of the fullest panel; [8]: the rows' lengths squared and summed, 64 b
     LaunchFillI32(status, 16, 0, s);
     if (transposed) {
         // The CSC arrays of A are the CSR arrays of A^T: from here on the matrix is that copy.
@@ -2754,8 +2766,9 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
     if (rcScatter != OPSPARSE_OK) {
         return rcScatter;
     }
-    // entries of the largest row block, long rows summed on their own, rows without entries, block numbers in use
-    int32_t tail[4] = {0, 0, 0, 0};
+    // entries of the largest row block, long rows summed on their own, rows without entries, block numbers in use, entries
+    // of the fullest panel
+    int32_t tail[5] = {0, 0, 0, 0, 0};
     if (hipMemcpyAsync(tail, status + 3, sizeof(tail), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         (void)hipGetLastError();
@@ -2783,6 +2796,7 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
     p.numEmptyRows = tail[2];
     p.streamedBlocks = l.streamed ? 1 : 0;
     p.usedRowBlocks = tail[3];
+    p.panelStart[0] = tail[4] - (nnz - head[2]) / l.P;
     p.numLongRows = head[1];
     p.rows = rows;
     p.nnz = nnz;

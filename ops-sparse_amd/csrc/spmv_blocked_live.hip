@@ -1271,7 +1271,7 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
     if (plan.liveValues == 0 || plan.transposed != 0 || a.vals == nullptr) {
         return OPSPARSE_E_INVALID;  // (this layout is the one with live values, for op(A) = A)
     }
-    const int32_t splits = GatherSplits(l.P, a.nnz);
+    const int32_t splits = GatherSplits(l.P, a.nnz, 0);
     // long rows: summed from the caller's own arrays (header[1] of them, counted by the analysis)
     const bool longRows = plan.numLongRows > 0;
     if (longRows && plan.liveValues != 0 && (a.vals == nullptr || a.colInd == nullptr)) {

@@ -33,8 +33,9 @@ inline int CheckLaunch()
 int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valType, int32_t outType,
                   int32_t computeIsInt);
 
-// Workgroups a column panel in the first kernel of the two blocked layouts (spmv_blocked.hip).
-int32_t GatherSplits(int64_t P, int64_t nnz);
+// Workgroups a column panel in the first kernel of the two blocked layouts (spmv_blocked.hip); `excess`: entries of the
+// fullest panel above the mean.
+int32_t GatherSplits(int64_t P, int64_t nnz, int64_t excess);
 
 // BLOCKED_LIVE launch (spmv_blocked_live.hip): values and x of valType (fp32 / fp16 / bf16), y fp32 or of valType.
 namespace live_layout {

@@ -1033,3 +1033,47 @@ def test_hubs_over_few_panels_are_summed_by_whole_workgroups(osa, gpu_ctx, dtype
         assert oracle.max_rel_err(got[0].numpy(), gold) <= 1e-5
     else:  # the fp64 sum rounded once: half a unit in the last place
         assert np.all(np.abs(got[0].float().numpy() - gold) <= 1.001 * 2.0 ** -8 * np.maximum(np.abs(gold), 2.0 ** -14))
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("live", [False, True])
+def test_panels_of_very_different_fullness(osa, gpu_ctx, live, transposed):
+    """Four fifths of the entries in one of nineteen panels of the inputs, none in another: the analysis tells the launches
+    how much fuller it is, and the panels are cut into more parts than those of an even matrix."""
+    dev, stream, handle = gpu_ctx
+    L = osa.lib()
+    outputs, inputs = 280_000, 600_000
+    rng = np.random.default_rng(81)
+    lengths = rng.integers(0, 24, outputs)
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(65_536, inputs, nnz).astype(np.int32)            # (panel 0: a few, panel 1: none)
+    colind[rng.random(nnz) < 0.8] = 3 * 32768 + 17
+    colind[:5] = [0, 32_767, 5, 98_304, 131_071]
+    val = rng.uniform(-1, 1, nnz).astype(np.float32)
+    x, y0 = rng.uniform(-1, 1, inputs).astype(np.float32), rng.uniform(-1, 1, outputs).astype(np.float32)
+    d_arrays, shape = (rowptr, colind, val), (outputs, inputs)
+    if transposed:
+        import scipy.sparse as sp
+        t = sp.csr_matrix((val, colind, rowptr), shape=shape).tocsc()
+        d_arrays, shape = (t.indptr.astype(np.int32), t.indices.astype(np.int32), t.data), (inputs, outputs)
+    d = [to_dev(np.ascontiguousarray(a), dev) for a in d_arrays]
+    flags = (osa.OPSPARSE_BLOCKED_TRANSPOSE if transposed else 0) | (osa.OPSPARSE_BLOCKED_LIVE_VALUES if live else 0)
+    need = L.opsparse_spmv_csr_blocked_workspace_bytes(*shape, nnz, flags)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    plan = osa.OpsparseSpmvPlan()
+    pv = lambda a: ctypes.c_void_p(a.data_ptr())
+    sp_ = ctypes.c_void_p(stream.cuda_stream)
+    assert L.opsparse_spmv_csr_blocked_analyse(pv(d[0]), pv(d[1]), pv(d[2]), *shape, nnz, flags, pv(ws), need,
+                                               ctypes.byref(plan), sp_) == 0
+    fullest = int(np.bincount(colind >> 15).max())
+    assert plan.panelStart[0] == fullest - nnz // plan.numPanels
+    d_x, d_y = to_dev(x, dev), to_dev(y0, dev)
+    scalar = lambda v: osa.OpsparseScalar(v, None, 0, 0)
+    assert L.opsparse_spmv_csr_launch(ctypes.byref(plan), int(transposed), pv(d[0]), pv(d[1]), pv(d[2]), pv(d_x), pv(d_y),
+                                      *shape, nnz, scalar(1.5), scalar(-0.5), osa.OPSPARSE_F32, osa.OPSPARSE_F32, 0, pv(ws),
+                                      need, sp_) == 0
+    stream.synchronize()
+    gold = oracle.spmv_f64(outputs, inputs, rowptr, colind, val, x, y0, 1.5, -0.5)
+    assert oracle.max_rel_err(d_y.cpu().numpy(), gold) <= 1e-5
