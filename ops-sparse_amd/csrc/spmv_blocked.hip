@@ -86,11 +86,16 @@ constexpr int64_t kStreamBlocksWanted = 8192;
 constexpr int64_t kStreamMinChunkEntries = 16;
 constexpr int64_t kStreamMaxRowPanelEntries = 12;
 // Uneven rows: the mean length of an entry's row is this many times the mean row's, and such a row has half an entry or
-// more in a panel.  They meet themselves in the instructions of the stream: 4 M x 4 M power-law rows 155 us streamed,
-// 120 in windowed blocks, 300 K x 300 K ones 73 and 38; rows of 8 or 32 entries each 122 and 130, 106 and 113; 8 M
-// power-law rows with few long ones among them (a quarter of an entry in a panel) 251 and 302.
+// more in a panel.  They meet themselves in the instructions of the stream (4 M x 4 M power-law rows 155 us streamed, 120
+// in windowed blocks, 300 K x 300 K ones 82 and 46), the more the more uneven they are; the windowed blocks, which are
+// smaller, have more padding, the more the shorter their chunks are.  Below 20 entries a (panel, block) chunk the product
+// of the two measures decides as well: 5 M rows of 13.4 over 153 panels, 18 a chunk, nine times as uneven and 0.72 in a
+// panel, 253 us streamed and 276 windowed; 6 M of 8, 13 a chunk, 30 times and 0.74, 214 and 195; 3 M of 3.8, 20 a chunk,
+// 13 times and 0.53, 70 and 62.
 constexpr double kStreamMaxUnevenness = 4.0;
 constexpr double kStreamUnevenRowPanelEntries = 0.5;
+constexpr int64_t kStreamUnevenChunkEntries = 20;
+constexpr double kStreamUnevenProduct = 9.0;
 constexpr int kStreamThreads = 64;                // a wavefront a workgroup: nothing is shared, nothing waits
 constexpr int kTurnThreads = 256;
 constexpr uint32_t kStreamPadRow = 0x7ffu;        // row field of a padding position (rows take 10 of its 11 bits)
@@ -2618,8 +2623,11 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
         }
         const double entries = sums[1] > 0 ? static_cast<double>(sums[1]) : 1.0;
         const double weighted = static_cast<double>(sums[0]) / entries;  // mean length of an entry's row
-        if (weighted > kStreamMaxUnevenness * entries / static_cast<double>(outputs) &&
-            weighted > kStreamUnevenRowPanelEntries * static_cast<double>(l.P)) {
+        const double unevenness = weighted * static_cast<double>(outputs) / entries;
+        const double inPanel = weighted / static_cast<double>(l.P);
+        if (unevenness > kStreamMaxUnevenness && inPanel > kStreamUnevenRowPanelEntries &&
+            (nnz / (static_cast<int64_t>(windowed.P) * windowed.B) >= kStreamUnevenChunkEntries ||
+             unevenness * inPanel > kStreamUnevenProduct)) {
             l = windowed;
             fallsBack = true;
         }
