@@ -202,11 +202,19 @@ bool PrefersWholeRows(const aclsparseSpMatDescr *A, const OpsparseSpmmPlan &plan
         return false;
     }
     if (elemBytes == 2) {
-        // fp16 keeps the slabs, tuned on c5, except under local rows of 6 entries or more (us, slabs / rows, pipelined:
-        // 7-point mesh of 1.1 M rows n = 24 106 / 74, n = 32 110 / 84, n = 64 174 / 154, n = 256 641 / 597; 9-point
-        // n = 64 252 / 228; band of 12 n = 32 75 / 50, n = 128 176 / 184, n = 256 363 / 325; 32 random columns a row
-        // n = 32 292 / 412)
-        if (mean < 6.0) {
+        // fp16 keeps the slabs, tuned on c5, except under local rows of 12 entries or more (us, slabs / rows, pipelined:
+        // band of 12 n = 64 45 / 35, n = 128 71 / 63, n = 256 144 / 143; 27-point mesh n = 64 203 / 145, n = 256 612 /
+        // 508; 32 random columns a row n = 32 292 / 412) and shorter ones where the table had the rows ahead.  Up to 128
+        // bytes of B a row, from 6 entries: 7-point mesh of 1 M rows n = 32 110 / 84, n = 64 160 / 143, 9-point n = 64
+        // 121 / 119.  Up to 256, from 10 entries (band of 10 n = 96 46 / 43) or with rows enough for several turns of
+        // the pipeline (7-point, 1 M rows, n = 128 298 / 280; 9-point of 2.3 M rows n = 112 712 / 645, of 720 K rows
+        // n = 96 196 / 209; band of 7, 300 K rows, n = 128 72 / 77).  Above 384, not 9-point meshes: 7-point n = 224
+        // 565 / 516, band of 10 94 / 85, 9-point 1248 / 1299.  In between, from 12: 9-point n = 160 966 / 1154, band of
+        // 10 74 / 78, 7-point 919 / 963.
+        const bool ninePoint = mean >= 8.0 && mean < 10.0;
+        const bool ahead = rowBytes <= 128 || (rowBytes <= 256 && (mean >= 10.0 || A->rows >= 786432)) ||
+                           (rowBytes > 384 && !ninePoint);
+        if (mean < 6.0 || (mean < 12.0 && !ahead)) {
             return false;
         }
     } else {

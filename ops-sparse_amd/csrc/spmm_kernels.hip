@@ -1604,19 +1604,29 @@ bool Small32(const SpmmArgs &a, size_t elementBytes)
     return static_cast<uint64_t>(a.k) * static_cast<uint64_t>(a.ldb) * elementBytes < (1ull << 32);
 }
 
+// Turns of a workgroup of the pipelined kernel: as many as leave the chip eight rounds of workgroups, up to kPipelineTurns.
+int32_t PipelineTurns(int64_t rows, int groups)
+{
+    const int64_t fill = (rows + groups - 1) / groups / (8 * 2048);
+    return static_cast<int32_t>(fill < 1 ? 1 : (fill > kPipelineTurns ? kPipelineTurns : fill));
+}
+
 // Whether the rows of an analysed matrix are worked by the pipelined kernel.  Two-byte elements: always, up to 32 lanes a
 // group (us, one row after the other / pipelined: 27-point mesh of 614 K rows, n = 32 155 / 132, n = 64 247 / 178, n = 256
 // 736 / 605; 7-point of 1.1 M rows 96 / 84, 174 / 154, 696 / 597; band of 20 57 / 46, 97 / 71, 307 / 255).  fp32, whose
 // other kernel keeps eight wavefronts on a SIMD where this one keeps five: rows of 16 entries on up to 8 lanes (27-point
-// n = 16 176 / 151, n = 32 165 / 153; 12 entries 66.4 / 66.7, 8 random ones 181 / 186), of 24 on 16 lanes (27-point
-// n = 64 263 / 249, 20 entries 105 / 111), and any on 32 (n = 128: 7-point 436 / 405, 9-point 659 / 580).
+// n = 16 176 / 151, n = 32 165 / 153; 12 entries 66.4 / 66.7, 8 random ones 181 / 186), of 30 on 16 lanes (bands, n = 48:
+// of 24 73 / 75, of 30 46 / 44, of 50 78 / 71, of 100 88 / 76; 27-point of 420 K rows, n = 36 130 / 137), and on 32 any
+// (n = 128: 7-point 436 / 405, 9-point 659 / 580) but rows of fewer than 12 in matrices so small that a group has one
+// turn, which leaves nothing to pipeline (150 K rows of 8, n = 100 48 / 52; 100 K of 12 44 / 43).
 template <typename ValT, int L>
 bool RowsArePipelined(const SpmmArgs &a)
 {
     if (a.plan == nullptr || a.nnz <= 0 || a.rows <= 0 || L > 32) {
         return false;
     }
-    const int64_t shortest = sizeof(ValT) == 2 || L == 32 ? 0 : (L == 16 ? 24 : 16);
+    const bool oneTurn = PipelineTurns(a.rows, kBlockThreads / L) == 1;
+    const int64_t shortest = sizeof(ValT) == 2 ? 0 : (L == 32 ? (oneTurn ? 12 : 0) : (L == 16 ? 30 : 16));
     return a.nnz >= shortest * a.rows;
 }
 
@@ -1624,10 +1634,8 @@ template <typename ValT, typename CT, typename AccT, int V, int L>
 int LaunchRowPipeline(const SpmmArgs &a, bool binned)
 {
     constexpr int kGroups = kBlockThreads / L;
-    // Turns a workgroup: as many as leave the chip eight rounds of workgroups, up to kPipelineTurns.
     const int64_t tiles = (a.rows + kGroups - 1) / kGroups;
-    const int64_t fill = tiles / (8 * 2048);
-    const int32_t turns = static_cast<int32_t>(fill < 1 ? 1 : (fill > kPipelineTurns ? kPipelineTurns : fill));
+    const int32_t turns = PipelineTurns(a.rows, kGroups);
     const uint32_t grid = static_cast<uint32_t>((tiles + turns - 1) / turns);
     auto launch = [&](auto tag) {
         constexpr bool kSmall = decltype(tag)::value;
