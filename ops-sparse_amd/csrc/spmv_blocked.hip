@@ -2149,41 +2149,10 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
         const char *env = std::getenv("OPS_SPARSE_BLOCKED_WINDOW");
         return env != nullptr ? std::atoll(env) : 0;
     }();
-    // (the blocks are cut at seven eighths of the window, plus the row in which the cut falls: nearly all fit one)
-    l.size = kNumRowsSizes - 1;
-    for (int i = 0; i < kNumRowsSizes - 1; ++i) {
-        const int64_t blocks = (rows >> kRowsSizes[i].rowLog) + nnz / (kRowsSizes[i].window * 7 / 8) + 1;
-        if (nnz / (P * blocks) >= kRowsSizes[i].chunk) {
-            l.size = i;
-            break;
-        }
-    }
-    int64_t window = cutEnv > 0 ? cutEnv : kRowsSizes[l.size].window * 7 / 8;
-    window = window > kMaxBlockEntries / 2 ? kMaxBlockEntries / 2 : window;
-    // Values that the layout keeps (frozen values, either op(A)) are kept in block order and streamed by a wavefront
-    // a block; values read where the caller has them need the windowed blocks, which read them in row order.
-    const bool noStream = std::getenv("OPS_SPARSE_BLOCKED_NO_STREAM") != nullptr;  // tuning switch
-    l.streamed = stream && !live && !noStream;
-    if (l.streamed) {
-        // Streamed blocks are cut by their rows; the entry cut is there for matrices of few, long rows, which would
-        // otherwise make fewer blocks than the chip has wavefronts: about 8192 blocks of 4096 entries at least.
-        const int64_t byRows = rows >> kStreamRowLog;
-        int64_t cut = byRows >= kStreamBlocksWanted / 2 ? kStreamWindow : nnz / (kStreamBlocksWanted - byRows);
-        cut = cut < kStreamMinWindow ? kStreamMinWindow : (cut > kStreamWindow ? kStreamWindow : cut);
-        cut = cutEnv > 0 ? cutEnv : cut;
-        // They pay where a (panel, block) chunk has 16 entries on average (smaller ones are mostly padding, and a
-        // block of 2^10 rows has a quarter of the entries of a windowed one: many panels and few entries a row
-        // are the windowed blocks' case) and where a row does not put more than 16 entries into a panel on
-        // average (such rows meet themselves in every instruction of the stream: 200 000 rows of 300 entries over
-        // 19 panels 228 us streamed, 202 us windowed; over 31 panels 200 either way).
-        const int64_t blocks = ((rows + kStreamRows - 1) >> kStreamRowLog) + nnz / cut + 1;
-        if (nnz / (P * blocks) < kStreamMinChunkEntries || nnz / rows / P > kStreamMaxRowPanelEntries) {
-            l.streamed = false;
-        } else {
-            window = cut;
-        }
-    }
-    l.rowLog = l.streamed ? kStreamRowLog : kRowsSizes[l.size].rowLog;
+    // A block ends behind 2^rowLog rows, behind `window` entries and, where the values are read in place in row order,
+    // behind a long row: `blocks` without these, the positions of all chunks in 32 bits with them.
+    auto blocksOf = [&](int32_t rowLog, int64_t cut) { return ((rows + (int64_t{1} << rowLog) - 1) >> rowLog) + nnz / cut + 1; };
+    auto numbered = [&](int64_t B) { return P * B + 1 <= INT32_MAX && nnz + kLaneEntries * P * B <= INT32_MAX - 65536; };
     // The values a launch reads: the caller's own (live values, op(A) = A), the transposed copy (op(A) = A^T), or,
     // for op(A) = A with frozen values, a compact copy without the long rows' values, whose entries are stored a
     // second time with their values.
@@ -2210,13 +2179,43 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
             l.frozenLong = frozenCopy;
         }
     }
-    // a block ends behind 2^rowLog rows, behind `window` entries and, where the values are read in place in row
-    // order, behind a long row
-    const bool cutBehindLong = !l.frozenLong && !l.streamed;
-    const int64_t B = ((rows + (int64_t{1} << l.rowLog) - 1) >> l.rowLog) + nnz / window + 1 + (cutBehindLong ? l.maxLong : 0);
-    if (P * B + 1 > INT32_MAX || nnz + kLaneEntries * P * B > INT32_MAX - 65536 ||
-        nnz / (P * (B - (cutBehindLong ? l.maxLong : 0))) < kMinChunkEntries) {
-        return BlockedLayout{};
+    // Values that the layout keeps (frozen values, either op(A)) are kept in block order and streamed by a wavefront
+    // a block; values read where the caller has them need the windowed blocks, which read them in row order.
+    const bool noStream = std::getenv("OPS_SPARSE_BLOCKED_NO_STREAM") != nullptr;  // tuning switch
+    int64_t window = 0, B = 0;
+    if (stream && !live && !noStream) {
+        // Streamed blocks are cut by their rows; the entry cut is there for matrices of few, long rows, which would
+        // otherwise make fewer blocks than the chip has wavefronts: about 8192 blocks of 4096 entries at least.
+        const int64_t byRows = rows >> kStreamRowLog;
+        int64_t cut = byRows >= kStreamBlocksWanted / 2 ? kStreamWindow : nnz / (kStreamBlocksWanted - byRows);
+        cut = cut < kStreamMinWindow ? kStreamMinWindow : (cut > kStreamWindow ? kStreamWindow : cut);
+        cut = cutEnv > 0 ? cutEnv : cut;
+        window = cut;
+        // They pay where a (panel, block) chunk has 16 entries on average (smaller ones are mostly padding, and a
+        // block of 2^10 rows has a quarter of the entries of a windowed one: many panels and few entries a row
+        // are the windowed blocks' case) and where a row does not put more than 12 entries into a panel on
+        // average (such rows meet themselves in every instruction of the stream: 200 000 rows of 300 entries over
+        // 19 panels 228 us streamed, 202 us windowed; over 31 panels 200 either way).
+        B = blocksOf(kStreamRowLog, window);
+        l.streamed = numbered(B) && nnz / (P * B) >= kStreamMinChunkEntries && nnz / rows / P <= kStreamMaxRowPanelEntries;
+        l.rowLog = kStreamRowLog;
+    }
+    if (!l.streamed) {
+        // (the blocks are cut at seven eighths of the window, plus the row in which the cut falls: nearly all fit one)
+        const int64_t behindLong = l.frozenLong ? 0 : l.maxLong;
+        l.size = -1;
+        for (int i = 0; i < kNumRowsSizes && l.size < 0; ++i) {
+            window = cutEnv > 0 ? cutEnv : kRowsSizes[i].window * 7 / 8;
+            window = window > kMaxBlockEntries / 2 ? kMaxBlockEntries / 2 : window;
+            l.rowLog = kRowsSizes[i].rowLog;
+            const int64_t blocks = blocksOf(l.rowLog, window);
+            const int64_t least = kRowsSizes[i].chunk > kMinChunkEntries ? kRowsSizes[i].chunk : kMinChunkEntries;
+            B = blocks + behindLong;
+            l.size = numbered(B) && nnz / (P * blocks) >= least ? i : -1;
+        }
+        if (l.size < 0) {
+            return BlockedLayout{};
+        }
     }
     l.P = static_cast<int32_t>(P);
     l.B = static_cast<int32_t>(B);

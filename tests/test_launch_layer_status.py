@@ -261,3 +261,18 @@ def test_coosort_buffer_has_room_for_the_offsets_scan_of_short_rows(L):
                 20_963_328, 33_000_000, 400_000_000, (1 << 31) - 1):
         array = (4 * nnz + 255) // 256 * 256
         assert L.opsparse_coosort_workspace_bytes(nnz) - 256 + array >= L.opsparse_csr2csc_workspace_bytes(1, nnz - 1, nnz)
+
+
+def test_blocked_layout_takes_a_larger_row_block_where_a_smaller_one_does_not_fit(L, osa):
+    """The windowed row blocks come in three sizes.  A size whose chunks are long enough only by a count of blocks rounded
+    down, or whose padded positions have no 32-bit numbers, must not keep the matrix from a larger one: every matrix that
+    blocks of 2^12 rows and 12 544 entries fit has the layout."""
+    live = osa.OPSPARSE_BLOCKED_LIVE_VALUES
+    for rows, cols, nnz in ((3_292_434, 14_019_549, 12_130_224), (134_217_728, 8_388_608, 1_200_000_000),
+                            (12_313, 1_059_523, 1_944_376_814), (3_464_661, 10_295_313, 1_362_892_024),
+                            (54_818_341, 2_128_157, 1_746_358_107), (2_607_130, 9_598_310, 1_325_596_402)):
+        panels = (cols + 32767) // 32768
+        blocks = (rows + 4095) // 4096 + nnz // 12544 + 1
+        assert nnz // (panels * blocks) >= 8 and nnz + 8 * panels * blocks < (1 << 31) - 65536 - (1 << 24)
+        assert L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, live) > 0
+        assert L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, 0) > 0
