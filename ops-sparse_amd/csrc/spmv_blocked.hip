@@ -84,7 +84,8 @@ constexpr int32_t kStreamWindow = 65536;          // a block is also cut whereve
 constexpr int32_t kStreamMinWindow = 4096;        // (of this, where the matrix has few rows: MakeBlockedLayout)
 constexpr int64_t kStreamBlocksWanted = 8192;
 constexpr int64_t kStreamMinChunkEntries = 16;
-constexpr int64_t kStreamMaxRowPanelEntries = 12;
+constexpr int64_t kStreamMaxRowPanelEntries = 16;  // of a row in a panel, on average: up to here the stream applies,
+constexpr int64_t kStreamBestRowPanelEntries = 12; // and up to here it comes before the windowed blocks
 // Uneven rows: the mean length of an entry's row is this many times the mean row's, and such a row has half an entry or
 // more in a panel.  They meet themselves in the instructions of the stream (4 M x 4 M power-law rows 155 us streamed, 120
 // in windowed blocks, 300 K x 300 K ones 82 and 46), the more the more uneven they are; the windowed blocks, which are
@@ -2193,9 +2194,10 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
         window = cut;
         // They pay where a (panel, block) chunk has 16 entries on average (smaller ones are mostly padding, and a
         // block of 2^10 rows has a quarter of the entries of a windowed one: many panels and few entries a row
-        // are the windowed blocks' case) and where a row does not put more than 12 entries into a panel on
+        // are the windowed blocks' case) and where a row does not put more than 16 entries into a panel on
         // average (such rows meet themselves in every instruction of the stream: 200 000 rows of 300 entries over
-        // 19 panels 228 us streamed, 202 us windowed; over 31 panels 200 either way).
+        // 19 panels 228 us streamed, 202 us windowed; over 31 panels, ten in a panel, 200 either way: from 13 on the
+        // analysis takes the stream for the matrices alone that the windowed blocks refuse).
         B = blocksOf(kStreamRowLog, window);
         l.streamed = numbered(B) && nnz / (P * B) >= kStreamMinChunkEntries && nnz / rows / P <= kStreamMaxRowPanelEntries;
         l.rowLog = kStreamRowLog;
@@ -2538,7 +2540,8 @@ size_t opsparse_spmv_csr_blocked_resident_bytes(int64_t rows, int64_t cols, int6
     return static_cast<size_t>(resident);
 }
 
-// `unevenToWindows`: frozen values of uneven rows go into windowed blocks where both forms apply.
+// `unevenToWindows`: frozen values of uneven rows, or of rows with many entries in a panel, go into windowed blocks where
+// both forms apply.
 static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, const void *csrValues, int64_t rows,
                           int64_t cols, int64_t nnz, int32_t flags, void *workspace, size_t workspaceBytes,
                           void *scratchSpace, size_t scratchBytes, bool unevenToWindows, OpsparseSpmvPlan *plan, void *stream)
@@ -2610,7 +2613,10 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
     }
     // From here on: `outputs` rows, `inputs` columns, the arrays rowOffsets / colInd / csrValues.
     bool fallsBack = false;
-    if (l.streamed && windowed.P != 0 && unevenToWindows) {
+    if (l.streamed && windowed.P != 0 && unevenToWindows && nnz / outputs / l.P > kStreamBestRowPanelEntries) {
+        l = windowed;
+        fallsBack = true;
+    } else if (l.streamed && windowed.P != 0 && unevenToWindows) {
         hipLaunchKernelGGL(RowSquaresKernel, dim3(GridOf(outputs, kBlockThreads * 16, 2048)), dim3(kBlockThreads), 0, s,
                            rowOffsets, outputs, l.longMinRow > 0 ? l.longMinRow : INT32_MAX,
                            reinterpret_cast<unsigned long long *>(status + 8));

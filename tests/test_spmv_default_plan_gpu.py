@@ -1077,3 +1077,37 @@ def test_panels_of_very_different_fullness(osa, gpu_ctx, live, transposed):
     stream.synchronize()
     gold = oracle.spmv_f64(outputs, inputs, rowptr, colind, val, x, y0, 1.5, -0.5)
     assert oracle.max_rel_err(d_y.cpu().numpy(), gold) <= 1e-5
+
+
+@pytest.mark.parametrize("per_row,long_row,streamed", [(105, False, 1), (130, False, 0), (130, True, 1)])
+def test_frozen_rows_with_many_entries_in_a_panel(osa, gpu_ctx, per_row, long_row, streamed):
+    """Nine panels.  Rows of up to 12 entries in a panel on average are streamed, of 13 - 16 go into windowed blocks; with a
+    row of 70 000 entries whose columns do not ascend, which fits no window, those are streamed as well."""
+    dev, stream, handle = gpu_ctx
+    L = osa.lib()
+    rows, cols = 20_000, 270_000
+    rng = np.random.default_rng(per_row)
+    lengths = np.full(rows, per_row)
+    if long_row:
+        lengths[123] = 70_000
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(0, cols, nnz).astype(np.int32)
+    val, x, y0 = (rng.uniform(-1, 1, n).astype(np.float32) for n in (nnz, cols, rows))
+    d = [to_dev(a, dev) for a in (rowptr, colind, val)]
+    need = L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, 0)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    plan = osa.OpsparseSpmvPlan()
+    pv = lambda a: ctypes.c_void_p(a.data_ptr())
+    sp_ = ctypes.c_void_p(stream.cuda_stream)
+    assert L.opsparse_spmv_csr_blocked_analyse(pv(d[0]), pv(d[1]), pv(d[2]), rows, cols, nnz, 0, pv(ws), need,
+                                               ctypes.byref(plan), sp_) == 0
+    assert plan.streamedBlocks == streamed
+    d_x, d_y = to_dev(x, dev), to_dev(y0, dev)
+    scalar = lambda v: osa.OpsparseScalar(v, None, 0, 0)
+    assert L.opsparse_spmv_csr_launch(ctypes.byref(plan), 0, pv(d[0]), pv(d[1]), pv(d[2]), pv(d_x), pv(d_y), rows, cols, nnz,
+                                      scalar(1.5), scalar(-0.5), osa.OPSPARSE_F32, osa.OPSPARSE_F32, 0, pv(ws), need, sp_) == 0
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, cols, rowptr, colind, val, x, y0, 1.5, -0.5)
+    assert oracle.max_rel_err(d_y.cpu().numpy(), gold) <= 1e-5
