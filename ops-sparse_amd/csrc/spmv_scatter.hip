@@ -43,9 +43,10 @@ constexpr int kPanelSlots = 256;                // pass 2 runs a workgroup a com
 constexpr int kMaxOutCols = 20000;              // columns of A per output panel at most: 156 KiB of fp64 sums
 constexpr int kKeyLog = 15;                     // bits of a local column in the sort keys
 constexpr int kStageBytes = 128 << 10;          // the products of a piece staged in LDS
-constexpr int kMaxPanels = 3800;                // the chunk tables of a piece in LDS
+constexpr int64_t kMaxCols = int64_t{1} << 25;
+constexpr int kMaxPanels = static_cast<int>((kMaxCols + kPanelSlots * kMaxOutCols - 1) / (kPanelSlots * kMaxOutCols)) * kPanelSlots;
 constexpr int64_t kMinPanels = 16;              // of 2^14 columns: below 2^18 columns the products go to y as atomics
-constexpr int64_t kMaxChunks = int64_t{1} << 26;  // panels x pieces: the chunk tables
+constexpr int64_t kMaxChunks = int64_t{3} << 25;  // panels x pieces: the chunk tables (2^31 entries over 15 M columns)
 // A column with more entries than this is left to the ordered layout over the transposed copy, which sums such a
 // column as a long row: here all its products would queue for one address of LDS.
 constexpr int32_t kMaxColumnEntries = 8192;
@@ -96,7 +97,7 @@ int32_t ValueTypeOf(int32_t flags)
 ScatterLayout MakeLayout(int64_t rows, int64_t cols, int64_t nnz, int32_t valueType)
 {
     ScatterLayout l{};
-    if (rows <= 0 || cols <= 0 || nnz <= 0 || nnz > INT32_MAX - 65536 || rows >= INT32_MAX || cols > (int64_t{1} << 25)) {
+    if (rows <= 0 || cols <= 0 || nnz <= 0 || nnz > INT32_MAX - 65536 || rows >= INT32_MAX || cols > kMaxCols) {
         return l;
     }
     // Panels of 2^14 columns made 306 workgroups of 5 M columns, two rounds of the chip for 1.2 rounds of work (pass 2
@@ -108,7 +109,7 @@ ScatterLayout MakeLayout(int64_t rows, int64_t cols, int64_t nnz, int32_t valueT
     const int64_t piece = kStageBytes / pb;
     const int64_t Q = (nnz + piece - 1) / piece;
     const int64_t units = (cols + 16383) >> 14;
-    if (units < MinPanels() || P > kMaxPanels || P * Q > kMaxChunks) {
+    if (units < MinPanels() || P * Q > kMaxChunks) {
         return l;
     }
     l.units = static_cast<int32_t>(units);

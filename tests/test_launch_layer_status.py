@@ -276,3 +276,14 @@ def test_blocked_layout_takes_a_larger_row_block_where_a_smaller_one_does_not_fi
         assert nnz // (panels * blocks) >= 8 and nnz + 8 * panels * blocks < (1 << 31) - 65536 - (1 << 24)
         assert L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, live) > 0
         assert L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, 0) > 0
+
+
+def test_scatter_layout_takes_every_entry_count_up_to_15_million_columns(L, osa):
+    """The output panels are 256 or a multiple; the bound of the chunk tables (panels x pieces) leaves room for 2^31 entries
+    up to 768 panels, and never for fewer than panels of 2^14 columns and 2^26 chunks would."""
+    f16 = osa.OPSPARSE_BLOCKED_VALUES_F16
+    for cols, nnz, flags in ((15_360_000, (1 << 31) - (1 << 17), 0), (10_706_930, 1_643_024_120, 0),
+                             (15_423_709, 1_136_269_937, 0), (16_151_713, 1_109_875_767, 0), (20_480_000, 870_000_000, 0),
+                             (25_600_000, 700_000_000, 0), (1 << 25, 530_000_000, 0), (20_803_146, 1_724_544_368, f16)):
+        assert L.opsparse_spmv_csr_scatter_workspace_bytes(3_000_000, cols, nnz, flags) > 0
+    assert L.opsparse_spmv_csr_scatter_workspace_bytes(3_000_000, (1 << 25) + 1, 530_000_000, 0) == 0
