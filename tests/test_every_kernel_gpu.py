@@ -602,68 +602,64 @@ def test_frozen_layout_with_int32_values(osa, gpu_ctx, int_compute, streamed, mo
             assert oracle.max_rel_err(d_y.cpu().numpy(), gold) <= 1e-5
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("narrow_y", [False, True])
-def test_atomics_layout_with_32_bit_positions_and_16_bit_values(osa, gpu_ctx, dtype, narrow_y, monkeypatch):
-    """The default plan's layout on fp16 / bf16 values with the positions of the entries kept in 32 bits
-    (live_layout::SpmvBlockReduceKernel<true, false, ValT, OutT>; 16 bits are the rule, 32 what a row block of
-    65 535 positions and more takes, asked for here by the switch)."""
+def _run_atomics_layout(osa, gpu_ctx, rows, cols, rowptr, colind, dtype, out_dtype, alpha, beta, seed):
+    """The layout whose row blocks are summed with atomics, analysed and launched directly (the default algorithm takes it
+    only for a matrix that the ordered layout refuses): checks one product and returns the plan."""
     dev, stream, handle = gpu_ctx
     L = osa.lib()
-    monkeypatch.setenv("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "0")
-    monkeypatch.setenv("OPS_SPARSE_BLOCKED_NO_SHORT_POSITIONS", "1")
-    monkeypatch.delenv("OPS_SPARSE_SPMV_REPEATABLE", raising=False)
-    rows, cols = 300_000, 1_400_000
-    rowptr, colind = _wide_matrix(rows, cols, 71, long_rows=[(9, 30_000)])
     nnz = colind.size
-    rng = np.random.default_rng(72)
-    out_dtype = dtype if narrow_y else torch.float32
+    rng = np.random.default_rng(seed)
     val, x = _as_seen(rng.uniform(-1, 1, nnz), dtype), _as_seen(rng.uniform(-1, 1, cols), dtype)
     y0 = _as_seen(rng.uniform(-1, 1, rows), out_dtype)
     d = [to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev, dtype), to_dev(x, dev, dtype)]
     d_y = to_dev(y0, dev, out_dtype)
-    op = osa.SpmvOp(handle, osa.Csr(rows, cols, d[0], d[1], d[2]), osa.DnVec(d[3]), osa.DnVec(d_y))
-    assert op.buffer.numel() == L.opsparse_spmv_csr_live_workspace_bytes(rows, cols, nnz)
-    op(1.5, 0.5)
+    need = L.opsparse_spmv_csr_live_workspace_bytes(rows, cols, nnz)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    plan = osa.OpsparseSpmvPlan()
+    pv, sp = lambda t: ctypes.c_void_p(t.data_ptr()), ctypes.c_void_p(stream.cuda_stream)
+    flag, kind = {torch.float32: (0, osa.OPSPARSE_F32), torch.float16: (osa.OPSPARSE_BLOCKED_VALUES_F16, osa.OPSPARSE_F16),
+                  torch.bfloat16: (osa.OPSPARSE_BLOCKED_VALUES_BF16, osa.OPSPARSE_BF16)}[dtype]
+    assert L.opsparse_spmv_csr_live_analyse(pv(d[0]), pv(d[1]), pv(d[2]), rows, cols, nnz, flag, pv(ws), need,
+                                            ctypes.byref(plan), sp) == 0
+    assert plan.kernel == osa.OPSPARSE_SPMV_BLOCKED_LIVE
+    scalar = lambda v: osa.OpsparseScalar(v, None, 0, 0)
+    assert L.opsparse_spmv_csr_launch(ctypes.byref(plan), 0, pv(d[0]), pv(d[1]), pv(d[2]), pv(d[3]), pv(d_y), rows, cols,
+                                      nnz, scalar(alpha), scalar(beta), kind,
+                                      osa.OPSPARSE_F32 if out_dtype == torch.float32 else kind, 0, pv(ws), need, sp) == 0
     stream.synchronize()
-    _check_spmv(d_y.cpu().float().numpy(), rows, cols, rowptr, colind, val, x, y0, 1.5, 0.5, out_dtype)
+    _check_spmv(d_y.cpu().float().numpy(), rows, cols, rowptr, colind, val, x, y0, alpha, beta, out_dtype)
+    return plan
 
 
 @pytest.mark.parametrize("dtype,narrow_y", [(torch.float32, False), (torch.float16, False), (torch.float16, True),
                                             (torch.bfloat16, False), (torch.bfloat16, True)])
-def test_atomics_layout_with_many_long_rows_in_one_block(osa, gpu_ctx, dtype, narrow_y, monkeypatch):
+@pytest.mark.parametrize("short_positions", [True, False])
+def test_atomics_layout_with_either_kind_of_positions(osa, gpu_ctx, dtype, narrow_y, short_positions, monkeypatch):
+    """Every type of values and y with the positions of the entries kept in 16 and in 32 bits
+    (live_layout::SpmvBlockReduceKernel<true, Short, ValT, OutT>; 16 bits are the rule, 32 what a row block of
+    65 535 positions and more takes, asked for here by the switch)."""
+    if not short_positions:
+        monkeypatch.setenv("OPS_SPARSE_BLOCKED_NO_SHORT_POSITIONS", "1")
+    rows, cols = 300_000, 1_400_000
+    rowptr, colind = _wide_matrix(rows, cols, 71, long_rows=[(9, 30_000)])
+    plan = _run_atomics_layout(osa, gpu_ctx, rows, cols, rowptr, colind, dtype, dtype if narrow_y else torch.float32, 1.5,
+                               0.5, 72)
+    assert plan.liveValues == (2 if short_positions else 1) and plan.numLongRows == 1
+
+
+@pytest.mark.parametrize("dtype,narrow_y", [(torch.float32, False), (torch.float16, False), (torch.float16, True),
+                                            (torch.bfloat16, False), (torch.bfloat16, True)])
+def test_atomics_layout_with_many_long_rows_in_one_block(osa, gpu_ctx, dtype, narrow_y):
     """200 neighbouring rows of 4200 .. 5000 ascending entries among short ones: more long rows than the workgroup
     of a row block adds up itself (64), so their partial sums are left to live_layout::SpmvLongRowSumKernel<OutT>,
     a wavefront a row."""
-    dev, stream, handle = gpu_ctx
-    L = osa.lib()
-    monkeypatch.setenv("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "0")
-    monkeypatch.delenv("OPS_SPARSE_SPMV_REPEATABLE", raising=False)
     rows, cols = 300_000, 1_400_000
     rng = np.random.default_rng(81)
     long_rows = [(5000 + i, int(n)) for i, n in enumerate(rng.integers(4200, 5000, 200))]
     rowptr, colind = _wide_matrix(rows, cols, 82, long_rows=long_rows)
-    nnz = colind.size
-    out_dtype = dtype if narrow_y else torch.float32
-    val, x = _as_seen(rng.uniform(-1, 1, nnz), dtype), _as_seen(rng.uniform(-1, 1, cols), dtype)
-    y0 = _as_seen(rng.uniform(-1, 1, rows), out_dtype)
-    d = [to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev, dtype), to_dev(x, dev, dtype)]
-    need = L.opsparse_spmv_csr_live_workspace_bytes(rows, cols, nnz)
-    ws = torch.empty(need, dtype=torch.uint8, device=dev)
-    plan = osa.OpsparseSpmvPlan()
-    pv = lambda t: ctypes.c_void_p(t.data_ptr())
-    flag = {torch.float32: 0, torch.float16: osa.OPSPARSE_BLOCKED_VALUES_F16,
-            torch.bfloat16: osa.OPSPARSE_BLOCKED_VALUES_BF16}[dtype]
-    assert L.opsparse_spmv_csr_live_analyse(pv(d[0]), pv(d[1]), pv(d[2]), rows, cols, nnz, flag, pv(ws), need,
-                                            ctypes.byref(plan), ctypes.c_void_p(stream.cuda_stream)) == 0
+    plan = _run_atomics_layout(osa, gpu_ctx, rows, cols, rowptr, colind, dtype, dtype if narrow_y else torch.float32, -1.5,
+                               0.75, 83)
     assert plan.numLongRows == 200 and plan.numDeferredLongRows > 0
-    del ws
-    d_y = to_dev(y0, dev, out_dtype)
-    op = osa.SpmvOp(handle, osa.Csr(rows, cols, d[0], d[1], d[2]), osa.DnVec(d[3]), osa.DnVec(d_y))
-    assert op.buffer.numel() == need
-    op(-1.5, 0.75)
-    stream.synchronize()
-    _check_spmv(d_y.cpu().float().numpy(), rows, cols, rowptr, colind, val, x, y0, -1.5, 0.75, out_dtype)
 
 
 @pytest.mark.parametrize("elem", [1, 2, 4])

@@ -1,8 +1,9 @@
 """The plan aclsparseSpMVPreprocess picks for ACL_SPARSE_SPMV_ALG_DEFAULT on a large matrix with scattered
-columns: a blocked-gather layout with live values — the one whose row blocks add with atomics (plan kernel
-BLOCKED_LIVE) for op(A) = A and floating-point values, the ordered one (BLOCKED_GATHER, the same bits from every
-call) with OPS_SPARSE_SPMV_REPEATABLE in the environment, for op(A) = A^T, for int32 values and under
-aclsparseSpMVOp.  The contract under test: a caller that follows the
+columns: the ordered blocked-gather layout with live values (BLOCKED_GATHER, the same bits from every call), and for a
+matrix that it refuses - a row of more than 65 534 entries whose columns do not ascend - with op(A) = A and
+floating-point values the one whose row blocks add with atomics (BLOCKED_LIVE), in the same buffer; not with
+OPS_SPARSE_SPMV_REPEATABLE in the environment, for int32 values or under aclsparseSpMVOp, which ask for room for the
+ordered layout alone.  The contract under test: a caller that follows the
 reference's call pattern (GetBufferSize, Preprocess, SpMV with the default algorithm) may change the values in
 place, or hand the descriptor a new values array, between calls, and always gets the product of the values as
 they are at the call.  An explicit ACL_SPARSE_SPMV_CSR_ALG2 request holds a copy of the values: there
@@ -35,8 +36,9 @@ def _default_bytes(osa, rows, cols, nnz, repeatable):
     return L.opsparse_spmv_csr_live_workspace_bytes(rows, cols, nnz)
 
 
-@pytest.fixture(params=[False, True], ids=["atomics", "repeatable"])
+@pytest.fixture(params=[False, True], ids=["default", "repeatable"])
 def repeatable(request, monkeypatch):
+    """The default algorithm as it is, with a buffer for either layout, and asked for repeatable sums."""
     if request.param:
         monkeypatch.setenv("OPS_SPARSE_SPMV_REPEATABLE", "1")
     else:
@@ -718,23 +720,29 @@ def test_atomics_layout_with_32_bit_positions(osa, gpu_ctx, how, monkeypatch):
     assert L.opsparse_spmv_csr_live_analyse(pv(d[0]), pv(d[1]), pv(d[2]), rows, cols, nnz, 0, pv(ws), need,
                                             ctypes.byref(plan), ctypes.c_void_p(stream.cuda_stream)) == 0
     assert plan.kernel == osa.OPSPARSE_SPMV_BLOCKED_LIVE and plan.liveValues == 1
-    del ws
     d_y = to_dev(y0, dev)
     op = osa.SpmvOp(handle, osa.Csr(rows, cols, d[0], d[1], d[2]), osa.DnVec(d[3]), osa.DnVec(d_y))
     assert op.buffer.numel() == need
-    for values, alpha, beta in ((val, 1.0, 0.0), ((val * np.float32(-2.0)).astype(np.float32), 0.5, 1.5)):
+    scalar = lambda v: osa.OpsparseScalar(v, None, 0, 0)
+    for values, alpha, beta, direct in ((val, 1.0, 0.0, True), ((val * np.float32(-2.0)).astype(np.float32), 0.5, 1.5, True),
+                                        (val, 1.0, 0.0, False), ((val * np.float32(-2.0)).astype(np.float32), 0.5, 1.5, False)):
         d[2].copy_(torch.from_numpy(values))
         d_y.copy_(torch.from_numpy(y0))
-        op(alpha, beta)
+        if direct:  # the plan analysed above (the default algorithm has the ordered layout where no block is too long)
+            assert L.opsparse_spmv_csr_launch(ctypes.byref(plan), 0, pv(d[0]), pv(d[1]), pv(d[2]), pv(d[3]), pv(d_y), rows,
+                                              cols, nnz, scalar(alpha), scalar(beta), osa.OPSPARSE_F32, osa.OPSPARSE_F32, 0,
+                                              pv(ws), need, ctypes.c_void_p(stream.cuda_stream)) == 0
+        else:
+            op(alpha, beta)
         stream.synchronize()
         gold = oracle.spmv_f64(rows, cols, rowptr, colind, values, x, y0, alpha, beta)
         assert oracle.max_rel_err(d_y.cpu().numpy(), gold) <= 1e-5
 
 
 def test_ordered_live_layout_only_where_x_is_out_of_reach_of_the_caches(osa, gpu_ctx, monkeypatch):
-    """The layout with live values and ordered sums (aclsparseSpMVOp DEFAULT / ALG1, and the default algorithm asked
-    for repeatable sums) is slower than the one with atomics; against the row-wise kernels it pays from 2.6 M
-    columns on.  Below that aclsparseSpMVOp_bufferSize answers 0 for these algorithms, as the reference does."""
+    """Of fewer than 7 M entries the layout with live values and ordered sums (aclsparseSpMVOp DEFAULT / ALG1, and the
+    default algorithm asked for repeatable sums) is taken from 2.6 M columns on.  Below that
+    aclsparseSpMVOp_bufferSize answers 0 for these algorithms, as the reference does."""
     dev, stream, handle = gpu_ctx
     L = osa.lib()
     rows, cols = 320_000, 1_500_000

@@ -21,9 +21,9 @@ ULP = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}
 
 @pytest.fixture(autouse=True)
 def _small_matrices(monkeypatch):
-    """The layout is taken from 128 output panels (2 M columns) and, by the default algorithm, from 7 M entries on;
-    the matrices here have 19 panels and 3 M entries so that the oracle stays quick.  Both switches are read at every
-    size query and analysis."""
+    """The layout is taken from 2^18 columns (16 units of 2^14) and, by the default algorithm, from 7 M entries on; the
+    matrices here have 19 units and 3 M entries so that the oracle stays quick.  Both switches are read at every size
+    query and analysis."""
     monkeypatch.setenv("OPS_SPARSE_SCATTER_MIN_PANELS", "8")
     monkeypatch.setenv("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "0")
     monkeypatch.delenv("OPS_SPARSE_SPMV_REPEATABLE", raising=False)
@@ -66,7 +66,7 @@ def _code(osa, dtype):
 @pytest.mark.parametrize("dtype,narrow_y", [(torch.float32, False), (torch.float16, False), (torch.float16, True),
                                             (torch.bfloat16, False), (torch.bfloat16, True)])
 def test_scatter_layout_through_the_launch_layer(osa, gpu_ctx, dtype, narrow_y):
-    """Analysis and launch through the raw entry points, every type pair: the plan's shape (19 panels of 2^14 columns,
+    """Analysis and launch through the raw entry points, every type pair: the plan's shape (19 units of 2^14 columns,
     pieces of 128 KiB of products), the products for two pairs of scalars, and again after the values changed in place (the
     layout holds none).  The split form of the analysis leaves the same plan."""
     dev, stream, _ = gpu_ctx
