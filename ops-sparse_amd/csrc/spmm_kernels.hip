@@ -1616,7 +1616,8 @@ int32_t PipelineTurns(int64_t rows, int groups)
 // 736 / 605; 7-point of 1.1 M rows 96 / 84, 174 / 154, 696 / 597; band of 20 57 / 46, 97 / 71, 307 / 255).  fp32, whose
 // other kernel keeps eight wavefronts on a SIMD where this one keeps five: rows of 16 entries on up to 8 lanes (27-point
 // n = 16 176 / 151, n = 32 165 / 153; 12 entries 66.4 / 66.7, 8 random ones 181 / 186), of 30 on 16 lanes (bands, n = 48:
-// of 24 73 / 75, of 30 46 / 44, of 50 78 / 71, of 100 88 / 76; 27-point of 420 K rows, n = 36 130 / 137), and on 32 any
+// of 24 73 / 75, of 30 46 / 44, of 50 78 / 71, of 100 88 / 76; 27-point of 420 K rows, n = 36 130 / 137) and of 24 in small
+// matrices (27-point, n = 48 / 64: 16 K rows 10.3 / 7.6, 76 K 34.7 / 32.7, 125 K 54.6 / 53.8), and on 32 any
 // (n = 128: 7-point 436 / 405, 9-point 659 / 580) but rows of fewer than 12 in matrices so small that a group has one
 // turn, which leaves nothing to pipeline (150 K rows of 8, n = 100 48 / 52; 100 K of 12 44 / 43).
 template <typename ValT, int L>
@@ -1626,7 +1627,8 @@ bool RowsArePipelined(const SpmmArgs &a)
         return false;
     }
     const bool oneTurn = PipelineTurns(a.rows, kBlockThreads / L) == 1;
-    const int64_t shortest = sizeof(ValT) == 2 ? 0 : (L == 32 ? (oneTurn ? 12 : 0) : (L == 16 ? 30 : 16));
+    const int64_t on16 = a.rows <= (int64_t{1} << 17) ? 24 : 30;
+    const int64_t shortest = sizeof(ValT) == 2 ? 0 : (L == 32 ? (oneTurn ? 12 : 0) : (L == 16 ? on16 : 16));
     return a.nnz >= shortest * a.rows;
 }
 
