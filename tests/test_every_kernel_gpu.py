@@ -479,6 +479,24 @@ def test_spmm_slab_kernel_with_64_bit_gather_addresses_every_width(osa, gpu_ctx,
         torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("types", ["f32", "f16_f16", "f16_f32"])
+def test_spmm_pipelined_rows_with_64_bit_gather_addresses_every_width(osa, gpu_ctx, types, monkeypatch):
+    """The same B of 4 GiB under rows of 10 - 50 entries worked whole by a lane group: SpmmRowPipelineKernel<..., V, L, false>
+    for L = 2 .. 32."""
+    monkeypatch.setenv("OPS_SPARSE_SPMM_NO_SLAB", "1")
+    monkeypatch.setenv("OPS_SPARSE_SPMM_NO_NARROW", "1")
+    m, k = 1200, 1 << 20
+    ldb = 4096 // torch.empty(0, dtype=SPMM_TYPES[types][0]).element_size()
+    rng = np.random.default_rng(5)
+    used = np.unique(np.concatenate([[0, k - 1], rng.integers(0, k, 4094)])).astype(np.int64)
+    for n in _spmm_widths(types)[:5]:
+        p = RawSpmm(osa, gpu_ctx, types, m, k, n, rng.integers(10, 51, m), seed=n, used_rows=used, ldb=ldb)
+        assert p.d_B.numel() * p.d_B.element_size() == 1 << 32 and p.nnz >= 24 * m
+        p.launch_and_check(p.analyse(), 1.5, -0.5)
+        del p
+        torch.cuda.empty_cache()
+
+
 NARROW_WIDTHS = {"f32": (4, 8), "f16_f16": (8, 16), "f16_f32": (8, 16)}      # one and two 16-byte pieces a row of B
 
 

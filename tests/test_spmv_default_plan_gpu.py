@@ -1,7 +1,7 @@
 """The plan aclsparseSpMVPreprocess picks for ACL_SPARSE_SPMV_ALG_DEFAULT on a large matrix with scattered
 columns: the ordered blocked-gather layout with live values (BLOCKED_GATHER, the same bits from every call), and for a
-matrix that it refuses - a row of more than 65 534 entries whose columns do not ascend - with op(A) = A and
-floating-point values the one whose row blocks add with atomics (BLOCKED_LIVE), in the same buffer; not with
+matrix that it refuses - a row of more than 65 534 entries whose columns do not ascend, or chunks too short for it -
+with op(A) = A and floating-point values the one whose row blocks add with atomics (BLOCKED_LIVE), in the same buffer; not with
 OPS_SPARSE_SPMV_REPEATABLE in the environment, for int32 values or under aclsparseSpMVOp, which ask for room for the
 ordered layout alone.  The contract under test: a caller that follows the
 reference's call pattern (GetBufferSize, Preprocess, SpMV with the default algorithm) may change the values in
@@ -572,12 +572,13 @@ def _value_flag(osa, dtype):
 
 @pytest.mark.parametrize("dtype,narrow_y", [(torch.float32, False), (torch.float16, False), (torch.float16, True),
                                             (torch.bfloat16, True)])
-def test_default_plan_for_the_transposed_product(osa, gpu_ctx, dtype, narrow_y):
-    """y = alpha * A^T x + beta * y with the default algorithm on a matrix whose updates of y are scattered:
-    Preprocess transposes A into the buffer, keeps for every entry of the copy where its value sits in csrValues,
+def test_default_plan_for_the_transposed_product(osa, gpu_ctx, dtype, narrow_y, monkeypatch):
+    """y = alpha * A^T x + beta * y with the default algorithm, asked for repeatable sums, on a matrix whose updates of y
+    are scattered: Preprocess transposes A into the buffer, keeps for every entry of the copy where its value sits in csrValues,
     and every call refreshes the copy's values from the caller's array before it runs the ordered kernels (no atomics
     on y).  Values changed in place and a replaced values array are followed; the transposed plan does not serve
     op(A) = A (that call runs without it, same buffer)."""
+    monkeypatch.setenv("OPS_SPARSE_SPMV_REPEATABLE", "1")
     dev, stream, handle = gpu_ctx
     L = osa.lib()
     rows, cols = 1_400_000, 300_000                          # A^T: 300 000 rows, x of 1.4 M elements
