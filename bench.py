@@ -354,6 +354,28 @@ def make_config(wl, torch, dev, which, scale):
     return cfg
 
 
+def live_layout_of(osa, torch, dev, stream, A, tflag):
+    """The layout with live values that Preprocess builds for A, by the raw analyses it makes in the same order: (name,
+    resident bytes)."""
+    import ctypes
+    L, rows, cols, nnz = osa.lib(), A["rows"], A["cols"], int(A["colind"].numel())
+    live = tflag | osa.OPSPARSE_BLOCKED_LIVE_VALUES
+    ptrs = [ctypes.c_void_p(A[k].data_ptr()) for k in ("rowptr", "colind", "values")]
+    sp, plan = ctypes.c_void_p(stream.cuda_stream), osa.OpsparseSpmvPlan()
+    if tflag and not any(k in os.environ for k in ("OPS_SPARSE_SPMV_REPEATABLE", "OPS_SPARSE_SPMV_NO_SCATTER")):
+        need = L.opsparse_spmv_csr_scatter_workspace_bytes(rows, cols, nnz, live)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+        if need and L.opsparse_spmv_csr_scatter_analyse(*ptrs[:2], rows, cols, nnz, live, ctypes.c_void_p(ws.data_ptr()), need,
+                                                        ctypes.byref(plan), sp) == osa.OPSPARSE_OK:
+            return "scatter_live", L.opsparse_spmv_csr_scatter_resident_bytes(rows, cols, nnz, live)
+    need = L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, live)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    if need and L.opsparse_spmv_csr_blocked_analyse(*ptrs, rows, cols, nnz, live, ctypes.c_void_p(ws.data_ptr()), need,
+                                                    ctypes.byref(plan), sp) == osa.OPSPARSE_OK:
+        return "blocked_gather_live_values", L.opsparse_spmv_csr_blocked_resident_bytes(rows, cols, nnz, live)
+    return "blocked_live_atomics", L.opsparse_spmv_csr_live_resident_bytes(rows, cols, nnz)
+
+
 def run_workload(args, osa, wl, torch, dev, stream, handle, key, cpu_cache):
     """One workload: Preprocess once, then rounds of `--steps` calls; returns the fields of its JSON object."""
     which, layout, transpose, env = WORKLOADS[key]
@@ -408,7 +430,8 @@ def run_workload(args, osa, wl, torch, dev, stream, handle, key, cpu_cache):
             preprocess_ms = dt      # GetBufferSize + buffer allocation + Preprocess: what a second matrix costs
         sets.append((op, out_t))
     if not is_spmm:
-        # which plan Preprocess chose shows in the buffer it asked for
+        # whether Preprocess took a re-stored layout shows in the buffer it asked for, and which one from the plan that the
+        # same analysis makes of the same arrays
         L = osa.lib()
         got = sets[0][0].buffer.numel() if sets[0][0].buffer is not None else 0
         tflag = osa.OPSPARSE_BLOCKED_TRANSPOSE if transpose else 0
@@ -421,21 +444,8 @@ def run_workload(args, osa, wl, torch, dev, stream, handle, key, cpu_cache):
         resident = None
         if layout == "blocked_gather":
             resident = L.opsparse_spmv_csr_blocked_resident_bytes(rows, cols, nnz, tflag)
-        elif layout == "csr" and atomics_live and got == atomics_live:
-            # the default algorithm found the gathers scattered: live values, row blocks summed with LDS atomics
-            layout = "blocked_live_atomics"
-            resident = L.opsparse_spmv_csr_live_resident_bytes(rows, cols, nnz)
-        elif layout == "csr" and ordered_live and got == ordered_live:
-            # ... or the same with every row summed in a fixed order (asked for, op(A) = A^T, int32)
-            layout = "blocked_gather_live_values"
-            resident = L.opsparse_spmv_csr_blocked_resident_bytes(rows, cols, nnz,
-                                                                  tflag | osa.OPSPARSE_BLOCKED_LIVE_VALUES)
-            scatter = L.opsparse_spmv_csr_scatter_resident_bytes(rows, cols, nnz, 0) if transpose else 0
-            if scatter and "OPS_SPARSE_SPMV_REPEATABLE" not in os.environ and "OPS_SPARSE_SPMV_NO_SCATTER" not in os.environ:
-                # op(A) = A^T where the last bit may vary: inside the same buffer Preprocess builds the layout that
-                # sorts the products by output panel (no column of the benchmark matrices is full enough to refuse it)
-                layout = "scatter_live"
-                resident = scatter
+        elif layout == "csr" and got and got in (atomics_live, ordered_live):
+            layout, resident = live_layout_of(osa, torch, dev, stream, A, tflag)
         ncols = 1
         bytes_alg = wl.spmv_bytes_alg(rows, cols, nnz, vb, 4, 4, beta != 0)
         bytes_gather = wl.spmv_bytes_gather(rows, cols, nnz, vb, 4, 4, beta != 0)
