@@ -297,18 +297,22 @@ aclsparseStatus_t aclsparseDnMatSetValues(aclsparseDnMatDescr_t dnMatDescr, void
  * kernel on the handle's stream, uses the handle's workspace (created on first
  * use) and synchronises the stream once; inside a stream capture it does none of
  * that and answers the ordinary plan's size.  Preprocess synchronises the stream
- * (once for the ordinary plan, up to four times for a re-stored layout) and
+ * (once for the ordinary plan; where a layout is re-stored, for the sample, up to
+ * four times an analysis, and for a second whole analysis where the matrix turns
+ * out not to be one for the first layout) and
  * must not be captured; aclsparseSpMV itself only enqueues kernels.
  *
  * Repeatability [ref: include/cann_ops_sparse.h:151-164]: ACL_SPARSE_SPMV_CSR_ALG2
  * gives bit-wise the same y from every call on the same data, for either op(A)
  * (the reference promises it for op(A) = A only).  So do ALG_DEFAULT / CSR_ALG1
  * with op(A) = A wherever the plan is row-wise or merge-path (every unprepared
- * call, every matrix under 7 M entries or with local columns) and for int32.
- * The plans that add in the order their wavefronts arrive are the default
- * algorithm's re-stored layouts on floating-point data (op(A) = A: row blocks
- * summed with LDS atomics; op(A) = A^T over more than 2 M columns: products
- * sorted by output panel and summed with LDS atomics) and op(A) = A^T without
+ * call, every matrix under 7 M entries or with local columns), for int32, and
+ * for nearly every re-stored matrix.  The plans that add in the order their
+ * wavefronts arrive are, on floating-point data with the default algorithm,
+ * op(A) = A where the ordered layout refuses the matrix (a row of more than
+ * 65 534 entries in descending order of columns, say: row blocks summed with LDS
+ * atomics), the re-stored op(A) = A^T over more than 2^18 columns (products
+ * sorted by output panel and summed with LDS atomics), and op(A) = A^T without
  * Preprocess (fp32 atomics on y): there the last bit of an element may differ
  * between two calls, as the reference says of CSR_ALG1.
  * OPS_SPARSE_SPMV_REPEATABLE=1 in the environment makes Preprocess choose

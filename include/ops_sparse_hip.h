@@ -210,9 +210,12 @@ int opsparse_spmv_csr_panels_analyse(const int32_t *rowOffsets, const int32_t *c
  *       are then stored a second time panel by panel, which halves what they cost.  Frozen values are kept in the
  *       order the second kernel streams them (plan->streamedBlocks = 1: row blocks of 2^10 rows, a wavefront
  *       each) where a (panel, block) chunk then still holds 16 entries, a row at most 12 a panel on average, and the
- *       rows are not so uneven that many entries lie in rows that meet themselves in one instruction of the stream;
- *       else, like live values, they are read in row order through a window in LDS by a workgroup a block of 2^12
- *       rows (which cannot hold a row of more than 65 534 entries: see OPSPARSE_E_UNSUPPORTED below).
+ *       rows are not so uneven that many entries lie in rows that meet themselves in one instruction of the stream
+ *       (the mean length of an entry's row against the mean row's, weighed against the chunks' length where these are
+ *       short); else, like live values, they are read in row order through a window in LDS by a workgroup a block of
+ *       2^10, 2^11 or 2^12 rows, the smallest whose chunks are long enough (which cannot hold a row of more than
+ *       65 534 entries: see OPSPARSE_E_UNSUPPORTED below).  Frozen rows of 13 to 16 entries a panel, or uneven ones,
+ *       that the windowed blocks refuse are streamed.
  *   OPSPARSE_BLOCKED_TRANSPOSE (= 1, so that a plain 0 / 1 "transpose" still reads right)  the layout of
  *       y = alpha * A^T * x + beta * y: the analysis transposes the matrix into the workspace (the CSC arrays of A
  *       are the CSR arrays of A^T) and builds the layout of that copy; no atomics on y.  With live values it keeps
@@ -223,8 +226,10 @@ int opsparse_spmv_csr_panels_analyse(const int32_t *rowOffsets, const int32_t *c
  * summed by the first kernel instead of going through the row blocks.  Returns OPSPARSE_E_INVALID for a column
  * index outside [0, cols), OPSPARSE_E_UNSUPPORTED for a matrix with a row of more than 65 534 entries that cannot
  * go the long rows' way (its columns do not ascend) where the blocks are the windowed ones.  Synchronises `stream`
- * twice (once more for op(A) = A^T, and for frozen values) and allocates nothing.  Launches touch only the first opsparse_spmv_csr_blocked_resident_bytes() of the workspace; the rest
- * serves the analysis and may be handed back afterwards.
+ * twice (once more for op(A) = A^T, and once more where it measures how uneven frozen rows are; a matrix that the
+ * windowed blocks refuse and the stream takes is analysed twice) and allocates nothing.  Launches touch only the first
+ * opsparse_spmv_csr_blocked_resident_bytes() of the workspace; the rest serves the analysis and may be handed back
+ * afterwards.
  */
 #define OPSPARSE_BLOCKED_TRANSPOSE 1
 #define OPSPARSE_BLOCKED_LIVE_VALUES 2
@@ -248,8 +253,9 @@ int opsparse_spmv_csr_blocked_analyse_split(const int32_t *rowOffsets, const int
  * BLOCKED_LIVE analysis (fp32, fp16 or bf16 values and x, op(A) = A, values read in place at every launch): the
  * layout of the plan kernel OPSPARSE_SPMV_BLOCKED_LIVE, whose second kernel adds into LDS with atomics in the order
  * the wavefronts get there.  The two byte counts are room for it and, in its place, for the BLOCKED_GATHER layout with
- * live values of the same matrix.  Same applicability bounds as BLOCKED_GATHER
- * except that a chunk needs 8 entries on average; `flags`: OPSPARSE_BLOCKED_VALUES_F16 / _BF16 only.  Synchronises
+ * live values of the same matrix, which is taken first where the default algorithm asks for this one; what is left to it
+ * are the matrices that BLOCKED_GATHER refuses, among them those whose (panel, block) chunks are too short there: its
+ * blocks hold up to 2^12 rows and 20 000 entries, and a chunk of these needs 8 entries on average; `flags`: OPSPARSE_BLOCKED_VALUES_F16 / _BF16 only.  Synchronises
  * `stream` twice.  No counterpart in the reference.
  */
 size_t opsparse_spmv_csr_live_workspace_bytes(int64_t rows, int64_t cols, int64_t nnz);

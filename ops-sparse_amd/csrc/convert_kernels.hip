@@ -1856,8 +1856,8 @@ int opsparse_csr2csc_launch(int64_t m, int64_t n, int64_t nnz, const void *csrVa
     // Stable sort by column of (column; row, value): the pair travels with its key, 8 bytes a pass and entry more
     // than a source position would, and the last pass writes rows and values where they belong — no gather by
     // position at the end, which cost two cache-line fills per entry (33.5 M entries: 2.9 -> 1.9 ms).
-    // Up to eight bits a pass, the tile ordered through LDS before it leaves (33.5 M entries over 2^20 columns:
-    // three passes instead of five, 1.2 ms).
+    // Up to ten bits a pass (WidePassesOf), the tile ordered through LDS before it leaves (33.5 M entries over 2^20
+    // columns: three passes of seven bits, 0.78 ms).
     const auto [passes, perPass] = WidePassesOf(KeyBits(n), nnz);
     const RadixPairIo io{rowOfPos, csrVal, cscRowInd, cscVal, valueBytes};
     const int32_t *keysIn = csrColInd;
@@ -1885,11 +1885,13 @@ int opsparse_csr2csc_launch(int64_t m, int64_t n, int64_t nnz, const void *csrVa
 //
 // aclsparseXcoosortByRow / ByColumn (sparse/coosort/arch35/coosort_host.cpp:309-371; the order is the one of
 // test/coosort/arch35/coosort_golden.h:52-85): a stable sort of (primary, secondary, P) triples, signed keys,
-// ascending in the primary key and, among equal ones, in the secondary.  Least-significant-key first: the 8-bit
+// ascending in the primary key and, among equal ones, in the secondary.  Least-significant-key first: the wide
 // passes of csr2csc over the secondary key, the primary key and P travelling as the pair, then over the primary
-// key with the secondary key and P as the pair; the last pass writes the caller's three arrays.  The keys are
-// taken relative to their minimum, found on the device first, so that a pass count follows from the range the
-// indices really span (one read-back of four integers: the call synchronises its stream once).
+// key with the secondary key and P as the pair; the last pass writes the caller's three arrays.  Where there are
+// 2^20 entries or more and a sample says that they lie in short rows, the passes run over the primary key only and
+// csrsort's kernels order each row in place (kRowsFirstLongest).  The keys are taken relative to their minimum,
+// found on the device first, so that a pass count follows from the range the indices really span (one read-back of
+// five integers, the ranges and the sample's count: the call synchronises its stream once).
 
 }  // extern "C"
 

@@ -178,7 +178,8 @@ void TrimToWorkspace(aclsparseHandle_t handle, RestoredChoice *choice, int64_t r
 // entries or more, an x the layout applies to, and a sample of the columns that says the gathers are scattered:
 // one short kernel and a synchronisation of the handle's stream), else none.  `repeatable`: the caller promises
 // the same bits from every execution (aclsparseSpMVOp): BLOCKED_GATHER; else BLOCKED_LIVE where it exists
-// (op(A) = A, floating-point values), which AnalyseRestored takes for what BLOCKED_GATHER refuses.
+// (op(A) = A, floating-point values): the same ordered layout in a buffer with room for either, and only for a matrix
+// that it refuses (AnalyseRestored) the one that adds with LDS atomics.
 RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffsets, const int32_t *colInd, int64_t rows,
                               int64_t cols, int64_t nnz, bool transpose, int32_t valueType, bool repeatable);
 // The size-query record of a matrix (OpsparseSpmvSized): written by the queries, asked by Preprocess / createDescr.

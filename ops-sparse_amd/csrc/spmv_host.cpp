@@ -273,9 +273,12 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
     if (off || rowOffsets == nullptr || colInd == nullptr) {
         return {0, 0, false};
     }
-    // Below 7 M entries the merge path on the caller's own arrays is as fast or faster (1 M rows x 4 entries: 30 us
-    // against 44 with the layout; 1.5 M x 4: 51 against 57; 2 M x 4: 87 against 71).  Tuning override, read at
-    // every call: OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ.
+    // Below 7 M entries the row-wise kernels on the caller's own arrays run, which need no analysis and no buffer.  They
+    // are the faster ones over a small x only (fp32, rows of 8 scattered entries, us a call, row-wise / layout: 2.1 M
+    // entries over 300 K columns 14 / 19, 1.1 M 19 / 19, 2 M 26 / 19, 8 M 40 / 23; 4 M entries 24 / 28, 30 / 29,
+    // 42 / 29, 69 / 31; 6.5 M entries 36 / 37, 45 / 37, 66 / 37, 109 / 41): with the present kernels the layout is ahead
+    // from about 1.5 M columns at any of these sizes, so the line is a cautious one.  Tuning override, read at every
+    // call: OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ.
     const char *minEnv = std::getenv("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ");
     if (nnz < (minEnv != nullptr ? std::atoll(minEnv) : kMinDefaultNnz)) {
         return {0, 0, false};
