@@ -1075,13 +1075,14 @@ __device__ __forceinline__ void SortRowInGroup(int64_t begin, int64_t len, int32
 constexpr int kSortRowsPerGroup = 8;
 
 template <int G, bool Packed>
-__global__ __launch_bounds__(kBlockThreads) void SortShortRowsKernel(const int32_t *__restrict__ rowPtr, int64_t m,
-                                                                    int64_t nnz, int32_t base, int32_t *colInd,
-                                                                    int32_t *perm, int32_t *counters,
-                                                                    int32_t *__restrict__ midList,
-                                                                    int32_t *__restrict__ longList)
+__global__ __launch_bounds__(kBlockThreads, 8) void SortShortRowsKernel(const int32_t *__restrict__ rowPtr, int64_t m,
+                                                                       int64_t nnz, int32_t base, int32_t *colInd,
+                                                                       int32_t *perm, int32_t *counters,
+                                                                       int32_t *__restrict__ midList,
+                                                                       int32_t *__restrict__ longList)
 {
     constexpr int R = kSortRowsPerGroup;
+    constexpr int kWaveRows = kWave / G * R;  // rows of a wavefront
     const int32_t g = threadIdx.x % G;
     const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * (kBlockThreads / G) + threadIdx.x / G) * R;
     int32_t off[R + 1];
@@ -1091,7 +1092,11 @@ __global__ __launch_bounds__(kBlockThreads) void SortShortRowsKernel(const int32
     }
     int64_t begin[R], len[R];
     int32_t col[R], pay[R];
-    uint32_t mids = 0, longs = 0;  // the group's rows for the lists
+    // The wavefront's rows for midList from the front, for longList from the back; how many.
+    __shared__ int32_t listed[kBlockThreads / kWave][kWaveRows];
+    __shared__ int32_t counts[kBlockThreads / kWave][2];
+    const int32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    int32_t nMid = 0, nLong = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int64_t row = row0 + r;
@@ -1104,16 +1109,57 @@ __global__ __launch_bounds__(kBlockThreads) void SortShortRowsKernel(const int32
                 len[r] = 0;  // nothing to sort, or bounds that do not describe a range of the arrays
             }
         }
-        if (len[r] > G) {
-            mids |= len[r] <= kSortWaveRow && g == 0 ? 1u << r : 0u;
-            longs |= len[r] > kSortWaveRow && g == 0 ? 1u << r : 0u;
-            len[r] = 0;
+        if (__ballot(len[r] > G) != 0) {
+            const bool mid = g == 0 && len[r] > G && len[r] <= kSortWaveRow, isLong = g == 0 && len[r] > kSortWaveRow;
+            const uint64_t inMid = __ballot(mid), inLong = __ballot(isLong), below = (uint64_t{1} << lane) - 1;
+            if (mid) {
+                listed[wave][nMid + __popcll(inMid & below)] = static_cast<int32_t>(row);
+            } else if (isLong) {
+                listed[wave][kWaveRows - 1 - nLong - __popcll(inLong & below)] = static_cast<int32_t>(row);
+            }
+            nMid += __popcll(inMid);
+            nLong += __popcll(inLong);
+            len[r] = len[r] > G ? 0 : len[r];
         }
         col[r] = 0;
         pay[r] = 0;
         if (g < len[r]) {
             col[r] = colInd[begin[r] + g];
             pay[r] = perm[begin[r] + g];
+        }
+    }
+    // The workgroup's rows take their places in the lists with one addition a list, while the entries are on their way.
+    // An addition a row, to the same two words, was served one after the other, 10 ns each (33 M entries, 4.4 random ones a
+    // row, of which 4 % of the rows do not fit eight lanes: 3116 us, 422 now).  Behind the sort, with barriers that wait for
+    // its stores, this cost equal rows up to 8 % (2 M rows of 13: 156 us without any lists, 167, 158 now; 4 M of 5: 135,
+    // 145, 136); with counters in LDS and the work left to the wavefront that arrives last, half as much.  So a wavefront has a
+    // piece of LDS and counts of its own, and one barrier, of LDS alone, is all they share.  Eight wavefronts a SIMD, as
+    // without lists.
+    if (lane < 2) {
+        counts[wave][lane] = lane == 0 ? nMid : nLong;
+    }
+    LdsBarrier();
+    if (wave < 2) {
+        // wavefront 0 writes midList, wavefront 1 longList
+        int32_t all = 0;
+#pragma unroll 1
+        for (int w = 0; w < kBlockThreads / kWave; ++w) {
+            all += counts[w][wave];
+        }
+        if (all > 0) {
+            int32_t at = 0;
+            if (lane == 0) {
+                at = atomicAdd(counters + wave, all);
+            }
+            at = __shfl(at, 0);
+#pragma unroll 1
+            for (int w = 0; w < kBlockThreads / kWave; ++w) {
+                const int32_t n = counts[w][wave];
+                for (int32_t i = lane; i < n; i += kWave) {
+                    (wave == 0 ? midList : longList)[at + i] = listed[w][wave == 0 ? i : kWaveRows - 1 - i];
+                }
+                at += n;
+            }
         }
     }
     // every lane takes part in the shuffles; groups without a row sort padding
@@ -1123,35 +1169,6 @@ __global__ __launch_bounds__(kBlockThreads) void SortShortRowsKernel(const int32
         if (g < len[r]) {
             colInd[begin[r] + g] = col[r];
             perm[begin[r] + g] = pay[r];
-        }
-    }
-    // The listed rows of a workgroup take their places with one addition a list.  An addition a row, to the same two words,
-    // was served one after the other, 10 ns each: with 4.4 random entries a row, of which 4 % of the rows do not fit eight
-    // lanes, coosort of 33 M entries took 4257 us, 1552 now (2780 by the passes over both keys); equal rows as before.
-    __shared__ int32_t count[2], first[2];
-    if (threadIdx.x < 2) {
-        count[threadIdx.x] = 0;
-    }
-    __syncthreads();
-    int32_t at[2] = {0, 0};
-    if (mids != 0) {
-        at[0] = atomicAdd(&count[0], __popc(mids));
-    }
-    if (longs != 0) {
-        at[1] = atomicAdd(&count[1], __popc(longs));
-    }
-    __syncthreads();
-    if (threadIdx.x < 2 && count[threadIdx.x] > 0) {
-        first[threadIdx.x] = atomicAdd(counters + threadIdx.x, count[threadIdx.x]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if ((mids >> r & 1u) != 0) {
-            midList[first[0] + at[0]++] = static_cast<int32_t>(row0 + r);
-        }
-        if ((longs >> r & 1u) != 0) {
-            longList[first[1] + at[1]++] = static_cast<int32_t>(row0 + r);
         }
     }
 }
