@@ -71,12 +71,11 @@ struct OpsparseSpmmBinding {
     int64_t stagingBytes = 0;  // room behind the plan's tables for row-major copies of B / C (0: none)
     int64_t widestN = 0;       // the widest C the buffer has been analysed for: its tables fit that width and less
     // One or two columns of B and C that are vectors in memory run as SpMV calls: their plan, and where in the
-    // buffer its workspace lies (0: the buffer was not preprocessed for such operands).
+    // buffer its workspace lies (0 bytes: the buffer was not preprocessed for such operands).
     OpsparseSpmvPlan vectorPlan{};
     int64_t vectorOff = 0;
     int64_t vectorBytes = 0;
-    // Rows that repeat: where in the buffer their lists lie (0: none), and how many lists and distances there are.
-    int64_t offsetOff = 0;
+    // Rows that repeat: how many lists, which lie at the start of the buffer (0: none), and distances there are.
     int32_t offsetPatterns = 0, offsetDistances = 0;
     int64_t offsetReach = 0;  // the furthest distance
     int32_t offsetRuns = 0;   // how the distances fall into runs

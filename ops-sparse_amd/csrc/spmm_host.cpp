@@ -237,6 +237,29 @@ bool PrefersWholeRows(const aclsparseSpMatDescr *A, const OpsparseSpmmPlan &plan
     return scattered < 250;
 }
 
+int64_t Align256(int64_t v)
+{
+    return (v + 255) / 256 * 256;
+}
+
+// Bytes at the start of the buffer for the lists of a matrix whose rows repeat, or for the SpMV plan that one or two columns
+// run under.  By the sizes of A alone, not by the operands: a buffer sized for a wide B serves a narrower one, and nothing
+// tells Preprocess which operands the buffer it is given was sized for.  (0: no such matrix by its sizes; the SpMV plan
+// then lies behind everything else, in buffers sized for such columns.)
+int64_t FrontBytes(const aclsparseSpMatDescr *A)
+{
+    return (A->valueType == ACL_FLOAT || A->valueType == ACL_FLOAT16) &&
+                   opsparse_spmv_csr_offsets_workspace_bytes(A->rows, A->cols, A->nnz) > 0
+               ? Align256(static_cast<int64_t>(opsparse_spmv_csr_workspace_bytes(A->rows, A->nnz)))
+               : 0;
+}
+
+// Where the plan's tables, and the staging area behind them, begin.
+void *Tables(const aclsparseSpMatDescr *A, void *buffer)
+{
+    return static_cast<unsigned char *>(buffer) + FrontBytes(A);
+}
+
 // Row statistics and long-row tables for width n into `buffer`; binds the buffer to A.
 aclsparseStatus_t BuildPlan(const aclsparseSpMatDescr *A, int64_t n, int64_t elemBytes, void *buffer,
                             hipStream_t stream)
@@ -252,43 +275,34 @@ aclsparseStatus_t BuildPlan(const aclsparseSpMatDescr *A, int64_t n, int64_t ele
     // Nothing says how large the caller's buffer is: it was sized by GetBufferSize for this matrix and width, and the
     // analysis lays out exactly what GetBufferSize counted (one reduction over the row offsets, no allocation).
     const size_t bytes = static_cast<size_t>(INT64_MAX);
-    const int rc = opsparse_spmm_csr_analyse(static_cast<const int32_t *>(A->rowOffsets), A->rows, A->nnz, n, buffer,
+    void *const tables = Tables(A, buffer);
+    const int rc = opsparse_spmm_csr_analyse(static_cast<const int32_t *>(A->rowOffsets), A->rows, A->nnz, n, tables,
                                              bytes, OPSPARSE_SPMM_AUTO, &plan, stream);
     if (rc != OPSPARSE_OK) {
         opsparse::LogError("aclsparseSpMM: analysis failed (%d)", rc);
         return FromLaunch(rc);
     }
     const int32_t maxRow = plan.maxRowNnz;
-    if (PrefersWholeRows(A, plan, n, elemBytes, buffer, stream)) {
+    if (PrefersWholeRows(A, plan, n, elemBytes, tables, stream)) {
         // a plan without tables: the launch layer then takes a lane group a row
         const int again = opsparse_spmm_csr_analyse(static_cast<const int32_t *>(A->rowOffsets), A->rows, A->nnz, n,
-                                                    buffer, bytes, OPSPARSE_SPMM_ROW_SPLIT, &plan, stream);
+                                                    tables, bytes, OPSPARSE_SPMM_ROW_SPLIT, &plan, stream);
         if (again != OPSPARSE_OK) {
             return FromLaunch(again);
         }
     }
-    A->spmm.widestN = (A->spmm.buffer == buffer && A->spmm.widestN > n) ? A->spmm.widestN : n;
+    if (A->spmm.buffer != buffer) {
+        A->spmm.widestN = 0;
+        A->spmm.offsetPatterns = 0;
+    }
+    A->spmm.widestN = A->spmm.widestN > n ? A->spmm.widestN : n;
     A->spmm.buffer = buffer;
     A->spmm.plan = plan;
     A->spmm.stagingBytes = 0;
     A->spmm.vectorOff = 0;
     A->spmm.vectorBytes = 0;
-    A->spmm.offsetOff = 0;
     A->spmm.maxRowNnz = maxRow;
     return ACL_SPARSE_STATUS_SUCCESS;
-}
-
-int64_t Align256(int64_t v)
-{
-    return (v + 255) / 256 * 256;
-}
-
-// Room for the lists of a matrix whose rows repeat (0: not for these operands).
-size_t OffsetBytes(const aclsparseSpMatDescr *A, const aclsparseDnMatDescr *C, const SpmmTypes &t)
-{
-    return C->cols >= 1 && C->cols <= opsparse::kOffsetMaxColumns && t.valType != OPSPARSE_I8
-               ? opsparse_spmv_csr_offsets_workspace_bytes(A->rows, A->cols, A->nnz)
-               : 0;
 }
 
 bool ScalarIsZero(const void *host, aclDataType computeType)
@@ -301,15 +315,14 @@ bool ScalarIsZero(const void *host, aclDataType computeType)
 bool OffsetsTake(const aclsparseSpMatDescr *A, int64_t n, int64_t ldb, int64_t ldc, const void *B, const void *C,
                  const SpmmTypes &t)
 {
-    return A->spmm.offsetOff > 0 && A->nnz > 0 && opsparse::OffsetSpmmTakes(n, ldb, ldc, B, C, t.valType, t.cType);
+    return A->spmm.offsetPatterns > 0 && A->nnz > 0 && opsparse::OffsetSpmmTakes(n, ldb, ldc, B, C, t.valType, t.cType);
 }
 int RunOffsets(const aclsparseSpMatDescr *A, int64_t n, int64_t ldb, int64_t ldc, const void *B, void *C,
                OpsparseScalar alpha, OpsparseScalar beta, const SpmmTypes &t, const void *buffer, hipStream_t stream)
 {
     const opsparse::OffsetSpmmArgs a{static_cast<const int32_t *>(A->rowOffsets), A->values, B, C, A->rows, A->cols, n,
                                      A->nnz, ldb, ldc, alpha, beta,
-                                     static_cast<const unsigned char *>(buffer) + A->spmm.offsetOff,
-                                     A->spmm.offsetPatterns, A->spmm.offsetDistances, A->spmm.offsetReach, A->spmm.offsetRuns, stream};
+                                     static_cast<const unsigned char *>(buffer), A->spmm.offsetPatterns, A->spmm.offsetDistances, A->spmm.offsetReach, A->spmm.offsetRuns, stream};
     return opsparse::LaunchOffsetSpmm(a, t.valType, t.cType);
 }
 
@@ -319,7 +332,7 @@ int RunStaged(const Staging &g, const aclsparseSpMatDescr *A, const aclsparseDnM
               const aclsparseDnMatDescr *C, aclsparseOperation_t opB, OpsparseScalar alpha, OpsparseScalar beta,
               const SpmmTypes &t, bool betaIsZero, void *buffer, hipStream_t stream)
 {
-    auto *base = static_cast<unsigned char *>(buffer);
+    auto *base = static_cast<unsigned char *>(Tables(A, buffer));
     const int64_t k = A->cols, m = A->rows, n = C->cols;
     const bool bColMajor = (B->order == ACL_SPARSE_ORDER_COL) != (opB == ACL_SPARSE_OP_TRANSPOSE);
     const bool cColMajor = C->order == ACL_SPARSE_ORDER_COL;
@@ -352,7 +365,7 @@ int RunStaged(const Staging &g, const aclsparseSpMatDescr *A, const aclsparseDnM
         rc = opsparse_spmm_csr_launch(&A->spmm.plan, static_cast<const int32_t *>(A->rowOffsets),
                                       static_cast<const int32_t *>(A->colInd), A->values, bUse, cUse, m, k, nRun, A->nnz,
                                       ldb, ldc, 0, g.c ? 0 : (cColMajor ? 1 : 0), 0, alpha, beta, t.valType, t.cType,
-                                      buffer, static_cast<size_t>(A->spmm.plan.bytes), stream);
+                                      base, static_cast<size_t>(A->spmm.plan.bytes), stream);
     }
     if (rc == OPSPARSE_OK && g.c) {
         rc = opsparse_dense_restage(cUse, C->values, m, n, n, g.nPadded, 0, C->ld, cColMajor ? 1 : 0,
@@ -389,12 +402,12 @@ aclsparseStatus_t aclsparseSpMMGetBufferSize(aclsparseHandle_t handle, aclsparse
                                                      handle != nullptr ? handle->stream : nullptr, size);
     if (rc == OPSPARSE_OK) {
         *size += static_cast<size_t>(MakeStaging(matA, matB, matC, opB, t, static_cast<int64_t>(*size)).bytes);
-        if (ColumnsAreVectors(matA, matB, matC, opB, t)) {
+        if (const int64_t front = FrontBytes(matA)) {
+            *size += static_cast<size_t>(front);
+        } else if (ColumnsAreVectors(matA, matB, matC, opB, t)) {
             // behind everything else: the workspace of the SpMV plan the columns run under
             *size = static_cast<size_t>(Align256(static_cast<int64_t>(*size))) +
                     opsparse_spmv_csr_workspace_bytes(matA->rows, matA->nnz);
-        } else if (const size_t lists = OffsetBytes(matA, matC, t)) {
-            *size = static_cast<size_t>(Align256(static_cast<int64_t>(*size))) + lists;
         }
     }
     return FromLaunch(rc);
@@ -421,9 +434,11 @@ aclsparseStatus_t aclsparseSpMMPreprocess(aclsparseHandle_t handle, aclsparseOpe
     if (built == ACL_SPARSE_STATUS_SUCCESS) {
         // the buffer was sized by GetBufferSize for these operands: their staging area exists
         matA->spmm.stagingBytes = MakeStaging(matA, matB, matC, opB, t, matA->spmm.plan.bytes).bytes;
+        matA->spmm.offsetPatterns = 0;
+        const int64_t front = FrontBytes(matA);
         if (ColumnsAreVectors(matA, matB, matC, opB, t)) {
-            // (GetBufferSize counted this region for these operands)
-            const int64_t off = Align256(matA->spmm.plan.bytes + matA->spmm.stagingBytes);
+            // (GetBufferSize counted this region: at the start for every operand, or at the end for these)
+            const int64_t off = front > 0 ? 0 : Align256(matA->spmm.plan.bytes + matA->spmm.stagingBytes);
             const size_t bytes = opsparse_spmv_csr_workspace_bytes(matA->rows, matA->nnz);
             OpsparseSpmvPlan vectorPlan{};
             const int rc = opsparse_spmv_csr_analyse(static_cast<const int32_t *>(matA->rowOffsets), matA->rows,
@@ -439,20 +454,17 @@ aclsparseStatus_t aclsparseSpMMPreprocess(aclsparseHandle_t handle, aclsparseOpe
                 matA->spmm.vectorOff = off;
                 matA->spmm.vectorBytes = static_cast<int64_t>(bytes);
             }
-        } else if (OffsetBytes(matA, matC, t) > 0 && stream != nullptr && matA->colInd != nullptr &&
-                   std::getenv("OPS_SPARSE_SPMM_NO_OFFSETS") == nullptr) {
-            // (the same: behind the plan's tables and the staging area)
-            const int64_t off = Align256(matA->spmm.plan.bytes + matA->spmm.stagingBytes);
+        } else if (front > 0 && matC->cols >= 1 && matC->cols <= opsparse::kOffsetMaxColumns && stream != nullptr &&
+                   matA->colInd != nullptr && std::getenv("OPS_SPARSE_SPMM_NO_OFFSETS") == nullptr) {
             opsparse::OffsetFound found;
             const int rc = opsparse::AnalyseOffsetRows(static_cast<const int32_t *>(matA->rowOffsets),
                                                        static_cast<const int32_t *>(matA->colInd), matA->rows, matA->cols,
                                                        matA->nnz, matA->spmm.maxRowNnz,
-                                                       static_cast<unsigned char *>(buffer) + off, &found, stream);
+                                                       static_cast<unsigned char *>(buffer), &found, stream);
             if (rc != OPSPARSE_OK) {
                 return FromLaunch(rc);
             }
             if (found.patterns > 0) {
-                matA->spmm.offsetOff = off;
                 matA->spmm.offsetPatterns = found.patterns;
                 matA->spmm.offsetDistances = found.distances;
                 matA->spmm.offsetRuns = opsparse::OffsetRuns(found);
@@ -489,14 +501,15 @@ aclsparseStatus_t aclsparseSpMM(aclsparseHandle_t handle, aclsparseOperation_t o
     bool staged = bound && g.bytes > 0 && g.bytes <= matA->spmm.stagingBytes && matA->spmm.plan.n == g.nPadded &&
                   matA->nnz > 0;
     const OpsparseSpmmPlan *plan = &matA->spmm.plan;
+    void *const tables = Tables(matA, buffer);
     // A few row-major fp32 columns under a plan cut for the kernel for narrow B: that kernel reads and writes rows of
     // any width up to 8, leading dimension and 4-byte alignment where they are, and the copies through the staging
     // area are saved.
     const bool direct = staged && opB == ACL_SPARSE_OP_NON_TRANSPOSE && matB->order == ACL_SPARSE_ORDER_ROW &&
                         matC->order == ACL_SPARSE_ORDER_ROW &&
-                        opsparse_spmm_csr_narrow_rows(plan, buffer, matC->cols, matA->nnz, t.valType, t.cType) != 0;
+                        opsparse_spmm_csr_narrow_rows(plan, tables, matC->cols, matA->nnz, t.valType, t.cType) != 0;
     // Rows that repeat: the kernel for them takes row-major operands of any width where they are.
-    const bool vectors = bound && matA->spmm.vectorOff > 0 && matA->spmm.vectorPlan.rows == matA->rows &&
+    const bool vectors = bound && matA->spmm.vectorBytes > 0 && matA->spmm.vectorPlan.rows == matA->rows &&
                          matA->spmm.vectorPlan.nnz == matA->nnz && ColumnsAreVectors(matA, matB, matC, opB, t);
     const bool offsets = bound && !vectors && opB == ACL_SPARSE_OP_NON_TRANSPOSE && matB->order == ACL_SPARSE_ORDER_ROW &&
                          matC->order == ACL_SPARSE_ORDER_ROW &&
@@ -530,7 +543,7 @@ aclsparseStatus_t aclsparseSpMM(aclsparseHandle_t handle, aclsparseOperation_t o
     const OpsparseSpmmBinding &bind = matA->spmm;
     if (offsets) {
         rc = RunOffsets(matA, matC->cols, matB->ld, matC->ld, matB->values, matC->values, a, b, t, buffer, handle->stream);
-    } else if (vectors && bind.vectorOff > 0) {
+    } else if (vectors && bind.vectorBytes > 0) {
         const int64_t bStep = matB->order == ACL_SPARSE_ORDER_COL ? matB->ld : 0;
         const int64_t cStep = matC->order == ACL_SPARSE_ORDER_COL ? matC->ld : 0;
         rc = OPSPARSE_OK;
@@ -553,7 +566,7 @@ aclsparseStatus_t aclsparseSpMM(aclsparseHandle_t handle, aclsparseOperation_t o
             static_cast<const int32_t *>(matA->colInd), matA->values, matB->values, matC->values, matA->rows,
             matA->cols, matC->cols, matA->nnz, matB->ld, matC->ld, matB->order == ACL_SPARSE_ORDER_COL ? 1 : 0,
             matC->order == ACL_SPARSE_ORDER_COL ? 1 : 0, opB == ACL_SPARSE_OP_TRANSPOSE ? 1 : 0, a, b, t.valType,
-            t.cType, buffer, plan != nullptr ? static_cast<size_t>(plan->bytes) : 0, handle->stream);
+            t.cType, tables, plan != nullptr ? static_cast<size_t>(plan->bytes) : 0, handle->stream);
     }
     if (rc != OPSPARSE_OK) {
         opsparse::LogError("aclsparseSpMM: launch failed (%d)", rc);

@@ -228,6 +228,29 @@ def test_spmv_status_table(osa, L, handle):
 
 # --------------------------------------------------------------------- SpMM
 
+@pytest.mark.parametrize("value_type", ["ACL_FLOAT", "ACL_FLOAT16"])
+def test_spmm_buffer_of_any_width_holds_the_lists_of_every_other(osa, L, value_type):
+    """What Preprocess may write for one width has to fit what a size query for another answered: beside the plan's own 256
+    bytes the lists of a matrix whose rows repeat, or the SpMV plan of a single column, whichever is larger.  (2000 rows with
+    2000 entries: no row can be long, so the query does not touch the device.)"""
+    vt = getattr(osa, value_type)
+    _, A = make_csr(osa, L, rows=2000, cols=2000, nnz=2000, vt=vt)
+    room = L.opsparse_spmv_csr_workspace_bytes(2000, 2000)
+    assert room >= L.opsparse_spmv_csr_offsets_workspace_bytes(2000, 2000, 2000) > 2000
+    sizes = []
+    for n in (1, 8, 64, 256, 264, 512, 4096):
+        _, B = make_mat(osa, L, rows=2000, cols=n, ld=n, vt=vt)
+        _, C = make_mat(osa, L, rows=2000, cols=n, ld=n)
+        size = ctypes.c_size_t(0)
+        assert L.aclsparseSpMMGetBufferSize(*spmm_args(osa, None, A, B, C), ctypes.byref(size)) == 0
+        assert size.value >= room + 256, n
+        sizes.append(size.value)
+        L.aclsparseDestroyDnMat(B)
+        L.aclsparseDestroyDnMat(C)
+    assert sizes[2] == sizes[-1]                     # whole pieces: nothing in it depends on the width
+    L.aclsparseDestroySpMat(A)
+
+
 def spmm_args(osa, h, A, B, C, opa=0, opb=0, ct=None, alg=0):
     return (h, opa, opb, None, A, B, None, C, osa.ACL_FLOAT if ct is None else ct, alg)
 

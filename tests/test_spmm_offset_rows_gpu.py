@@ -147,6 +147,39 @@ def test_one_buffer_for_several_widths_and_live_values(osa, gpu_ctx):
         assert bool((buf[size.value:] == 0x77).all())
 
 
+@pytest.mark.parametrize("sized_for,then", [(512, 64), (260, 256), (512, 1), (64, 1), (1, 64)])
+def test_buffer_sized_for_another_width_holds_the_lists(osa, gpu_ctx, sized_for, then):
+    """GetBufferSize for one width, Preprocess and SpMM for another (one column: SpMV calls), in exactly that many bytes."""
+    dev, stream, handle = gpu_ctx
+    rng, rows = np.random.default_rng(3), 40_000
+    d = np.array([-200, -1, 0, 1, 200])
+    cols = np.arange(rows)[:, None] + d
+    ok = (cols >= 0) & (cols < rows)
+    rowptr, colind = np.concatenate([[0], np.cumsum(ok.sum(1))]).astype(np.int32), cols[ok].astype(np.int32)
+    val = rng.uniform(-1, 1, colind.size).astype(np.float32)
+    A = osa.Csr(rows, rows, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev))
+    one, none, size = ctypes.c_float(1.0), ctypes.c_float(0.0), ctypes.c_size_t(0)
+
+    def call(n):
+        B, C = rng.uniform(-1, 1, rows * n).astype(np.float32), to_dev(np.zeros(rows * n, np.float32), dev)
+        Bd, Cd = osa.DnMat(rows, n, n, to_dev(B, dev)), osa.DnMat(rows, n, n, C)
+        return B, C, (Bd, Cd), (handle.h, osa.ACL_SPARSE_OP_NON_TRANSPOSE, osa.ACL_SPARSE_OP_NON_TRANSPOSE, ctypes.byref(one), A.d,
+                                Bd.d, ctypes.byref(none), Cd.d, osa.ACL_FLOAT, osa.ACL_SPARSE_SPMM_ALG_DEFAULT)
+
+    _, _, keep, common = call(sized_for)
+    assert osa.lib().aclsparseSpMMGetBufferSize(*common, ctypes.byref(size)) == 0
+    buf = torch.full((size.value + (1 << 20),), 0x77, dtype=torch.uint8, device=dev)
+    for n in (then, sized_for):
+        B, C, keep, common = call(n)
+        if n == then:
+            assert osa.lib().aclsparseSpMMPreprocess(*common, buf.data_ptr()) == 0
+        assert osa.lib().aclsparseSpMM(*common, buf.data_ptr()) == 0
+        stream.synchronize()
+        gold = oracle.spmm_f64(rows, n, rowptr, colind, val, B, n, np.zeros(rows * n, np.float32), n, 1.0, 0.0)
+        assert oracle.max_rel_err(C.cpu().numpy(), gold) <= 1e-5
+    assert bool((buf[size.value:] == 0x77).all())
+
+
 @pytest.mark.parametrize("types,n", [("f32", 128), ("f32", 256), ("f16", 256), ("f16_f32", 256)])
 def test_five_scattered_distances_under_wide_b(osa, gpu_ctx, types, n):
     """Few distances that are no star's: one row a lane under 32 and 64 pieces as well."""
