@@ -358,6 +358,14 @@ aclsparseStatus_t aclsparseSpMV(aclsparseHandle_t handle, aclsparseOperation_t o
  * preprocesses into that buffer first.  buffer == NULL gives
  * INSUFFICIENT_RESOURCES.  alpha / beta follow the handle's pointer mode;
  * NULL is read as 0 [ref: spmm_host.cpp:62-74].
+ *
+ * The values of A, B and C are read where the caller has them at every call and
+ * may change between calls.  The sparsity structure of A may not, in place, after
+ * Preprocess: where the rows of A repeat (a mesh operator, as above under SpMV)
+ * Preprocess leaves a byte a row in the buffer and the calls read that instead of
+ * the column indices.  Call Preprocess again for another structure.
+ * Preprocess launches a few kernels, synchronises the stream (up to four times)
+ * and must not be captured.
  */
 aclsparseStatus_t aclsparseSpMMGetBufferSize(aclsparseHandle_t handle, aclsparseOperation_t opA,
                                              aclsparseOperation_t opB, const void *alpha,
@@ -400,7 +408,10 @@ aclsparseStatus_t aclsparseSpMM(aclsparseHandle_t handle, aclsparseOperation_t o
  *                 small matrix).
  *   createDescr   snapshots matA's pointers and sizes (not its values: they may
  *                 change between executions, except under ALG2); ALG2 needs
- *                 `buffer`, which must stay valid until destroyDescr.
+ *                 `buffer`, which must stay valid until destroyDescr.  Under
+ *                 ALG2, or with a buffer, the sparsity structure must stay as it
+ *                 was, too: executions may read what createDescr left in the
+ *                 buffer instead of the column indices.
  *   createPlan    only the identity epilogue: a non-NULL LTO buffer or a
  *                 non-zero size gives NOT_SUPPORTED.
  *   destroy*      NULL is accepted and gives SUCCESS.
