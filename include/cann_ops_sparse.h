@@ -309,13 +309,13 @@ aclsparseStatus_t aclsparseDnMatSetValues(aclsparseDnMatDescr_t dnMatDescr, void
  * Repeatability [ref: include/cann_ops_sparse.h:151-164]: ACL_SPARSE_SPMV_CSR_ALG2
  * gives bit-wise the same y from every call on the same data, for either op(A)
  * (the reference promises it for op(A) = A only).  So do ALG_DEFAULT / CSR_ALG1
- * with op(A) = A wherever the plan is row-wise or merge-path (every unprepared
- * call, every matrix under 2 M entries or with local columns), for int32, and
+ * with op(A) = A for every unprepared call, every matrix under 7 M entries or
+ * with local columns, for int32, and
  * for nearly every re-stored matrix.  The plans that add in the order their
  * wavefronts arrive are, on floating-point data with the default algorithm,
- * op(A) = A where the ordered layout refuses the matrix (a row of more than
- * 65 534 entries in descending order of columns, say: row blocks summed with LDS
- * atomics), the re-stored op(A) = A^T over more than 2^18 columns (products
+ * op(A) = A with 7 M entries or more where the ordered layout refuses the matrix
+ * (a row of more than 65 534 entries in descending order of columns, say: row
+ * blocks summed with LDS atomics), the re-stored op(A) = A^T over more than 2^18 columns (products
  * sorted by output panel and summed with LDS atomics), and op(A) = A^T without
  * Preprocess (fp32 atomics on y): there the last bit of an element may differ
  * between two calls, as the reference says of CSR_ALG1.

@@ -306,8 +306,9 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
     }
     // Results that may differ in the last bit between calls (the reference's ALG_DEFAULT / CSR_ALG1 of aclsparseSpMV)
     // may fall back to the layout whose row blocks add with atomics, where there is one: op(A) = A, floating-point data.
-    // Its bytes are room for the ordered one, too.
-    const bool atomics = !repeatable && !transpose && valueType != OPSPARSE_I32;
+    // Its bytes are room for the ordered one, too.  Not below 7 M entries: the kernels that such a matrix has otherwise
+    // repeat their sums, and where the ordered layout refuses it they take it.
+    const bool atomics = !repeatable && !transpose && valueType != OPSPARSE_I32 && !small;
     const size_t bytes =
         atomics ? opsparse_spmv_csr_live_workspace_bytes(rows, cols, nnz)
                 : opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, BlockedFlags(transpose, true, valueType));
