@@ -80,6 +80,7 @@ struct OpsparseSpmmBinding {
     int64_t offsetReach = 0;  // the furthest distance
     int32_t offsetRuns = 0;   // how the distances fall into runs
     int32_t maxRowNnz = 0;  // entries of the longest row (a plan without tables does not say)
+    bool wholeRows = false;  // the plan was cut for whole rows (PrefersWholeRows)
 };
 
 // reference: sparse/common/aclsparse_handle_internal.h:56-72
@@ -198,10 +199,13 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
 void RememberSized(aclsparseConstSpMatDescr_t matA, const RestoredChoice &choice, bool transpose, int32_t valueType);
 bool SizedFor(aclsparseConstSpMatDescr_t matA, const RestoredChoice &choice, bool transpose, int32_t valueType);
 // The second look at a matrix that the row-wise kernels would serve: `plan` becomes an OPSPARSE_SPMV_OFFSET_ROWS one where
-// its rows repeat.  `buffer` has opsparse_spmv_csr_workspace_bytes().  OPS_SPARSE_SPMV_NO_OFFSETS in the environment skips
-// it (tuning, tests of the row-wise kernels).
+// its rows repeat and that is the faster plan.  `buffer` has opsparse_spmv_csr_workspace_bytes().  OPS_SPARSE_SPMV_NO_OFFSETS
+// in the environment skips it (tuning, tests of the row-wise kernels).
 int LookForOffsets(const int32_t *rowOffsets, const int32_t *colInd, int64_t rows, int64_t cols, int64_t nnz, void *buffer,
                    OpsparseSpmvPlan *plan, void *stream);
+// OPS_SPARSE_OFFSETS_ANY_SIZE in the environment: Preprocess and createDescr take the lists of repeating rows wherever there
+// are such lists, also where other kernels are faster (tuning, tests of these kernels at small sizes).
+bool OffsetsAtAnySize();
 // valueType: the OPSPARSE_* type of the values and of x.
 RestoredChoice PickRestoredLayout(int64_t rows, int64_t cols, int64_t nnz, bool transpose, int32_t valueType);
 // `scratch` / `scratchBytes`: where the analysis works when the buffer only has room for what the launches keep

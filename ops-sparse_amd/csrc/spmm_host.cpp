@@ -283,7 +283,8 @@ aclsparseStatus_t BuildPlan(const aclsparseSpMatDescr *A, int64_t n, int64_t ele
         return FromLaunch(rc);
     }
     const int32_t maxRow = plan.maxRowNnz;
-    if (PrefersWholeRows(A, plan, n, elemBytes, tables, stream)) {
+    const bool wholeRows = PrefersWholeRows(A, plan, n, elemBytes, tables, stream);
+    if (wholeRows) {
         // a plan without tables: the launch layer then takes a lane group a row
         const int again = opsparse_spmm_csr_analyse(static_cast<const int32_t *>(A->rowOffsets), A->rows, A->nnz, n,
                                                     tables, bytes, OPSPARSE_SPMM_ROW_SPLIT, &plan, stream);
@@ -302,7 +303,69 @@ aclsparseStatus_t BuildPlan(const aclsparseSpMatDescr *A, int64_t n, int64_t ele
     A->spmm.vectorOff = 0;
     A->spmm.vectorBytes = 0;
     A->spmm.maxRowNnz = maxRow;
+    A->spmm.wholeRows = wholeRows;
     return ACL_SPARSE_STATUS_SUCCESS;
+}
+
+// Where the lists of a matrix whose rows repeat are ahead of the plan that was just made for a C of n columns.  us a launch,
+// plan / lists:
+//   - one 16-byte piece of B a row: n = 4 of 80 K rows 5-point mesh 4.2 / 4.5, 7-point 4.6 / 6.2, 9-point 5.6 / 5.6, 27-point 11.1 / 12.4,
+//     of 160 K 5.4 / 5.2, 6.2 / 6.1, 9.1 / 6.5, 18.6 / 12.0; 3 distances of 320 K 5.9 / 6.3, of 2.5 M 28.1 / 29.8; fp16 n = 8 of 80 K
+//     7-point 7.8 / 9.1, 9-point 9.9 / 7.6, of 160 K 10.9 / 8.7, 16.5 / 9.4;
+//   - two: n = 8 of 80 K rows 4.5 / 5.0, 5.9 / 5.6, 7.0 / 6.2, 14.7 / 10.7, 5-point of 160 K 7.7 / 6.4; fp16 n = 16 5-point of 80 K 10.2 / 7.4;
+//   - row-major fp32 rows that are not whole 16-byte pieces, which the plan copies: ahead at every size, n = 33 of 5000 rows 5-point
+//     11.1 / 4.6, 27-point 15.8 / 9.2, of 290 K 120 / 33, 188 / 114;
+//   - slabs staged through LDS: ahead at every size, 5-point n = 128 of 2000 rows 27 / 6, of 320 K 127 / 80; 7-point n = 256 75 / 7,
+//     312 / 198; fp16 5-point n = 64 25 / 7, 69 / 48, 9-point n = 128 35 / 8, 137 / 108; only fp16 under lists with many empty
+//     steps is behind (10 distances, which are 18 steps, n = 128 of 40 K rows 23 / 21, of 150 K 57 / 60, of 500 K 166 / 180);
+//   - whole rows, fp16: behind nearly everywhere (7-point of 320 K rows n = 32 24 / 36, 27-point n = 64 102 / 141);
+//   - whole rows, fp32, by the list: 5-point mesh of 80 K rows n = 16 6.8 / 6.1, n = 32 9.4 / 8.9, n = 64 15.0 / 13.8, of 40 K 4.6 / 5.2,
+//     4.9 / 6.1, 9.8 / 9.1; 9-point of 160 K 13.7 / 13.7, 23.8 / 24.0, 34.7 / 32.2, n = 128 75 / 53, of 80 K 10.1 / 8.5, 14.4 / 12.6,
+//     19.5 / 21.1; 7-point n = 16 of 320 K 20.1 / 21.1, of 640 K 37.5 / 32.9, n = 32 28.9 / 30.1 and 64 / 49, n = 64 of 160 K 28.9 / 29.7,
+//     of 320 K 65 / 45, n = 128 64 / 60 and 127 / 93; longer lists n = 16: 27-point of 40 K 11.0 / 10.2, of 80 K 21 / 16, 19-point
+//     7.0 / 9.0, 14.7 / 14.0, 15 distances of 320 K 37 / 36, of
+//     640 K 76 / 57, and 10, which are 18 steps, 49 / 51, of 1.25 M 102 / 84; n = 32: 27-point of 160 K 40 / 46, of 320 K 80 / 75, 19-point
+//     61 / 66, of 640 K 125 / 107; n = 64: 27-point of 160 K 68 / 74, 19-point 59 / 64, of 320 K 136 / 107, 116 / 100;
+//   - beyond 64 columns only where there is a kernel for two rows a lane (of 320 K rows, n = 128, 27-point 224 / 188, but 19-point
+//     190 / 210, 15 distances n = 256 351 / 553).
+// `copied`: the plan copies rows that the kernel for lists takes where they are.  `mayHaveRuns`: two rows a lane.
+bool ListsAhead(const aclsparseSpMatDescr *A, int64_t n, int64_t elemBytes, int32_t distances, bool copied, bool mayHaveRuns)
+{
+    const int64_t pieces = (n * elemBytes + 15) / 16;
+    const int64_t chunk = distances <= 5 ? 5 : distances <= 7 ? 7 : 9, steps = (distances + chunk - 1) / chunk * chunk;
+    const bool emptySteps = 2 * steps * A->rows > 3 * A->nnz;
+    if (opsparse::OffsetsAtAnySize()) {
+        return true;
+    }
+    const int64_t k16 = int64_t{1} << 14;
+    if (pieces == 1) {
+        return distances >= 4 && A->rows >= (distances < 8 ? 9 * k16 : 6 * k16);
+    }
+    if (pieces == 2) {
+        return distances >= 3 && A->rows >= (distances <= 5 && elemBytes == 4 ? 8 * k16 : 4 * k16);
+    }
+    if (copied) {
+        return true;
+    }
+    if (!A->spmm.wholeRows) {
+        return elemBytes == 4 || !emptySteps || A->rows < int64_t{1} << 17;
+    }
+    if (elemBytes == 2) {
+        return false;
+    }
+    int64_t least;
+    if (distances <= 5) {
+        least = !emptySteps ? 4 : pieces <= 4 ? 32 : 8;
+    } else if (distances <= 7) {
+        least = pieces <= 4 ? 32 : pieces <= 8 ? 24 : 9;
+    } else if (distances <= 9) {
+        least = pieces <= 8 ? 4 : 8;
+    } else if (pieces <= 4) {
+        least = emptySteps ? 64 : distances >= 18 ? 4 : 32;
+    } else {
+        least = pieces <= 8 ? 24 : pieces <= 32 ? 16 : 8;
+    }
+    return A->rows >= least * k16 && (pieces <= 16 || mayHaveRuns);
 }
 
 bool ScalarIsZero(const void *host, aclDataType computeType)
@@ -436,6 +499,8 @@ aclsparseStatus_t aclsparseSpMMPreprocess(aclsparseHandle_t handle, aclsparseOpe
         matA->spmm.stagingBytes = MakeStaging(matA, matB, matC, opB, t, matA->spmm.plan.bytes).bytes;
         matA->spmm.offsetPatterns = 0;
         const int64_t front = FrontBytes(matA);
+        const bool copied = matA->spmm.stagingBytes > 0 && t.valType == OPSPARSE_F32 && opB == ACL_SPARSE_OP_NON_TRANSPOSE &&
+                            matB->order == ACL_SPARSE_ORDER_ROW && matC->order == ACL_SPARSE_ORDER_ROW;
         if (ColumnsAreVectors(matA, matB, matC, opB, t)) {
             // (GetBufferSize counted this region: at the start for every operand, or at the end for these)
             const int64_t off = front > 0 ? 0 : Align256(matA->spmm.plan.bytes + matA->spmm.stagingBytes);
@@ -455,7 +520,8 @@ aclsparseStatus_t aclsparseSpMMPreprocess(aclsparseHandle_t handle, aclsparseOpe
                 matA->spmm.vectorBytes = static_cast<int64_t>(bytes);
             }
         } else if (front > 0 && matC->cols >= 1 && matC->cols <= opsparse::kOffsetMaxColumns && stream != nullptr &&
-                   matA->colInd != nullptr && std::getenv("OPS_SPARSE_SPMM_NO_OFFSETS") == nullptr) {
+                   matA->colInd != nullptr && std::getenv("OPS_SPARSE_SPMM_NO_OFFSETS") == nullptr &&
+                   ListsAhead(matA, matA->spmm.plan.n, ElementBytes(t.valType), matA->spmm.maxRowNnz, copied, true)) {
             opsparse::OffsetFound found;
             const int rc = opsparse::AnalyseOffsetRows(static_cast<const int32_t *>(matA->rowOffsets),
                                                        static_cast<const int32_t *>(matA->colInd), matA->rows, matA->cols,
@@ -464,10 +530,12 @@ aclsparseStatus_t aclsparseSpMMPreprocess(aclsparseHandle_t handle, aclsparseOpe
             if (rc != OPSPARSE_OK) {
                 return FromLaunch(rc);
             }
-            if (found.patterns > 0) {
+            const int32_t runs = opsparse::OffsetRuns(found);
+            if (found.patterns > 0 && ListsAhead(matA, matA->spmm.plan.n, ElementBytes(t.valType), found.distances, copied,
+                                                 runs != opsparse::kOffsetRunsAny)) {
                 matA->spmm.offsetPatterns = found.patterns;
                 matA->spmm.offsetDistances = found.distances;
-                matA->spmm.offsetRuns = opsparse::OffsetRuns(found);
+                matA->spmm.offsetRuns = runs;
                 const int64_t back = -static_cast<int64_t>(found.distance[0]), on = found.distance[found.distances - 1];
                 matA->spmm.offsetReach = back > on ? back : on;
             }

@@ -222,17 +222,44 @@ int32_t BlockedFlags(bool transpose, bool liveValues, int32_t valueType)
                                          : 0);
 }
 
+// Where the product by lists is the faster one (us a launch, row-wise / lists; below, the chains of a tile's loads outweigh the
+// bytes saved, and most of all in the first and last tiles, whose distances reach out of the matrix):
+//   5-point mesh of 80 K rows 4.4 / 5.1, 150 K 5.0 / 5.6, 300 K 5.9 / 5.8, 700 K 9.9 / 7.7; 7-point 4.6 / 5.9 (39 K), 5.6 / 6.1,
+//   7.3 / 7.1, 13.1 / 9.5; 9-point 4.8 / 6.8 (40 K), 6.5 / 6.9, 8.7 / 7.8, 15.1 / 10.7;
+//   longer lists have one row a lane and half the chains: 15 distances of 40 K rows 5.1 / 5.7, 80 K 6.2 / 6.0, 150 K 8.1 / 6.7; 27
+//   5.9 / 7.1, 7.9 / 8.1, 11.7 / 8.5, 300 K 19.5 / 10.8; 19, which are 27 steps, 5.8 / 6.9 (80 K), 8.1 / 7.3.
+// Rows that have few of the distances: two lists of 3 (of 2) that share nothing, 300 K rows 5.8 / 6.3 (4.8 / 5.3), 1 M rows 13.3 / 9.8
+// (8.8 / 7.8).
+bool OffsetsAheadBySize(int64_t rows, int64_t nnz)
+{
+    return rows >= (int64_t{1} << 18) || (rows >= 3 * (int64_t{1} << 15) && nnz > 9 * rows);
+}
+bool OffsetsAheadByLists(int64_t rows, int64_t nnz, int32_t distances)
+{
+    if (distances > 18 && distances < 24) {
+        return rows >= (int64_t{1} << 17);
+    }
+    return distances > 9 || 2 * distances * rows <= 3 * nnz || rows >= (int64_t{1} << 19);
+}
+
 int LookForOffsets(const int32_t *rowOffsets, const int32_t *colInd, int64_t rows, int64_t cols, int64_t nnz, void *buffer,
                    OpsparseSpmvPlan *plan, void *stream)
 {
     const size_t bytes = opsparse_spmv_csr_offsets_workspace_bytes(rows, cols, nnz);
+    const bool anySize = OffsetsAtAnySize();
     if (plan->kernel != OPSPARSE_SPMV_STREAM_ROWS || plan->longRowsBeside != 0 || bytes == 0 || colInd == nullptr ||
-        std::getenv("OPS_SPARSE_SPMV_NO_OFFSETS") != nullptr) {
+        (!anySize && !OffsetsAheadBySize(rows, nnz)) || std::getenv("OPS_SPARSE_SPMV_NO_OFFSETS") != nullptr) {
         return OPSPARSE_OK;
     }
+    const OpsparseSpmvPlan rowWise = *plan;
     const int rc = opsparse_spmv_csr_offsets_analyse(rowOffsets, colInd, rows, cols, nnz, buffer, bytes, plan, stream);
+    if (rc == OPSPARSE_OK && !anySize && !OffsetsAheadByLists(rows, nnz, plan->numDistances)) {
+        *plan = rowWise;
+    }
     return rc == OPSPARSE_E_UNSUPPORTED ? OPSPARSE_OK : rc;
 }
+
+bool OffsetsAtAnySize() { return std::getenv("OPS_SPARSE_OFFSETS_ANY_SIZE") != nullptr; }
 
 void RememberSized(aclsparseConstSpMatDescr_t matA, const RestoredChoice &choice, bool transpose, int32_t valueType)
 {

@@ -11,9 +11,16 @@ import torch
 
 import oracle
 from helpers import run_spmm, to_dev
-from test_spmv_offset_rows_gpu import _matrix, _spread
+from test_spmv_offset_rows_gpu import _matrix, _spread, follows_lists, repeating_rows
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _lists_at_any_size(monkeypatch):
+    """Preprocess takes the lists where they are the faster plan, which small matrices' seldom are."""
+    monkeypatch.setenv("OPS_SPARSE_OFFSETS_ANY_SIZE", "1")
+
 
 DTYPES = {"f32": (torch.float32, torch.float32), "f16": (torch.float16, torch.float16), "f16_f32": (torch.float16, torch.float32)}
 
@@ -185,3 +192,83 @@ def test_five_scattered_distances_under_wide_b(osa, gpu_ctx, types, n):
     """Few distances that are no star's: one row a lane under 32 and 64 pieces as well."""
     rowptr, colind = _matrix(1500, 1500, [[-30, -7, 0, 9, 40]], np.zeros(1500, int))
     _run(osa, gpu_ctx, rowptr, colind, 1500, n, types, 0.5)
+
+
+STAR9 = [-40, -39, -38, -1, 0, 1, 38, 39, 40]                 # a 9-point box
+TEN, TWENTY = [*STAR9, 80], sorted({7 * i for i in range(-10, 10)})
+
+
+@pytest.mark.parametrize("distances,types,n,rows,lists", [
+    # one piece of B a row, two pieces
+    (STAR2, "f32", 4, 147_456, True), (STAR2, "f32", 3, 147_455, False), ([-1, 0, 1], "f32", 4, 200_000, False),
+    (TWENTY, "f32", 4, 98_304, True), (STAR9, "f16", 8, 98_303, False), ([-1, 0, 1], "f32", 8, 1 << 17, True),
+    (STAR2, "f32", 8, (1 << 17) - 1, False), (STAR2, "f16", 16, 1 << 16, True), (STAR3, "f32", 8, (1 << 16) - 1, False),
+    # ragged rows, which the other kernels work on copies of
+    (STAR2, "f32", 33, 1024, True), (TWENTY, "f32", 50, 1024, True),
+    # whole rows, by the list and the width
+    (STAR2, "f32", 16, 1 << 16, True), (STAR2, "f32", 64, (1 << 16) - 1, False), ([-1, 0, 1], "f32", 16, (1 << 19) - 1, False),
+    ([-1, 0, 1], "f32", 16, 1 << 19, True), (STAR9, "f32", 32, 1 << 16, True), (STAR9, "f32", 64, (1 << 17) - 1, False),
+    (STAR3, "f32", 12, (1 << 19) - 1, False), (STAR3, "f32", 12, 1 << 19, True), (STAR3, "f32", 32, 393_215, False),
+    (STAR3, "f32", 32, 393_216, True), (STAR3, "f32", 64, 147_455, False), (STAR3, "f32", 64, 147_456, True),
+    (TWENTY, "f32", 16, 1 << 16, True), (TWENTY, "f32", 16, (1 << 16) - 1, False), (TEN, "f32", 16, (1 << 20) - 1, False),
+    (TEN, "f32", 16, 1 << 20, True), (TEN, "f32", 32, 393_215, False), (TEN, "f32", 64, 1 << 18, True),
+    # wider: slabs give way at every size, whole rows only to two rows a lane
+    (STAR2, "f32", 128, 1024, True), (STAR9, "f32", 128, 1 << 17, True), (STAR9, "f32", 128, (1 << 17) - 1, False),
+    (TEN, "f32", 128, 1 << 18, False), (STAR9, "f32", 256, 2000, True),
+    # fp16: where the plan is slabs
+    (STAR2, "f16", 64, 2000, True), (TEN, "f16", 128, (1 << 17) - 1, True), (TEN, "f16", 128, 1 << 17, False), (STAR9, "f16", 64, 1 << 18, False), (TWENTY, "f16_f32", 64, 1 << 18, False)])
+def test_either_side_of_every_bound(osa, gpu_ctx, monkeypatch, distances, types, n, rows, lists):
+    """Which matrices Preprocess takes lists of, seen from outside: once it has run, other column indices in place are not
+    looked at by the kernel that has lists."""
+    monkeypatch.delenv("OPS_SPARSE_OFFSETS_ANY_SIZE")
+    dev, stream, handle = gpu_ctx
+    val_dtype, c_dtype = DTYPES[types]
+    rowptr, colind = repeating_rows(rows, distances, dev)
+    B, C = torch.ones(rows, n, dtype=val_dtype, device=dev), torch.zeros(rows, n, dtype=c_dtype, device=dev)
+    B[0] = 0
+    A = osa.Csr(rows, rows, rowptr, colind, torch.ones(colind.numel(), dtype=val_dtype, device=dev))
+    op = osa.SpmmOp(handle, A, osa.DnMat(rows, n, n, B.view(-1)), osa.DnMat(rows, n, n, C.view(-1)))
+    assert follows_lists(lambda: op(1.0, 0.0), C, rowptr, colind, stream) == lists
+
+
+@pytest.mark.parametrize("where", ["a", "b", "beyond_a_list"])
+@pytest.mark.parametrize("types,n,stencil", [("f32", 4, STAR2), ("f32", 33, STAR3), ("f32", 128, STAR2), ("f32", 256, BOX3), ("f16", 16, STAR3),
+                                             ("f16_f32", 128, BOX2)])
+def test_infinities_and_nan(osa, gpu_ctx, types, n, stencil, where):
+    """NaN and infinities in A, in B, and in rows of B that a row's list leaves out although its neighbours' lists name them:
+    where the plain product has them and nowhere else.  (fp16 C is clamped: infinities become 65504.)"""
+    val_dtype, c_dtype = DTYPES[types]
+    rows, rng = 3001, np.random.default_rng(n)
+    lists = [stencil, [d for d in stencil if d != 1], [d for d in stencil if d != stencil[0]]]
+    choose = np.where(np.arange(rows) % 5 == 3, 1 + np.arange(rows) // 5 % 2, 0)
+    if where == "beyond_a_list":
+        choose[:] = np.where(np.arange(rows) % 2 == 0, 1, choose)      # no even row has distance 1 ...
+        lists[0] = lists[2] = [0]                                      # ... and the odd ones only their own column
+        lists[1] = [d for d in stencil if d % 2 == 0]
+    rowptr, colind = _matrix(rows, rows, lists, choose)
+    val = _seen(rng.uniform(-1, 1, colind.size), val_dtype)
+    B = _seen(rng.uniform(-1, 1, (rows, n)), val_dtype)
+    bad = np.array([np.nan, np.inf, -np.inf], np.float32)
+    if where == "a":
+        val[rng.choice(val.size, 40, replace=False)] = bad[np.arange(40) % 3]
+    else:
+        at = 2 * rng.choice(rows // 2, 30, replace=False) + 1          # odd rows of B
+        B[at] = bad[np.arange(30) % 3][:, None]
+    dev, stream, handle = gpu_ctx
+    d = [to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev, val_dtype)]
+    A, C = osa.Csr(rows, rows, *d), torch.zeros(rows * n, dtype=c_dtype, device=dev)
+    op = osa.SpmmOp(handle, A, osa.DnMat(rows, n, n, to_dev(B.ravel(), dev, val_dtype)), osa.DnMat(rows, n, n, C))
+    op(1.0, 0.0)
+    stream.synchronize()
+    got = C.float().cpu().numpy().reshape(rows, n)
+    gold = np.zeros((rows, n))
+    with np.errstate(invalid="ignore"):
+        entry_row = np.repeat(np.arange(rows), np.diff(rowptr))
+        np.add.at(gold, entry_row, val[:, None].astype(np.float64) * B[colind].astype(np.float64))
+    if c_dtype == torch.float16:
+        gold = np.clip(gold, -65504.0, 65504.0)                        # (NaN stays NaN)
+    assert np.array_equal(np.isnan(got), np.isnan(gold)) and np.array_equal(np.isinf(got), np.isinf(gold))
+    fine = np.isfinite(gold)
+    assert fine.any() and not (fine.all() and c_dtype != torch.float16)
+    assert np.allclose(got[fine], gold[fine], rtol=2.0 ** -10 if c_dtype == torch.float16 else 1e-5, atol=1e-5)
+    assert np.array_equal(np.sign(got[np.isinf(gold)]), np.sign(gold[np.isinf(gold)]))

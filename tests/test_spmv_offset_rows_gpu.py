@@ -40,6 +40,38 @@ def _spread(n, reach, seed):
     return sorted(d)
 
 
+def repeating_rows(rows, distances, dev, others=None):
+    """Row offsets and columns, on the device, of the matrix whose row r has the distances that stay inside; stretches of 64
+    rows in turns have `others` instead."""
+    r = torch.arange(rows, device=dev)[:, None]
+    every = sorted(set(distances) | set(others or []))
+    cols = r + torch.tensor(every, device=dev)
+    has = torch.tensor([[d in l for d in every] for l in (distances, others or distances)], device=dev)
+    ok = (cols >= 0) & (cols < rows) & has[r[:, 0] // 64 % 2]
+    ends = torch.cumsum(ok.sum(1), 0)
+    return torch.cat([ends.new_zeros(1), ends]).int(), cols[ok].int()
+
+
+def follows_lists(call, out, rowptr, colind, stream):
+    """Does `call` multiply by what Preprocess saw (True) or by the column indices as they are?  All ones, but the first
+    element (row) of x (B): with every index set to 0 in place, the sums over the indices are 0.  Row sums either way."""
+    call()
+    stream.synchronize()
+    counts = (rowptr[1:] - rowptr[:-1]).float()
+    touched = torch.zeros_like(counts).index_add_(0, torch.repeat_interleave(torch.arange(counts.numel(), device=colind.device),
+                                                                             rowptr.diff().long()), (colind == 0).float())
+    want = (counts - touched).view(-1, *[1] * (out.dim() - 1))
+    assert bool((out.float() == want).all())
+    kept = colind.clone()
+    colind.zero_()
+    call()
+    stream.synchronize()
+    colind.copy_(kept)
+    lists = bool((out.float() == want).all())
+    assert lists or not bool(out.any())
+    return lists
+
+
 def _offsets_plan(m, want=True):
     osa = m.osa
     plan = m.analyse(osa.OPSPARSE_SPMV_STREAM_ROWS)
@@ -150,6 +182,7 @@ def test_public_calls_follow_the_values_and_agree_with_the_row_wise_plan(osa, gp
     y0 = workloads.uniform(3, rows, -1.0, 1.0, dev)
     csr = osa.Csr(rows, rows, behind(A["rowptr"]), behind(A["colind"]), values)
     got = {}
+    monkeypatch.setenv("OPS_SPARSE_OFFSETS_ANY_SIZE", "1")   # (at this size the row-wise plan is the faster one)
     for switch in (False, True):
         if switch:
             monkeypatch.setenv("OPS_SPARSE_SPMV_NO_OFFSETS", "1")
@@ -190,3 +223,33 @@ def test_launch_wants_the_buffer_of_the_plan(osa, gpu_ctx):
             m.d_y.data_ptr(), rows, rows, m.nnz, S(1), S(0), osa.OPSPARSE_F32, osa.OPSPARSE_F32, 0)
     assert m.L.opsparse_spmv_csr_launch(*args, None, 0, m.sp) == osa.OPSPARSE_E_WORKSPACE
     assert m.L.opsparse_spmv_csr_launch(*args, m.ws.data_ptr(), plan.bytes - 1, m.sp) == osa.OPSPARSE_E_WORKSPACE
+
+
+FIVE, NINE, TEN = [-40, -1, 0, 1, 40], [-40, -39, -38, -1, 0, 1, 38, 39, 40], list(range(-5, 5))
+TWENTY = list(range(-10, 10))
+
+
+@pytest.mark.parametrize("entry", ["spmv", "alg2", "spmvop_alg2", "spmm"])
+@pytest.mark.parametrize("distances,rows,lists", [
+    (FIVE, 1 << 18, True), (FIVE, (1 << 18) - 1, False), (NINE, (1 << 18) - 1, False), (TEN, 98_304, True),
+    (TEN, 98_303, False), (TWENTY, (1 << 17) - 1, False), (TWENTY, 1 << 17, True), ("in turns", (1 << 19) - 64, False), ("in turns", 1 << 19, True)])
+def test_either_side_of_every_bound(osa, gpu_ctx, monkeypatch, entry, distances, rows, lists):
+    """Which matrices Preprocess / createDescr take lists of, seen from outside: column indices that change in place
+    afterwards are not looked at where there are lists.  "in turns": stretches of rows with three and four of six distances."""
+    monkeypatch.delenv("OPS_SPARSE_OFFSETS_ANY_SIZE", raising=False)
+    dev, stream, handle = gpu_ctx
+    if distances == "in turns":
+        rowptr, colind = repeating_rows(rows, [-3, 2, 9], dev, [-2, 5, 9, 11])
+    else:
+        rowptr, colind = repeating_rows(rows, distances, dev)
+    A = osa.Csr(rows, rows, rowptr, colind, torch.ones(colind.numel(), device=dev))
+    x, y = torch.ones(rows, device=dev), torch.zeros(rows, device=dev)
+    x[0] = 0
+    X, Y = osa.DnVec(x), osa.DnVec(y)
+    if entry == "spmvop_alg2":
+        op = osa.SpmvOpPlan(handle, A, X, Y, Y, alg=osa.ACL_SPARSE_SPMVOP_ALG2)
+    elif entry == "spmm":
+        op = osa.SpmmOp(handle, A, osa.DnMat(rows, 1, 1, x), osa.DnMat(rows, 1, 1, y))
+    else:
+        op = osa.SpmvOp(handle, A, X, Y, alg=osa.ACL_SPARSE_SPMV_CSR_ALG2 if entry == "alg2" else osa.ACL_SPARSE_SPMV_ALG_DEFAULT)
+    assert follows_lists(lambda: op(1.0, 0.0), y, rowptr, colind, stream) == lists
