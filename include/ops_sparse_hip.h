@@ -94,7 +94,7 @@ typedef OPSPARSE_ABI_ENUM(OpsparseSpmvKernel) {
                                       into fp64 sums in LDS with atomics.  26 bytes of traffic per entry, none on y;
                                       fp32 / fp16 / bf16, values read where the caller has them; like the reference's
                                       transposed kernel the last bit of a result may differ between two calls */
-    OPSPARSE_SPMV_OFFSET_ROWS = 9   /* rows of at most 48 entries that repeat (a mesh operator): the columns of row r
+    OPSPARSE_SPMV_OFFSET_ROWS = 9   /* rows of at most 32 entries that repeat (a mesh operator): the columns of row r
                                       are r plus one of at most 128 lists of distances, and a byte a row names the
                                       list; the column indices are not read.  op(A) = A, every type of STREAM_ROWS,
                                       values read where the caller has them */
@@ -303,8 +303,10 @@ int opsparse_spmv_csr_scatter_analyse_split(const int32_t *rowOffsets, const int
 /*
  * OFFSET_ROWS analysis, a second look at a matrix that opsparse_spmv_csr_analyse made a STREAM_ROWS plan of: do its
  * rows repeat?  bytes of the workspace, 0 where the sizes alone rule it out; `plan` is that plan, which the analysis
- * turns into an OFFSET_ROWS one or, returning OPSPARSE_E_UNSUPPORTED, leaves as it is (more than 128 different lists of
- * distances col - row, a table of more than 3072 of them, a column outside [0, cols), short rows among long ones).
+ * turns into an OFFSET_ROWS one or, returning OPSPARSE_E_UNSUPPORTED, leaves as it is: rows of more than 32 entries, columns
+ * of a row that do not ascend, a column outside [0, cols), more than 128 different lists of distances col - row (or more
+ * than 33 among 64 neighbouring rows), more than 32 different distances in all of them, or more than twice as many of
+ * these as a row has entries on average.
  * Every entry of the matrix is checked; rowOffsets / colInd must be the same at the launches, which read rowOffsets and
  * the values but not colInd.  Synchronises `stream` once; the launches need the whole workspace.  No counterpart in the
  * reference.

@@ -7,8 +7,9 @@
 //
 // us a call, beta != 0, row-wise kernels / here: 5-point 2048 x 2048 39.6 / 26.4 (5.2 TB/s of the bytes it needs), 9-point
 // 1500 x 1501 38.6 / 23.4, 7-point 125 x 131 x 127 31.3 / 20.0, 27-point 131 x 127 x 129 125 / 56 (4.6 TB/s), bf16 118 /
-// 47, 83 x 141 x 109 71 / 31; below some 250 000 points (27: 90 000) the row-wise kernels are ahead.  The analysis reads the columns twice: Preprocess of
-// the first takes 0.37 ms instead of 0.18, of the 27-point one 0.60 instead of 0.19, of a matrix that is none 0.05 - 0.1 more.
+// 47, 83 x 141 x 109 71 / 31; below some 250 000 points (27: 90 000) the row-wise kernels are ahead, and Preprocess keeps them.
+// The analysis reads the columns twice: Preprocess of the first takes 0.37 ms instead of 0.18, of the 27-point one 0.60 instead
+// of 0.19, of a matrix that is none 0.05 - 0.1 more.
 //
 // No counterpart in the reference, whose kernels read a column index an entry
 // (sparse/spmv/arch22/kernels/spmv_kernel.h:27-310).
@@ -309,7 +310,9 @@ using Some = typename std::conditional<sizeof(T) == 4, typename std::conditional
                                        typename std::conditional<V == 2, Short2U, uint16_t>::type>::type;
 
 struct OffsetList {
-    int32_t d[kOffsetMaxDistances];  // all distances in ascending order, zeros behind them
+    // all distances in ascending order, and the last one again behind them: the loads there stay in range, and the bound of
+    // a tile's columns is the entry of the compiled width
+    int32_t d[kOffsetMaxDistances];
 };
 
 // A wavefront walks over tiles of 128 consecutive rows, a lane taking two neighbours.  The distances of all lists, in
