@@ -12,7 +12,7 @@ import torch
 
 import oracle
 from helpers import to_dev
-from test_every_kernel_gpu import SPMV_TYPES, RawSpmv
+from test_every_kernel_gpu import SPMV_TYPES, RawSpmv, _type_code
 
 pytestmark = pytest.mark.gpu
 
@@ -253,3 +253,45 @@ def test_either_side_of_every_bound(osa, gpu_ctx, monkeypatch, entry, distances,
     else:
         op = osa.SpmvOp(handle, A, X, Y, alg=osa.ACL_SPARSE_SPMV_CSR_ALG2 if entry == "alg2" else osa.ACL_SPARSE_SPMV_ALG_DEFAULT)
     assert follows_lists(lambda: op(1.0, 0.0), y, rowptr, colind, stream) == lists
+
+
+@pytest.mark.parametrize("where", ["a", "x", "beyond_a_list"])
+@pytest.mark.parametrize("types", ["f32", "bf16_bf16", "f16_f32"])
+@pytest.mark.parametrize("distances", [5, 9, 27])
+def test_infinities_and_nan(osa, gpu_ctx, distances, types, where):
+    """NaN and infinities in A, in x, and in elements of x that a row's list leaves out although its neighbours' lists name
+    them: in y where the plain product has them and nowhere else."""
+    rows, rng = 3001, np.random.default_rng(distances)
+    every = _spread(distances, 40, 1)
+    lists = [every, [d for d in every if d != every[1]], every[1:]]
+    choose = np.where(np.arange(rows) % 5 == 3, 1 + np.arange(rows) // 5 % 2, 0)
+    if where == "beyond_a_list":
+        lists = [[0], [d for d in every if d % 2 == 0], every[:1] + [0]]   # even rows: even distances
+        choose = np.where(np.arange(rows) % 2 == 0, 1, 0)
+    rowptr, colind = _matrix(rows, rows, lists, choose)
+    m = RawSpmv(osa, gpu_ctx, rowptr, colind, rows, types, seed=distances)
+    row_wise = m.analyse(osa.OPSPARSE_SPMV_STREAM_ROWS)      # (keeps nothing in the workspace)
+    plan = _offsets_plan(m)
+    bad = torch.tensor([float("nan"), float("inf"), -float("inf")], device=m.dev)
+    if where == "a":
+        at = torch.from_numpy(rng.choice(m.nnz, 40, replace=False)).to(m.dev)
+        m.d_val[at] = bad[torch.arange(40, device=m.dev) % 3].to(m.d_val.dtype)
+    else:
+        at = torch.from_numpy(2 * rng.choice(rows // 2, 30, replace=False) + 1).to(m.dev)
+        m.d_x[at] = bad[torch.arange(30, device=m.dev) % 3].to(m.d_x.dtype)
+    S = lambda v: osa.OpsparseScalar(float(v), None, 0, 0)
+    got = []
+    for p in (plan, row_wise):
+        assert m.L.opsparse_spmv_csr_launch(ctypes.byref(p), 0, m.d_rp.data_ptr(), m.d_ci.data_ptr(), m.d_val.data_ptr(),
+                                            m.d_x.data_ptr(), m.d_y.data_ptr(), rows, rows, m.nnz, S(1), S(0),
+                                            _type_code(osa, m.val_dtype), _type_code(osa, m.out_dtype), 0, m.ws.data_ptr(),
+                                            m.ws.numel(), m.sp) == osa.OPSPARSE_OK
+        m.stream.synchronize()
+        got.append(m.d_y.float().clone())
+    assert bool(got[1].isfinite().any()) and not bool(got[1].isfinite().all())
+    assert torch.equal(got[0].isnan(), got[1].isnan()) and torch.equal(got[0].isinf(), got[1].isinf())
+    # (fp64 sums in another order, rounded once: two units in the last place, or what 32 terms below 1 leave behind)
+    ulp = 2.0 ** -7 if m.out_dtype == torch.bfloat16 else 2.0 ** -22
+    fine = got[1].isfinite()
+    assert bool(((got[0] - got[1])[fine].abs() <= 2 * ulp * got[1][fine].abs() + 1e-12).all())
+    assert torch.equal(got[0][got[1].isinf()], got[1][got[1].isinf()])
