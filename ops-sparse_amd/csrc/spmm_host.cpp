@@ -319,13 +319,17 @@ aclsparseStatus_t BuildPlan(const aclsparseSpMatDescr *A, int64_t n, int64_t ele
 //     312 / 198; fp16 5-point n = 64 25 / 7, 69 / 48, 9-point n = 128 35 / 8, 137 / 108; only fp16 under lists with many empty
 //     steps is behind (10 distances, which are 18 steps, n = 128 of 40 K rows 23 / 21, of 150 K 57 / 60, of 500 K 166 / 180);
 //   - whole rows, fp16: behind nearly everywhere (7-point of 320 K rows n = 32 24 / 36, 27-point n = 64 102 / 141);
-//   - whole rows, fp32, by the list: 5-point mesh of 80 K rows n = 16 6.8 / 6.1, n = 32 9.4 / 8.9, n = 64 15.0 / 13.8, of 40 K 4.6 / 5.2,
-//     4.9 / 6.1, 9.8 / 9.1; 9-point of 160 K 13.7 / 13.7, 23.8 / 24.0, 34.7 / 32.2, n = 128 75 / 53, of 80 K 10.1 / 8.5, 14.4 / 12.6,
-//     19.5 / 21.1; 7-point n = 16 of 320 K 20.1 / 21.1, of 640 K 37.5 / 32.9, n = 32 28.9 / 30.1 and 64 / 49, n = 64 of 160 K 28.9 / 29.7,
-//     of 320 K 65 / 45, n = 128 64 / 60 and 127 / 93; longer lists n = 16: 27-point of 40 K 11.0 / 10.2, of 80 K 21 / 16, 19-point
-//     7.0 / 9.0, 14.7 / 14.0, 15 distances of 320 K 37 / 36, of
-//     640 K 76 / 57, and 10, which are 18 steps, 49 / 51, of 1.25 M 102 / 84; n = 32: 27-point of 160 K 40 / 46, of 320 K 80 / 75, 19-point
-//     61 / 66, of 640 K 125 / 107; n = 64: 27-point of 160 K 68 / 74, 19-point 59 / 64, of 320 K 136 / 107, 116 / 100;
+//   - whole rows, fp32, by the list and the width (a lane group has a power of two of lanes, so that n = 24 idles as many as 32 uses):
+//     5-point mesh of 100 K rows n = 12 7.0 / 7.7, n = 24 9.9 / 10.7, n = 48 17.4 / 17.2, of 150 K 8.8 / 8.1, 13.7 / 14.2, 23.9 / 21.4, of
+//     250 K 14.6 / 12.3, 20.3 / 18.5, 44 / 33, of 80 K n = 16 6.8 / 6.1, n = 64 15.0 / 13.8;
+//     7-point of 150 K 10.4 / 10.4, 15.0 / 16.4, 25.7 / 27.3, of 250 K 16.5 / 14.7, 21.8 / 23.0, 45 / 39, of 400 K 24 / 22, 34 / 32, 73 / 50,
+//     n = 16 of 320 K 20.1 / 21.1, of 640 K 37.5 / 32.9;
+//     9-point of 70 K 7.5 / 8.0, 13.4 / 11.7, 17.4 / 22.4, of 100 K 10.8 / 9.2, 15.6 / 13.4, 23.0 / 23.3, n = 96 41 / 36, of 250 K 21 / 16,
+//     32 / 26, 57 / 45, 111 / 76;
+//     27-point of 70 K 18.5 / 14.2, 19.4 / 21.8, 31 / 44, 45 / 83, of 250 K 56 / 36, 59 / 57, 102 / 97, 166 / 173, of 400 K 91 / 56, 94 / 76,
+//     161 / 125, 250 / 214; 19 distances, which are 27 steps, n = 16 of 40 K 7.0 / 9.0, of 80 K 14.7 / 14.0, n = 32 of 320 K 61 / 66, of
+//     640 K 125 / 107, n = 64 of 160 K 59 / 64, of 320 K 116 / 100; 15, 18 steps, n = 16 of 320 K 37 / 36, of 640 K 76 / 57; 10, 18 steps,
+//     n = 16 of 640 K 49 / 51, of 1.25 M 102 / 84;
 //   - beyond 64 columns only where there is a kernel for two rows a lane (of 320 K rows, n = 128, 27-point 224 / 188, but 19-point
 //     190 / 210, 15 distances n = 256 351 / 553).
 // `copied`: the plan copies rows that the kernel for lists takes where they are.  `mayHaveRuns`: two rows a lane.
@@ -355,15 +359,15 @@ bool ListsAhead(const aclsparseSpMatDescr *A, int64_t n, int64_t elemBytes, int3
     }
     int64_t least;
     if (distances <= 5) {
-        least = !emptySteps ? 4 : pieces <= 4 ? 32 : 8;
+        least = emptySteps ? (pieces <= 4 ? 32 : 8) : pieces == 3 ? 8 : pieces == 4 ? 5 : pieces <= 8 ? 10 : 6;
     } else if (distances <= 7) {
-        least = pieces <= 4 ? 32 : pieces <= 8 ? 24 : 9;
+        least = pieces == 3 ? 10 : pieces == 4 ? 32 : pieces <= 8 ? 24 : pieces <= 16 ? 12 : 9;
     } else if (distances <= 9) {
-        least = pieces <= 8 ? 4 : 8;
+        least = pieces <= 8 ? 5 : 6;
     } else if (pieces <= 4) {
         least = emptySteps ? 64 : distances >= 18 ? 4 : 32;
     } else {
-        least = pieces <= 8 ? 24 : pieces <= 32 ? 16 : 8;
+        least = pieces <= 8 ? (steps == distances ? 16 : 24) : pieces <= 32 ? 16 : 8;
     }
     return A->rows >= least * k16 && (pieces <= 16 || mayHaveRuns);
 }

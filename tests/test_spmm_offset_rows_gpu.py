@@ -195,7 +195,7 @@ def test_five_scattered_distances_under_wide_b(osa, gpu_ctx, types, n):
 
 
 STAR9 = [-40, -39, -38, -1, 0, 1, 38, 39, 40]                 # a 9-point box
-TEN, TWENTY = [*STAR9, 80], sorted({7 * i for i in range(-10, 10)})
+TEN, TWENTY, TWENTY_SEVEN = [*STAR9, 80], [7 * i for i in range(-10, 10)], [7 * i for i in range(-13, 14)]
 
 
 @pytest.mark.parametrize("distances,types,n,rows,lists", [
@@ -206,14 +206,16 @@ TEN, TWENTY = [*STAR9, 80], sorted({7 * i for i in range(-10, 10)})
     # ragged rows, which the other kernels work on copies of
     (STAR2, "f32", 33, 1024, True), (TWENTY, "f32", 50, 1024, True),
     # whole rows, by the list and the width
-    (STAR2, "f32", 16, 1 << 16, True), (STAR2, "f32", 64, (1 << 16) - 1, False), ([-1, 0, 1], "f32", 16, (1 << 19) - 1, False),
-    ([-1, 0, 1], "f32", 16, 1 << 19, True), (STAR9, "f32", 32, 1 << 16, True), (STAR9, "f32", 64, (1 << 17) - 1, False),
-    (STAR3, "f32", 12, (1 << 19) - 1, False), (STAR3, "f32", 12, 1 << 19, True), (STAR3, "f32", 32, 393_215, False),
-    (STAR3, "f32", 32, 393_216, True), (STAR3, "f32", 64, 147_455, False), (STAR3, "f32", 64, 147_456, True),
+    (STAR2, "f32", 12, (1 << 17) - 1, False), (STAR2, "f32", 16, 81_920, True), (STAR2, "f32", 24, 163_839, False),
+    (STAR2, "f32", 64, 98_304, True), (STAR2, "f32", 64, 98_303, False), ([-1, 0, 1], "f32", 16, (1 << 19) - 1, False),
+    ([-1, 0, 1], "f32", 16, 1 << 19, True), (STAR9, "f32", 32, 81_920, True), (STAR9, "f32", 64, 98_303, False),
+    (STAR3, "f32", 12, 163_840, True), (STAR3, "f32", 16, (1 << 19) - 1, False), (STAR3, "f32", 32, 393_215, False),
+    (STAR3, "f32", 32, 393_216, True), (STAR3, "f32", 64, 196_607, False), (STAR3, "f32", 64, 196_608, True),
     (TWENTY, "f32", 16, 1 << 16, True), (TWENTY, "f32", 16, (1 << 16) - 1, False), (TEN, "f32", 16, (1 << 20) - 1, False),
     (TEN, "f32", 16, 1 << 20, True), (TEN, "f32", 32, 393_215, False), (TEN, "f32", 64, 1 << 18, True),
+    (TWENTY_SEVEN, "f32", 32, 1 << 18, True), (TWENTY_SEVEN, "f32", 32, (1 << 18) - 1, False),
     # wider: slabs give way at every size, whole rows only to two rows a lane
-    (STAR2, "f32", 128, 1024, True), (STAR9, "f32", 128, 1 << 17, True), (STAR9, "f32", 128, (1 << 17) - 1, False),
+    (STAR2, "f32", 128, 1024, True), (STAR9, "f32", 128, 98_304, True), (STAR9, "f32", 128, 98_303, False),
     (TEN, "f32", 128, 1 << 18, False), (STAR9, "f32", 256, 2000, True),
     # fp16: where the plan is slabs
     (STAR2, "f16", 64, 2000, True), (TEN, "f16", 128, (1 << 17) - 1, True), (TEN, "f16", 128, 1 << 17, False), (STAR9, "f16", 64, 1 << 18, False), (TWENTY, "f16_f32", 64, 1 << 18, False)])
