@@ -364,7 +364,7 @@ aclsparseStatus_t aclsparseSpMV(aclsparseHandle_t handle, aclsparseOperation_t o
  * Preprocess: where the rows of A repeat (a mesh operator, as above under SpMV)
  * Preprocess leaves a byte a row in the buffer and the calls read that instead of
  * the column indices.  Call Preprocess again for another structure.
- * Preprocess launches a few kernels, synchronises the stream (up to four times)
+ * Preprocess launches a few kernels, synchronises the stream (up to five times)
  * and must not be captured.
  */
 aclsparseStatus_t aclsparseSpMMGetBufferSize(aclsparseHandle_t handle, aclsparseOperation_t opA,
