@@ -33,7 +33,7 @@
 // the caller (or the copy described below) has them.  val * x is exact in
 // fp64; the additions of a row are made in an order that the layout fixes —
 // inside a lane in stored order, across the lanes of a wavefront by a scan of
-// fixed shape, across wavefronts and windows by one thread in ascending order
+// fixed shape, across wavefronts and windows in ascending order
 // — so two calls on the same data give the same bits, and a row is rounded
 // once.  Integer data is summed with wrap-around in 32 bits.
 //
@@ -185,22 +185,53 @@ __device__ __forceinline__ Uint4 LoadFourRaw(const ValT *p)
     }
 }
 
-// y[row] = alpha * sum + beta * yIn[row].
+// alpha * sum + beta * old.
 template <typename OutT, typename AccT>
-__device__ __forceinline__ void StoreOut(OutT *y, const OutT *yIn, int64_t row, AccT sum, AccT alpha, AccT beta)
+__device__ __forceinline__ OutT Scaled(AccT sum, AccT alpha, AccT beta, OutT old)
 {
     if constexpr (std::is_same<AccT, uint32_t>::value) {
         uint32_t o = alpha * sum;
         if (beta != 0u) {
-            o += beta * static_cast<uint32_t>(yIn[row]);
+            o += beta * static_cast<uint32_t>(old);
         }
-        y[row] = static_cast<OutT>(static_cast<int32_t>(o));
+        return static_cast<OutT>(static_cast<int32_t>(o));
     } else {
         double o = alpha * sum;
         if (beta != 0.0) {
-            o += beta * ToAcc<double>(yIn[row]);
+            o += beta * ToAcc<double>(old);
         }
-        y[row] = FromAcc<OutT>(o);
+        return FromAcc<OutT>(o);
+    }
+}
+
+// y[row] = alpha * sum + beta * yIn[row].
+template <typename OutT, typename AccT>
+__device__ __forceinline__ void StoreOut(OutT *y, const OutT *yIn, int64_t row, AccT sum, AccT alpha, AccT beta)
+{
+    OutT old{};
+    if (beta != AccT(0)) {
+        old = yIn[row];
+    }
+    y[row] = Scaled<OutT, AccT>(sum, alpha, beta, old);
+}
+
+// The same for the rows row0 + row[0 .. N) that are below row0 + nRows; what it reads of yIn it asks for together.
+template <int N, typename OutT, typename AccT>
+__device__ __forceinline__ void StoreRows(OutT *y, const OutT *yIn, int64_t row0, int32_t nRows, const int32_t (&row)[N],
+                                          const AccT (&sum)[N], AccT alpha, AccT beta)
+{
+    OutT old[N] = {};
+    if (beta != AccT(0)) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            old[u] = yIn[row0 + (row[u] < nRows ? row[u] : 0)];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        if (row[u] < nRows) {
+            y[row0 + row[u]] = Scaled<OutT, AccT>(sum[u], alpha, beta, old[u]);
+        }
     }
 }
 
@@ -246,14 +277,20 @@ __device__ __forceinline__ double DppMove(double old, double src)
                                                  static_cast<uint32_t>(__double2hiint(src)));
     return __hiloint2double(static_cast<int>(hi), static_cast<int>(lo));
 }
-__device__ __forceinline__ uint32_t ReadLane63(uint32_t v)
+// (`lane` the same in all lanes)
+__device__ __forceinline__ uint32_t ReadLane(uint32_t v, int lane)
 {
-    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), kWave - 1));
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
 }
-__device__ __forceinline__ double ReadLane63(double v)
+__device__ __forceinline__ double ReadLane(double v, int lane)
 {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), kWave - 1),
-                            __builtin_amdgcn_readlane(__double2loint(v), kWave - 1));
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+template <typename T>
+__device__ __forceinline__ T ReadLane63(T v)
+{
+    return ReadLane(v, kWave - 1);
 }
 
 // One step of the segmented scan: v and `fresh` of the lanes that the move reaches take the lane's at the given
@@ -317,7 +354,7 @@ __device__ __forceinline__ void SegRound(const int32_t (&k)[kSegEntries], const 
 // What a wavefront leaves of its stretch for the one thread that joins the stretches: the sum of its first run
 // (which may go on from the stretch before) and of the run still open at its end.  ends: [2 * wave] head,
 // [2 * wave + 1] tail; a key of kNoKey: none.
-struct SegEnds {
+struct __align__(16) SegEnds {
     int32_t key[2 * (kBlkThreads / kWave)];
     uint64_t sum[2 * (kBlkThreads / kWave)];
 };
@@ -376,40 +413,6 @@ __device__ __forceinline__ void SegJoin(const SegEnds &ends, int waves, int32_t 
             }
             pendKey = tk;
             pendSum = SlotToAcc<AccT>(ends.sum[2 * w + 1]);
-        }
-    }
-}
-
-// SegJoin by the lanes of one wavefront: lane w fetches what wavefront w left, the joining itself runs on values
-// passed from lane to lane in turn (the same order, the same sums); lane 0 writes.  All 64 lanes call it.
-template <typename AccT, typename OutFn>
-__device__ __forceinline__ void SegJoinWave(const SegEnds &ends, int waves, int lane, int32_t &pendKey, AccT &pendSum,
-                                            OutFn &&out)
-{
-    const int w = lane < waves ? lane : 0;
-    const int32_t hkMine = ends.key[2 * w], tkMine = ends.key[2 * w + 1];
-    const uint64_t hsMine = ends.sum[2 * w], tsMine = ends.sum[2 * w + 1];
-    for (int i = 0; i < waves; ++i) {
-        const int32_t hk = __shfl(hkMine, i), tk = __shfl(tkMine, i);
-        const uint64_t hs = __shfl(static_cast<unsigned long long>(hsMine), i);
-        const uint64_t ts = __shfl(static_cast<unsigned long long>(tsMine), i);
-        if (hk != kNoKey) {
-            if (pendKey == hk) {
-                pendSum += SlotToAcc<AccT>(hs);
-            } else {
-                if (pendKey != kNoKey && lane == 0) {
-                    out(pendKey, pendSum);
-                }
-                pendKey = hk;
-                pendSum = SlotToAcc<AccT>(hs);
-            }
-        }
-        if (tk != kNoKey) {
-            if (pendKey != kNoKey && lane == 0) {
-                out(pendKey, pendSum);
-            }
-            pendKey = tk;
-            pendSum = SlotToAcc<AccT>(ts);
         }
     }
 }
@@ -1519,6 +1522,22 @@ __device__ __forceinline__ int ChunkOf(const int32_t *tabD, int32_t P, int32_t p
     return lo;
 }
 
+// A constant put together where it is used (kept in registers from the kernel's start on it makes the compiler spill others).
+__device__ __forceinline__ uint64_t MadeHere(uint64_t v)
+{
+    uint32_t lo = static_cast<uint32_t>(v), hi = static_cast<uint32_t>(v >> 32);
+    asm volatile("" : "+v"(lo), "+v"(hi));
+    return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// Four entries loaded `ahead` places in front of where they belong, put there (ahead <= 0: they are; what is moved in from
+// behind the array's last entry is zero).
+__device__ __forceinline__ Uint4 ShiftedFour(Uint4 v, int32_t ahead)
+{
+    const Uint4 by1 = Uint4{v.y, v.z, v.w, 0u}, by2 = Uint4{v.z, v.w, 0u, 0u}, by3 = Uint4{v.w, 0u, 0u, 0u};
+    return ahead <= 0 ? v : ahead == 1 ? by1 : ahead == 2 ? by2 : ahead == 3 ? by3 : Uint4{0u, 0u, 0u, 0u};
+}
+
 // The sum of a long row's partial sums, lane by lane in panel order and then across the lanes, the same way at
 // every call; every lane returns it.
 template <typename AccT>
@@ -1547,7 +1566,8 @@ __device__ __forceinline__ AccT LongRowTotal(const uint64_t *__restrict__ from, 
 constexpr int kLaneRun = 16;        // consecutive entries a lane sums in one round of phase 2
 constexpr int kBigRound = kWave * kLaneRun;
 constexpr int kStagePasses = 2;     // passes over a block's positions whose loads a wavefront has in flight at a time
-constexpr uint64_t kJoinMark = 0x7ff8dead0000beefull;  // rowSum of a row that the joining thread writes
+constexpr int kOutAtOnce = 4;       // rows that a lane writes at a time
+constexpr uint64_t kJoinMark = 0x7ff8dead0000beefull;  // rowSum of a row that several wavefronts have pieces of
 
 template <typename ValT, typename OutT>
 struct BlockRowsArgs {
@@ -1581,10 +1601,19 @@ struct BlockRowsArgs {
 // lane takes kLaneRun consecutive entries of the window into registers; behind a barrier the window's memory serves
 // as rowSum[key - first key of the window].  (3) A lane adds its entries up run by run, in stored order; a run that
 // begins and ends inside the lane is a row's sum and goes to rowSum.  The runs at the lanes' edges are joined by a
-// segmented scan over the wavefront, the ones at the wavefronts' edges by one thread (SegJoin), which writes those
-// rows itself.  (4) rowSum goes out, a key a lane.
+// segmented scan over the wavefront, the ones at the wavefronts' edges by the lanes of wavefront 0, which write those rows
+// themselves.  (4) rowSum goes out, a key a lane.
+//
+// Bound by the length of a block's turn: the workgroups that fit a compute unit wait for one another's memory, and a
+// register that the compiler spills waits behind every load in flight.  The small size fits six wavefronts a SIMD (80
+// registers), the others four, all without spills.  31 M entries over 4 M rows (small blocks) 100 -> 90 us, 65 M over 8.4 M
+// (middle ones) 235 -> 219, of which 18 us were 20 bytes of spilled registers in the middle size; the rest is the join of the
+// wavefronts' edges by lanes side by side (one lane after the other had each wait for an old y) and the end of the value
+// array read without a second path around every load.  A workgroup that stays and takes block after block, with the next
+// block's tables and places asked for ahead, is slower (160 -> 179 us a call): its wavefronts meet at one more barrier, where
+// all of them wait for the last row written.  So are sums in memory of their own, without the barrier in front of them (172).
 template <int kSize, typename ValT, typename OutT, typename AccT>
-__global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 5 : 4) void SpmvBlockRowsKernel(
+__global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 6 : 4) void SpmvBlockRowsKernel(
     const BlockRowsArgs<ValT, OutT> a)
 {
     constexpr bool kIntData = std::is_same<ValT, int32_t>::value;
@@ -1636,7 +1665,7 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 5 : 4) void
         }
     }
     const int32_t nB = m.nEntries;  // entries of the block
-    int32_t pendKey = kNoKey;  // (wavefront 0: the row that is still open across the wavefronts and windows)
+    int32_t pendKey = kNoKey;  // (wavefront 0: the row that is still open behind a window, and its sum so far)
     AccT pendSum = AccT(0);
     // (whatever the tables hold, a row outside the block is never written)
     auto outKey = [&](int32_t key, AccT sum) {
@@ -1711,29 +1740,21 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 5 : 4) void
                 }
             }
         }
-        // the values: four at a time at any entry of the block that is at least four in front of the array's end
-        // (a lane behind the block's last entry reads its first ones; what it reads is not used)
+        // the values: four at a time; the four at the end of the array start early enough to lie inside it and are put
+        // into their places when they are used (a lane behind the block's last entry reads its first ones; what it
+        // reads is not used)
         Uint4 vraw[kMaxRounds][kLaneRun / 4];
-        const bool atArrayEnd = static_cast<int64_t>(m.base) + nB + 4 > a.valEntries;
+        const int64_t last4 = a.valEntries - m.base - 4;  // (where the last four start, from the block's first entry)
+        const int32_t lastFour = last4 < INT32_MAX ? static_cast<int32_t>(last4) : INT32_MAX;
+        const bool atArrayEnd = nB > lastFour;
 #pragma unroll
         for (int u = 0; u < kMaxRounds; ++u) {
             const int32_t q = w0 + (rBeg + u) * kBigRound + lane * kLaneRun;
             const ValT *from = a.vals + m.base;
 #pragma unroll
             for (int f = 0; f < kLaneRun / 4; ++f) {
-                const int32_t qf = q + 4 * f;
-                if (!atArrayEnd) {
-                    vraw[u][f] = LoadFourRaw(from + (qf < nEnd ? qf : 0));
-                } else {
-                    vraw[u][f] = Uint4{0, 0, 0, 0};
-                    if (qf + 4 <= nEnd) {
-                        vraw[u][f] = LoadFourRaw(from + qf);
-                    } else if (qf < nEnd) {
-                        vraw[u][f].x = ToRaw(from[qf]);
-                        vraw[u][f].y = qf + 1 < nEnd ? ToRaw(from[qf + 1]) : 0u;
-                        vraw[u][f].z = qf + 2 < nEnd ? ToRaw(from[qf + 2]) : 0u;
-                    }
-                }
+                const int32_t qf = q + 4 * f < nEnd ? q + 4 * f : 0;
+                vraw[u][f] = LoadFourRaw(from + (qf < lastFour ? qf : lastFour));
             }
         }
         if (w0 > 0) {
@@ -1804,6 +1825,12 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 5 : 4) void
                 int32_t key = before[u] + static_cast<int32_t>(b & 1u);  // of the lane's first entry
                 const int32_t key0 = key;
                 bool headOpen = true;
+                if (atArrayEnd) {
+#pragma unroll
+                    for (int f = 0; f < kLaneRun / 4; ++f) {
+                        vraw[u][f] = ShiftedFour(vraw[u][f], q + 4 * f - lastFour);
+                    }
+                }
 #pragma unroll
                 for (int j = 0; j < kLaneRun; ++j) {
                     if (j > 0 && ((b >> j) & 1u) != 0) {
@@ -1849,27 +1876,62 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 5 : 4) void
             }
         }
         if (lane == 0) {
-            // to the joining thread its two ends; and in rowSum a mark for both: theirs is not a sum to write out
+            // its two ends for whoever joins the pieces; and in rowSum a mark for both rows: theirs is not a whole sum
             SegLeave<AccT>(ends, wave, firstKey, carryKey, firstKey == carryKey, carrySum);
             if (firstKey != kNoKey) {
-                park(firstKey, kJoinMark);
-                park(carryKey, kJoinMark);
+                const uint64_t mark = MadeHere(kJoinMark);
+                park(firstKey, mark);
+                park(carryKey, mark);
             }
         }
         LdsBarrier();
+        const bool last = w0 + kW >= nB;
         if (wave == 0) {
-            SegJoinWave<AccT>(ends, kWaves, lane, pendKey, pendSum, outKey);
-        }
-        const int32_t keyStop = keyEnd - keyWin < static_cast<int32_t>(kSums) ? keyEnd : keyWin + static_cast<int32_t>(kSums) - 1;
-        for (int32_t key = keyWin + 1 + tid; key <= keyStop; key += kThreads) {
-            const uint64_t sum = rowSum[key - keyWin];
-            if (sum != kJoinMark) {
-                outKey(key, SlotToAcc<AccT>(sum));
+            // The rows with an edge of a wavefront in them, an edge a lane: the first edge of a row adds up its pieces in
+            // ascending order, behind what the window before left of it.  The last row of a window may go on in the next.
+            const int32_t key = lane < 2 * kWaves ? ends.key[lane < 2 * kWaves ? lane : 0] : kNoKey;
+            uint32_t same = 0;
+#pragma unroll
+            for (int e = 0; e < 2 * kWaves; ++e) {
+                same |= (__builtin_amdgcn_readlane(key, e) == key ? 1u : 0u) << e;
+            }
+            const bool firstEdge = key != kNoKey && (same & ((1u << (lane & 31)) - 1u)) == 0;
+            AccT sum = pendSum;
+            bool any = key == pendKey;
+            for (uint32_t in = firstEdge ? same : 0u; in != 0; in &= in - 1) {
+                const AccT part = SlotToAcc<AccT>(ends.sum[__ffs(static_cast<int>(in)) - 1]);
+                sum = any ? sum + part : part;
+                any = true;
+            }
+            if (pendKey != kNoKey && lane == 0 && key != pendKey) {
+                outKey(pendKey, pendSum);  // (it ended with the window before)
+            }
+            if (firstEdge && (last || key != keyEnd)) {
+                outKey(key, sum);
+            }
+            if (!last) {
+                const uint64_t open = __ballot(firstEdge && key == keyEnd);
+                pendKey = keyEnd;
+                pendSum = ReadLane(sum, __ffsll(static_cast<long long>(open)) - 1);
             }
         }
-    }
-    if (tid == 0 && pendKey != kNoKey) {
-        outKey(pendKey, pendSum);
+        // The others a key a lane, kOutAtOnce rows of a lane asked for together.
+        for (int32_t key0 = keyWin + 1; key0 <= keyEnd; key0 += kOutAtOnce * kThreads) {
+            int32_t rowOf[kOutAtOnce];
+            AccT sumOf[kOutAtOnce];
+#pragma unroll
+            for (int u = 0; u < kOutAtOnce; ++u) {
+                const int32_t key = key0 + tid + u * kThreads;
+                rowOf[u] = kBlockRows;
+                sumOf[u] = AccT(0);
+                if (key <= keyEnd && key <= kBlockRows) {  // (so it is, whatever the tables hold: there is room for it)
+                    const uint64_t slot = rowSum[key - keyWin];
+                    rowOf[u] = slot != kJoinMark ? ordRow[key] : kBlockRows;
+                    sumOf[u] = SlotToAcc<AccT>(slot);
+                }
+            }
+            StoreRows<kOutAtOnce, OutT, AccT>(a.y, a.yIn, row0, nRows, rowOf, sumOf, alpha, beta);
+        }
     }
 }
 

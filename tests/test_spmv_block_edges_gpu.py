@@ -1,0 +1,50 @@
+"""Windowed row blocks at their edges: the four values at the end of the value array, which a lane loads from further in front,
+and rows whose pieces lie in several wavefronts and several windows of a block, with an old y to be scaled."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import to_dev
+
+pytestmark = pytest.mark.gpu
+
+COLS = 1_400_000
+
+
+def _matrix(rows, tail, spans, seed):
+    """Short rows; `spans`: rows of many entries, their columns in no order, so that they stay in the blocks; the last rows hold
+    `tail` entries each."""
+    rng = np.random.default_rng(seed)
+    lengths = rng.integers(0, 16, rows)
+    for row, n in spans.items():
+        lengths[row] = n
+    lengths[-2:] = tail
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    return rowptr, rng.integers(0, COLS, nnz).astype(np.int32), rng
+
+
+@pytest.mark.parametrize("tail", [1, 2, 3, 4, 7, 16, 17, 0])
+@pytest.mark.parametrize("dtype,alg", [("f32", "default"), ("f16", "default"), ("f32", "frozen")])
+def test_last_values_of_the_array_and_rows_across_windows(osa, gpu_ctx, monkeypatch, tail, dtype, alg):
+    for name in ("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "OPS_SPARSE_ORDERED_LIVE_MIN_COLS"):
+        monkeypatch.setenv(name, "0")
+    monkeypatch.setenv("OPS_SPARSE_BLOCKED_NO_STREAM", "1")
+    dev, stream, handle = gpu_ctx
+    rows = 300_001
+    spans = {5: 300, 1000: 4096, 1001: 4097, 40_000: 9000, 80_000: 20_000, 80_001: 3, rows - 4: 6000}
+    rowptr, colind, rng = _matrix(rows, tail, spans, 100 + tail)
+    nnz = colind.size
+    kind = {"f32": torch.float32, "f16": torch.float16}[dtype]
+    val, x = (torch.from_numpy(rng.uniform(-1, 1, n).astype(np.float32)).to(kind).float().numpy() for n in (nnz, COLS))
+    y0 = rng.uniform(-1, 1, rows).astype(np.float32)
+    y = to_dev(y0, dev)
+    A = osa.Csr(rows, COLS, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev, kind))
+    op = osa.SpmvOp(handle, A, osa.DnVec(to_dev(x, dev, kind)), osa.DnVec(y),
+                    alg=osa.ACL_SPARSE_SPMV_CSR_ALG2 if alg == "frozen" else osa.ACL_SPARSE_SPMV_ALG_DEFAULT)
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, nnz)
+    op(1.5, -0.5)
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, COLS, rowptr, colind, val, x, y0, 1.5, -0.5)
+    assert oracle.max_rel_err(y.cpu().numpy(), gold) <= 1e-5
