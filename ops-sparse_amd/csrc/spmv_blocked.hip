@@ -419,19 +419,20 @@ __device__ __forceinline__ void SegJoin(const SegEnds &ends, int waves, int32_t 
 
 // ---- row blocks ------------------------------------------------------------------------------------------------
 
-// Windowed row blocks come in three sizes: the entries of a block whose gathered x a phase-2 workgroup holds in LDS at a
-// time (the window), the rows of a block at most, and the workgroup's threads.  Small blocks: more workgroups a compute
-// unit, whose waits for memory and at barriers fall at different times.  Large ones: longer chunks (less padding, fewer
-// lines of gathered x shared between blocks).  The layout takes the smallest whose chunks are long enough.  A call with
-// live values, small / middle / large: 31 M entries over 123 panels (20 / 37 / 73 a chunk) 159 / 166 / 176 us; 24 M over
-// 46 panels (64 a chunk and more) 96 / 109 / 118; 65 M over 256 panels (9.7 / 18 / 35) 343 / 335 / 334; 34 M over 256
-// (7.5 / 14 / 28) does not fit the small size and takes 243 / 254.
+// Windowed row blocks come in two sizes: the entries of a block whose gathered x a phase-2 workgroup holds in LDS at a
+// time (the window), the rows of a block at most, the workgroup's threads and the wavefronts a SIMD that its registers leave
+// room for.  The ordinary size gives every wavefront one round of its window and all of a block's positions in one turn, and
+// three workgroups fit a compute unit.  A call, ordinary size / 4096 entries and 256 threads, six workgroups a compute unit, the
+// faster of the smaller ones: 31 M entries over 123 panels 140 / 144 us, 47 M frozen over 183 162 / 169, 24 M over 123 103 / 111,
+// 32 M over 62 124 / 124; against 7168 entries and 256 threads, two rounds and two turns: 65 M over 256 277 / 291.  The large one is
+// for chunks that would be short: more entries of a block in a panel, less padding, fewer lines of gathered x shared between
+// blocks.
 struct RowsSize {
-    int32_t window, rowLog, threads;
+    int32_t window, rowLog, threads, waves;
     int64_t chunk;  // entries of a (panel, block) chunk, on average, from which the size is taken
 };
-constexpr RowsSize kRowsSizes[] = {{4096, 10, 256, 10}, {7168, 11, 256, 8}, {14336, 12, 512, 0}};
-constexpr int kNumRowsSizes = 3;
+constexpr RowsSize kRowsSizes[] = {{8192, 11, 512, 6, 8}, {14336, 12, 512, 4, 0}};
+constexpr int kNumRowsSizes = 2;
 
 // What the workgroup of a row block needs to know before anything else, in one piece.
 struct BlockMeta {
@@ -451,16 +452,13 @@ struct BlockMeta {
 __host__ __device__ __forceinline__ int32_t BlockBitsOff(int32_t short0, int32_t b) { return ((short0 >> 5) & ~3) + 8 * b; }
 __host__ __device__ __forceinline__ int32_t BlockOrdOff(int32_t row0, int32_t b) { return ((row0 + 7) & ~7) + 16 * b; }
 
-// Row block of a row: blocks of 2^rowLog rows, cut again wherever the row's first entry passes a multiple of the entry
-// window (`offsets`: the row offsets without the entries of long rows), and, with `longBefore` (the number of long
-// rows among rows 0 .. r), behind every long row.  Monotone in the row number.
-__device__ __forceinline__ int32_t RowBlockOf(const int32_t *__restrict__ offsets, int32_t row, int32_t window,
-                                              int32_t numBlocks, const int32_t *__restrict__ longBefore, int32_t rowLog)
+// Row block of a row.  Windowed blocks: `blockOf` says (RowBlockCutsKernel).  Streamed ones: blocks of 2^rowLog rows, cut again
+// wherever the row's first entry passes a multiple of the entry window (`offsets`: the row offsets without the entries of long
+// rows).  Monotone in the row number.
+__device__ __forceinline__ int32_t RowBlockOf(const int32_t *__restrict__ blockOf, const int32_t *__restrict__ offsets,
+                                              int32_t row, int32_t window, int32_t numBlocks, int32_t rowLog)
 {
-    int32_t b = (row >> rowLog) + offsets[row] / window;
-    if (longBefore != nullptr && row > 0) {
-        b += longBefore[row - 1];
-    }
+    const int32_t b = blockOf != nullptr ? blockOf[row] : (row >> rowLog) + offsets[row] / window;
     return b < 0 ? 0 : (b < numBlocks ? b : numBlocks - 1);  // in range whatever the arrays hold
 }
 
@@ -500,7 +498,7 @@ __global__ __launch_bounds__(kBlockThreads) void IotaKernel(int32_t *__restrict_
 __global__ __launch_bounds__(kBlockThreads) void BlockedChunkKeysKernel(
     const int32_t *__restrict__ colSorted, const int32_t *__restrict__ pos, const int32_t *__restrict__ rowOfPos,
     const int32_t *__restrict__ offsets, int64_t nnz, int64_t cols, int32_t numBlocks, int32_t window,
-    const int32_t *__restrict__ longBefore, int32_t cutBehindLong, int32_t rowLog, uint16_t *__restrict__ colLocal,
+    const int32_t *__restrict__ longBefore, const int32_t *__restrict__ blockOf, int32_t rowLog, uint16_t *__restrict__ colLocal,
     int32_t *__restrict__ chunkKey, int32_t *__restrict__ rowOfSrc, int32_t *__restrict__ status)
 {
     const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
@@ -515,8 +513,7 @@ __global__ __launch_bounds__(kBlockThreads) void BlockedChunkKeysKernel(
             atomicOr(status, 1);
             chunkKey[i] = -1;
         } else {
-            chunkKey[i] = (col >> kPanelLog) * numBlocks +
-                          RowBlockOf(offsets, row, window, numBlocks, cutBehindLong != 0 ? longBefore : nullptr, rowLog);
+            chunkKey[i] = (col >> kPanelLog) * numBlocks + RowBlockOf(blockOf, offsets, row, window, numBlocks, rowLog);
         }
     }
 }
@@ -726,10 +723,43 @@ __global__ __launch_bounds__(kBlockThreads) void BlockedTablesKernel(const int32
     }
 }
 
+// Where the windowed row blocks begin: flags[row] = 1 (zero before).  A block ends where the entries of its rows reach
+// `window`, in front of a row that would make it too long for 16-bit slots, behind 2^rowLog rows, behind a long row (longBefore,
+// or NULL) and at a multiple of kCutRows rows; each starts where the one before ends.  (Cut at multiples of either bound the blocks of 65 M entries over 8.4 M rows held 4 200 entries of 6 272,
+// and there were 12 500 instead of 8 400: a block's length in entries pays for what it waits for at its start.)  A wavefront
+// walks the kCutRows rows that are its own; two looks at 64 rows each find a block's end, 50 - 100 us for all of them.
+// No more blocks than numbers of them (rows / 2^rowLog + entries / window and one behind every long row): cut at the multiples
+// of both bounds they are that many, a greedy block that starts in or behind one of those ends no earlier, and a row too long
+// for the slots of its block is several windows long.
+constexpr int32_t kCutRows = 1 << 16;
+
+__global__ __launch_bounds__(kWave) void RowBlockCutsKernel(const int32_t *__restrict__ offsets, int32_t rows, int32_t window,
+                                                            const int32_t *__restrict__ longBefore, int32_t rowLog,
+                                                            int32_t *__restrict__ flags)
+{
+    const int lane = threadIdx.x;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kCutRows;
+    const int32_t end = static_cast<int32_t>(first + kCutRows < rows ? first + kCutRows : rows);
+    const int32_t step = (1 << rowLog) / kWave;  // (16 - 64)
+    for (int32_t row = static_cast<int32_t>(first); row < end;) {
+        if (lane == 0) {
+            flags[row] = 1;
+        }
+        const int32_t base = offsets[row], longs = longBefore != nullptr && row > 0 ? longBefore[row - 1] : 0;
+        // does row r go on with the block?  (no: nor does any behind it)
+        auto goesOn = [&](int32_t r) {
+            return r < end && r - row < (1 << rowLog) && offsets[r] - base < window && offsets[r + 1] - base <= kMaxBlockEntries &&
+                   (longBefore == nullptr || longBefore[r - 1] == longs);
+        };
+        const int32_t near = row + step * __popcll(__ballot(goesOn(row + (lane + 1) * step)));
+        row = near + 1 + __popcll(__ballot(lane < step && goesOn(near + 1 + lane)));
+    }
+}
+
 // blockRow[b] = first row of row block b (blockRow pre-filled with `rows`).
-__global__ __launch_bounds__(kBlockThreads) void BlockedRowBlocksKernel(const int32_t *__restrict__ offsets,
+__global__ __launch_bounds__(kBlockThreads) void BlockedRowBlocksKernel(const int32_t *__restrict__ blockOf,
+                                                                        const int32_t *__restrict__ offsets,
                                                                         int32_t rows, int32_t window, int32_t B,
-                                                                        const int32_t *__restrict__ longBefore,
                                                                         int32_t rowLog, int32_t *__restrict__ blockRow)
 {
     const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -737,8 +767,8 @@ __global__ __launch_bounds__(kBlockThreads) void BlockedRowBlocksKernel(const in
         return;
     }
     const int32_t row = static_cast<int32_t>(r);
-    const int32_t cur = RowBlockOf(offsets, row, window, B, longBefore, rowLog);
-    const int32_t prev = row > 0 ? RowBlockOf(offsets, row - 1, window, B, longBefore, rowLog) : -1;
+    const int32_t cur = RowBlockOf(blockOf, offsets, row, window, B, rowLog);
+    const int32_t prev = row > 0 ? RowBlockOf(blockOf, offsets, row - 1, window, B, rowLog) : -1;
     for (int32_t b = prev + 1; b <= cur; ++b) {
         blockRow[b] = row;
     }
@@ -1605,15 +1635,15 @@ struct BlockRowsArgs {
 // themselves.  (4) rowSum goes out, a key a lane.
 //
 // Bound by the length of a block's turn: the workgroups that fit a compute unit wait for one another's memory, and a
-// register that the compiler spills waits behind every load in flight.  The small size fits six wavefronts a SIMD (80
-// registers), the others four, all without spills.  31 M entries over 4 M rows (small blocks) 100 -> 90 us, 65 M over 8.4 M
-// (middle ones) 235 -> 219, of which 18 us were 20 bytes of spilled registers in the middle size; the rest is the join of the
-// wavefronts' edges by lanes side by side (one lane after the other had each wait for an old y) and the end of the value
-// array read without a second path around every load.  A workgroup that stays and takes block after block, with the next
-// block's tables and places asked for ahead, is slower (160 -> 179 us a call): its wavefronts meet at one more barrier, where
-// all of them wait for the last row written.  So are sums in memory of their own, without the barrier in front of them (172).
+// register that the compiler spills waits behind every load in flight (no size spills any).  65 M entries over 8.4 M rows,
+// live values, 235 us at first; 219 without 20 bytes of spilled registers, with the wavefronts' edges joined by lanes side by
+// side (one after the other had each wait for an old y) and the end of the value array read without a second path around every
+// load; 189 with the blocks cut one after the other (RowBlockCutsKernel); 176 with one round a wavefront and one turn a block.
+// 31 M over 4 M rows 100 -> 79.  A workgroup that stays and takes block after block, with the next block's tables and places
+// asked for ahead, is slower (160 -> 179 us a call): its wavefronts meet at one more barrier, where all of them wait for the
+// last row written.  So are sums in memory of their own, without the barrier in front of them (172).
 template <int kSize, typename ValT, typename OutT, typename AccT>
-__global__ __launch_bounds__(kRowsSizes[kSize].threads, kSize == 0 ? 6 : 4) void SpmvBlockRowsKernel(
+__global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves) void SpmvBlockRowsKernel(
     const BlockRowsArgs<ValT, OutT> a)
 {
     constexpr bool kIntData = std::is_same<ValT, int32_t>::value;
@@ -2539,10 +2569,8 @@ int LaunchBlocked(const SpmvArgs &a, const OpsparseSpmvPlan &plan, int32_t valTy
             const auto threads = dim3(kRowsSizes[l.size].threads);
             if (l.size == 0) {
                 hipLaunchKernelGGL((SpmvBlockRowsKernel<0, ValT, OutT, AccT>), grid, threads, 0, a.stream, args);
-            } else if (l.size == 1) {
-                hipLaunchKernelGGL((SpmvBlockRowsKernel<1, ValT, OutT, AccT>), grid, threads, 0, a.stream, args);
             } else {
-                hipLaunchKernelGGL((SpmvBlockRowsKernel<2, ValT, OutT, AccT>), grid, threads, 0, a.stream, args);
+                hipLaunchKernelGGL((SpmvBlockRowsKernel<1, ValT, OutT, AccT>), grid, threads, 0, a.stream, args);
             }
             if (plan.numEmptyRows > 0) {
                 hipLaunchKernelGGL((SpmvEmptyRowsKernel<OutT, AccT>),
@@ -2751,6 +2779,14 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
     }
     // where the values are read in place a long row ends its block, so that a block's other entries are one piece
     const int32_t *cutBehind = (longBefore != nullptr && !l.frozenLong && !l.streamed) ? longBefore : nullptr;
+    int32_t *blockOf = nullptr;
+    if (!l.streamed) {
+        blockOf = ints(l.emptyFlagsOff);  // (the rows without entries are listed by now)
+        LaunchFillI32(blockOf, outputs, 0, s);
+        hipLaunchKernelGGL(RowBlockCutsKernel, dim3(GridOf(outputs, kCutRows, INT32_MAX)), dim3(kWave), 0, s, offsets,
+                           static_cast<int32_t>(outputs), l.window, cutBehind, l.rowLog, blockOf);
+        LaunchInclusiveScanI32(blockOf, blockOf, outputs, -1, scratch, s);
+    }
     // Entries in (panel, original position) order: stable 4-bit radix passes over the panel number.
     const int32_t *firstKeys = colInd;
     if (longBefore != nullptr) {
@@ -2770,7 +2806,7 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
     int32_t *chunkKey = keys[1 - cur], *rowOfSrc = poss[1 - cur];
     hipLaunchKernelGGL(BlockedChunkKeysKernel, dim3(GridOf(nnz, kBlockThreads, 16384)), dim3(kBlockThreads), 0, s,
                        keys[cur], pos, rowOfPos, offsets, nnz, inputs, l.B, l.window, longBefore,
-                       cutBehind != nullptr ? 1 : 0, l.rowLog, colLocal, chunkKey, rowOfSrc, status);
+                       blockOf, l.rowLog, colLocal, chunkKey, rowOfSrc, status);
     if (longBefore != nullptr && l.frozenLong) {
         hipLaunchKernelGGL(LongRowPanelsKernel, dim3(GridOf(l.P, kBlockThreads, INT32_MAX)), dim3(kBlockThreads), 0, s,
                            keys[cur], nnz, l.P, l.maxLong, static_cast<int32_t>(l.P) << kPanelLog, ints(l.longChunkOff));
@@ -2797,7 +2833,7 @@ static int AnalyseBlocked(const int32_t *rowOffsets, const int32_t *colInd, cons
                   static_cast<int32_t>((l.streamed ? kStreamPadRow : kPadSlot) * 0x10001u), s);
     LaunchFillI32(blockRow, l.B + 1, static_cast<int32_t>(outputs), s);
     hipLaunchKernelGGL(BlockedRowBlocksKernel, dim3(GridOf(outputs, kBlockThreads, INT32_MAX)), dim3(kBlockThreads), 0, s,
-                       offsets, static_cast<int32_t>(outputs), l.window, l.B, cutBehind, l.rowLog, blockRow);
+                       blockOf, offsets, static_cast<int32_t>(outputs), l.window, l.B, l.rowLog, blockRow);
     if (longBefore != nullptr) {
         hipLaunchKernelGGL(BlockedLongFirstKernel, dim3(GridOf(l.B + 1, kBlockThreads, INT32_MAX)), dim3(kBlockThreads), 0,
                            s, blockRow, longBefore, l.B, ints(l.longFirstOff));

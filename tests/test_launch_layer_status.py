@@ -264,7 +264,7 @@ def test_coosort_buffer_has_room_for_the_offsets_scan_of_short_rows(L):
 
 
 def test_blocked_layout_takes_a_larger_row_block_where_a_smaller_one_does_not_fit(L, osa):
-    """The windowed row blocks come in three sizes.  A size whose chunks are long enough only by a count of blocks rounded
+    """The windowed row blocks come in two sizes.  A size whose chunks are long enough only by a count of blocks rounded
     down, or whose padded positions have no 32-bit numbers, must not keep the matrix from a larger one: every matrix that
     blocks of 2^12 rows and 12 544 entries fit has the layout."""
     live = osa.OPSPARSE_BLOCKED_LIVE_VALUES

@@ -48,3 +48,33 @@ def test_last_values_of_the_array_and_rows_across_windows(osa, gpu_ctx, monkeypa
     stream.synchronize()
     gold = oracle.spmv_f64(rows, COLS, rowptr, colind, val, x, y0, 1.5, -0.5)
     assert oracle.max_rel_err(y.cpu().numpy(), gold) <= 1e-5
+
+
+@pytest.mark.parametrize("rows,longest,ends", [(65_536, 76, False), (65_537, 76, True), (131_071, 40, False), (400_000, 12, True)])
+def test_where_the_blocks_are_cut(osa, gpu_ctx, monkeypatch, rows, longest, ends):
+    """Blocks end at every 65 536 rows, behind their most rows (a stretch of rows of one entry and none) and behind long rows
+    (one beside another, the first and the last row of the matrix, either side of row 65 536)."""
+    for name in ("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "OPS_SPARSE_ORDERED_LIVE_MIN_COLS"):
+        monkeypatch.setenv(name, "0")
+    dev, stream, handle = gpu_ctx
+    rng = np.random.default_rng(rows)
+    lengths = rng.integers(0, longest + 1, rows)
+    lengths[20_000:26_500] = rng.integers(0, 2, 6500)
+    long_rows = [0, 30_000, 30_001, 65_535, rows - 1] if ends else [40_000]
+    lengths[long_rows] = 64 * (COLS // 32768 + 1) + 4096
+    if rows > 131_072:
+        lengths[131_071:131_074] = [7167, 7168, 7169]  # (their columns in no order: they stay in the blocks)
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(0, COLS, nnz).astype(np.int32)
+    for r in long_rows:
+        colind[rowptr[r]:rowptr[r + 1]].sort()
+    val, x = rng.uniform(-1, 1, nnz).astype(np.float32), rng.uniform(-1, 1, COLS).astype(np.float32)
+    y = torch.full((rows,), float("nan"), device=dev)
+    A = osa.Csr(rows, COLS, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev))
+    op = osa.SpmvOp(handle, A, osa.DnVec(to_dev(x, dev)), osa.DnVec(y))
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, nnz)
+    op(1.0, 0.0)
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, COLS, rowptr, colind, val, x, np.zeros(rows, np.float32), 1.0, 0.0)
+    assert oracle.max_rel_err(y.cpu().numpy(), gold) <= 1e-5

@@ -872,8 +872,8 @@ SIZES = {"small": (260_000, 300_000), "middle": (200_000, 9_830_400), "large": (
                                        (torch.bfloat16, torch.bfloat16), (torch.int32, torch.int32),
                                        (torch.int32, torch.float32)])
 def test_every_size_of_the_windowed_row_blocks(osa, gpu_ctx, size, dtype, out):
-    """The windowed blocks come in three sizes by how many entries a (panel, block) chunk gets (10, 300 and 699 panels
-    here): blocks of up to 1024, 2048 and 4096 rows and 4096, 7168 and 14 336 entries a window.  Rows of 0 - 22 entries;
+    """The windowed blocks come in two sizes by how many entries a (panel, block) chunk gets (10 and 300 panels, and 699
+    here): blocks of up to 2048 and 4096 rows and 8192 and 14 336 entries a window.  Rows of 0 - 22 entries;
     a run of empty rows longer than a block; rows of 5000 and 20 000 unsorted entries, which fill several windows; a row of
     20 000 ascending ones (a long row).  Every type of values and of y."""
     dev, stream, handle = gpu_ctx
