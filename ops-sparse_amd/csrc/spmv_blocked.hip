@@ -258,6 +258,8 @@ constexpr int32_t kNoKey = INT32_MAX;  // an entry outside the stream; `store` i
 // Lane-to-lane moves inside the vector ALU (data-parallel primitives): the lanes that the control word gives no
 // source, and the rows that the row mask leaves out, receive `old`.
 constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
+constexpr int kDppQuadSwap1 = 0xb1;    // the lanes of a quad 1, 0, 3, 2
+constexpr int kDppQuadSwap2 = 0x4e;    // 2, 3, 0, 1
 constexpr int kDppWaveShr1 = 0x138;    // every lane from the lane before it; lane 0 has no source
 constexpr int kDppRowBcast15 = 0x142;  // lane 15 of every row of 16 lanes to all lanes of the next row
 constexpr int kDppRowBcast31 = 0x143;  // lane 31 to all lanes of rows 2 and 3
@@ -1560,6 +1562,37 @@ __device__ __forceinline__ uint64_t MadeHere(uint64_t v)
     return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
+// Among the four lanes of a quad: piece j of lane i becomes piece i of lane j.
+// (the moves are made by all lanes, whichever of them keep the result)
+template <int kCtrl>
+__device__ __forceinline__ Uint4 QuadMove(Uint4 v)
+{
+    return Uint4{DppMove<kCtrl, 0xf>(0u, v.x), DppMove<kCtrl, 0xf>(0u, v.y), DppMove<kCtrl, 0xf>(0u, v.z),
+                 DppMove<kCtrl, 0xf>(0u, v.w)};
+}
+template <int kCtrl>
+__device__ __forceinline__ void QuadExchange(Uint4 &a, Uint4 &b, bool second)
+{
+    const Uint4 aMoved = QuadMove<kCtrl>(a), bMoved = QuadMove<kCtrl>(b);
+    a = Uint4{second ? bMoved.x : a.x, second ? bMoved.y : a.y, second ? bMoved.z : a.z, second ? bMoved.w : a.w};
+    b = Uint4{second ? b.x : aMoved.x, second ? b.y : aMoved.y, second ? b.z : aMoved.z, second ? b.w : aMoved.w};
+}
+__device__ __forceinline__ void QuadTranspose(Uint4 &p0, Uint4 &p1, Uint4 &p2, Uint4 &p3)
+{
+    const bool odd = (threadIdx.x & 1) != 0, upper = (threadIdx.x & 2) != 0;
+    QuadExchange<kDppQuadSwap1>(p0, p1, odd);
+    QuadExchange<kDppQuadSwap1>(p2, p3, odd);
+    QuadExchange<kDppQuadSwap2>(p0, p2, upper);
+    QuadExchange<kDppQuadSwap2>(p1, p3, upper);
+}
+
+// A value made anew wherever this stands: what follows from it is not kept in registers over a loop.
+__device__ __forceinline__ int MadeAnew(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // Four entries loaded `ahead` places in front of where they belong, put there (ahead <= 0: they are; what is moved in from
 // behind the array's last entry is zero).
 __device__ __forceinline__ Uint4 ShiftedFour(Uint4 v, int32_t ahead)
@@ -1638,8 +1671,9 @@ struct BlockRowsArgs {
 // register that the compiler spills waits behind every load in flight (no size spills any).  65 M entries over 8.4 M rows,
 // live values, 235 us at first; 219 without 20 bytes of spilled registers, with the wavefronts' edges joined by lanes side by
 // side (one after the other had each wait for an old y) and the end of the value array read without a second path around every
-// load; 189 with the blocks cut one after the other (RowBlockCutsKernel); 176 with one round a wavefront and one turn a block.
-// 31 M over 4 M rows 100 -> 79.  A workgroup that stays and takes block after block, with the next block's tables and places
+// load; 189 with the blocks cut one after the other (RowBlockCutsKernel); 176 with one round a wavefront and one turn a block; 165
+// with the values loaded by quads of lanes: 780 MB, 4.7 TB/s, at which more workgroups a compute unit (64 registers, four instead of
+// three) no longer help.  31 M over 4 M rows 100 -> 74.  A workgroup that stays and takes block after block, with the next block's tables and places
 // asked for ahead, is slower (160 -> 179 us a call): its wavefronts meet at one more barrier, where all of them wait for the
 // last row written.  So are sums in memory of their own, without the barrier in front of them (172).
 template <int kSize, typename ValT, typename OutT, typename AccT>
@@ -1705,6 +1739,8 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
         }
     };
     for (int32_t w0 = 0; w0 < nB; w0 += kW) {
+        // (what follows from the lane is worked out where it is used: kept over the loop it would make the compiler spill)
+        const int tid = MadeAnew(threadIdx.x), lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
         const int32_t nEnd = nB - w0 < kW ? nB : w0 + kW;  // the window holds the entries [w0, nEnd)
         const int32_t rounds = (nEnd - w0 + kBigRound - 1) / kBigRound;
         const int32_t perWave = (rounds + kWaves - 1) / kWaves;
@@ -1770,6 +1806,9 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
                 }
             }
         }
+        // (the lanes of a quad load the quad's 64 entries together, 64 bytes an instruction, and exchange them when they are
+        // used: a lane's own 16 entries one after the other are four loads of 64 lines each)
+        const int32_t loadFirst = (lane & ~3) * kLaneRun + (lane & 3) * 4;
         // the values: four at a time; the four at the end of the array start early enough to lie inside it and are put
         // into their places when they are used (a lane behind the block's last entry reads its first ones; what it
         // reads is not used)
@@ -1779,11 +1818,11 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
         const bool atArrayEnd = nB > lastFour;
 #pragma unroll
         for (int u = 0; u < kMaxRounds; ++u) {
-            const int32_t q = w0 + (rBeg + u) * kBigRound + lane * kLaneRun;
+            const int32_t q = w0 + (rBeg + u) * kBigRound + loadFirst;
             const ValT *from = a.vals + m.base;
 #pragma unroll
             for (int f = 0; f < kLaneRun / 4; ++f) {
-                const int32_t qf = q + 4 * f < nEnd ? q + 4 * f : 0;
+                const int32_t qf = q + f * kLaneRun < nEnd ? q + f * kLaneRun : 0;
                 vraw[u][f] = LoadFourRaw(from + (qf < lastFour ? qf : lastFour));
             }
         }
@@ -1804,6 +1843,17 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
         }
         LdsBarrier();
         // ---- the window's entries into registers
+#pragma unroll
+        for (int u = 0; u < kMaxRounds; ++u) {
+            if (atArrayEnd) {
+#pragma unroll
+                for (int f = 0; f < kLaneRun / 4; ++f) {
+                    vraw[u][f] = ShiftedFour(vraw[u][f], w0 + (rBeg + u) * kBigRound + loadFirst + f * kLaneRun - lastFour);
+                }
+            }
+            QuadTranspose(vraw[u][0], vraw[u][1], vraw[u][2], vraw[u][3]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (their exchange before the window's loads: else the compiler spills)
         uint32_t xraw[kMaxRounds][kLaneRun];
         uint32_t bits[kMaxRounds];
         int32_t before[kMaxRounds];
@@ -1855,12 +1905,6 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
                 int32_t key = before[u] + static_cast<int32_t>(b & 1u);  // of the lane's first entry
                 const int32_t key0 = key;
                 bool headOpen = true;
-                if (atArrayEnd) {
-#pragma unroll
-                    for (int f = 0; f < kLaneRun / 4; ++f) {
-                        vraw[u][f] = ShiftedFour(vraw[u][f], q + 4 * f - lastFour);
-                    }
-                }
 #pragma unroll
                 for (int j = 0; j < kLaneRun; ++j) {
                     if (j > 0 && ((b >> j) & 1u) != 0) {
