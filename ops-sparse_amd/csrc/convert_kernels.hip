@@ -662,6 +662,9 @@ __device__ __forceinline__ auto WideVals(P *pairs, int64_t n)
     return reinterpret_cast<std::conditional_t<std::is_const<P>::value, const uint32_t, uint32_t> *>(pairs) + n;
 }
 
+typedef uint32_t Uint2U __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint64_t Record __attribute__((aligned(4)));  // (a caller's buffer may begin at any 4-byte-aligned address)
+
 // A tile's entries as the loads deliver them: lane l of wavefront w holds entries 512 w + l, 512 w + 64 + l, ...
 template <int T>
 struct WideTileRegs {
@@ -722,10 +725,12 @@ struct WideLds {
     int32_t waveSums[WideShape<T>::kWaves];
 };
 
-// Puts the tile held in registers into the LDS arrays in the order of its digits.  Ends with a barrier.
-template <int T>
-__device__ __forceinline__ void WideOrder(WideLds<T> &lds, const WideTileRegs<T> &r, int32_t shift, int32_t mask,
-                                          int32_t bits)
+// rank[i]: the place in the order of the tile's digits of the thread's entry i, whose digit is dig[i]; lds.outOf: where the
+// entries of a digit go, less their places there.  Ends with a barrier, behind which lds.counters is free.
+template <int T, typename Lds>
+__device__ __forceinline__ void WideRank(Lds &lds, const uint32_t (&dig)[kWideItems],
+                                         const int32_t (&first)[WideShape<T>::kPer], int32_t mask, int32_t bits,
+                                         uint32_t (&rank)[kWideItems])
 {
     constexpr int kPer = WideShape<T>::kPer, kWaves = WideShape<T>::kWaves;
     const int tid = threadIdx.x, lane = tid % kWave;
@@ -734,11 +739,9 @@ __device__ __forceinline__ void WideOrder(WideLds<T> &lds, const WideTileRegs<T>
     for (int32_t d = lane; d < digits; d += kWave) {
         mine[d] = 0;
     }
-    uint32_t dig[kWideItems];
     uint64_t peers[kWideItems];
 #pragma unroll
     for (int i = 0; i < kWideItems; ++i) {
-        dig[i] = WideDigit(r.key[i], shift, mask);
         peers[i] = ~uint64_t{0};
     }
     for (int32_t b = 0; b < bits; ++b) {
@@ -753,7 +756,6 @@ __device__ __forceinline__ void WideOrder(WideLds<T> &lds, const WideTileRegs<T>
         }
     }
     // (a wavefront's own counters: LDS serves a wavefront's instructions in their order)
-    uint32_t rank[kWideItems];
 #pragma unroll
     for (int i = 0; i < kWideItems; ++i) {
         const uint32_t below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(peers[i] >> 32),
@@ -788,7 +790,7 @@ __device__ __forceinline__ void WideOrder(WideLds<T> &lds, const WideTileRegs<T>
         for (int j = 0; j < kPer; ++j) {
             const int32_t d = tid * kPer + j;
             if (d < digits) {
-                lds.outOf[d] = r.first[j] - run;
+                lds.outOf[d] = first[j] - run;
                 constexpr int kAtOnce = 4;
 #pragma unroll
                 for (int w0 = 0; w0 < kWaves; w0 += kAtOnce) {
@@ -812,6 +814,19 @@ __device__ __forceinline__ void WideOrder(WideLds<T> &lds, const WideTileRegs<T>
         rank[i] += static_cast<uint32_t>(mine[dig[i]]);
     }
     LdsBarrier();  // the counters make room for the entries
+}
+
+// Puts the tile held in registers into the LDS arrays in the order of its digits.  Ends with a barrier.
+template <int T>
+__device__ __forceinline__ void WideOrder(WideLds<T> &lds, const WideTileRegs<T> &r, int32_t shift, int32_t mask,
+                                          int32_t bits)
+{
+    uint32_t dig[kWideItems], rank[kWideItems];
+#pragma unroll
+    for (int i = 0; i < kWideItems; ++i) {
+        dig[i] = WideDigit(r.key[i], shift, mask);
+    }
+    WideRank<T>(lds, dig, r.first, mask, bits, rank);
 #pragma unroll
     for (int i = 0; i < kWideItems; ++i) {
         lds.key[rank[i]] = r.key[i];
@@ -853,42 +868,33 @@ __device__ __forceinline__ void WideWrite(const WideLds<T> &lds, int64_t tile, i
     }
 }
 
-// One pass; the payload modes are those of RadixScatterKernel (pairs only), VB the bytes of a value in the arrays
-// that the first pass reads and the last one writes (a template parameter: a branch on it among the loads would
-// leave the compiler unable to count what is in flight).  prefix is the scanned table of WideCountKernel:
-// prefix[digit * numTiles + tile] is the first output position of the tile's entries of that digit.  Every XCD has a
-// range of tiles, its workgroups take neighbouring tiles of it in the same turn, and a workgroup has the loads of its
-// next tile in flight while it writes the current one.  The tile that the end of the array cuts short is done last,
-// by workgroup 0, with bounds checks.
-template <int T, int Mode, int VB>
-__global__ __launch_bounds__(T) void WideScatterKernel(
-    const int32_t *__restrict__ keysIn, const RadixPair *__restrict__ pairsIn, int32_t *__restrict__ keysOut,
-    RadixPair *__restrict__ pairsOut, int64_t n, int32_t keyBase, int32_t shift, int32_t mask, int32_t bits,
-    const int32_t *__restrict__ prefix, int64_t numTiles, RadixPairIo io)
+// The tiles of a pass.  Every XCD has a range of tiles, its workgroups take neighbouring tiles of it in the same turn, and a
+// workgroup has the loads of its next tile in flight while it writes the current one: two sets of registers used in turn.  The
+// tile that the end of the array cuts short is done last, by workgroup 0, with bounds checks.
+template <int T, typename Regs, typename Fetch, typename Order, typename Write>
+__device__ __forceinline__ void WideTurns(int64_t n, int64_t numTiles, Fetch &&fetch, Order &&order, Write &&write)
 {
-    __shared__ WideLds<T> lds;
     const int64_t fullTiles = n / WideShape<T>::kTile;
-    WideTileRegs<T> r;
+    Regs r;
     const uint32_t xcds = gridDim.x < kNumXcd ? gridDim.x : kNumXcd;
     const uint32_t xcd = blockIdx.x % xcds;
     const int64_t step = (gridDim.x - xcd + xcds - 1) / xcds;
     const int64_t tileEnd = fullTiles * (xcd + 1) / xcds;
     int64_t tile = fullTiles * xcd / xcds + blockIdx.x / xcds;
-    // The loads of the next tile are on their way while the current one is ordered and written: two sets of registers
-    // used in turn.  (The last turn fetches its own tile again rather than branch around the loads: a wait for "all
-    // but what was issued since" needs one straight path.)
-    auto turn = [&](WideTileRegs<T> &now, WideTileRegs<T> &next) {
+    // (The last turn fetches its own tile again rather than branch around the loads: a wait for "all but what was issued
+    // since" needs one straight path.)
+    auto turn = [&](Regs &now, Regs &next) {
         const int64_t ahead = tile + step < tileEnd ? tile + step : tile;
-        WideFetch<T, Mode, VB, true>(next, ahead, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
+        fetch(next, ahead, std::true_type{});
         __builtin_amdgcn_sched_barrier(0);  // the loads are issued here, not where the scheduler finds room later
-        WideOrder<T>(lds, now, shift, mask, bits);
-        WideWrite<T, Mode, VB, true>(lds, tile, n, shift, mask, keysOut, pairsOut, io);
+        order(now, tile, std::true_type{});
+        write(tile, std::true_type{});
         LdsBarrier();  // the tile's LDS is free again
         tile += step;
     };
     if (tile < tileEnd) {
-        WideFetch<T, Mode, VB, true>(r, tile, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
-        WideTileRegs<T> other;
+        fetch(r, tile, std::true_type{});
+        Regs other;
         // the first turn stands outside the loop: entered from here, with no stores behind the loads, the loop's
         // wait for the loads would be a wait for everything, the stores of the turn before included
         turn(r, other);
@@ -901,9 +907,211 @@ __global__ __launch_bounds__(T) void WideScatterKernel(
         }
     }
     if (blockIdx.x == 0 && fullTiles < numTiles) {
-        WideFetch<T, Mode, VB, false>(r, fullTiles, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles, io);
-        WideOrder<T>(lds, r, shift, mask, bits);
-        WideWrite<T, Mode, VB, false>(lds, fullTiles, n, shift, mask, keysOut, pairsOut, io);
+        fetch(r, fullTiles, std::false_type{});
+        order(r, fullTiles, std::false_type{});
+        write(fullTiles, std::false_type{});
+    }
+}
+
+// One pass; the payload modes are those of RadixScatterKernel (pairs only), VB the bytes of a value in the arrays
+// that the first pass reads and the last one writes (a template parameter: a branch on it among the loads would
+// leave the compiler unable to count what is in flight).  prefix is the scanned table of WideCountKernel:
+// prefix[digit * numTiles + tile] is the first output position of the tile's entries of that digit.
+template <int T, int Mode, int VB>
+__global__ __launch_bounds__(T) void WideScatterKernel(
+    const int32_t *__restrict__ keysIn, const RadixPair *__restrict__ pairsIn, int32_t *__restrict__ keysOut,
+    RadixPair *__restrict__ pairsOut, int64_t n, int32_t keyBase, int32_t shift, int32_t mask, int32_t bits,
+    const int32_t *__restrict__ prefix, int64_t numTiles, RadixPairIo io)
+{
+    __shared__ WideLds<T> lds;
+    WideTurns<T, WideTileRegs<T>>(
+        n, numTiles,
+        [&](WideTileRegs<T> &r, int64_t tile, auto full) {
+            WideFetch<T, Mode, VB, decltype(full)::value>(r, tile, keysIn, pairsIn, n, keyBase, shift, mask, prefix, numTiles,
+                                                          io);
+        },
+        [&](const WideTileRegs<T> &r, int64_t, auto) { WideOrder<T>(lds, r, shift, mask, bits); },
+        [&](int64_t tile, auto full) {
+            WideWrite<T, Mode, VB, decltype(full)::value>(lds, tile, n, shift, mask, keysOut, pairsOut, io);
+        });
+}
+
+// ------------------------------- passes in front of buckets that are ordered in LDS
+// Where the last bits of a key are ordered bucket by bucket (below), a pass need not carry the bits that the passes before have
+// ordered by: an entry's bucket is where it stands.  What travels is a record of 8 bytes, the low bits of the key above the
+// payload in one word and the value in the other, and between two passes a byte beside it, the second pass's digit, which is
+// also all that its count has to read.  Bound by memory: 12 bytes an entry in and 9 out, 9 and 8, where key, row and value were
+// 12 in and 12 out in either pass; a tile's run in a bucket is a piece of one array instead of three.
+struct PackIo {
+    const int32_t *keys;  // first pass: keyBase + key, payload and value of every entry
+    int32_t keyBase;
+    const int32_t *pays;
+    const void *vals;
+    const uint8_t *digitsIn;  // second pass
+    const Record *recsIn;
+    uint8_t *digitsOut;  // first pass of two
+    Record *recsOut;
+    int64_t n;
+    int32_t low, payBits;  // bits of a key below its bucket; of a payload (together 32 at most)
+    int32_t nextShift;     // first pass of two: the second one's digit is what is above this bit of a key
+};
+
+enum PackMode { kPackOnly = 0, kPackFirst = 1, kPackSecond = 2 };
+
+template <int T, int Mode>
+struct PackRegs {
+    uint32_t key[kWideItems], pay[kWideItems], val[kWideItems];
+    int32_t first[WideShape<T>::kPer];
+};
+template <int T>
+struct PackRegs<T, kPackSecond> {
+    uint64_t rec[kWideItems];
+    uint32_t digit[kWideItems];
+    int32_t first[WideShape<T>::kPer];
+};
+
+// Low bits of a key above its payload, and the value.
+__device__ __forceinline__ uint64_t PackedRecord(uint32_t word, uint32_t val)
+{
+    return (static_cast<uint64_t>(val) << 32) | word;
+}
+
+template <int T>
+struct PackLds {
+    union {
+        int32_t counters[WideShape<T>::kWaves << kWideMaxBits];
+        struct {
+            uint64_t rec[WideShape<T>::kTile];
+            uint16_t digit[WideShape<T>::kTile];  // kPackFirst: the next pass's above the lower eight bits
+        };
+    };
+    int32_t outOf[1 << kWideMaxBits];
+    int32_t waveSums[WideShape<T>::kWaves];
+};
+
+// prefix, shift, mask, bits: as WideScatterKernel; the first digit of two has eight bits at most.
+template <int T, int Mode, int VB>
+__global__ __launch_bounds__(T, 4) void PackScatterKernel(PackIo io, int32_t shift, int32_t mask, int32_t bits,
+                                                          const int32_t *__restrict__ prefix, int64_t numTiles)
+{
+    __shared__ PackLds<T> lds;
+    constexpr int kTile = WideShape<T>::kTile, kPer = WideShape<T>::kPer;
+    const uint32_t lowMask = (1u << io.low) - 1u;
+    auto fetch = [&](PackRegs<T, Mode> &r, int64_t tile, auto full) {
+        const int tid = MadeAnew(threadIdx.x);
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const int32_t d = tid * kPer + j;
+            r.first[j] = prefix[static_cast<int64_t>(d <= mask ? d : mask) * numTiles + tile];
+        }
+        const int64_t wave0 = tile * kTile + tid / kWave * (kWave * kWideItems) + tid % kWave;
+#pragma unroll
+        for (int i = 0; i < kWideItems; ++i) {
+            // (a slot past the end reads the last entry)
+            const int64_t at = decltype(full)::value || wave0 + i * kWave < io.n ? wave0 + i * kWave : io.n - 1;
+            if constexpr (Mode == kPackSecond) {
+                r.rec[i] = __builtin_nontemporal_load(io.recsIn + at);
+                r.digit[i] = LoadStream(io.digitsIn + at);
+            } else {
+                r.key[i] = static_cast<uint32_t>(LoadStream(io.keys + at));
+                r.pay[i] = static_cast<uint32_t>(LoadStream(io.pays + at));
+                r.val[i] = 0;
+                if constexpr (VB == 4) {
+                    r.val[i] = LoadStream(static_cast<const uint32_t *>(io.vals) + at);
+                } else if constexpr (VB == 2) {
+                    r.val[i] = static_cast<const uint16_t *>(io.vals)[at];
+                } else if constexpr (VB == 1) {
+                    r.val[i] = static_cast<const uint8_t *>(io.vals)[at];
+                }
+            }
+        }
+    };
+    auto order = [&](const PackRegs<T, Mode> &r, int64_t tile, auto full) {
+        const int tid = MadeAnew(threadIdx.x);
+        uint32_t dig[kWideItems], rank[kWideItems];
+        const int64_t wave0 = tile * kTile + tid / kWave * (kWave * kWideItems) + tid % kWave;
+#pragma unroll
+        for (int i = 0; i < kWideItems; ++i) {
+            if constexpr (Mode == kPackSecond) {
+                dig[i] = r.digit[i] & static_cast<uint32_t>(mask);
+            } else {
+                dig[i] = WideDigit(Rebased(static_cast<int32_t>(r.key[i]), io.keyBase), shift, mask);
+            }
+            // a slot past the end gets the largest digit, so that it sorts behind every real entry
+            dig[i] = decltype(full)::value || wave0 + i * kWave < io.n ? dig[i] : static_cast<uint32_t>(mask);
+        }
+        WideRank<T>(lds, dig, r.first, mask, bits, rank);
+#pragma unroll
+        for (int i = 0; i < kWideItems; ++i) {
+            if constexpr (Mode == kPackSecond) {
+                lds.rec[rank[i]] = r.rec[i];
+                lds.digit[rank[i]] = static_cast<uint16_t>(dig[i]);
+            } else {
+                const uint32_t key = static_cast<uint32_t>(Rebased(static_cast<int32_t>(r.key[i]), io.keyBase));
+                lds.rec[rank[i]] = PackedRecord(((key & lowMask) << io.payBits) | r.pay[i], r.val[i]);
+                lds.digit[rank[i]] = static_cast<uint16_t>(Mode == kPackFirst ? dig[i] | (key >> io.nextShift << 8) : dig[i]);
+            }
+        }
+        LdsBarrier();
+    };
+    auto write = [&](int64_t tile, auto full) {
+        const int tid = MadeAnew(threadIdx.x);
+        const int32_t valid = decltype(full)::value ? kTile : static_cast<int32_t>(io.n - tile * kTile);
+#pragma unroll
+        for (int i = 0; i < kWideItems; ++i) {
+            const int32_t p = i * T + tid;
+            if (decltype(full)::value || p < valid) {  // the real entries are the first `valid` slots of the ordered tile
+                const uint32_t digit = lds.digit[p];
+                const int64_t dst = static_cast<int64_t>(lds.outOf[Mode == kPackFirst ? digit & 0xffu : digit] + p);
+                io.recsOut[dst] = lds.rec[p];
+                if constexpr (Mode == kPackFirst) {
+                    io.digitsOut[dst] = static_cast<uint8_t>(digit >> 8);
+                }
+            }
+        }
+    };
+    WideTurns<T, PackRegs<T, Mode>>(io.n, numTiles, fetch, order, write);
+}
+
+// WideCountKernel's table from the digits that the first pass left: a thread takes eight of a tile's together.
+template <int T>
+__global__ __launch_bounds__(T) void DigitCountKernel(const uint8_t *__restrict__ digits, int64_t n, int32_t mask,
+                                                      int32_t *__restrict__ table, int64_t numTiles)
+{
+    constexpr int kTile = WideShape<T>::kTile;
+    static_assert(kWideItems == 8, "eight digits a load");
+    __shared__ int32_t hist[kWideCountTiles << 8];
+    const int32_t count = mask + 1;
+    for (int32_t i = threadIdx.x; i < kWideCountTiles * count; i += T) {
+        hist[i] = 0;
+    }
+    const int64_t firstTile = static_cast<int64_t>(XcdContiguousTile(blockIdx.x, gridDim.x)) * kWideCountTiles;
+    Uint2U eight[kWideCountTiles];
+#pragma unroll
+    for (int j = 0; j < kWideCountTiles; ++j) {
+        const int64_t at = (firstTile + j) * kTile + 8 * threadIdx.x;
+        eight[j] = *reinterpret_cast<const Uint2U *>(digits + (at < n ? at : 0));  // (the array's room ends on such a piece)
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kWideCountTiles; ++j) {
+        const int64_t at = (firstTile + j) * kTile + 8 * threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t d = ((i < 4 ? eight[j].x : eight[j].y) >> (8 * (i % 4))) & static_cast<uint32_t>(mask);
+            atomicAdd(&hist[j * count + d], at + i < n ? 1 : 0);
+        }
+    }
+    __syncthreads();
+    for (int32_t i = threadIdx.x; i < kWideCountTiles * count; i += T) {
+        const int64_t tile = firstTile + i % kWideCountTiles;
+        if (tile < numTiles) {
+            const int32_t d = i / kWideCountTiles;
+            table[1 + static_cast<int64_t>(d) * numTiles + tile] = hist[i % kWideCountTiles * count + d];
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        table[0] = 0;
     }
 }
 
@@ -1089,8 +1297,8 @@ __device__ __forceinline__ void SortRowInGroup(int64_t begin, int64_t len, int32
 // keys, and a bucket of a few thousand entries is ordered in LDS by one workgroup.  It leaves as one piece, whole lines,
 // where a pass writes a run of tens of entries for each of its buckets; the starts of its keys are the offsets that
 // another two passes over the sorted keys found by counting, and the sorted keys themselves need not be written where
-// nobody asks for them.  Bound by memory: 12 bytes an entry in, 8 (csr2csc) or 12 (coosort) out, three or two workgroups a
-// compute unit, one of which loads while another orders.
+// nobody asks for them.  Bound by memory: 8 bytes an entry in, 8 (csr2csc) or 12 (coosort) out, three or two workgroups a
+// compute unit, one of which loads while another orders; coosort's by its vector instructions, which sort the rows.
 //
 // Buckets that do not fit go on lists.  Of up to kFinishLarge entries: a workgroup twice as large orders them.  Beyond (hubs):
 // three kernels count, scan and scatter pieces of kFinishMost entries as a pass does its tiles.  With nothing on the lists
@@ -1127,8 +1335,8 @@ struct FinishList {
 constexpr int kFinishLengths = 32;  // ints from `large` on that are zero at the start: the lists' lengths, csrsort's counters
 
 struct FinishIo {
-    const int32_t *keys;   // zero-based, in the order of their upper bits
-    const RadixPair *pairs;
+    const Record *recs;  // in the order of the keys' upper bits: low bits of the key above the payload, and the value
+    int32_t payBits;
     int64_t n;
     const int32_t *starts;  // bucket b begins at starts[b * startStride]; there is one more than buckets
     int64_t startStride;
@@ -1208,6 +1416,12 @@ __device__ __forceinline__ void FinishRows(const Lds &lds, const FinishIo &io, i
     }
 }
 
+// The low bits of the key that a record holds.
+__device__ __forceinline__ int32_t FinishDigit(uint64_t rec, int32_t payBits, int32_t mask)
+{
+    return static_cast<int32_t>(static_cast<uint32_t>(rec) >> payBits) & mask;
+}
+
 // Orders the `len` entries at `first` by the low bits of their keys and writes them: a whole bucket (Big = false) where it
 // stands, a piece of one where the scanned table says.
 template <int T, bool Keys, int VB, bool Big, bool Digits, int Lanes>
@@ -1220,19 +1434,14 @@ __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, co
     // have the largest digit and so come behind every entry
     const int32_t rounds = (len + T - 1) / T;
     const int32_t at0 = wave * rounds * kWave + lane;
-    int32_t key[kFinishItems];
-    RadixPair pay[kFinishItems];
+    // (no branch around a load: a slot past the end reads the last entry)
+    uint64_t rec[kFinishItems];
+    const int32_t lastSlot = len > 0 ? len - 1 : 0;
 #pragma unroll
     for (int i = 0; i < kFinishItems; ++i) {
         const int32_t slot = at0 + i * kWave;
-        const int64_t at = static_cast<int64_t>(first) + (slot < len ? slot : len - 1);
-        key[i] = 0;
-        pay[i] = RadixPair{0, 0u};
-        if (i < rounds) {
-            key[i] = LoadStream(io.keys + at);
-            // (zeros travel as values where there are none: without this load the compiler spills)
-            pay[i] = RadixPair{LoadStream(WideRows(io.pairs) + at), LoadStream(WideVals(io.pairs, io.n) + at)};
-        }
+        const int64_t at = static_cast<int64_t>(first) + (slot < lastSlot ? slot : lastSlot);
+        rec[i] = __builtin_nontemporal_load(io.recs + (at < io.n ? at : io.n - 1));
     }
     int32_t *mine = lds.counters + wave * digits;
     for (int32_t d = lane; d < digits; d += kWave) {
@@ -1246,11 +1455,12 @@ __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, co
 #pragma unroll
     for (int i = 0; i < kFinishItems; ++i) {
         rank[i] = 0;
-        key[i] = at0 + i * kWave < len ? key[i] & mask : mask;
+        rec[i] = at0 + i * kWave < len ? rec[i] : ~uint64_t{0};
         if (i < rounds) {
+            const int32_t key = FinishDigit(rec[i], io.payBits, mask);
             uint64_t peers = ~uint64_t{0};
             for (int32_t b = 0; b < io.low; ++b) {
-                const uint32_t ones = static_cast<uint32_t>(__builtin_amdgcn_sbfe(key[i], b, 1));
+                const uint32_t ones = static_cast<uint32_t>(__builtin_amdgcn_sbfe(key, b, 1));
                 const uint64_t m = __ballot(ones != 0);
                 // peers & ~(m ^ ones)
                 const uint32_t lo = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(peers), static_cast<uint32_t>(m), ones, 0x90);
@@ -1259,12 +1469,12 @@ __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, co
             }
             const uint32_t below = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(peers >> 32),
                                                              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(peers), 0));
-            const uint32_t before = static_cast<uint32_t>(mine[key[i]]);
+            const uint32_t before = static_cast<uint32_t>(mine[key]);
             rank[i] = before + below;
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
             __builtin_amdgcn_wave_barrier();
             if (below == 0) {
-                mine[key[i]] = static_cast<int32_t>(before + __popcll(peers));
+                mine[key] = static_cast<int32_t>(before + __popcll(peers));
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
             __builtin_amdgcn_wave_barrier();
@@ -1325,17 +1535,17 @@ __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, co
 #pragma unroll
     for (int i = 0; i < kFinishItems; ++i) {
         if (i < rounds) {
-            rank[i] += static_cast<uint32_t>(mine[key[i]]);
+            rank[i] += static_cast<uint32_t>(mine[FinishDigit(rec[i], io.payBits, mask)]);
         }
     }
     LdsBarrier();  // the counters make room for the entries
 #pragma unroll
     for (int i = 0; i < kFinishItems; ++i) {
         if (i < rounds) {
-            lds.row[rank[i]] = pay[i].row;
-            lds.val[rank[i]] = pay[i].val;
+            lds.row[rank[i]] = static_cast<int32_t>(static_cast<uint32_t>(rec[i]) & ((1u << io.payBits) - 1u));
+            lds.val[rank[i]] = static_cast<uint32_t>(rec[i] >> 32);
             if constexpr ((Keys && Lanes == 0) || Big) {
-                lds.digit[rank[i]] = static_cast<uint16_t>(key[i]);
+                lds.digit[rank[i]] = static_cast<uint16_t>(FinishDigit(rec[i], io.payBits, mask));
             }
         }
     }
@@ -1432,17 +1642,17 @@ __global__ __launch_bounds__(kFinishThreads) void FinishCountKernel(FinishIo io)
         int32_t len;
         const int32_t first = FinishPieceAt(io, piece, &bucket, &len);
         // all loads ahead of the LDS atomics; an entry past the end reads the last one and counts for nothing
-        int32_t key[kFinishItems];
+        uint64_t rec[kFinishItems];
 #pragma unroll
         for (int i = 0; i < kFinishItems; ++i) {
             const int32_t at = i * kFinishThreads + threadIdx.x;
-            key[i] = io.keys[static_cast<int64_t>(first) + (at < len ? at : len - 1)];
+            rec[i] = io.recs[static_cast<int64_t>(first) + (at < len ? at : len - 1)];
         }
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < kFinishItems; ++i) {
             const int32_t at = i * kFinishThreads + threadIdx.x;
-            atomicAdd(&hist[key[i] & (digits - 1)], at < len ? 1 : 0);
+            atomicAdd(&hist[FinishDigit(rec[i], io.payBits, digits - 1)], at < len ? 1 : 0);
         }
         __syncthreads();
         for (int32_t d = threadIdx.x; d < digits; d += kFinishThreads) {
@@ -1546,9 +1756,9 @@ __global__ __launch_bounds__(kFinishLargeThreads) void FinishListsKernel(FinishI
 // Where the buckets of two passes begin, without a look at every key: between the passes the entries with lower digit dl are
 // one stretch, and of those with upper digit dh the second pass puts as many in front of (dh, dl) as its table has for the
 // tiles in front of the stretch, and as lie in the stretch's first tile in front of it.  A workgroup a lower digit.
-// `keys`: what the second pass read; starts[buckets] = n and the lists' lengths = 0 come from here, too.
-__global__ __launch_bounds__(kFinishScanThreads) void FinishStartsKernel(const int32_t *__restrict__ keys, int64_t n,
-                                                                    int64_t tile, int64_t numTiles, int32_t low,
+// `upper`: the digits that the second pass read; starts[buckets] = n and the lists' lengths = 0 come from here, too.
+__global__ __launch_bounds__(kFinishScanThreads) void FinishStartsKernel(const uint8_t *__restrict__ upper, int64_t n,
+                                                                    int64_t tile, int64_t numTiles,
                                                                     int32_t lowerBits, int32_t upperBits,
                                                                     const int32_t *__restrict__ lowerPrefix,
                                                                     const int32_t *__restrict__ upperPrefix,
@@ -1564,16 +1774,16 @@ __global__ __launch_bounds__(kFinishScanThreads) void FinishStartsKernel(const i
     const int64_t t = stretch / tile;
     // (all loads of a turn ahead of the LDS atomics)
     for (int64_t i0 = t * tile; i0 < stretch; i0 += kWideItems * kFinishScanThreads) {
-        int32_t key[kWideItems];
+        uint32_t digit[kWideItems];
 #pragma unroll
         for (int j = 0; j < kWideItems; ++j) {
             const int64_t i = i0 + j * kFinishScanThreads + threadIdx.x;
-            key[j] = keys[i < stretch ? i : stretch - 1];
+            digit[j] = upper[i < stretch ? i : stretch - 1];
         }
 #pragma unroll
         for (int j = 0; j < kWideItems; ++j) {
             const int64_t i = i0 + j * kFinishScanThreads + threadIdx.x;
-            atomicAdd(&hist[WideDigit(key[j], low + lowerBits, digits - 1)], i < stretch ? 1 : 0);
+            atomicAdd(&hist[digit[j] & static_cast<uint32_t>(digits - 1)], i < stretch ? 1 : 0);
         }
     }
     __syncthreads();
@@ -2024,6 +2234,18 @@ int64_t WideTiles(int64_t n)
 }
 int64_t WideTableInts(int64_t n) { return (WideTiles(n) << kWideMaxBits) + 1; }
 
+// ... of the passes that leave records.  Half as many as the other passes of many entries have: two workgroups a compute unit,
+// one of which loads while the other orders, and runs that are as long, in bytes, as theirs of three arrays (17 M triples over 1 M
+// rows 865 us with 1024, 777 with 512; 33.5 M 2032 and 2029; 3.3 M over 300 000 with 256 707, with 512 626).  A table of theirs has
+// at most as many ints as one of ten bits of the others': twice the tiles, but nine bits in one pass of so many entries, and eight
+// in each of two.
+int PackThreads(int64_t n) { return n >= (int64_t{1} << 20) ? 512 : 256; }
+int64_t PackTiles(int64_t n)
+{
+    const int64_t tile = static_cast<int64_t>(PackThreads(n)) * kWideItems;
+    return (n + tile - 1) / tile;
+}
+
 // Passes of a sort of n entries over `keyBits` bits of key, and the bits each takes.  At least two: a first pass that
 // reads the sources and a last one that writes the outputs.  The passes share the key's bits evenly: the fewer buckets
 // a pass has, the longer the runs its tiles write.  (Nine bits at most where the workgroups are large: 20 bits of 33.5 M
@@ -2141,23 +2363,28 @@ int32_t KeyBits(int64_t n)
 }
 
 // How a stable sort by keys in [0, numKeys) ends in LDS: `high` upper bits in one or two passes, `low` bits at the end.
-// Taken where that saves a pass.  kFinishMean leaves a fifth of the room for buckets fuller than the average (with three
+// Taken where that saves a pass, and where it saves none from 5 M entries on: the passes in front of buckets move less (triples,
+// the same number of passes, plain / with buckets: 4 M over 100 000 rows 433 / 451 us, 6 M over 300 000 630 / 601, 6 M over 600 000
+// 642 / 596, 9.6 M over 200 000 795 / 714).  kFinishMean leaves a fifth of the room for buckets fuller than the average (with three
 // fifths, and one more bit in the passes: 33.5 M entries 683 us, 651 so); below kFinishLeast the workgroups' start and end
 // outweigh their work.
 struct FinishPlan {
     bool use;
-    int32_t passes, low, lowerBits, upperBits;
+    int32_t passes, low, lowerBits, upperBits, payBits;
     int64_t buckets;
 };
 constexpr int64_t kFinishMean = kFinishMost * 4 / 5;
 constexpr int64_t kFinishLeast = 512;
+constexpr int64_t kFinishSamePasses = 5 << 20;
 constexpr int64_t kFinishMin = 1 << 14;  // entries (the lists' room in the second pair buffer is counted from here)
 
-FinishPlan FinishPlanOf(int64_t numKeys, int64_t n)
+FinishPlan FinishPlanOf(int64_t numKeys, int64_t n, int32_t payBits)
 {
     FinishPlan f{};
     const int32_t keyBits = KeyBits(numKeys);
     int32_t low = keyBits - 1 < kFinishMaxBits ? keyBits - 1 : kFinishMaxBits;
+    low = low < 32 - payBits ? low : 32 - payBits;  // (the two share a word)
+    f.payBits = payBits;
     auto mean = [&](int32_t bits) {  // entries of a bucket
         return static_cast<double>(n) * static_cast<double>(int64_t{1} << bits) / static_cast<double>(numKeys);
     };
@@ -2173,7 +2400,8 @@ FinishPlan FinishPlanOf(int64_t numKeys, int64_t n)
     f.lowerBits = f.passes == 1 ? high : (high + 1) / 2;
     f.upperBits = high - f.lowerBits;
     f.buckets = int64_t{1} << high;
-    f.use = f.passes < WidePassesOf(keyBits, n).passes;
+    const int32_t plain = WidePassesOf(keyBits, n).passes;
+    f.use = f.passes < plain || (f.passes == plain && n >= kFinishSamePasses);
     return f;
 }
 
@@ -2207,6 +2435,43 @@ void LaunchSortListedRows(const int32_t *rowPtr, int32_t base, int64_t n, int32_
                        static_cast<int32_t *>(nullptr));
 }
 
+template <int T, int Mode>
+void LaunchPackPassOf(const PackIo &io, int32_t valueBytes, int32_t shift, int32_t bits, int32_t *table, int32_t *scratch,
+                      hipStream_t s)
+{
+    const int32_t mask = (1 << bits) - 1;
+    const int64_t numTiles = PackTiles(io.n);
+    const auto counts = dim3(static_cast<uint32_t>((numTiles + kWideCountTiles - 1) / kWideCountTiles));
+    if (Mode == kPackSecond) {
+        hipLaunchKernelGGL(DigitCountKernel<T>, counts, dim3(T), 0, s, io.digitsIn, io.n, mask, table, numTiles);
+    } else {
+        hipLaunchKernelGGL(WideCountKernel<T>, counts, dim3(T), 0, s, io.keys, io.n, io.keyBase, shift, mask, table, numTiles);
+    }
+    LaunchInclusiveScan(table, table, (numTiles << bits) + 1, 0, scratch, s);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(WideScatterBlocks(io.n, T)), dim3(T), 0, s, io, shift, mask, bits, table, numTiles);
+    };
+    if constexpr (Mode == kPackSecond) {
+        launch(PackScatterKernel<T, Mode, 4>);
+    } else {
+        switch (valueBytes) {
+            case 4: launch(PackScatterKernel<T, Mode, 4>); break;
+            case 2: launch(PackScatterKernel<T, Mode, 2>); break;
+            case 1: launch(PackScatterKernel<T, Mode, 1>); break;
+            default: launch(PackScatterKernel<T, Mode, 0>); break;
+        }
+    }
+}
+
+// One pass of a sort that ends in LDS; table: WideTableInts(n) ints.
+template <int Mode>
+void LaunchPackPass(const PackIo &io, int32_t valueBytes, int32_t shift, int32_t bits, int32_t *table, int32_t *scratch,
+                    hipStream_t s)
+{
+    const auto launch = PackThreads(io.n) == 512 ? LaunchPackPassOf<512, Mode> : LaunchPackPassOf<256, Mode>;
+    launch(io, valueBytes, shift, bits, table, scratch, s);
+}
+
 struct FinishSort {
     const int32_t *keysIn;  // keyBase + key
     int32_t keyBase;
@@ -2218,12 +2483,12 @@ struct FinishSort {
     int64_t n, numKeys;
 };
 
-// keys[], pairs[]: n keys and n pairs each; table: WideTableInts(n).  The entries pass through the first of the buffers and
+// keys[], pairs[]: 4 n and 8 n bytes each; table: WideTableInts(n).  The entries pass through the first of the buffers and
 // lie in the second when the last kernels start, whose lists then use the first pair buffer; `ptr` may be keys[0].
 void LaunchFinishSort(const FinishSort &sort, const FinishPlan &plan, int32_t *const *keys, void *const *pairs,
                       int32_t *table, int32_t *scratch, hipStream_t s)
 {
-    const int64_t n = sort.n, numTiles = WideTiles(n), most = n / kFinishMost + 1;  // (buckets on a list: fewer)
+    const int64_t n = sort.n, numTiles = PackTiles(n), most = n / kFinishMost + 1;  // (buckets on a list: fewer)
     FinishIo io{};
     auto *at = static_cast<int32_t *>(pairs[0]);
     auto take = [&](int64_t ints) {
@@ -2248,27 +2513,41 @@ void LaunchFinishSort(const FinishSort &sort, const FinishPlan &plan, int32_t *c
         io.midList = take(n / 2);
         io.longList = take(n / kSortWaveRow);
     }
+    PackIo pack{};
+    pack.keys = sort.keysIn;
+    pack.keyBase = sort.keyBase;
+    pack.pays = sort.io.rowSrc;
+    pack.vals = sort.io.valSrc;
+    pack.n = n;
+    pack.low = plan.low;
+    pack.payBits = plan.payBits;
+    pack.nextShift = plan.low + plan.lowerBits;
+    auto *last = static_cast<Record *>(pairs[1]);
     if (plan.passes == 1) {
-        LaunchWidePairPass(kPayPairFirst, sort.keysIn, nullptr, keys[1], pairs[1], n, sort.keyBase, plan.low,
-                           plan.lowerBits, table, scratch, sort.io, s);
+        pack.recsOut = last;
+        LaunchPackPass<kPackOnly>(pack, sort.io.valueBytes, plan.low, plan.lowerBits, table, scratch, s);
         LaunchFill(io.list.large, kFinishLengths, 0, s);
         io.starts = table;
         io.startStride = numTiles;
     } else {
         // (up to eight bits each: the tables of both passes fit where one of ten bits does)
         int32_t *upper = table + (numTiles << plan.lowerBits) + 1;
-        LaunchWidePairPass(kPayPairFirst, sort.keysIn, nullptr, keys[0], pairs[0], n, sort.keyBase, plan.low,
-                           plan.lowerBits, table, scratch, sort.io, s);
-        LaunchWidePairPass(kPayPair, keys[0], pairs[0], keys[1], pairs[1], n, 0, plan.low + plan.lowerBits,
-                           plan.upperBits, upper, scratch, sort.io, s);
-        hipLaunchKernelGGL(FinishStartsKernel, dim3(1u << plan.lowerBits), dim3(kFinishScanThreads), 0, s, keys[0], n,
-                           static_cast<int64_t>(WideThreads(n)) * kWideItems, numTiles, plan.low, plan.lowerBits,
-                           plan.upperBits, table, upper, starts, io.list);
+        auto *digits = reinterpret_cast<uint8_t *>(keys[0]);
+        pack.recsOut = static_cast<Record *>(pairs[0]);
+        pack.digitsOut = digits;
+        LaunchPackPass<kPackFirst>(pack, sort.io.valueBytes, plan.low, plan.lowerBits, table, scratch, s);
+        pack.recsIn = pack.recsOut;
+        pack.digitsIn = digits;
+        pack.recsOut = last;
+        LaunchPackPass<kPackSecond>(pack, 4, 0, plan.upperBits, upper, scratch, s);
+        hipLaunchKernelGGL(FinishStartsKernel, dim3(1u << plan.lowerBits), dim3(kFinishScanThreads), 0, s, digits, n,
+                           static_cast<int64_t>(PackThreads(n)) * kWideItems, numTiles, plan.lowerBits, plan.upperBits, table,
+                           upper, starts, io.list);
         io.starts = starts;
         io.startStride = 1;
     }
-    io.keys = keys[1];
-    io.pairs = static_cast<const RadixPair *>(pairs[1]);
+    io.recs = last;
+    io.payBits = plan.payBits;
     io.n = n;
     io.low = plan.low;
     io.numKeys = sort.numKeys;
@@ -2558,7 +2837,7 @@ int opsparse_csr2csc_launch(int64_t m, int64_t n, int64_t nnz, const void *csrVa
     // Up to ten bits a pass (WidePassesOf), the tile ordered through LDS before it leaves, and the last bits in LDS where
     // that saves a pass (33.5 M entries over 2^20 columns: three passes of seven bits 0.80 ms, two and the last bits 0.65).
     const RadixPairIo io{rowOfPos, csrVal, cscRowInd, cscVal, valueBytes};
-    const FinishPlan plan = FinishPlanOf(n, nnz);
+    const FinishPlan plan = FinishPlanOf(n, nnz, KeyBits(m + indexBase));
     if (plan.use) {
         const FinishSort sort{csrColInd, indexBase, io, nullptr, 0, cscColPtr, indexBase, nnz, n};
         LaunchFinishSort(sort, plan, keys, pairs, table, tiles, s);
@@ -2853,7 +3132,7 @@ int opsparse_coosort_launch(int64_t nnz, int32_t byRow, int32_t *cooRows, int32_
         // the entries instead of one a digit.
         int32_t *rowPtr = keys[0];  // (the passes' buffers are free when it is written)
         const int64_t bound = static_cast<int64_t>(r[3]) + 1;
-        const FinishPlan plan = FinishPlanOf(span, nnz);
+        const FinishPlan plan = FinishPlanOf(span, nnz, KeyBits(bound));
         const bool rowsToo = plan.use && SortPacked(bound, 0, kWave);
         if (plan.use) {
             const FinishSort sort{primary, r[0], RadixPairIo{secondary, perm, secondary, perm, 4}, primary,

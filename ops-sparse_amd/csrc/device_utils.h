@@ -149,6 +149,13 @@ __device__ __forceinline__ T GroupSumDyn(T v, int g)
     return v;
 }
 
+// A value made anew wherever this stands: what follows from it is not kept in registers over a loop.
+__device__ __forceinline__ int MadeAnew(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // A workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every global load and store
 // the wavefront has in flight; this one leaves them outstanding (a tile's loads issued ahead of their use).
 __device__ __forceinline__ void LdsBarrier()

@@ -1586,13 +1586,6 @@ __device__ __forceinline__ void QuadTranspose(Uint4 &p0, Uint4 &p1, Uint4 &p2, U
     QuadExchange<kDppQuadSwap2>(p1, p3, upper);
 }
 
-// A value made anew wherever this stands: what follows from it is not kept in registers over a loop.
-__device__ __forceinline__ int MadeAnew(int v)
-{
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
 // Four entries loaded `ahead` places in front of where they belong, put there (ahead <= 0: they are; what is moved in from
 // behind the array's last entry is zero).
 __device__ __forceinline__ Uint4 ShiftedFour(Uint4 v, int32_t ahead)

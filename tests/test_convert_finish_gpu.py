@@ -85,3 +85,23 @@ def test_coosort_buckets(osa, gpu_ctx, nnz, m, dense, hub, wide, by_row):
             at = at[:-count]
     rows, cols = (primary - 3, secondary) if by_row else (secondary, primary - 3)
     run_coosort(osa, gpu_ctx, 1 << 30, 1 << 30, rows, cols, by_row, perm=rng.permutation(nnz).astype(np.int32))
+
+
+@pytest.mark.parametrize("m,n,nnz,base", [
+    ((1 << 22) - 1, 262_143, 400_001, 1),    # the payload takes 22 bits, the low bits of a key ten
+    ((1 << 22) - 1, (1 << 20) - 77, 5_300_003, 0), (1 << 22, (1 << 20) - 77, 5_300_003, 1),  # 22 and 23 bits; one pass fewer or none
+    (1 << 24, 300_000, 5_242_880, 1), (3, 300_000, 5_242_879, 0)])
+def test_csr2csc_rows_of_many_bits(osa, gpu_ctx, m, n, nnz, base):
+    rng = np.random.default_rng(m + n)
+    rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, m - 1)), [nnz]]).astype(np.int32)
+    run_csr2csc(osa, gpu_ctx, m, n, rowptr + base, columns("uniform", n, nnz, rng) + base,
+                rng.uniform(-1, 1, nnz).astype(np.float32), np.float32, True, base)
+
+
+@pytest.mark.parametrize("span,cols,nnz", [(400_000, 1 << 22, 2_000_000), (700_000, (1 << 26) - 2, 5_300_000),
+                                           (500_000, 1 << 27, 9_000_000), (700_000, (1 << 31) - 2, 5_300_000)])
+def test_coosort_columns_of_many_bits(osa, gpu_ctx, span, cols, nnz):
+    rng = np.random.default_rng(span + nnz)
+    rows, c = rng.integers(0, span, nnz).astype(np.int32), rng.integers(0, cols, nnz).astype(np.int32)
+    c[:2] = [0, cols - 1]
+    run_coosort(osa, gpu_ctx, span, cols, rows, c, True, perm=rng.permutation(nnz).astype(np.int32))
