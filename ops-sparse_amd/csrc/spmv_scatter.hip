@@ -53,6 +53,7 @@ constexpr int32_t kMaxColumnEntries = 8192;
 
 typedef float Float4 __attribute__((ext_vector_type(4)));
 typedef uint32_t Uint4 __attribute__((ext_vector_type(4)));
+typedef uint32_t Uint4U __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte load at any dword
 typedef unsigned short Ushort4 __attribute__((ext_vector_type(4)));
 
 struct ScatterLayout {
@@ -297,32 +298,26 @@ __global__ __launch_bounds__(kBlockThreads) void EntryMetaKernel(const int32_t *
 
 // ---------------------------------------------------------------------------------------------- the two passes
 
+// Four consecutive values as they lie in memory, and one of them.
 template <typename ValT>
-__device__ __forceinline__ void LoadFour(const ValT *p, float out[4]);
+struct FourOf {
+    typedef Short4U Type;
+};
 template <>
-__device__ __forceinline__ void LoadFour<float>(const float *p, float out[4])
+struct FourOf<float> {
+    typedef Float4U Type;
+};
+__device__ __forceinline__ float OneOf(const Float4U &v, int j, float) { return v[j]; }
+__device__ __forceinline__ float OneOf(const Short4U &v, int j, Half)
 {
-    const Float4U v = __builtin_nontemporal_load(reinterpret_cast<const Float4U *>(p));
-    out[0] = v.x, out[1] = v.y, out[2] = v.z, out[3] = v.w;
+    const uint16_t bits = v[j];
+    Half h;
+    __builtin_memcpy(&h, &bits, 2);
+    return static_cast<float>(h);
 }
-template <>
-__device__ __forceinline__ void LoadFour<Half>(const Half *p, float out[4])
+__device__ __forceinline__ float OneOf(const Short4U &v, int j, Bf16)
 {
-    const Short4U v = __builtin_nontemporal_load(reinterpret_cast<const Short4U *>(p));
-    for (int j = 0; j < 4; ++j) {
-        const uint16_t bits = v[j];
-        Half h;
-        __builtin_memcpy(&h, &bits, 2);
-        out[j] = static_cast<float>(h);
-    }
-}
-template <>
-__device__ __forceinline__ void LoadFour<Bf16>(const Bf16 *p, float out[4])
-{
-    const Short4U v = __builtin_nontemporal_load(reinterpret_cast<const Short4U *>(p));
-    for (int j = 0; j < 4; ++j) {
-        out[j] = __uint_as_float(static_cast<uint32_t>(v[j]) << 16);
-    }
+    return __uint_as_float(static_cast<uint32_t>(v[j]) << 16);
 }
 
 template <typename ValT>
@@ -333,8 +328,13 @@ __device__ __forceinline__ float WidenOne(ValT v)
 
 // Pass 1: the products of a workgroup's pieces (a step apart, below) written to `inter` in panel order.  One
 // workgroup a compute unit (the staging area is most of its LDS), so nothing else would cover the time a piece's
-// loads are on their way: the workgroup asks for the next piece's values and slots before it writes the current one
-// out (one piece after the other: 309 us on the 8 M x 8 M power-law matrix).
+// loads are on their way: before it writes a piece out, the workgroup asks for what it needs of the next one, fp32
+// values also for the x of their rows, whose numbers it has asked for a piece earlier.  No load stands in a branch (the
+// compiler would wait for it there): the lanes past the end of a piece read its last four entries again, and put the same
+// products into the same places.
+//
+// Bound by memory, 16 bytes an entry (fp32).  39 M entries of a 5 M x 5 M power-law matrix: 153 us while the loads of the next
+// piece stood in a branch and x was gathered when a piece began, 130 now.
 template <typename ValT, typename ProdT>
 __global__ __launch_bounds__(kThreads) void ScatterProductsKernel(const ValT *__restrict__ vals, const ValT *__restrict__ x,
                                                                   const uint32_t *__restrict__ meta,
@@ -345,88 +345,150 @@ __global__ __launch_bounds__(kThreads) void ScatterProductsKernel(const ValT *__
 {
     constexpr int kPiece = kStageBytes / static_cast<int>(sizeof(ProdT));
     constexpr int kRounds = kPiece / (kThreads * 4);  // a thread takes 4 consecutive entries a round
+    constexpr bool kXAhead = sizeof(ProdT) == 8;      // (twice the entries of 16 bits would not fit the registers)
+    constexpr int kTables = (kMaxPanels + kThreads) / kThreads;  // panels' table entries a thread
+    typedef typename FourOf<ValT>::Type Four;
+    typedef Uint4 Metas[kRounds];
     __shared__ __align__(16) ProdT stage[kPiece];
     __shared__ int32_t base[kMaxPanels + 1];
-    __shared__ int32_t dst[kMaxPanels];
-    const int t = threadIdx.x;
-    constexpr int kChunkLanes = 16;
-    Uint4 m[kRounds];
-    float v[kRounds][4];
-    // values and slots of piece q into registers: every load is issued whatever the piece's length (those past its end
-    // re-read its first entries and are not used), so that none waits for another
-    auto fetch = [&](int32_t q) {
-        const int64_t first = static_cast<int64_t>(q) * kPiece;
-        const int32_t count = nnz - first < kPiece ? static_cast<int32_t>(nnz - first) : kPiece;
-#pragma unroll
-        for (int r = 0; r < kRounds; ++r) {
-            const int32_t k = (r * kThreads + t) * 4;
-            if (k + 4 <= count) {
-                m[r] = __builtin_nontemporal_load(reinterpret_cast<const Uint4 *>(meta + first + k));
-                LoadFour<ValT>(vals + first + k, v[r]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const bool in = k + j < count;
-                    m[r][j] = in ? meta[first + k + j] : 0u;
-                    v[r][j] = in ? WidenOne<ValT>(vals[first + k + j]) : 0.0f;
-                }
-            }
+    __shared__ int32_t dst[kMaxPanels + 1];
+    // a last piece of fewer than four entries: an entry a thread, without the staging area
+    const int32_t few = static_cast<int32_t>(nnz % kPiece) < 4 ? static_cast<int32_t>(nnz % kPiece) : 0;
+    if (blockIdx.x == 0 && static_cast<int32_t>(threadIdx.x) < few) {
+        const int32_t q = Q - 1;
+        const int64_t at = static_cast<int64_t>(q) * kPiece + threadIdx.x;
+        const int32_t slot = static_cast<int32_t>(meta[at] & 0xffffu);
+        const int32_t *bases = pieceBase + static_cast<int64_t>(q) * (P + 1);
+        int32_t p = 0;
+        while (p + 1 < P && bases[p + 1] <= slot) {
+            ++p;
         }
-    };
+        inter[chunkDst[static_cast<int64_t>(q) * P + p] + slot - bases[p]] =
+            static_cast<ProdT>(WidenOne<ValT>(vals[at])) * static_cast<ProdT>(WidenOne<ValT>(x[pieceRow[q] + (meta[at] >> 16)]));
+    }
+    const int32_t pieces = few > 0 ? Q - 1 : Q;
     // The workgroups of an XCD take neighbouring pieces in the same turn: their chunks of a panel follow one another in
     // memory, and the line between two chunks is completed in the L2 the workgroups share (5 M x 5 M power-law matrix,
     // 39 M entries: 158 -> 147 us).
     const uint32_t xcds = gridDim.x < kNumXcd ? gridDim.x : kNumXcd;
     const uint32_t xcd = blockIdx.x % xcds;
     const int32_t step = static_cast<int32_t>((gridDim.x - xcd + xcds - 1) / xcds);
-    const int32_t qEnd = static_cast<int32_t>(static_cast<int64_t>(Q) * (xcd + 1) / xcds);
-    int32_t q = static_cast<int32_t>(static_cast<int64_t>(Q) * xcd / xcds + blockIdx.x / xcds);
-    if (q < qEnd) {
-        fetch(q);
+    const int32_t qEnd = static_cast<int32_t>(static_cast<int64_t>(pieces) * (xcd + 1) / xcds);
+    int32_t q = static_cast<int32_t>(static_cast<int64_t>(pieces) * xcd / xcds + blockIdx.x / xcds);
+    if (q >= qEnd) {
+        return;
     }
-    for (; q < qEnd; q += step) {
-        const int64_t first = static_cast<int64_t>(q) * kPiece;
+    Metas mA, mB;  // of the piece at hand and (kXAhead) of the next
+    Four v[kRounds];
+    ValT xv[kRounds][4];
+    int32_t baseAhead[kTables], dstAhead[kTables];
+    // where the thread's entries of round r are, in the last piece its last four where there would be none; of a piece behind
+    // the workgroup's last (asked for, not used) everyone's are the same, one line for all
+    auto placeOf = [&](int32_t piece, int r) {
+        const int64_t first = static_cast<int64_t>(piece < qEnd ? piece : 0) * kPiece;
         const int32_t count = nnz - first < kPiece ? static_cast<int32_t>(nnz - first) : kPiece;
-        for (int32_t p = t; p <= P; p += kThreads) {
-            base[p] = pieceBase[static_cast<int64_t>(q) * (P + 1) + p];
-        }
-        for (int32_t p = t; p < P; p += kThreads) {
-            dst[p] = chunkDst[static_cast<int64_t>(q) * P + p];
-        }
-        const ValT *xRow = x + pieceRow[q];
-        float xv[kRounds][4];
+        const int32_t last = piece < qEnd ? count - 4 : 0;
+        const int32_t k = (r * kThreads + MadeAnew(threadIdx.x)) * 4;
+        return first + (k < last ? k : last);
+    };
+    auto askMetas = [&](int32_t piece, Metas &m) {
 #pragma unroll
         for (int r = 0; r < kRounds; ++r) {
-            const int32_t k = (r * kThreads + t) * 4;
+            m[r] = __builtin_nontemporal_load(reinterpret_cast<const Uint4U *>(meta + placeOf(piece, r)));
+        }
+    };
+    auto askValues = [&](int32_t piece) {
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            v[r] = __builtin_nontemporal_load(reinterpret_cast<const Four *>(vals + placeOf(piece, r)));
+        }
+#pragma unroll
+        for (int r = 0; r < kTables; ++r) {
+            const int32_t p = r * kThreads + MadeAnew(threadIdx.x);
+            const int64_t row = piece < qEnd ? piece : 0;
+            baseAhead[r] = pieceBase[row * (P + 1) + (p <= P ? p : P)];
+            dstAhead[r] = chunkDst[row * P + (p < P ? p : P - 1)];
+        }
+    };
+    auto askX = [&](int32_t piece, const Metas &m) {
+        const ValT *xRow = x + pieceRow[piece < qEnd ? piece : 0];
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                xv[r][j] = k + j < count ? WidenOne<ValT>(xRow[m[r][j] >> 16]) : 0.0f;
+                xv[r][j] = xRow[m[r][j] >> 16];
+            }
+        }
+    };
+    auto turn = [&](Metas &now, Metas &next) {
+        const int32_t q1 = q + step, q2 = q1 + step;
+        if constexpr (!kXAhead) {
+            askX(q, now);
+        }
+        const int t = MadeAnew(threadIdx.x);
+#pragma unroll
+        for (int r = 0; r < kTables; ++r) {
+            const int32_t p = r * kThreads + t;
+            if (p <= P) {
+                base[p] = baseAhead[r];
+                dst[p] = dstAhead[r];
             }
         }
 #pragma unroll
         for (int r = 0; r < kRounds; ++r) {
-            const int32_t k = (r * kThreads + t) * 4;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                if (k + j < count) {
-                    stage[m[r][j] & 0xffffu] = static_cast<ProdT>(v[r][j]) * static_cast<ProdT>(xv[r][j]);
-                }
+                stage[now[r][j] & 0xffffu] =
+                    static_cast<ProdT>(OneOf(v[r], j, ValT{})) * static_cast<ProdT>(WidenOne<ValT>(xv[r][j]));
             }
         }
-        __syncthreads();
-        if (q + step < qEnd) {
-            fetch(q + step);
+        LdsBarrier();
+        askValues(q1);
+        if constexpr (kXAhead) {
+            askX(q1, next);
+            askMetas(q2, now);
+        } else {
+            askMetas(q1, next);
         }
+        __builtin_amdgcn_sched_barrier(0);  // (asked for here, not where the scheduler finds room later)
         // kChunkLanes lanes a chunk: the piece's products of one panel, 32 or 64 on average, contiguous in the staging
-        // area and in memory (64 lanes a chunk: 166 us, 32 and 16: 155, on 39 M entries)
+        // area and in memory (64 lanes a chunk: 166 us, 32 and 16: 155, on 39 M entries); kAtOnce products of a lane together
+        constexpr int kChunkLanes = 16, kAtOnce = 4;
         for (int32_t p = t / kChunkLanes; p < P; p += kThreads / kChunkLanes) {
             const int32_t s0 = base[p], s1 = base[p + 1];
             ProdT *out = inter + dst[p];
-            for (int32_t k = s0 + t % kChunkLanes; k < s1; k += kChunkLanes) {
-                out[k - s0] = stage[k];
+            for (int32_t k = s0 + t % kChunkLanes; k < s1; k += kAtOnce * kChunkLanes) {
+                ProdT prod[kAtOnce];
+#pragma unroll
+                for (int u = 0; u < kAtOnce; ++u) {
+                    prod[u] = stage[k + u * kChunkLanes < s1 ? k + u * kChunkLanes : k];
+                }
+#pragma unroll
+                for (int u = 0; u < kAtOnce; ++u) {
+                    if (k + u * kChunkLanes < s1) {
+                        out[k + u * kChunkLanes - s0] = prod[u];
+                    }
+                }
             }
         }
-        __syncthreads();
+        LdsBarrier();
+        q += step;
+    };
+    askMetas(q, mA);
+    askValues(q);
+    if constexpr (kXAhead) {
+        askX(q, mA);
+        askMetas(q + step, mB);
+    }
+    while (true) {
+        turn(mA, mB);
+        if (q >= qEnd) {
+            break;
+        }
+        turn(mB, mA);
+        if (q >= qEnd) {
+            break;
+        }
     }
 }
 

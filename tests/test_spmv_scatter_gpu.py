@@ -246,3 +246,25 @@ def test_output_panels_of_every_round_count(osa, gpu_ctx, cols):
     scatter = L.opsparse_spmv_csr_scatter_workspace_bytes(rows, cols, colind.size, 0)
     assert 0 < scatter < buf.numel() and _untouched_from(buf, scatter)
     call(val, 1.5, -0.5)
+
+
+@pytest.mark.parametrize("tail", [0, 1, 2, 3, 4, 5, 16_381])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_last_piece_of_a_few_entries(osa, gpu_ctx, dtype, tail):
+    """A last piece of 1 - 3 entries has no four to load together; longer ones read their last four again.  As many pieces as
+    give some workgroups one and some two of them."""
+    dev, stream, handle = gpu_ctx
+    rows, cols = 270_001, 300_000
+    nnz = 200 * PIECE[dtype] + tail if dtype == torch.float32 else 130 * PIECE[dtype] + tail
+    rng = np.random.default_rng(tail + 1)
+    rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz - 1, rows - 1)), [nnz]]).astype(np.int32)
+    colind = rng.integers(0, cols, nnz).astype(np.int32)
+    val, x = _seen(rng.uniform(-1, 1, nnz), dtype), _seen(rng.uniform(-1, 1, rows), dtype)
+    y0 = rng.uniform(-1, 1, cols).astype(np.float32)
+    y = to_dev(y0, dev)
+    A = osa.Csr(rows, cols, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev, dtype))
+    op = osa.SpmvOp(handle, A, osa.DnVec(to_dev(x, dev, dtype)), osa.DnVec(y), op=osa.ACL_SPARSE_OP_TRANSPOSE)
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, nnz)
+    op(1.5, -0.5)
+    stream.synchronize()
+    _check(y.cpu().numpy(), oracle.spmv_trans_f64(rows, cols, rowptr, colind, val, x, y0, 1.5, -0.5), torch.float32)
