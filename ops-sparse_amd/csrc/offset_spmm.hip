@@ -119,7 +119,9 @@ struct TileWalk {
 // us a call, the kernels for any columns / here: 5-point 2048 x 2048 n = 4 78 / 48 (the 320 MB it cannot do without at
 // 6.6 TB/s), n = 8 120 / 88; 7-point 125 x 131 x 127 n = 16 131 / 97, n = 32 213 / 169; 9-point 900 x 901 n = 64 190 / 134;
 // 27-point 71 x 77 x 79 n = 8 61 / 37, n = 64 184 / 156.  Wide B is bound by the instructions and waits of a pass (4 - 5
-// wavefronts a SIMD): with every gather sent to the row itself and no C written n = 32 still takes 110 us.
+// wavefronts a SIMD): with every gather sent to the row itself and no C written n = 32 still takes 110 us.  Passes whose rows
+// all have every distance, as inside a mesh, go without a branch an entry, one distance's elements widened at a time (9-point 1300 x
+// 1200 n = 24 120 -> 105, n = 64 127 -> 114; 27-point 100 x 100 x 101 n = 4 47 -> 43, n = 64 153 -> 142; 7-point n = 12 82 -> 76).
 template <typename ValT, typename CT, int P, typename Shape>
 __global__ __launch_bounds__(kBlockThreads) void SpmmOffsetRowsKernel(
     const int32_t *__restrict__ rowOffsets, const ValT *__restrict__ vals, const ValT *__restrict__ B, CT *C, int64_t rows,
@@ -338,7 +340,7 @@ __global__ __launch_bounds__(kBlockThreads) void SpmmOffsetRowsKernel(
                     AccT acc[V] = {};
                     const RowInfo mine = info[l];
                     int32_t at = mine.at;
-                    for (int32_t k0 = 0; k0 < distances; k0 += U) {
+                    auto chunk = [&](int32_t k0) {
                         Piece<ValT, V> b[U];
 #pragma unroll
                         for (int u = 0; u < U; ++u) {
@@ -346,20 +348,52 @@ __global__ __launch_bounds__(kBlockThreads) void SpmmOffsetRowsKernel(
                         }
                         const uint32_t bits = mine.mask >> k0;
                         ValT v[U];
+                        constexpr uint32_t kAll = (1u << U) - 1;
+                        if (__all((bits & kAll) == kAll)) {
 #pragma unroll
-                        for (int u = 0; u < U; ++u) {
-                            v[u] = staged[at];
-                            at += (bits >> u) & 1;
-                        }
+                            for (int u = 0; u < U; ++u) {
+                                v[u] = staged[at + u];
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                        for (int u = 0; u < U; ++u) {
-                            if (((bits >> u) & 1) != 0) {
+                            for (int u = 0; u < U; ++u) {
                                 const AccT w = ToAcc<AccT>(v[u]);
 #pragma unroll
                                 for (int i = 0; i < V; ++i) {
                                     acc[i] += w * ToAcc<AccT>(b[u].e[i]);
                                 }
+                                __builtin_amdgcn_sched_barrier(0);  // (what a distance widens is not kept beside the next one's)
                             }
+                            at += U;
+                        } else {
+#pragma unroll
+                            for (int u = 0; u < U; ++u) {
+                                v[u] = staged[at];
+                                at += (bits >> u) & 1;
+                            }
+#pragma unroll
+                            for (int u = 0; u < U; ++u) {
+                                // (opaque, so that its conversions are not made ahead of the branch for both of its arms)
+                                Int4U raw;
+                                __builtin_memcpy(&raw, b[u].e, 16);
+                                asm volatile("" : "+v"(raw));
+                                Piece<ValT, V> here;
+                                __builtin_memcpy(here.e, &raw, 16);
+                                if (((bits >> u) & 1) != 0) {
+                                    const AccT w = ToAcc<AccT>(v[u]);
+#pragma unroll
+                                    for (int i = 0; i < V; ++i) {
+                                        acc[i] += w * ToAcc<AccT>(here.e[i]);
+                                    }
+                                }
+                            }
+                        }
+                    };
+                    if constexpr (Shape::kMost == U) {
+                        chunk(0);
+                    } else {
+                        for (int32_t k0 = 0; k0 < distances; k0 += U) {
+                            chunk(k0);
                         }
                     }
                     finish(acc, r0 + l);
