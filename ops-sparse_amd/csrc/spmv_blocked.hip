@@ -131,10 +131,12 @@ typedef float Float4 __attribute__((ext_vector_type(4)));
 typedef unsigned short Ushort4 __attribute__((ext_vector_type(4)));
 typedef uint32_t Uint4 __attribute__((ext_vector_type(4)));
 typedef uint32_t Uint4U __attribute__((ext_vector_type(4), aligned(4)));  // a 16-byte load at any dword
+typedef uint32_t Uint4H __attribute__((ext_vector_type(4), aligned(2)));  // ... at any 16-bit value
 typedef uint32_t Uint2 __attribute__((ext_vector_type(2)));
+typedef uint32_t Uint2H __attribute__((ext_vector_type(2), aligned(2)));
 
 // ---- data as 32 raw bits -------------------------------------------------------------------------------------
-// x, gathered x and stored values travel as 32 raw bits: an fp32 (fp16 and bf16 widened, which is exact) or an int32.
+// x, gathered x and stored values are used as 32 raw bits: an fp32 (fp16 and bf16 widened, which is exact) or an int32.
 
 __device__ __forceinline__ uint32_t ToRaw(float v) { return __float_as_uint(v); }
 __device__ __forceinline__ uint32_t ToRaw(Half v) { return __float_as_uint(static_cast<float>(v)); }
@@ -169,19 +171,62 @@ __device__ __forceinline__ AccT SlotToAcc(uint64_t s)
     }
 }
 
-// Four consecutive values of the caller's array as raw bits, in one load (32-bit types: at any 4-byte-aligned
-// address; fp16 / bf16: at any 2-byte-aligned one).
+// Gathered x lies in memory in the width of x, fp16 and bf16 in the 16 bits they came in (finite or not, the same value when
+// widened again): both passes are bound by the bytes they move, of which an entry costs 10 instead of 14.  With it 16-bit values
+// are widened where they are used, not where they are loaded, which made every wavefront wait there.  Live values: 65 M bf16
+// entries of a power law over 8.4 M rows 258 -> 213 us, 60 M over 3 M equal rows 191 -> 145, 16 M over 1 M rows 76 -> 70; frozen,
+// windowed 157 -> 137 (6 M rows), streamed 182 -> 156 (60 M entries).
 template <typename ValT>
-__device__ __forceinline__ Uint4 LoadFourRaw(const ValT *p)
+using Stored = std::conditional_t<sizeof(ValT) == 4, uint32_t, uint16_t>;
+template <typename ValT>
+__device__ __forceinline__ uint32_t WidenRaw(uint32_t bits)  // (of 16-bit types: the low half of `bits`)
+{
+    if constexpr (sizeof(ValT) == 4) {
+        return bits;
+    } else {
+        const uint16_t low = static_cast<uint16_t>(bits);
+        ValT v;
+        __builtin_memcpy(&v, &low, 2);
+        return ToRaw(v);
+    }
+}
+template <typename ValT>
+__device__ __forceinline__ Stored<ValT> NarrowRaw(uint32_t raw)  // (of what WidenRaw gave)
+{
+    if constexpr (std::is_same<ValT, Half>::value) {
+        const Half v = static_cast<Half>(__uint_as_float(raw));
+        uint16_t bits;
+        __builtin_memcpy(&bits, &v, 2);
+        return bits;
+    } else if constexpr (sizeof(ValT) == 2) {
+        return static_cast<uint16_t>(raw >> 16);
+    } else {
+        return raw;
+    }
+}
+
+// Four consecutive values in one load, as they are stored (32-bit types: at any 4-byte-aligned address; fp16 / bf16: at
+// any 2-byte-aligned one), and widened.  Two steps: widening waits for the load.
+template <typename ValT>
+using StoredFour = std::conditional_t<sizeof(ValT) == 4, Uint4, Uint2>;
+template <typename ValT>
+__device__ __forceinline__ StoredFour<ValT> LoadFour(const ValT *p)
 {
     if constexpr (sizeof(ValT) == 4) {
         const Uint4U raw = __builtin_nontemporal_load(reinterpret_cast<const Uint4U *>(p));
         return Uint4{raw.x, raw.y, raw.z, raw.w};
     } else {
-        const Short4U raw = __builtin_nontemporal_load(reinterpret_cast<const Short4U *>(p));
-        ValT four[4];
-        __builtin_memcpy(four, &raw, 8);
-        return Uint4{ToRaw(four[0]), ToRaw(four[1]), ToRaw(four[2]), ToRaw(four[3])};
+        const Uint2H raw = __builtin_nontemporal_load(reinterpret_cast<const Uint2H *>(p));
+        return Uint2{raw.x, raw.y};
+    }
+}
+template <typename ValT>
+__device__ __forceinline__ Uint4 WidenFour(StoredFour<ValT> v)
+{
+    if constexpr (sizeof(ValT) == 4) {
+        return v;
+    } else {
+        return Uint4{WidenRaw<ValT>(v.x), WidenRaw<ValT>(v.x >> 16), WidenRaw<ValT>(v.y), WidenRaw<ValT>(v.y >> 16)};
     }
 }
 
@@ -1252,23 +1297,24 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
     __syncthreads();
     const int64_t len = e - a;
     const int64_t lo = a + len * part / splits, hi = a + len * (part + 1) / splits;
-    // Whole aligned groups of 4 entries go as 8-byte loads and 16-byte stores; what is left at
+    // Whole aligned groups of 4 entries go as 8-byte loads and 16-byte stores (8-byte ones of 16-bit x); what is left at
     // either end of [lo, hi) is done one by one.
+    auto *xgOut = reinterpret_cast<Stored<XT> *>(xg);
     const int64_t g0 = (lo + 3) >> 2, g1 = hi >> 2;
     if (lo < hi && g0 > g1) {
         if (tid < 4 && lo + tid < hi) {
-            xg[lo + tid] = xs[colLocal[lo + tid] & (kPanelCols - 1)];
+            xgOut[lo + tid] = NarrowRaw<XT>(xs[colLocal[lo + tid] & (kPanelCols - 1)]);
         }
     } else if (lo < hi) {
         if (tid < 4) {
             const int64_t i = lo + tid;
             if (i < g0 * 4) {
-                xg[i] = xs[colLocal[i] & (kPanelCols - 1)];
+                xgOut[i] = NarrowRaw<XT>(xs[colLocal[i] & (kPanelCols - 1)]);
             }
         } else if (tid < 8) {
             const int64_t i = g1 * 4 + (tid - 4);
             if (i < hi) {
-                xg[i] = xs[colLocal[i] & (kPanelCols - 1)];
+                xgOut[i] = NarrowRaw<XT>(xs[colLocal[i] & (kPanelCols - 1)]);
             }
         }
         for (int64_t g = g0; g < g1; g += kGatherBatch * kBlkThreads) {
@@ -1289,7 +1335,12 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
                 r.z = xs[c[u].z & (kPanelCols - 1)];
                 r.w = xs[c[u].w & (kPanelCols - 1)];
                 if (gg < g1) {
-                    *(reinterpret_cast<Uint4 *>(xg) + gg) = r;
+                    if constexpr (sizeof(XT) == 4) {
+                        *(reinterpret_cast<Uint4 *>(xg) + gg) = r;
+                    } else {
+                        *(reinterpret_cast<Ushort4 *>(xg) + gg) =
+                            Ushort4{NarrowRaw<XT>(r.x), NarrowRaw<XT>(r.y), NarrowRaw<XT>(r.z), NarrowRaw<XT>(r.w)};
+                    }
                 }
             }
         }
@@ -1440,19 +1491,20 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
         // is always four whole entries: it starts at most at i1 - 4 (never below 0), so the last group reads a
         // few entries in front of its own, and a group past the end re-reads the last one; `add` takes only the
         // entries that are the group's own.  No entry is ever fetched one by one.
-        auto request = [&](int32_t i0, int32_t i1, int32_t q, Int4U *c, Uint4 *v) {
+        auto request = [&](int32_t i0, int32_t i1, int32_t q, Int4U *c, StoredFour<XT> *v) {
             int64_t at = i0 + 4 * static_cast<int64_t>(q);
             at = at + 4 <= i1 ? at : static_cast<int64_t>(i1) - 4;
             at = at < 0 ? 0 : at;
             *c = __builtin_nontemporal_load(reinterpret_cast<const Int4U *>(colInd + at));
-            *v = LoadFourRaw(vals + at);
+            *v = LoadFour(vals + at);
         };
-        auto add = [&](int32_t i0, int32_t i1, int32_t q, const Int4U &c, const Uint4 &v, AccT *sum) {
+        auto add = [&](int32_t i0, int32_t i1, int32_t q, const Int4U &c, const StoredFour<XT> &stored, AccT *sum) {
             const int64_t own = i0 + 4 * static_cast<int64_t>(q);  // first entry of the group
             int64_t at = own + 4 <= i1 ? own : static_cast<int64_t>(i1) - 4;
             at = at < 0 ? 0 : at;
             const uint32_t mask = kPanelCols - 1;  // an entry of the group is in the panel by construction
             const int32_t cs[4] = {c.x, c.y, c.z, c.w};
+            const Uint4 v = WidenFour<XT>(stored);
             const uint32_t vs[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -1470,22 +1522,22 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
         if (k < tn) {
             int32_t i0 = pieceLo[k], i1 = pieceHi[k];
             Int4U cFirst;
-            Uint4 vFirst;
+            StoredFour<XT> vFirst;
             request(i0, i1, gt, &cFirst, &vFirst);
             while (true) {
                 const int32_t kn = k + stride;
                 const int32_t kk = kn < tn ? kn : k;
                 const int32_t j0 = pieceLo[kk], j1 = pieceHi[kk];
                 Int4U cAhead;
-                Uint4 vAhead;
+                StoredFour<XT> vAhead;
                 request(j0, j1, gt, &cAhead, &vAhead);
                 const int32_t n4 = (i1 - i0 + 3) >> 2;  // groups of the piece, the last one maybe short
                 AccT sum = AccT(0);
                 Int4U c = cFirst;
-                Uint4 v = vFirst;
+                StoredFour<XT> v = vFirst;
                 for (int32_t q = gt; q < n4; q += kLongLanes) {
                     Int4U cNext;
-                    Uint4 vNext;
+                    StoredFour<XT> vNext;
                     request(i0, i1, q + kLongLanes, &cNext, &vNext);
                     add(i0, i1, q, c, v, &sum);
                     c = cNext;
@@ -1515,7 +1567,7 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
             AccT sum = AccT(0);
             for (int32_t q = tid; q < n4; q += 2 * kBlkThreads) {
                 Int4U c[2];
-                Uint4 v[2];
+                StoredFour<XT> v[2];
                 request(i0, i1, q, &c[0], &v[0]);
                 request(i0, i1, q + kBlkThreads, &c[1], &v[1]);
                 add(i0, i1, q, c[0], v[0], &sum);
@@ -1571,13 +1623,27 @@ __device__ __forceinline__ Uint4 QuadMove(Uint4 v)
                  DppMove<kCtrl, 0xf>(0u, v.w)};
 }
 template <int kCtrl>
-__device__ __forceinline__ void QuadExchange(Uint4 &a, Uint4 &b, bool second)
+__device__ __forceinline__ Uint2 QuadMove(Uint2 v)
 {
-    const Uint4 aMoved = QuadMove<kCtrl>(a), bMoved = QuadMove<kCtrl>(b);
-    a = Uint4{second ? bMoved.x : a.x, second ? bMoved.y : a.y, second ? bMoved.z : a.z, second ? bMoved.w : a.w};
-    b = Uint4{second ? b.x : aMoved.x, second ? b.y : aMoved.y, second ? b.z : aMoved.z, second ? b.w : aMoved.w};
+    return Uint2{DppMove<kCtrl, 0xf>(0u, v.x), DppMove<kCtrl, 0xf>(0u, v.y)};
 }
-__device__ __forceinline__ void QuadTranspose(Uint4 &p0, Uint4 &p1, Uint4 &p2, Uint4 &p3)
+__device__ __forceinline__ Uint4 Select(bool first, Uint4 a, Uint4 b)
+{
+    return Uint4{first ? a.x : b.x, first ? a.y : b.y, first ? a.z : b.z, first ? a.w : b.w};
+}
+__device__ __forceinline__ Uint2 Select(bool first, Uint2 a, Uint2 b)
+{
+    return Uint2{first ? a.x : b.x, first ? a.y : b.y};
+}
+template <int kCtrl, typename Four>
+__device__ __forceinline__ void QuadExchange(Four &a, Four &b, bool second)
+{
+    const Four aMoved = QuadMove<kCtrl>(a), bMoved = QuadMove<kCtrl>(b);
+    a = Select(second, bMoved, a);
+    b = Select(second, b, aMoved);
+}
+template <typename Four>
+__device__ __forceinline__ void QuadTranspose(Four &p0, Four &p1, Four &p2, Four &p3)
 {
     const bool odd = (threadIdx.x & 1) != 0, upper = (threadIdx.x & 2) != 0;
     QuadExchange<kDppQuadSwap1>(p0, p1, odd);
@@ -1586,12 +1652,18 @@ __device__ __forceinline__ void QuadTranspose(Uint4 &p0, Uint4 &p1, Uint4 &p2, U
     QuadExchange<kDppQuadSwap2>(p1, p3, upper);
 }
 
-// Four entries loaded `ahead` places in front of where they belong, put there (ahead <= 0: they are; what is moved in from
+// Four values loaded `ahead` places in front of where they belong, put there (ahead <= 0: they are; what is moved in from
 // behind the array's last entry is zero).
 __device__ __forceinline__ Uint4 ShiftedFour(Uint4 v, int32_t ahead)
 {
     const Uint4 by1 = Uint4{v.y, v.z, v.w, 0u}, by2 = Uint4{v.z, v.w, 0u, 0u}, by3 = Uint4{v.w, 0u, 0u, 0u};
     return ahead <= 0 ? v : ahead == 1 ? by1 : ahead == 2 ? by2 : ahead == 3 ? by3 : Uint4{0u, 0u, 0u, 0u};
+}
+__device__ __forceinline__ Uint2 ShiftedFour(Uint2 v, int32_t ahead)
+{
+    const uint64_t all = (static_cast<uint64_t>(v.y) << 32) | v.x;
+    const uint64_t moved = ahead <= 0 ? all : ahead < 4 ? all >> (16 * ahead) : 0u;
+    return Uint2{static_cast<uint32_t>(moved), static_cast<uint32_t>(moved >> 32)};
 }
 
 // The sum of a long row's partial sums, lane by lane in panel order and then across the lanes, the same way at
@@ -1763,10 +1835,15 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
             for (int u = 0; u < kStagePasses; ++u) {
                 uint32_t at = static_cast<uint32_t>(src[u]);
                 at = at < static_cast<uint32_t>(a.xgEntries) ? at : 0u;  // (in range whatever the table holds)
-                const Uint4U v0 = *reinterpret_cast<const Uint4U *>(a.xg + at);
-                const Uint4U v1 = *reinterpret_cast<const Uint4U *>(a.xg + at + 4);
-                xa[u] = Uint4{v0.x, v0.y, v0.z, v0.w};
-                xb[u] = Uint4{v1.x, v1.y, v1.z, v1.w};
+                if constexpr (sizeof(ValT) == 4) {
+                    const Uint4U v0 = *reinterpret_cast<const Uint4U *>(a.xg + at);
+                    const Uint4U v1 = *reinterpret_cast<const Uint4U *>(a.xg + at + 4);
+                    xa[u] = Uint4{v0.x, v0.y, v0.z, v0.w};
+                    xb[u] = Uint4{v1.x, v1.y, v1.z, v1.w};
+                } else {
+                    const Uint4H v0 = *reinterpret_cast<const Uint4H *>(reinterpret_cast<const uint16_t *>(a.xg) + at);
+                    xa[u] = Uint4{v0.x, v0.y, v0.z, v0.w};
+                }
             }
         };
         auto drop = [&](int32_t start) {
@@ -1775,7 +1852,15 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
                 const int32_t mine = start + u * kWaves * kPassSpan + lane * kLaneEntries;
                 const uint32_t sl[8] = {slots[u].x & 0xffffu, slots[u].x >> 16, slots[u].y & 0xffffu, slots[u].y >> 16,
                                         slots[u].z & 0xffffu, slots[u].z >> 16, slots[u].w & 0xffffu, slots[u].w >> 16};
-                const uint32_t xv[8] = {xa[u].x, xa[u].y, xa[u].z, xa[u].w, xb[u].x, xb[u].y, xb[u].z, xb[u].w};
+                uint32_t xv[8];
+                if constexpr (sizeof(ValT) == 4) {
+                    xv[0] = xa[u].x; xv[1] = xa[u].y; xv[2] = xa[u].z; xv[3] = xa[u].w;
+                    xv[4] = xb[u].x; xv[5] = xb[u].y; xv[6] = xb[u].z; xv[7] = xb[u].w;
+                } else {
+                    const Uint4 lo = WidenFour<ValT>(Uint2{xa[u].x, xa[u].y}), hi = WidenFour<ValT>(Uint2{xa[u].z, xa[u].w});
+                    xv[0] = lo.x; xv[1] = lo.y; xv[2] = lo.z; xv[3] = lo.w;
+                    xv[4] = hi.x; xv[5] = hi.y; xv[6] = hi.z; xv[7] = hi.w;
+                }
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const uint32_t rel = sl[j] - static_cast<uint32_t>(w0);  // (a window is whole rounds: the
@@ -1805,7 +1890,7 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
         // the values: four at a time; the four at the end of the array start early enough to lie inside it and are put
         // into their places when they are used (a lane behind the block's last entry reads its first ones; what it
         // reads is not used)
-        Uint4 vraw[kMaxRounds][kLaneRun / 4];
+        StoredFour<ValT> vraw[kMaxRounds][kLaneRun / 4];
         const int64_t last4 = a.valEntries - m.base - 4;  // (where the last four start, from the block's first entry)
         const int32_t lastFour = last4 < INT32_MAX ? static_cast<int32_t>(last4) : INT32_MAX;
         const bool atArrayEnd = nB > lastFour;
@@ -1816,7 +1901,7 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
 #pragma unroll
             for (int f = 0; f < kLaneRun / 4; ++f) {
                 const int32_t qf = q + f * kLaneRun < nEnd ? q + f * kLaneRun : 0;
-                vraw[u][f] = LoadFourRaw(from + (qf < lastFour ? qf : lastFour));
+                vraw[u][f] = LoadFour(from + (qf < lastFour ? qf : lastFour));
             }
         }
         if (w0 > 0) {
@@ -1910,7 +1995,8 @@ __global__ __launch_bounds__(kRowsSizes[kSize].threads, kRowsSizes[kSize].waves)
                         ++key;
                         run = AccT(0);
                     }
-                    const uint32_t v4[4] = {vraw[u][j / 4].x, vraw[u][j / 4].y, vraw[u][j / 4].z, vraw[u][j / 4].w};
+                    const Uint4 wide = WidenFour<ValT>(vraw[u][j / 4]);
+                    const uint32_t v4[4] = {wide.x, wide.y, wide.z, wide.w};
                     const AccT prod = RawToAcc<AccT, kIntData>(v4[j % 4]) * RawToAcc<AccT, kIntData>(xraw[u][j]);
                     run += q + j < nEnd ? prod : AccT(0);
                 }
@@ -2061,7 +2147,7 @@ __global__ __launch_bounds__(kStreamThreads) void SpmvBlockStreamKernel(const Bl
         }
     }
     struct Piece {
-        Uint4 v[2], x[2];
+        StoredFour<ValT> v[2], x[2];
         Uint2 f[2];
     };
     struct Sources {
@@ -2093,8 +2179,12 @@ __global__ __launch_bounds__(kStreamThreads) void SpmvBlockStreamKernel(const Bl
             // that xg has behind it: those are padding positions)
             int32_t src = from.at[s] + (at & 4);
             src = src < 0 ? 0 : (src < a.xgEntries ? src : a.xgEntries);
-            piece.v[s] = LoadFourRaw(a.valD + at);
-            piece.x[s] = *reinterpret_cast<const Uint4U *>(a.xg + src);
+            piece.v[s] = LoadFour(a.valD + at);
+            if constexpr (sizeof(ValT) == 4) {
+                piece.x[s] = *reinterpret_cast<const Uint4U *>(a.xg + src);
+            } else {
+                piece.x[s] = *reinterpret_cast<const Uint2H *>(reinterpret_cast<const uint16_t *>(a.xg) + src);
+            }
             piece.f[s] = __builtin_nontemporal_load(reinterpret_cast<const Uint2 *>(a.field + at));
         }
         return piece;
@@ -2102,8 +2192,9 @@ __global__ __launch_bounds__(kStreamThreads) void SpmvBlockStreamKernel(const Bl
     auto process = [&](const Piece &cur, int32_t start) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            const uint32_t vr[4] = {cur.v[s].x, cur.v[s].y, cur.v[s].z, cur.v[s].w};
-            const uint32_t xr[4] = {cur.x[s].x, cur.x[s].y, cur.x[s].z, cur.x[s].w};
+            const Uint4 v4 = WidenFour<ValT>(cur.v[s]), x4 = WidenFour<ValT>(cur.x[s]);
+            const uint32_t vr[4] = {v4.x, v4.y, v4.z, v4.w};
+            const uint32_t xr[4] = {x4.x, x4.y, x4.z, x4.w};
             // positions behind the block's last (a lane then holds the block's last four again): padding
             const bool inside = start + s * kSub + lane * 4 < dEnd;
             const Uint2 fs = inside ? cur.f[s] : Uint2{kStreamPadRow * 0x10001u, kStreamPadRow * 0x10001u};

@@ -105,3 +105,26 @@ def test_coosort_columns_of_many_bits(osa, gpu_ctx, span, cols, nnz):
     rows, c = rng.integers(0, span, nnz).astype(np.int32), rng.integers(0, cols, nnz).astype(np.int32)
     c[:2] = [0, cols - 1]
     run_coosort(osa, gpu_ctx, span, cols, rows, c, True, perm=rng.permutation(nnz).astype(np.int32))
+
+
+VALUES = [("FP32", True), ("FP16", True), ("INT8", True), ("FP32", False)]
+
+
+@pytest.mark.parametrize("val_type,numeric", VALUES)
+def test_csr2csc_two_packed_passes_of_the_smallest_workgroups(osa, gpu_ctx, val_type, numeric):
+    """21 column bits, ten of them in LDS, under 2^20 entries."""
+    n, nnz = (1 << 20) + 3, 700_001
+    rng = np.random.default_rng(5)
+    rowptr = np.array([0, nnz // 3, nnz // 3, nnz], np.int32)
+    val = _typed(rng.uniform(-1, 1, nnz).astype(np.float32), val_type)
+    run_csr2csc(osa, gpu_ctx, 3, n, rowptr + 1, columns("uniform", n, nnz, rng) + 1, val, NP_TYPE[val_type], numeric, 1)
+
+
+@pytest.mark.parametrize("val_type,numeric", VALUES)
+def test_csr2csc_of_few_entries_a_column_and_many_rows(osa, gpu_ctx, val_type, numeric):
+    """24 row bits leave eight for LDS, whose buckets would hold 128 entries: three passes of the largest workgroups."""
+    m, n, nnz = (1 << 23) + 7, (1 << 24) - 3, (1 << 23) + 5
+    rng = np.random.default_rng(6)
+    rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, m - 1)), [nnz]]).astype(np.int32)
+    val = _typed(rng.uniform(-1, 1, nnz).astype(np.float32), val_type)
+    run_csr2csc(osa, gpu_ctx, m, n, rowptr, columns("uniform", n, nnz, rng), val, NP_TYPE[val_type], numeric, 0)

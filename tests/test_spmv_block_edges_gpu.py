@@ -78,3 +78,41 @@ def test_where_the_blocks_are_cut(osa, gpu_ctx, monkeypatch, rows, longest, ends
     stream.synchronize()
     gold = oracle.spmv_f64(rows, COLS, rowptr, colind, val, x, np.zeros(rows, np.float32), 1.0, 0.0)
     assert oracle.max_rel_err(y.cpu().numpy(), gold) <= 1e-5
+
+
+@pytest.mark.parametrize("streamed", [False, True])
+@pytest.mark.parametrize("dtype,alg", [("f16", "default"), ("bf16", "default"), ("f16", "frozen"), ("bf16", "frozen")])
+def test_gathered_x_of_16_bits(osa, gpu_ctx, monkeypatch, dtype, alg, streamed):
+    """x of every bit pattern, from an odd 16-bit place on.  Eight entries of a row name one column and hold 1/8 each: y is that
+    element of x, bit for bit.  A long row over positive elements keeps its values behind the gathered x (frozen)."""
+    for name in ("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "OPS_SPARSE_ORDERED_LIVE_MIN_COLS"):
+        monkeypatch.setenv(name, "0")
+    if not streamed:
+        monkeypatch.setenv("OPS_SPARSE_BLOCKED_NO_STREAM", "1")
+    dev, stream, handle = gpu_ctx
+    kind = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    rng = np.random.default_rng(17)
+    rows, long_row, long_len = 300_001, 170_000, 20_000
+    bits = torch.from_numpy(((np.arange(COLS + 1) * 40503) % 65536).astype(np.uint16).view(np.int16))
+    x = bits.view(kind).to(dev)[1:]
+    x64 = bits.view(kind)[1:].double().numpy()
+    lengths = np.full(rows, 8)
+    lengths[long_row] = long_len
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    of_row = rng.integers(0, COLS, rows)
+    colind = np.repeat(of_row, lengths).astype(np.int32)
+    tame = np.flatnonzero((x64 > 0.01) & (x64 < 100.0))
+    colind[rowptr[long_row]:rowptr[long_row + 1]] = np.sort(rng.choice(tame, long_len, replace=False))
+    val = torch.full((colind.size,), 0.125, dtype=kind, device=dev)
+    y = torch.full((rows,), 7.0, device=dev)
+    A = osa.Csr(rows, COLS, to_dev(rowptr, dev), to_dev(colind, dev), val)
+    op = osa.SpmvOp(handle, A, osa.DnVec(x), osa.DnVec(y),
+                    alg=osa.ACL_SPARSE_SPMV_CSR_ALG2 if alg == "frozen" else osa.ACL_SPARSE_SPMV_ALG_DEFAULT)
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, colind.size)
+    op(1.0, 0.0)
+    stream.synchronize()
+    got, want = y.cpu().numpy(), x64[of_row].astype(np.float32)
+    want[long_row] = got[long_row]
+    assert np.array_equal(got, want, equal_nan=True)
+    total = 0.125 * x64[colind[rowptr[long_row]:rowptr[long_row + 1]]].sum()
+    assert abs(got[long_row] - total) <= 2 ** -23 * total  # (a sum in 64 bits, rounded once)
