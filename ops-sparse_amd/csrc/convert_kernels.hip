@@ -1378,15 +1378,15 @@ __device__ __forceinline__ void SortRowInGroup(int64_t begin, int64_t len, int32
 // these kernels end at once, 14 us for the three.
 //
 // 33.5 M entries over 2^20 keys: csr2csc 797 -> 651 us (the last pass with its count and scan, 213 us, and the counting of the
-// sorted columns, 70, became 133 us and 19 for the buckets' starts), coosort by row 991 -> 897; 400 K entries over 50 000
-// columns 95 -> 64 us, 5 M over 500 000, where no pass is saved, 191 either way.  Where half of the keys are met, so that every
-// bucket is twice as full as planned, the larger workgroups make it 772 -> 742 us (925 while such buckets went in pieces, 1139
+// sorted columns, 70, became 133 us and 19 for the buckets' starts), and 498 with packed records in front of the buckets (114 us);
+// 400 K entries over 50 000 columns 95 -> 64 us.  Before the records were packed: where half of the keys are met, so that every
+// bucket is twice as full as planned, the larger workgroups made it 772 -> 742 us (925 while such buckets went in pieces, 1139
 // with each entry of theirs written straight to its place); with a tenth of the entries in one column 1487 -> 762.
 //
 // coosort's rows lie side by side in LDS then, and those of up to 64 entries are sorted in registers on their way out; the
 // rest go on csrsort's lists.  A kernel over the sorted entries that did this read and wrote 8 bytes an entry once more: 33.5 M
 // entries, 32 a row, 897 -> 779 us, 8 a row over 4 M rows 904 -> 747 (without the digits in LDS there is room for three
-// workgroups a compute unit instead of two, too).
+// workgroups a compute unit instead of two, too).  With packed records in front and the faster networks 676 us, the buckets 225.
 
 constexpr int kFinishThreads = 512;
 constexpr int kFinishItems = 12;  // entries of a thread
@@ -2908,7 +2908,8 @@ int opsparse_csr2csc_launch(int64_t m, int64_t n, int64_t nnz, const void *csrVa
     // than a source position would, and the last pass writes rows and values where they belong — no gather by
     // position at the end, which cost two cache-line fills per entry (33.5 M entries: 2.9 -> 1.9 ms).
     // Up to ten bits a pass (WidePassesOf), the tile ordered through LDS before it leaves, and the last bits in LDS where
-    // that saves a pass (33.5 M entries over 2^20 columns: three passes of seven bits 0.80 ms, two and the last bits 0.65).
+    // that saves a pass or there are many entries (33.5 M over 2^20 columns: three passes of seven bits 0.80 ms, two over packed
+    // records and the last bits 0.50).
     const RadixPairIo io{rowOfPos, csrVal, cscRowInd, cscVal, valueBytes};
     const FinishPlan plan = FinishPlanOf(n, nnz, KeyBits(m + indexBase));
     if (plan.use) {

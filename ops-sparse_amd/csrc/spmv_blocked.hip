@@ -13,10 +13,10 @@
 //   phase 1  the entries' local column indices are stored a second time sorted
 //            by column panel (2^15 columns = 128 KiB of x).  A workgroup copies
 //            its panel's slice of x into LDS and writes xg[i] = x[col[i]] for
-//            the panel's entries: 2 bytes read, 4 bytes written per entry, both
-//            as linear streams.
-//   phase 2  rows are grouped into row blocks (at most 2^10 - 2^12 rows, cut also
-//            wherever the entry count passes a multiple of the entry window).
+//            the panel's entries: 2 bytes read, 4 bytes (of 16-bit x 2) written per
+//            entry, both as linear streams.
+//   phase 2  rows are grouped into row blocks (streamed: 2^10 rows; windowed: at most
+//            2^11 or 2^12 rows and a window's entries, one block cut after the other).
 //            The entries of a block are one contiguous piece of the values in
 //            row order, and a workgroup owns one block: it streams the block's
 //            xg — in (block, panel) order, one contiguous piece per (panel,
@@ -28,7 +28,7 @@
 //            the entries only.
 //
 // Every entry costs 16 bytes of traffic (2 + 4 in phase 1, 2 + 4 + 4 in phase
-// 2) against 8 algorithmic bytes plus a 128-byte line per gather in the
+// 2; of 16-bit data 10) against 8 algorithmic bytes plus a 128-byte line per gather in the
 // row-wise kernels.  No value is stored: every call reads the values where
 // the caller (or the copy described below) has them.  val * x is exact in
 // fp64; the additions of a row are made in an order that the layout fixes —
@@ -1737,7 +1737,7 @@ struct BlockRowsArgs {
 // live values, 235 us at first; 219 without 20 bytes of spilled registers, with the wavefronts' edges joined by lanes side by
 // side (one after the other had each wait for an old y) and the end of the value array read without a second path around every
 // load; 189 with the blocks cut one after the other (RowBlockCutsKernel); 176 with one round a wavefront and one turn a block; 165
-// with the values loaded by quads of lanes: 780 MB, 4.7 TB/s, at which more workgroups a compute unit (64 registers, four instead of
+// with the values loaded by quads of lanes: 746 MB, 4.5 TB/s, at which more workgroups a compute unit (64 registers, four instead of
 // three) no longer help.  31 M over 4 M rows 100 -> 74.  A workgroup that stays and takes block after block, with the next block's tables and places
 // asked for ahead, is slower (160 -> 179 us a call): its wavefronts meet at one more barrier, where all of them wait for the
 // last row written.  So are sums in memory of their own, without the barrier in front of them (172).
