@@ -118,10 +118,11 @@ constexpr int64_t kLongMinRowFrozen = 1024;
 constexpr int kLongLanes = 16;        // lanes that sum one (long row, panel) piece in phase 1
 constexpr int32_t kInBlockLongRows = 64;          // long rows a row block's own workgroup adds up at most
 // Live values: pieces of at least this many entries that are also longer than this many lane groups' shares of the
-// workgroup's long entries are added up by the whole workgroup.  A group takes 64 entries a round trip to memory, and the
+// workgroup's long entries are added up by the whole workgroup.  A group takes 256 entries a round trip to memory, and the
 // hub of a graph has thousands in a panel where there are few panels: 400 K x 400 K power-law rows, 24 entries a row, the
-// longest 100 000, 105 us a call, 64 with it (77 by the merge path); 1 M x 1 M, 8.6 M entries, 96 and 63.  With four
-// shares instead of six, 1.3 M x 1.3 M and 24 entries a row 159 us, 155 by groups alone.
+// longest 100 000, 105 us a call by groups of 64 a round trip, 64 with it, 59 with 256 (77 by the merge path); 1 M x 1 M, 8.6 M
+// entries, 96 and 63.  Pieces of 4096 and more only: 500 K rows, 8 M entries, the longest 200 000, 59 us, 51 so; pieces of 512 and
+// more, where groups took 64, 1 M rows of 16, the longest 50 000, 78 instead of 74: the workgroup takes them one after the other.
 constexpr int32_t kBigPiece = 2048;
 constexpr int32_t kBigPieceShares = 6;
 constexpr int32_t kMaxBigPieces = kBlkThreads / kLongLanes / kBigPieceShares + 1;
@@ -1535,7 +1536,26 @@ __global__ __launch_bounds__(kBlkThreads) void SpmvBlockGatherKernel(const uint1
                 AccT sum = AccT(0);
                 Int4U c = cFirst;
                 StoredFour<XT> v = vFirst;
-                for (int32_t q = gt; q < n4; q += kLongLanes) {
+                int32_t q = gt;
+                // a long piece: four requests on their way at a time, 256 entries a round trip (a hub of 200 000 entries over 92 panels,
+                // 23 M entries, a call 113 -> 105 us; 50 000 over 31 panels, 16 M entries, 74 -> 70; 65 M over 256 panels 266 -> 262)
+                while (q + 3 * kLongLanes < n4) {
+                    Int4U cs[4];
+                    StoredFour<XT> vs[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        request(i0, i1, q + (u + 1) * kLongLanes, &cs[u], &vs[u]);
+                    }
+                    add(i0, i1, q, c, v, &sum);
+#pragma unroll
+                    for (int u = 0; u < 3; ++u) {
+                        add(i0, i1, q + (u + 1) * kLongLanes, cs[u], vs[u], &sum);
+                    }
+                    c = cs[3];
+                    v = vs[3];
+                    q += 4 * kLongLanes;
+                }
+                for (; q < n4; q += kLongLanes) {
                     Int4U cNext;
                     StoredFour<XT> vNext;
                     request(i0, i1, q + kLongLanes, &cNext, &vNext);

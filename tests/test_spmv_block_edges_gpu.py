@@ -116,3 +116,36 @@ def test_gathered_x_of_16_bits(osa, gpu_ctx, monkeypatch, dtype, alg, streamed):
     assert np.array_equal(got, want, equal_nan=True)
     total = 0.125 * x64[colind[rowptr[long_row]:rowptr[long_row + 1]]].sum()
     assert abs(got[long_row] - total) <= 2 ** -23 * total  # (a sum in 64 bits, rounded once)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_pieces_of_long_rows_of_every_length(osa, gpu_ctx, monkeypatch, dtype):
+    """Live values: what a long row has in one panel is summed by 16 lanes, 64 entries a request and four requests at a time where
+    there are as many; the remainders on either side, and the end of the arrays."""
+    monkeypatch.setenv("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "0")
+    dev, stream, handle = gpu_ctx
+    kind = {"f32": torch.float32, "bf16": torch.bfloat16}[dtype]
+    rng = np.random.default_rng(23)
+    rows, cols, panel = 300_000, 1_000_000, 32768
+    pieces = [0, 1, 3, 63, 64, 65, 191, 192, 193, 195, 196, 197, 255, 256, 257, 447, 448, 449, 511, 512, 513, 1024, 1999, 2047]
+    lengths = rng.integers(6, 11, rows)
+    lengths[-1] = 0
+    own = {}
+    for k, n in enumerate(pieces):
+        row = rows - 1 if k == len(pieces) - 1 else 1000 + 7 * k  # (one of them ends where the arrays do)
+        other = np.sort(rng.choice(panel, 4096 - n, replace=False)) if k % 2 else np.sort(rng.choice(cols - 4 * panel, 4096 - n, replace=False) + 4 * panel)
+        own[row] = np.sort(np.concatenate([other, 2 * panel + rng.choice(panel, n, replace=False)]))
+        lengths[row] = 4096
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    colind = rng.integers(0, cols, int(rowptr[-1])).astype(np.int32)
+    for row, c in own.items():
+        colind[rowptr[row]:rowptr[row + 1]] = c
+    val, x = (torch.from_numpy(rng.uniform(0.5, 1, n).astype(np.float32)).to(kind).float().numpy() for n in (colind.size, cols))
+    y = torch.full((rows,), float("nan"), device=dev)
+    A = osa.Csr(rows, cols, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev, kind))
+    op = osa.SpmvOp(handle, A, osa.DnVec(to_dev(x, dev, kind)), osa.DnVec(y))
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, colind.size)
+    op(1.0, 0.0)
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, cols, rowptr, colind, val, x, np.zeros(rows, np.float32), 1.0, 0.0)
+    assert oracle.max_rel_err(y.cpu().numpy(), gold) <= 2 ** -23  # (sums in 64 bits, rounded once)
