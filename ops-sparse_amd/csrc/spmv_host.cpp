@@ -104,7 +104,7 @@ aclsparseStatus_t ValidateData(SpmvCall *c, aclDataType computeType)
 // CSR_ALG2 asks for one: the blocked-gather layout first, the column panels where that one does not fit the
 // matrix; both hold a copy of the values as they were at Preprocess.
 // ALG_DEFAULT / CSR_ALG1 get a layout with LIVE values (every call re-reads the caller's values, so nothing can go
-// stale) when the gathers of x are scattered: 0.27 ms against 1.1 ms for the merge path on an 8 M x 8 M power-law
+// stale) when the gathers of x are scattered: 0.26 ms against 1.1 ms for the merge path on an 8 M x 8 M power-law
 // matrix.  Its rows are summed in an order that the layout fixes.  A matrix with a row that this layout refuses gets, for
 // op(A) = A and floating-point values, the one whose row blocks add with LDS atomics: these algorithm values promise no
 // bit-wise repeatable result (reference include/cann_ops_sparse.h:57-60, only CSR_ALG2 is "deterministic").
