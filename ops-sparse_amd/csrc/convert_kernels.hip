@@ -942,6 +942,8 @@ __global__ __launch_bounds__(T) void WideScatterKernel(
 // payload in one word and the value in the other, and between two passes a byte beside it, the second pass's digit, which is
 // also all that its count has to read.  Bound by memory: 12 bytes an entry in and 9 out, 9 and 8, where key, row and value were
 // 12 in and 12 out in either pass; a tile's run in a bucket is a piece of one array instead of three.
+// Where the low bits and the payload take more than a word (more than 2^22 rows under ten low bits) the payload's top bits travel
+// in 16 bits of their own (Tops): 2 bytes an entry more into and out of every step behind the first.
 struct PackIo {
     const int32_t *keys;  // first pass: keyBase + key, payload and value of every entry
     int32_t keyBase;
@@ -951,22 +953,25 @@ struct PackIo {
     const Record *recsIn;
     uint8_t *digitsOut;  // first pass of two
     Record *recsOut;
+    const uint16_t *topsIn;  // Tops: what is above payBits of a payload, beside the records
+    uint16_t *topsOut;
     int64_t n;
-    int32_t low, payBits;  // bits of a key below its bucket; of a payload (together 32 at most)
+    int32_t low, payBits;  // bits of a key below its bucket; of a payload in the record (together 32 at most)
     int32_t nextShift;     // first pass of two: the second one's digit is what is above this bit of a key
 };
 
 enum PackMode { kPackOnly = 0, kPackFirst = 1, kPackSecond = 2 };
 
-template <int T, int Mode>
+template <int T, int Mode, bool Tops>
 struct PackRegs {
     uint32_t key[kWideItems], pay[kWideItems], val[kWideItems];
     int32_t first[WideShape<T>::kPer];
 };
-template <int T>
-struct PackRegs<T, kPackSecond> {
+template <int T, bool Tops>
+struct PackRegs<T, kPackSecond, Tops> {
     uint64_t rec[kWideItems];
     uint32_t digit[kWideItems];
+    uint32_t top[Tops ? kWideItems : 1];
     int32_t first[WideShape<T>::kPer];
 };
 
@@ -976,13 +981,14 @@ __device__ __forceinline__ uint64_t PackedRecord(uint32_t word, uint32_t val)
     return (static_cast<uint64_t>(val) << 32) | word;
 }
 
-template <int T>
+template <int T, bool Tops>
 struct PackLds {
     union {
         int32_t counters[WideShape<T>::kWaves << kWideMaxBits];
         struct {
             uint64_t rec[WideShape<T>::kTile];
-            uint16_t digit[WideShape<T>::kTile];  // kPackFirst: the next pass's above the lower eight bits
+            uint16_t digit[WideShape<T>::kTile * (Tops ? 2 : 1)];  // kPackFirst: the next pass's above the lower eight
+                                                                   // bits; behind the tile's digits its tops
         };
     };
     int32_t outOf[1 << kWideMaxBits];
@@ -990,14 +996,14 @@ struct PackLds {
 };
 
 // prefix, shift, mask, bits: as WideScatterKernel; the first digit of two has eight bits at most.
-template <int T, int Mode, int VB>
+template <int T, int Mode, int VB, bool Tops>
 __global__ __launch_bounds__(T, 4) void PackScatterKernel(PackIo io, int32_t shift, int32_t mask, int32_t bits,
                                                           const int32_t *__restrict__ prefix, int64_t numTiles)
 {
-    __shared__ PackLds<T> lds;
+    __shared__ PackLds<T, Tops> lds;
     constexpr int kTile = WideShape<T>::kTile, kPer = WideShape<T>::kPer;
     const uint32_t lowMask = (1u << io.low) - 1u;
-    auto fetch = [&](PackRegs<T, Mode> &r, int64_t tile, auto full) {
+    auto fetch = [&](PackRegs<T, Mode, Tops> &r, int64_t tile, auto full) {
         const int tid = MadeAnew(threadIdx.x);
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
@@ -1012,6 +1018,9 @@ __global__ __launch_bounds__(T, 4) void PackScatterKernel(PackIo io, int32_t shi
             if constexpr (Mode == kPackSecond) {
                 r.rec[i] = __builtin_nontemporal_load(io.recsIn + at);
                 r.digit[i] = LoadStream(io.digitsIn + at);
+                if constexpr (Tops) {
+                    r.top[i] = LoadStream(io.topsIn + at);
+                }
             } else {
                 r.key[i] = static_cast<uint32_t>(LoadStream(io.keys + at));
                 r.pay[i] = static_cast<uint32_t>(LoadStream(io.pays + at));
@@ -1026,7 +1035,7 @@ __global__ __launch_bounds__(T, 4) void PackScatterKernel(PackIo io, int32_t shi
             }
         }
     };
-    auto order = [&](const PackRegs<T, Mode> &r, int64_t tile, auto full) {
+    auto order = [&](const PackRegs<T, Mode, Tops> &r, int64_t tile, auto full) {
         const int tid = MadeAnew(threadIdx.x);
         uint32_t dig[kWideItems], rank[kWideItems];
         const int64_t wave0 = tile * kTile + tid / kWave * (kWave * kWideItems) + tid % kWave;
@@ -1046,9 +1055,16 @@ __global__ __launch_bounds__(T, 4) void PackScatterKernel(PackIo io, int32_t shi
             if constexpr (Mode == kPackSecond) {
                 lds.rec[rank[i]] = r.rec[i];
                 lds.digit[rank[i]] = static_cast<uint16_t>(dig[i]);
+                if constexpr (Tops) {
+                    lds.digit[kTile + rank[i]] = static_cast<uint16_t>(r.top[i]);
+                }
             } else {
                 const uint32_t key = static_cast<uint32_t>(Rebased(static_cast<int32_t>(r.key[i]), io.keyBase));
-                lds.rec[rank[i]] = PackedRecord(((key & lowMask) << io.payBits) | r.pay[i], r.val[i]);
+                const uint32_t pay = Tops ? r.pay[i] & ((1u << io.payBits) - 1u) : r.pay[i];
+                lds.rec[rank[i]] = PackedRecord(((key & lowMask) << io.payBits) | pay, r.val[i]);
+                if constexpr (Tops) {
+                    lds.digit[kTile + rank[i]] = static_cast<uint16_t>(r.pay[i] >> io.payBits);
+                }
                 lds.digit[rank[i]] = static_cast<uint16_t>(Mode == kPackFirst ? dig[i] | (key >> io.nextShift << 8) : dig[i]);
             }
         }
@@ -1064,13 +1080,16 @@ __global__ __launch_bounds__(T, 4) void PackScatterKernel(PackIo io, int32_t shi
                 const uint32_t digit = lds.digit[p];
                 const int64_t dst = static_cast<int64_t>(lds.outOf[Mode == kPackFirst ? digit & 0xffu : digit] + p);
                 io.recsOut[dst] = lds.rec[p];
+                if constexpr (Tops) {
+                    io.topsOut[dst] = lds.digit[kTile + p];
+                }
                 if constexpr (Mode == kPackFirst) {
                     io.digitsOut[dst] = static_cast<uint8_t>(digit >> 8);
                 }
             }
         }
     };
-    WideTurns<T, PackRegs<T, Mode>>(io.n, numTiles, fetch, order, write);
+    WideTurns<T, PackRegs<T, Mode, Tops>>(io.n, numTiles, fetch, order, write);
 }
 
 // WideCountKernel's table from the digits that the first pass left: a thread takes eight of a tile's together.
@@ -1409,6 +1428,7 @@ constexpr int kFinishLengths = 32;  // ints from `large` on that are zero at the
 
 struct FinishIo {
     const Record *recs;  // in the order of the keys' upper bits: low bits of the key above the payload, and the value
+    const uint16_t *tops;  // Tops: what is above payBits of the payloads
     int32_t payBits;
     int64_t n;
     const int32_t *starts;  // bucket b begins at starts[b * startStride]; there is one more than buckets
@@ -1497,7 +1517,7 @@ __device__ __forceinline__ int32_t FinishDigit(uint64_t rec, int32_t payBits, in
 
 // Orders the `len` entries at `first` by the low bits of their keys and writes them: a whole bucket (Big = false) where it
 // stands, a piece of one where the scanned table says.
-template <int T, bool Keys, int VB, bool Big, bool Digits, int Lanes>
+template <int T, bool Keys, int VB, bool Big, bool Tops, bool Digits, int Lanes>
 __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, const FinishIo &io, int32_t first, int32_t len,
                                             uint32_t bucket, const int32_t *__restrict__ places)
 {
@@ -1509,12 +1529,16 @@ __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, co
     const int32_t at0 = wave * rounds * kWave + lane;
     // (no branch around a load: a slot past the end reads the last entry)
     uint64_t rec[kFinishItems];
+    uint32_t top[Tops ? kFinishItems : 1];
     const int32_t lastSlot = len > 0 ? len - 1 : 0;
 #pragma unroll
     for (int i = 0; i < kFinishItems; ++i) {
         const int32_t slot = at0 + i * kWave;
         const int64_t at = static_cast<int64_t>(first) + (slot < lastSlot ? slot : lastSlot);
         rec[i] = __builtin_nontemporal_load(io.recs + (at < io.n ? at : io.n - 1));
+        if constexpr (Tops) {
+            top[i] = LoadStream(io.tops + (at < io.n ? at : io.n - 1));
+        }
     }
     int32_t *mine = lds.counters + wave * digits;
     for (int32_t d = lane; d < digits; d += kWave) {
@@ -1608,14 +1632,20 @@ __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, co
 #pragma unroll
     for (int i = 0; i < kFinishItems; ++i) {
         if (i < rounds) {
-            rank[i] += static_cast<uint32_t>(mine[FinishDigit(rec[i], io.payBits, mask)]);
+            // (Tops: the digit is worked out again: kept beside the record it would make the compiler spill)
+            const uint64_t again = Tops ? static_cast<uint32_t>(MadeAnew(static_cast<int>(rec[i]))) : rec[i];
+            rank[i] += static_cast<uint32_t>(mine[FinishDigit(again, io.payBits, mask)]);
         }
     }
     LdsBarrier();  // the counters make room for the entries
 #pragma unroll
     for (int i = 0; i < kFinishItems; ++i) {
         if (i < rounds) {
-            lds.row[rank[i]] = static_cast<int32_t>(static_cast<uint32_t>(rec[i]) & ((1u << io.payBits) - 1u));
+            uint32_t pay = static_cast<uint32_t>(rec[i]) & ((1u << io.payBits) - 1u);
+            if constexpr (Tops) {
+                pay |= top[i] << io.payBits;
+            }
+            lds.row[rank[i]] = static_cast<int32_t>(pay);
             lds.val[rank[i]] = static_cast<uint32_t>(rec[i] >> 32);
             if constexpr ((Keys && Lanes == 0) || Big) {
                 lds.digit[rank[i]] = static_cast<uint16_t>(FinishDigit(rec[i], io.payBits, mask));
@@ -1656,7 +1686,7 @@ __device__ __forceinline__ void FinishPiece(FinishLds<T, Digits, Lanes> &lds, co
 }
 
 // A workgroup a bucket (neighbouring buckets on one XCD).
-template <bool Keys, int VB, int Lanes = 0>
+template <bool Keys, int VB, int Lanes, bool Tops>
 __global__ __launch_bounds__(kFinishThreads, Keys && Lanes == 0 ? 4 : 6) void FinishBucketsKernel(FinishIo io)
 {
     __shared__ FinishLds<kFinishThreads, Keys && Lanes == 0, Lanes> lds;
@@ -1688,7 +1718,7 @@ __global__ __launch_bounds__(kFinishThreads, Keys && Lanes == 0 ? 4 : 6) void Fi
         }
         return;
     }
-    FinishPiece<kFinishThreads, Keys, VB, false>(lds, io, first, len, bucket, nullptr);
+    FinishPiece<kFinishThreads, Keys, VB, false, Tops>(lds, io, first, len, bucket, nullptr);
 }
 
 // The first position and the length of piece `i` of the list.
@@ -1804,7 +1834,7 @@ __global__ __launch_bounds__(kFinishScanThreads) void FinishScanKernel(FinishIo 
     }
 }
 
-template <bool Keys, int VB, int Lanes = 0>
+template <bool Keys, int VB, int Lanes, bool Tops>
 __global__ __launch_bounds__(kFinishLargeThreads) void FinishListsKernel(FinishIo io)
 {
     __shared__ FinishLds<kFinishLargeThreads, true, Lanes> lds;
@@ -1812,16 +1842,17 @@ __global__ __launch_bounds__(kFinishLargeThreads) void FinishListsKernel(FinishI
     for (int32_t i = blockIdx.x; i < large; i += gridDim.x) {
         const int32_t bucket = io.list.largeOf[i];
         const int32_t first = io.starts[bucket * io.startStride];
-        FinishPiece<kFinishLargeThreads, Keys, VB, false>(lds, io, first, io.starts[(bucket + 1) * io.startStride] - first,
-                                                          static_cast<uint32_t>(bucket), nullptr);
+        FinishPiece<kFinishLargeThreads, Keys, VB, false, Tops>(lds, io, first,
+                                                                io.starts[(bucket + 1) * io.startStride] - first,
+                                                                static_cast<uint32_t>(bucket), nullptr);
         LdsBarrier();
     }
     for (int32_t piece = blockIdx.x; piece < pieces; piece += gridDim.x) {
         uint32_t bucket;
         int32_t len;
         const int32_t first = FinishPieceAt(io, piece, &bucket, &len);
-        FinishPiece<kFinishLargeThreads, Keys, VB, true>(lds, io, first, len, bucket,
-                                                         io.list.table + (static_cast<int64_t>(piece) << io.low));
+        FinishPiece<kFinishLargeThreads, Keys, VB, true, Tops>(lds, io, first, len, bucket,
+                                                               io.list.table + (static_cast<int64_t>(piece) << io.low));
         LdsBarrier();
     }
 }
@@ -2309,13 +2340,18 @@ int64_t WideTableInts(int64_t n) { return (WideTiles(n) << kWideMaxBits) + 1; }
 
 // ... of the passes that leave records.  Half as many as the other passes of many entries have: two workgroups a compute unit,
 // one of which loads while the other orders, and runs that are as long, in bytes, as theirs of three arrays (17 M triples over 1 M
-// rows 865 us with 1024, 777 with 512; 33.5 M 2032 and 2029; 3.3 M over 300 000 with 256 707, with 512 626).  A table of theirs has
-// at most as many ints as one of ten bits of the others': twice the tiles, but nine bits in one pass of so many entries, and eight
-// in each of two.
-int PackThreads(int64_t n) { return n >= (int64_t{1} << 20) ? 512 : 256; }
-int64_t PackTiles(int64_t n)
+// rows 865 us with 1024, 777 with 512; 33.5 M 2032 and 2029; 3.3 M over 300 000 with 256 707, with 512 626).  With tops, whose keys
+// have many buckets, the run of a tile in one of them is a line with 1024 and half of one with 512: csr2csc of 12 M entries over
+// 8.4 M columns 426 us with 1024, 377 with 512, 33.6 M over 8.4 M 781 and 771, 48 M over 12 M 959 and 1023, 80 M over 20 M 1711 and
+// 1910.  A table of theirs has at most as many ints as one of ten bits of the others': twice the tiles, but nine bits in one pass
+// of so many entries, and eight in each of two.
+int PackThreads(int64_t n, bool tops)
 {
-    const int64_t tile = static_cast<int64_t>(PackThreads(n)) * kWideItems;
+    return tops && n >= int64_t{5} << 23 ? 1024 : n >= (int64_t{1} << 20) ? 512 : 256;
+}
+int64_t PackTiles(int64_t n, bool tops)
+{
+    const int64_t tile = static_cast<int64_t>(PackThreads(n, tops)) * kWideItems;
     return (n + tile - 1) / tile;
 }
 
@@ -2442,8 +2478,9 @@ int32_t KeyBits(int64_t n)
 // fifths, and one more bit in the passes: 33.5 M entries 683 us, 651 so); below kFinishLeast the workgroups' start and end
 // outweigh their work.
 struct FinishPlan {
-    bool use;
-    int32_t passes, low, lowerBits, upperBits, payBits;
+    bool use, tops;
+    int32_t passes, low, lowerBits, upperBits;
+    int32_t payBits;  // of a payload in the record; `tops`: the others travel beside it
     int64_t buckets;
 };
 constexpr int64_t kFinishMean = kFinishMost * 4 / 5;
@@ -2451,13 +2488,11 @@ constexpr int64_t kFinishLeast = 512;
 constexpr int64_t kFinishSamePasses = 5 << 20;
 constexpr int64_t kFinishMin = 1 << 14;  // entries (the lists' room in the second pair buffer is counted from here)
 
-FinishPlan FinishPlanOf(int64_t numKeys, int64_t n, int32_t payBits)
+FinishPlan FinishPlanWith(int64_t numKeys, int64_t n, int32_t payBits, int32_t mostLow)
 {
     FinishPlan f{};
     const int32_t keyBits = KeyBits(numKeys);
-    int32_t low = keyBits - 1 < kFinishMaxBits ? keyBits - 1 : kFinishMaxBits;
-    low = low < 32 - payBits ? low : 32 - payBits;  // (the two share a word)
-    f.payBits = payBits;
+    int32_t low = keyBits - 1 < mostLow ? keyBits - 1 : mostLow;
     auto mean = [&](int32_t bits) {  // entries of a bucket
         return static_cast<double>(n) * static_cast<double>(int64_t{1} << bits) / static_cast<double>(numKeys);
     };
@@ -2468,6 +2503,8 @@ FinishPlan FinishPlanOf(int64_t numKeys, int64_t n, int32_t payBits)
     if (n < kFinishMin || low < 1 || mean(low) < static_cast<double>(kFinishLeast) || high > 16) {
         return f;
     }
+    f.tops = payBits > 32 - low;
+    f.payBits = f.tops ? 32 - low : payBits;
     f.passes = high <= most ? 1 : 2;
     f.low = low;
     f.lowerBits = f.passes == 1 ? high : (high + 1) / 2;
@@ -2476,6 +2513,17 @@ FinishPlan FinishPlanOf(int64_t numKeys, int64_t n, int32_t payBits)
     const int32_t plain = WidePassesOf(keyBits, n).passes;
     f.use = f.passes < plain || (f.passes == plain && n >= kFinishSamePasses);
     return f;
+}
+
+// With tops where a word leaves a key two low bits fewer than it might have, or a pass more.  Without them, and the plain passes where those buckets are too small, csr2csc of 33.6 M entries, 8.4 M x 8.4 M, takes 909 us
+// (765 with), of 80 M, 20 M x 20 M, 2440 (1680), of 1 M over 1 M columns and 5 M rows 116 (77), coosort by row of 80 M, 20 M x 20 M,
+// 3450 (2120).  One bit fewer costs less than the tops: 20 M entries, 5 M x 5 M, 415 us without and 423 with.
+FinishPlan FinishPlanOf(int64_t numKeys, int64_t n, int32_t payBits)
+{
+    const int32_t room = 32 - payBits < kFinishMaxBits ? 32 - payBits : kFinishMaxBits;
+    const FinishPlan inWord = FinishPlanWith(numKeys, n, payBits, room);
+    const FinishPlan most = FinishPlanWith(numKeys, n, payBits, kFinishMaxBits);
+    return inWord.use && inWord.passes <= most.passes && inWord.low + 1 >= most.low ? inWord : most;
 }
 
 // Lanes per row from the mean row length: twice the mean, a power of two in [8, 64].
@@ -2508,12 +2556,12 @@ void LaunchSortListedRows(const int32_t *rowPtr, int32_t base, int64_t n, int32_
                        static_cast<int32_t *>(nullptr));
 }
 
-template <int T, int Mode>
+template <int T, int Mode, bool Tops>
 void LaunchPackPassOf(const PackIo &io, int32_t valueBytes, int32_t shift, int32_t bits, int32_t *table, int32_t *scratch,
                       hipStream_t s)
 {
     const int32_t mask = (1 << bits) - 1;
-    const int64_t numTiles = PackTiles(io.n);
+    const int64_t numTiles = PackTiles(io.n, Tops);
     const auto counts = dim3(static_cast<uint32_t>((numTiles + kWideCountTiles - 1) / kWideCountTiles));
     if (Mode == kPackSecond) {
         hipLaunchKernelGGL(DigitCountKernel<T>, counts, dim3(T), 0, s, io.digitsIn, io.n, mask, table, numTiles);
@@ -2525,13 +2573,13 @@ void LaunchPackPassOf(const PackIo &io, int32_t valueBytes, int32_t shift, int32
         hipLaunchKernelGGL(kernel, dim3(WideScatterBlocks(io.n, T)), dim3(T), 0, s, io, shift, mask, bits, table, numTiles);
     };
     if constexpr (Mode == kPackSecond) {
-        launch(PackScatterKernel<T, Mode, 4>);
+        launch(PackScatterKernel<T, Mode, 4, Tops>);
     } else {
         switch (valueBytes) {
-            case 4: launch(PackScatterKernel<T, Mode, 4>); break;
-            case 2: launch(PackScatterKernel<T, Mode, 2>); break;
-            case 1: launch(PackScatterKernel<T, Mode, 1>); break;
-            default: launch(PackScatterKernel<T, Mode, 0>); break;
+            case 4: launch(PackScatterKernel<T, Mode, 4, Tops>); break;
+            case 2: launch(PackScatterKernel<T, Mode, 2, Tops>); break;
+            case 1: launch(PackScatterKernel<T, Mode, 1, Tops>); break;
+            default: launch(PackScatterKernel<T, Mode, 0, Tops>); break;
         }
     }
 }
@@ -2541,7 +2589,13 @@ template <int Mode>
 void LaunchPackPass(const PackIo &io, int32_t valueBytes, int32_t shift, int32_t bits, int32_t *table, int32_t *scratch,
                     hipStream_t s)
 {
-    const auto launch = PackThreads(io.n) == 512 ? LaunchPackPassOf<512, Mode> : LaunchPackPassOf<256, Mode>;
+    const bool tops = io.topsOut != nullptr;
+    const int threads = PackThreads(io.n, tops);
+    auto launch = tops ? (threads == 256 ? LaunchPackPassOf<256, Mode, true> : LaunchPackPassOf<512, Mode, true>)
+                       : (threads == 256 ? LaunchPackPassOf<256, Mode, false> : LaunchPackPassOf<512, Mode, false>);
+    if constexpr (Mode != kPackOnly) {  // (so many entries take two passes)
+        launch = threads == 1024 ? LaunchPackPassOf<1024, Mode, true> : launch;
+    }
     launch(io, valueBytes, shift, bits, table, scratch, s);
 }
 
@@ -2561,7 +2615,7 @@ struct FinishSort {
 void LaunchFinishSort(const FinishSort &sort, const FinishPlan &plan, int32_t *const *keys, void *const *pairs,
                       int32_t *table, int32_t *scratch, hipStream_t s)
 {
-    const int64_t n = sort.n, numTiles = PackTiles(n), most = n / kFinishMost + 1;  // (buckets on a list: fewer)
+    const int64_t n = sort.n, numTiles = PackTiles(n, plan.tops), most = n / kFinishMost + 1;  // (buckets on a list: fewer)
     FinishIo io{};
     auto *at = static_cast<int32_t *>(pairs[0]);
     auto take = [&](int64_t ints) {
@@ -2596,8 +2650,11 @@ void LaunchFinishSort(const FinishSort &sort, const FinishPlan &plan, int32_t *c
     pack.payBits = plan.payBits;
     pack.nextShift = plan.low + plan.lowerBits;
     auto *last = static_cast<Record *>(pairs[1]);
+    // (between two passes the digits are the first n bytes of a key buffer, the tops the last 2 n)
+    auto *lastTops = plan.tops ? reinterpret_cast<uint16_t *>(keys[1]) : nullptr;
     if (plan.passes == 1) {
         pack.recsOut = last;
+        pack.topsOut = lastTops;
         LaunchPackPass<kPackOnly>(pack, sort.io.valueBytes, plan.low, plan.lowerBits, table, scratch, s);
         LaunchFill(io.list.large, kFinishLengths, 0, s);
         io.starts = table;
@@ -2608,18 +2665,22 @@ void LaunchFinishSort(const FinishSort &sort, const FinishPlan &plan, int32_t *c
         auto *digits = reinterpret_cast<uint8_t *>(keys[0]);
         pack.recsOut = static_cast<Record *>(pairs[0]);
         pack.digitsOut = digits;
+        pack.topsOut = plan.tops ? reinterpret_cast<uint16_t *>(digits + 2 * n) : nullptr;
         LaunchPackPass<kPackFirst>(pack, sort.io.valueBytes, plan.low, plan.lowerBits, table, scratch, s);
         pack.recsIn = pack.recsOut;
         pack.digitsIn = digits;
+        pack.topsIn = pack.topsOut;
         pack.recsOut = last;
+        pack.topsOut = lastTops;
         LaunchPackPass<kPackSecond>(pack, 4, 0, plan.upperBits, upper, scratch, s);
         hipLaunchKernelGGL(FinishStartsKernel, dim3(1u << plan.lowerBits), dim3(kFinishScanThreads), 0, s, digits, n,
-                           static_cast<int64_t>(PackThreads(n)) * kWideItems, numTiles, plan.lowerBits, plan.upperBits, table,
+                           static_cast<int64_t>(PackThreads(n, plan.tops)) * kWideItems, numTiles, plan.lowerBits, plan.upperBits, table,
                            upper, starts, io.list);
         io.starts = starts;
         io.startStride = 1;
     }
     io.recs = last;
+    io.tops = lastTops;
     io.payBits = plan.payBits;
     io.n = n;
     io.low = plan.low;
@@ -2636,29 +2697,33 @@ void LaunchFinishSort(const FinishSort &sort, const FinishPlan &plan, int32_t *c
         hipLaunchKernelGGL(FinishScanKernel, dim3(GridFor(most, 1, 512)), dim3(kFinishScanThreads), 0, s, io);
         hipLaunchKernelGGL(lists, dim3(GridFor(2 * most, 1, 256)), dim3(kFinishLargeThreads), 0, s, io);
     };
-    if (sort.rowBound > 0) {
-        switch (SortLanes(n, sort.numKeys)) {
-            case 8: launch(FinishBucketsKernel<true, 4, 8>, FinishListsKernel<true, 4, 8>); break;
-            case 16: launch(FinishBucketsKernel<true, 4, 16>, FinishListsKernel<true, 4, 16>); break;
-            case 32: launch(FinishBucketsKernel<true, 4, 32>, FinishListsKernel<true, 4, 32>); break;
-            default: launch(FinishBucketsKernel<true, 4, 64>, FinishListsKernel<true, 4, 64>); break;
+    auto finish = [&](auto withTops) {
+        constexpr bool Tops = decltype(withTops)::value;
+        if (sort.rowBound > 0) {
+            switch (SortLanes(n, sort.numKeys)) {
+                case 8: launch(FinishBucketsKernel<true, 4, 8, Tops>, FinishListsKernel<true, 4, 8, Tops>); break;
+                case 16: launch(FinishBucketsKernel<true, 4, 16, Tops>, FinishListsKernel<true, 4, 16, Tops>); break;
+                case 32: launch(FinishBucketsKernel<true, 4, 32, Tops>, FinishListsKernel<true, 4, 32, Tops>); break;
+                default: launch(FinishBucketsKernel<true, 4, 64, Tops>, FinishListsKernel<true, 4, 64, Tops>); break;
+            }
+        } else if (sort.keyOut != nullptr) {
+            launch(FinishBucketsKernel<true, 4, 0, Tops>, FinishListsKernel<true, 4, 0, Tops>);
+        } else {
+            switch (sort.io.valueBytes) {
+                case 4: launch(FinishBucketsKernel<false, 4, 0, Tops>, FinishListsKernel<false, 4, 0, Tops>); break;
+                case 2: launch(FinishBucketsKernel<false, 2, 0, Tops>, FinishListsKernel<false, 2, 0, Tops>); break;
+                case 1: launch(FinishBucketsKernel<false, 1, 0, Tops>, FinishListsKernel<false, 1, 0, Tops>); break;
+                default: launch(FinishBucketsKernel<false, 0, 0, Tops>, FinishListsKernel<false, 0, 0, Tops>); break;
+            }
         }
+    };
+    plan.tops ? finish(std::true_type{}) : finish(std::false_type{});
+    if (sort.rowBound > 0) {
         // the buffers that the entries lay in are csrsort's scratch now
         hipLaunchKernelGGL(SortMidRowsKernel<true>, dim3(kSortListBlocks), dim3(kBlockThreads), 0, s, sort.ptr, sort.base,
                            sort.io.rowOut, static_cast<int32_t *>(sort.io.valOut), io.rowCounters, io.midList);
         LaunchSortListedRows(sort.ptr, sort.base, sort.rowBound, sort.io.rowOut, static_cast<int32_t *>(sort.io.valOut),
                              keys[1], static_cast<int32_t *>(pairs[1]), io.rowCounters, io.midList, io.longList, s);
-        return;
-    }
-    if (sort.keyOut != nullptr) {
-        launch(FinishBucketsKernel<true, 4>, FinishListsKernel<true, 4>);
-        return;
-    }
-    switch (sort.io.valueBytes) {
-        case 4: launch(FinishBucketsKernel<false, 4>, FinishListsKernel<false, 4>); break;
-        case 2: launch(FinishBucketsKernel<false, 2>, FinishListsKernel<false, 2>); break;
-        case 1: launch(FinishBucketsKernel<false, 1>, FinishListsKernel<false, 1>); break;
-        default: launch(FinishBucketsKernel<false, 0>, FinishListsKernel<false, 0>); break;
     }
 }
 

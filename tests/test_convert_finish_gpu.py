@@ -122,9 +122,50 @@ def test_csr2csc_two_packed_passes_of_the_smallest_workgroups(osa, gpu_ctx, val_
 
 @pytest.mark.parametrize("val_type,numeric", VALUES)
 def test_csr2csc_of_few_entries_a_column_and_many_rows(osa, gpu_ctx, val_type, numeric):
-    """24 row bits leave eight for LDS, whose buckets would hold 128 entries: three passes of the largest workgroups."""
+    """24 row bits leave eight in a record, whose buckets would hold 128 entries: the rows' top bits travel beside it."""
     m, n, nnz = (1 << 23) + 7, (1 << 24) - 3, (1 << 23) + 5
     rng = np.random.default_rng(6)
     rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, m - 1)), [nnz]]).astype(np.int32)
     val = _typed(rng.uniform(-1, 1, nnz).astype(np.float32), val_type)
     run_csr2csc(osa, gpu_ctx, m, n, rowptr, columns("uniform", n, nnz, rng), val, NP_TYPE[val_type], numeric, 0)
+
+
+MANY = (1 << 23) + 9  # rows: 24 bits, of which 22 stand beside ten low bits of a key
+
+
+@pytest.mark.parametrize("val_type,numeric", VALUES)
+@pytest.mark.parametrize("n,nnz", [(400_003, 800_001), ((1 << 20) + 3, 700_001), (500_001, 1_200_003), ((1 << 21) + 3, 2_000_001),
+                                   ((1 << 25) + 3, 5 * (1 << 23) + 8195)])
+def test_csr2csc_top_bits_of_rows_beside_the_records(osa, gpu_ctx, n, nnz, val_type, numeric):
+    """One pass and two of every size of workgroup; the last one's two passes take eight bits each."""
+    rng = np.random.default_rng(nnz)
+    rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, MANY - 1)), [nnz]]).astype(np.int32)
+    val = _typed(rng.uniform(-1, 1, nnz).astype(np.float32), val_type)
+    run_csr2csc(osa, gpu_ctx, MANY, n, rowptr + 1, columns("uniform", n, nnz, rng) + 1, val, NP_TYPE[val_type], numeric, 1)
+
+
+@pytest.mark.parametrize("what", ["hubs", "few", "ends"])
+def test_csr2csc_top_bits_in_buckets_that_do_not_fit(osa, gpu_ctx, what):
+    n, nnz = (1 << 20) - 77, 3_000_001
+    rng = np.random.default_rng(8)
+    rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, MANY - 1)), [nnz]]).astype(np.int32)
+    run_csr2csc(osa, gpu_ctx, MANY, n, rowptr, columns(what, n, nnz, rng), rng.uniform(-1, 1, nnz).astype(np.float32),
+                np.float32, True, 0)
+
+
+@pytest.mark.parametrize("span,cols,nnz", [(700_001, 1 << 25, 2_500_000), (300_001, 1 << 25, 2_000_000),
+                                           (200_001, (1 << 26) - 2, 2_000_000), (100_001, (1 << 26) - 2, 1_850_000),
+                                           (2_000_000, (1 << 31) - 2, 5_300_000)])
+@pytest.mark.parametrize("hub", [0, 40_000])
+def test_coosort_top_bits_of_columns_beside_the_records(osa, gpu_ctx, span, cols, nnz, hub):
+    """Rows of every number of lanes, sorted where their bucket is, and rows whose columns do not fit their 32-bit keys; with
+    `hub`, a row that no workgroup orders and rows of 64, 65 and 66 entries."""
+    rng = np.random.default_rng(span)
+    rows, c = rng.integers(0, span, nnz).astype(np.int32), rng.integers(0, cols, nnz).astype(np.int32)
+    c[:2] = [0, cols - 1]
+    if hub:
+        at = rng.permutation(nnz)
+        for row, count in enumerate((hub, 64, 65, 66)):
+            rows[at[:count]] = 500 + row
+            at = at[count:]
+    run_coosort(osa, gpu_ctx, span, cols, rows, c, True, perm=rng.permutation(nnz).astype(np.int32))
