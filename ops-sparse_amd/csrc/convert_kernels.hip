@@ -2336,15 +2336,16 @@ int64_t WideTiles(int64_t n)
     const int64_t tile = static_cast<int64_t>(WideThreads(n)) * kWideItems;
     return (n + tile - 1) / tile;
 }
-int64_t WideTableInts(int64_t n) { return (WideTiles(n) << kWideMaxBits) + 1; }
+// Room for the table of a pass of ten bits, and for the two of the passes that leave records (PackTiles), a total behind each.
+int64_t WideTableInts(int64_t n) { return (WideTiles(n) << kWideMaxBits) + 2; }
 
 // ... of the passes that leave records.  Half as many as the other passes of many entries have: two workgroups a compute unit,
 // one of which loads while the other orders, and runs that are as long, in bytes, as theirs of three arrays (17 M triples over 1 M
 // rows 865 us with 1024, 777 with 512; 33.5 M 2032 and 2029; 3.3 M over 300 000 with 256 707, with 512 626).  With tops, whose keys
 // have many buckets, the run of a tile in one of them is a line with 1024 and half of one with 512: csr2csc of 12 M entries over
 // 8.4 M columns 426 us with 1024, 377 with 512, 33.6 M over 8.4 M 781 and 771, 48 M over 12 M 959 and 1023, 80 M over 20 M 1711 and
-// 1910.  A table of theirs has at most as many ints as one of ten bits of the others': twice the tiles, but nine bits in one pass
-// of so many entries, and eight in each of two.
+// 1910.  Their tables have as many counts as one of ten bits of the others' at most: from 2^23 entries on twice the tiles, but nine
+// bits in one pass, and eight in each of two.
 int PackThreads(int64_t n, bool tops)
 {
     return tops && n >= int64_t{5} << 23 ? 1024 : n >= (int64_t{1} << 20) ? 512 : 256;
@@ -2660,7 +2661,7 @@ void LaunchFinishSort(const FinishSort &sort, const FinishPlan &plan, int32_t *c
         io.starts = table;
         io.startStride = numTiles;
     } else {
-        // (up to eight bits each: the tables of both passes fit where one of ten bits does)
+        // (up to eight bits each: WideTableInts has room for both tables)
         int32_t *upper = table + (numTiles << plan.lowerBits) + 1;
         auto *digits = reinterpret_cast<uint8_t *>(keys[0]);
         pack.recsOut = static_cast<Record *>(pairs[0]);

@@ -40,8 +40,8 @@ def test_csr2csc_buckets(osa, gpu_ctx, n, nnz, val_type, numeric, what):
 
 
 @pytest.mark.parametrize("val_type,numeric", [("FP16", True), ("INT8", True), ("FP32", False)])
-def test_csr2csc_last_pass_of_the_largest_workgroups(osa, gpu_ctx, val_type, numeric):
-    """17 column bits: two passes either way, the last one writes the outputs."""
+def test_csr2csc_packed_passes_that_save_none(osa, gpu_ctx, val_type, numeric):
+    """17 column bits: two passes either way, over records and with buckets in LDS from 5 M entries on."""
     n, nnz = 100_000, (1 << 23) + 5
     rng = np.random.default_rng(3)
     rowptr = np.array([0, nnz // 3, nnz], np.int32)
@@ -118,6 +118,26 @@ def test_csr2csc_two_packed_passes_of_the_smallest_workgroups(osa, gpu_ctx, val_
     rowptr = np.array([0, nnz // 3, nnz // 3, nnz], np.int32)
     val = _typed(rng.uniform(-1, 1, nnz).astype(np.float32), val_type)
     run_csr2csc(osa, gpu_ctx, 3, n, rowptr + 1, columns("uniform", n, nnz, rng) + 1, val, NP_TYPE[val_type], numeric, 1)
+
+
+@pytest.mark.parametrize("val_type,numeric", VALUES)
+def test_csr2csc_plain_passes_of_the_largest_workgroups(osa, gpu_ctx, val_type, numeric):
+    """25 column bits, buckets of 429 entries on average: three passes over keys, rows and values, the last one writes the outputs."""
+    n, nnz = 20_000_003, (1 << 23) + 5
+    rng = np.random.default_rng(4)
+    rowptr = np.array([0, nnz // 3, nnz], np.int32)
+    val = _typed(rng.uniform(-1, 1, nnz).astype(np.float32), val_type)
+    run_csr2csc(osa, gpu_ctx, 2, n, rowptr, columns("uniform", n, nnz, rng), val, NP_TYPE[val_type], numeric, 0)
+
+
+def test_csr2csc_fullest_packed_passes(osa, gpu_ctx):
+    """Whole tiles and two digits of eight bits: the tables of both passes fill their room to the last number."""
+    m, n, nnz = 3_000_000, (1 << 25) + 3, 3 << 23
+    rng = np.random.default_rng(9)
+    rowptr = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, m - 1)), [nnz]]).astype(np.int32)
+    c = columns("uniform", n, nnz, rng)
+    c[:2] = [n - 1, 0]
+    run_csr2csc(osa, gpu_ctx, m, n, rowptr, c, rng.uniform(-1, 1, nnz).astype(np.float32), np.float32, True, 0)
 
 
 @pytest.mark.parametrize("val_type,numeric", VALUES)
