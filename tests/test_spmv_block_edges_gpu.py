@@ -52,8 +52,8 @@ def test_last_values_of_the_array_and_rows_across_windows(osa, gpu_ctx, monkeypa
 
 @pytest.mark.parametrize("rows,longest,ends", [(65_536, 76, False), (65_537, 76, True), (131_071, 40, False), (400_000, 12, True)])
 def test_where_the_blocks_are_cut(osa, gpu_ctx, monkeypatch, rows, longest, ends):
-    """Blocks end at every 65 536 rows, behind their most rows (a stretch of rows of one entry and none) and behind long rows
-    (one beside another, the first and the last row of the matrix, either side of row 65 536)."""
+    """Blocks end behind their most rows (65 536 are 32 times as many; a stretch of rows of one entry and none) and behind long
+    rows (one beside another, the first and the last row of the matrix)."""
     for name in ("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "OPS_SPARSE_ORDERED_LIVE_MIN_COLS"):
         monkeypatch.setenv(name, "0")
     dev, stream, handle = gpu_ctx
@@ -78,6 +78,35 @@ def test_where_the_blocks_are_cut(osa, gpu_ctx, monkeypatch, rows, longest, ends
     stream.synchronize()
     gold = oracle.spmv_f64(rows, COLS, rowptr, colind, val, x, np.zeros(rows, np.float32), 1.0, 0.0)
     assert oracle.max_rel_err(y.cpu().numpy(), gold) <= 1e-5
+
+
+@pytest.mark.parametrize("rows,least,longest,hubs", [
+    (30_000, 380, 420, 0), (131_072, 0, 36, 0), (131_073, 0, 36, 0), (262_145, 0, 16, 0), (70_000, 60, 80, 223), (70_000, 30, 40, 600),
+    (200_000, 10, 14, 900)])
+def test_where_a_stretch_of_blocks_ends(osa, gpu_ctx, monkeypatch, rows, least, longest, hubs):
+    """The blocks are cut by workgroups that take 65 536 rows, or 256 blocks' worth of entries (7168 a block), rows (2048) and long
+    rows: several such stretches in the same 65 536 rows, by entries and by long rows, and one."""
+    for name in ("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ", "OPS_SPARSE_ORDERED_LIVE_MIN_COLS"):
+        monkeypatch.setenv(name, "0")
+    dev, stream, handle = gpu_ctx
+    rng = np.random.default_rng(rows + hubs)
+    lengths = rng.integers(least, longest + 1, rows)
+    hub_rows = 1000 + np.arange(hubs) * 3
+    lengths[hub_rows] = 64 * (COLS // 32768 + 1) + 4096
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz = int(rowptr[-1])
+    colind = rng.integers(0, COLS, nnz).astype(np.int32)
+    for r in hub_rows:
+        colind[rowptr[r]:rowptr[r + 1]].sort()
+    val, x = rng.uniform(0.5, 1, nnz).astype(np.float32), rng.uniform(0.5, 1, COLS).astype(np.float32)
+    y = torch.full((rows,), float("nan"), device=dev)
+    A = osa.Csr(rows, COLS, to_dev(rowptr, dev), to_dev(colind, dev), to_dev(val, dev))
+    op = osa.SpmvOp(handle, A, osa.DnVec(to_dev(x, dev)), osa.DnVec(y))
+    assert op.buffer.numel() > osa.lib().opsparse_spmv_csr_workspace_bytes(rows, nnz)
+    op(1.0, 0.0)
+    stream.synchronize()
+    gold = oracle.spmv_f64(rows, COLS, rowptr, colind, val, x, np.zeros(rows, np.float32), 1.0, 0.0)
+    assert oracle.max_rel_err(y.cpu().numpy(), gold) <= 2 ** -23  # (sums in 64 bits, rounded once)
 
 
 @pytest.mark.parametrize("streamed", [False, True])
