@@ -2520,7 +2520,9 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
             const int64_t blocks = blocksOf(l.rowLog, window);
             const int64_t least = kRowsSizes[i].chunk > kMinChunkEntries ? kRowsSizes[i].chunk : kMinChunkEntries;
             B = blocks + behindLong;
-            l.size = numbered(B) && nnz / (P * blocks) >= least ? i : -1;
+            // (where a block's table of rows begins, and the rows that the cut of the blocks looks at behind the last, in 32 bits)
+            const bool rowsNumbered = rows + 16 * B <= INT32_MAX - 65536;
+            l.size = numbered(B) && rowsNumbered && nnz / (P * blocks) >= least ? i : -1;
         }
         if (l.size < 0) {
             return BlockedLayout{};

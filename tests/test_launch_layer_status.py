@@ -278,6 +278,18 @@ def test_blocked_layout_takes_a_larger_row_block_where_a_smaller_one_does_not_fi
         assert L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, 0) > 0
 
 
+def test_blocked_layout_numbers_the_tables_of_its_rows_in_32_bits(L, osa):
+    """A windowed block's table of rows begins at its first row plus 16 a block in front of it, and the cut of the blocks looks
+    up to 4096 rows past the last: matrices whose rows leave no room for that below 2^31 do not have the layout.  (Streamed
+    blocks have no such tables.)"""
+    live, transposed = osa.OPSPARSE_BLOCKED_LIVE_VALUES, osa.OPSPARSE_BLOCKED_TRANSPOSE
+    cols, nnz = (1 << 18) + 1, 200_000_000
+    for rows in (1_900_000_000, 2_000_000_000, 2_120_000_000, 2_130_000_000, 2_140_000_000, (1 << 31) - 4096, (1 << 31) - 2):
+        fits = rows + 16 * ((rows + 4095) // 4096 + nnz // 12544 + 1) <= (1 << 31) - 1 - 65536
+        assert (L.opsparse_spmv_csr_blocked_workspace_bytes(rows, cols, nnz, live) > 0) == fits, rows
+        assert (L.opsparse_spmv_csr_blocked_workspace_bytes(cols, rows, nnz, live | transposed) > 0) == fits, rows
+
+
 def test_scatter_layout_takes_every_entry_count_up_to_15_million_columns(L, osa):
     """The output panels are 256 or a multiple; the bound of the chunk tables (panels x pieces) leaves room for 2^31 entries
     up to 768 panels, and never for fewer than panels of 2^14 columns and 2^26 chunks would."""
