@@ -2549,7 +2549,9 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
     const int64_t padded = nnz + kLaneEntries * P * B;  // every chunk padded to a multiple of kLaneEntries
     l.padded = padded;
     l.colLocalOff = off; off += align(2 * nnz + 8);
-    l.xgOff = off; off += align(4 * nnz) + 256;  // a lane's 16-byte loads of xg may run 7 entries past a chunk
+    // (in the width of x; frozen values of long rows lie behind it in 32 bits.  A lane's 16-byte loads of xg may run 7 entries past
+    // a chunk.)
+    l.xgOff = off; off += align((l.frozenLong ? 4 : vb) * nnz) + 256;
     l.slotOff = off; off += align(2 * padded + 16);  // (the long entries' row numbers behind the block order)
     l.src8Off = off; off += align(4 * (padded / kLaneEntries + 2));
     l.metaOff = off; off += align(static_cast<int64_t>(sizeof(BlockMeta)) * (B + 1));

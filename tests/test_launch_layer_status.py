@@ -290,6 +290,19 @@ def test_blocked_layout_numbers_the_tables_of_its_rows_in_32_bits(L, osa):
         assert (L.opsparse_spmv_csr_blocked_workspace_bytes(cols, rows, nnz, live | transposed) > 0) == fits, rows
 
 
+def test_blocked_layout_holds_gathered_x_in_the_width_of_x(L, osa):
+    """16-bit x: two bytes an entry between the passes instead of four, except where frozen values keep those of long rows
+    behind them."""
+    live = osa.OPSPARSE_BLOCKED_LIVE_VALUES
+    rows, cols, nnz = 1_000_000, 1_000_000, 8_000_000
+    for f16 in (osa.OPSPARSE_BLOCKED_VALUES_F16, osa.OPSPARSE_BLOCKED_VALUES_BF16):
+        for size in (L.opsparse_spmv_csr_blocked_workspace_bytes, L.opsparse_spmv_csr_blocked_resident_bytes):
+            assert size(rows, cols, nnz, live) - size(rows, cols, nnz, live | f16) == 2 * nnz
+            # (op(A) = A^T: the copy's values, too)
+            transposed = live | osa.OPSPARSE_BLOCKED_TRANSPOSE
+            assert size(rows, cols, nnz, transposed) - size(rows, cols, nnz, transposed | f16) >= 4 * nnz
+
+
 def test_scatter_layout_takes_every_entry_count_up_to_15_million_columns(L, osa):
     """The output panels are 256 or a multiple; the bound of the chunk tables (panels x pieces) leaves room for 2^31 entries
     up to 768 panels, and never for fewer than panels of 2^14 columns and 2^26 chunks would."""
