@@ -118,8 +118,9 @@ struct TileWalk {
 //
 // us a call, the kernels for any columns / here: 5-point 2048 x 2048 n = 4 78 / 48 (the 320 MB it cannot do without at
 // 6.6 TB/s), n = 8 120 / 88; 7-point 125 x 131 x 127 n = 16 131 / 97, n = 32 213 / 169; 9-point 900 x 901 n = 64 190 / 134;
-// 27-point 71 x 77 x 79 n = 8 61 / 37, n = 64 184 / 156.  Wide B is bound by the instructions and waits of a pass (4 - 5
-// wavefronts a SIMD): with every gather sent to the row itself and no C written n = 32 still takes 110 us.  Passes whose rows
+// 27-point 71 x 77 x 79 n = 8 61 / 37, n = 64 184 / 156.  Wide B is bound by the data path of the vector memory, 86 % busy over a
+// call of n = 32 (its address path 80 %): a row of B passes it once a distance, wherever it comes from (with every gather sent
+// to the row itself and no C written n = 32 still takes 110 us).  Passes whose rows
 // all have every distance, as inside a mesh, go without a branch an entry, one distance's elements widened at a time (9-point 1300 x
 // 1200 n = 24 120 -> 105, n = 64 127 -> 114; 27-point 100 x 100 x 101 n = 4 47 -> 43, n = 64 153 -> 142; 7-point n = 12 82 -> 76).
 template <typename ValT, typename CT, int P, typename Shape>

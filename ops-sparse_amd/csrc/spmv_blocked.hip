@@ -399,9 +399,9 @@ __device__ __forceinline__ void SegRound(const int32_t (&k)[kSegEntries], const 
     carrySum = ReadLane63(v);
 }
 
-// What a wavefront leaves of its stretch for the one thread that joins the stretches: the sum of its first run
-// (which may go on from the stretch before) and of the run still open at its end.  ends: [2 * wave] head,
-// [2 * wave + 1] tail; a key of kNoKey: none.
+// What a wavefront leaves of its stretch for whoever joins the stretches (phase 1: a thread, phase 2: the lanes of a
+// wavefront): the sum of its first run (which may go on from the stretch before) and of the run still open at its end.
+// ends: [2 * wave] head, [2 * wave + 1] tail; a key of kNoKey: none.
 struct __align__(16) SegEnds {
     int32_t key[2 * (kBlkThreads / kWave)];
     uint64_t sum[2 * (kBlkThreads / kWave)];
@@ -472,14 +472,17 @@ __device__ __forceinline__ void SegJoin(const SegEnds &ends, int waves, int32_t 
 // room for.  The ordinary size gives every wavefront one round of its window and all of a block's positions in one turn, and
 // three workgroups fit a compute unit.  A call, ordinary size / 4096 entries and 256 threads, six workgroups a compute unit, the
 // faster of the smaller ones: 31 M entries over 123 panels 140 / 144 us, 47 M frozen over 183 162 / 169, 24 M over 123 103 / 111,
-// 32 M over 62 124 / 124; against 7168 entries and 256 threads, two rounds and two turns: 65 M over 256 277 / 291.  The large one is
-// for chunks that would be short: more entries of a block in a panel, less padding, fewer lines of gathered x shared between
-// blocks.
+// 32 M over 62 124 / 124; against 7168 entries and 256 threads, two rounds and two turns: 65 M over 256 277 / 291.  Few entries
+// gain by it, too: 5.6 M of a power law over 700 K rows 37.3 us, 39.4 in smaller blocks cut at multiples, 8 M over 1 M even rows
+// 37.7 and 41.9.  The large one is for chunks that would be short: more entries of a block in a panel, less padding, fewer lines of
+// gathered x shared between blocks.  It is taken where the ordinary one would have fewer than kMinChunkEntries in a (panel, block)
+// chunk, by the block numbers that there may be (a third of them stay unused, so chunks are half as long again): from 8 to 12,
+// ordinary / large, 22 M over 8.4 M rows 93 / 100 us, in bf16 72 / 86, 120 M over 16 M rows 515 / 513 and 341 / 361; from 5.5 to 8,
+// 33.6 M over 16 M rows 160 / 172 and 123 / 140, but 124 M over 25 M rows 590 / 575.
 struct RowsSize {
     int32_t window, rowLog, threads, waves;
-    int64_t chunk;  // entries of a (panel, block) chunk, on average, from which the size is taken
 };
-constexpr RowsSize kRowsSizes[] = {{8192, 11, 512, 6, 8}, {14336, 12, 512, 4, 0}};
+constexpr RowsSize kRowsSizes[] = {{8192, 11, 512, 6}, {14336, 12, 512, 4}};
 constexpr int kNumRowsSizes = 2;
 
 // What the workgroup of a row block needs to know before anything else, in one piece.
@@ -2518,11 +2521,10 @@ BlockedLayout MakeBlockedLayout(int64_t rows, int64_t cols, int64_t nnz, bool tr
             window = window > kMaxBlockEntries / 2 ? kMaxBlockEntries / 2 : window;
             l.rowLog = kRowsSizes[i].rowLog;
             const int64_t blocks = blocksOf(l.rowLog, window);
-            const int64_t least = kRowsSizes[i].chunk > kMinChunkEntries ? kRowsSizes[i].chunk : kMinChunkEntries;
             B = blocks + behindLong;
             // (where a block's table of rows begins, and the rows that the cut of the blocks looks at behind the last, in 32 bits)
             const bool rowsNumbered = rows + 16 * B <= INT32_MAX - 65536;
-            l.size = numbered(B) && rowsNumbered && nnz / (P * blocks) >= least ? i : -1;
+            l.size = numbered(B) && rowsNumbered && nnz / (P * blocks) >= kMinChunkEntries ? i : -1;
         }
         if (l.size < 0) {
             return BlockedLayout{};

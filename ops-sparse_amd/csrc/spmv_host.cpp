@@ -315,12 +315,12 @@ RestoredChoice PickLiveLayout(aclsparseHandle_t handle, const int32_t *rowOffset
     }
     // From 7 M entries on the layout is ahead wherever the gathers are scattered.  Of 2 to 7 M entries (fewer have no layout):
     // - op(A) = A^T, whose other kernels send every entry to a y of this many columns as an atomic (us a call, atomics / layout: graphs of
-    //   300 K rows, 2.4 M entries 164 / 28, of 1 M rows, 6 M entries 342 / 46; 600 K rows of 4 121 / 33; 2 M of 3 295 / 48);
-    // - uneven rows, which the merge path would work, from 2^19 rows and columns on (row-wise / layout: 530 K rows, 3.2 M
-    //   entries 41 / 26 and, with a row of 200 000, 75 / 48; 1.1 M, 2.2 M entries 71 / 26; 5 M, 5 M entries 161 / 74;
-    //   bf16, 700 K, 4.2 M entries 62 / 36; 300 K, 2.4 M entries 47 / 44);
-    // - even rows, over an x of 6 MiB and more (1.6 M rows of 2 32 / 30, of 4 57 / 41; 3.2 M of 2 88 / 50; but 1.1 M of 2
-    //   20 / 25, of 3 27 / 29, fp16 1.7 M of 3 33 / 39).
+    //   300 K rows, 2.4 M entries 157 / 29, of 1 M rows, 6 M entries 330 / 44; 600 K rows of 4 121 / 27; 2 M of 3 294 / 46);
+    // - uneven rows, which the merge path would work, from 2^19 rows and columns on (power laws with rows of up to 2000, row-wise /
+    //   layout: 530 K rows, 3.2 M entries 28 / 28 and, with a row of 132 000, 29 / 36; 1.1 M, 2.2 M entries 33 / 24; 4 M, 6.5 M
+    //   entries 131 / 49; 5 M, 5 M entries 97 / 48; bf16, 700 K, 4.2 M entries 33 / 27; 300 K, 2.4 M entries 24 / 26);
+    // - even rows, over an x of 6 MiB and more (1.6 M rows of 2 30 / 27, of 4 55 / 34; 3.2 M of 2 88 / 40; but 1.1 M of 2
+    //   18 / 21, of 3 26 / 26, 500 K of 8 25 / 27; fp16 1.7 M of 3 31 / 27, where the line is cautious).
     // Tuning override of the first bound, read at every call: OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ (nothing below it then).
     const char *minEnv = std::getenv("OPS_SPARSE_DEFAULT_BLOCKED_MIN_NNZ");
     const bool small = minEnv == nullptr && nnz < kMinDefaultNnz;

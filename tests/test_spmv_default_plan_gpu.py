@@ -863,7 +863,7 @@ def test_buffer_holds_only_what_the_calls_keep_when_the_handle_lends_the_scratch
         L.aclsparseSetWorkspace(handle.h, None, 0)
 
 
-SIZES = {"small": (260_000, 300_000), "middle": (200_000, 9_830_400), "large": (200_000, 22_900_000)}
+SIZES = {"10_panels": (260_000, 300_000, 5), "300_panels": (200_000, 9_830_400, 6), "699_panels": (200_000, 22_900_000, 5)}
 
 
 @pytest.mark.parametrize("size", list(SIZES))
@@ -873,12 +873,12 @@ SIZES = {"small": (260_000, 300_000), "middle": (200_000, 9_830_400), "large": (
                                        (torch.int32, torch.float32)])
 def test_every_size_of_the_windowed_row_blocks(osa, gpu_ctx, size, dtype, out):
     """The windowed blocks come in two sizes by how many entries a (panel, block) chunk gets (10 and 300 panels, and 699
-    here): blocks of up to 2048 and 4096 rows and 8192 and 14 336 entries a window.  Rows of 0 - 22 entries;
+    here): blocks of up to 2048 rows and 8192 entries a window, and of up to 4096 and 14 336.  Rows of 0 - 22 entries;
     a run of empty rows longer than a block; rows of 5000 and 20 000 unsorted entries, which fill several windows; a row of
     20 000 ascending ones (a long row).  Every type of values and of y."""
     dev, stream, handle = gpu_ctx
-    rows, cols = SIZES[size]
-    rng = np.random.default_rng(len(size) + 3 * (dtype == torch.float16))
+    rows, cols, seed = SIZES[size]
+    rng = np.random.default_rng(seed + 3 * (dtype == torch.float16))
     lengths = rng.integers(0, 23, rows)
     lengths[5000:9500] = 0
     lengths[[7, 1023, 1024, rows - 1]] = [5000, 20_000, 20_000, 5000]
