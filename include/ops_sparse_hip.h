@@ -204,8 +204,8 @@ int opsparse_spmv_csr_panels_analyse(const int32_t *rowOffsets, const int32_t *c
 
 /*
  * BLOCKED_GATHER analysis: bytes of the workspace, or 0 when the family does not apply (x must have more than 2^18
- * and at most 2^25 elements, the matrix at least two million entries, and a (panel, row block) chunk at least 8
- * entries on average).  Values and x are fp32, fp16, bf16 or int32 (`flags`); at the launches y is fp32 or of the
+ * and at most 2^25 elements, the matrix at least two million entries, a (panel, row block) chunk at least 8
+ * entries on average, and the rows stay 9 M below 2^31, where the blocks' tables are numbered in 32 bits).  Values and x are fp32, fp16, bf16 or int32 (`flags`); at the launches y is fp32 or of the
  * values' own type, int32 under the integer compute type.
  * The layout holds where the entries' columns sit in 2^15-column panels, the place of every entry in its row block,
  * and small tables by which a block's kernel tells its rows apart.  Every row is summed in an order that the layout
@@ -222,7 +222,7 @@ int opsparse_spmv_csr_panels_analyse(const int32_t *rowOffsets, const int32_t *c
  *       rows are not so uneven that many entries lie in rows that meet themselves in one instruction of the stream
  *       (the mean length of an entry's row against the mean row's, weighed against the chunks' length where these are
  *       short); else, like live values, they are read in row order through a window in LDS by a workgroup a block of
- *       2^10, 2^11 or 2^12 rows, the smallest whose chunks are long enough (which cannot hold a row of more than
+ *       2^11 or 2^12 rows at most, the smaller where its chunks are long enough (which cannot hold a row of more than
  *       65 534 entries: see OPSPARSE_E_UNSUPPORTED below).  Frozen rows of 13 to 16 entries a panel, or uneven ones,
  *       that the windowed blocks refuse are streamed.
  *   OPSPARSE_BLOCKED_TRANSPOSE (= 1, so that a plain 0 / 1 "transpose" still reads right)  the layout of

@@ -99,7 +99,8 @@ def test_csr2csc_rows_of_many_bits(osa, gpu_ctx, m, n, nnz, base):
 
 
 @pytest.mark.parametrize("span,cols,nnz", [(400_000, 1 << 22, 2_000_000), (700_000, (1 << 26) - 2, 5_300_000),
-                                           (500_000, 1 << 27, 9_000_000), (700_000, (1 << 31) - 2, 5_300_000)])
+                                           (500_000, 1 << 27, 9_000_000), (700_000, (1 << 31) - 2, 5_300_000),
+                                           (147_000, 1 << 26, 5_300_000)])  # (the bits of a column fit beside six of a row's)
 def test_coosort_columns_of_many_bits(osa, gpu_ctx, span, cols, nnz):
     rng = np.random.default_rng(span + nnz)
     rows, c = rng.integers(0, span, nnz).astype(np.int32), rng.integers(0, cols, nnz).astype(np.int32)
